@@ -23,13 +23,19 @@ LIB = os.path.join(PKG, "libtm.so")
 ARCH = "gfx950"
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I", INCLUDE, "-I", CSRC,
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
+# The FP64 kernels hold some two hundred 64-bit literals (their polynomials).  Hoisted
+# out of the cell loops they overflow the SGPRs and every use reads one back from a
+# VGPR lane (450 SGPR spills in the two-pass DP step, 134 VGPRs); left in place they
+# cost scalar moves beside the FP64 work (71 spills, 91 VGPRs).  The FP32 kernels'
+# literals are instruction operands: the same flag measured nothing there.
+NO_LICM = ["-mllvm", "-disable-machine-licm"]
 UNITS = {
-    "tm_kernels_f64.hip": ["-ffp-contract=off"],
+    "tm_kernels_f64.hip": ["-ffp-contract=off", *NO_LICM],
     "tm_kernels_f32.hip": ["-ffp-contract=fast"],
     "tm_ensemble.hip": ["-ffp-contract=off"],
     "tm_frames.hip": ["-ffp-contract=off"],
-    "tm_consumers.hip": ["-ffp-contract=off"],
-    "tm_movement.hip": ["-ffp-contract=off"],
+    "tm_consumers.hip": ["-ffp-contract=off", *NO_LICM],
+    "tm_movement.hip": ["-ffp-contract=off", *NO_LICM],
     "tm_api.cpp": ["-ffp-contract=off"],
     "tm_io.cpp": ["-ffp-contract=off"],
 }
