@@ -1592,11 +1592,13 @@ int default_variant(int model, int precision, int64_t total_cells)
         want = precision == TM_F64 ? "dp_f64_64x32_t256_x8aq_w6" : "dp_f32_128x24_t256_x8aq";
     } else {
         // Rietkerk: small lattices are latency-bound and want the single fused
-        // 16 x 16 launch; batches want the split step (each P* sampled once),
-        // in FP32 with the two-pass Dornic kernel on 128 x 24 tiles (C3 batch:
-        // 4.6e10 against 4.3e10 cell-updates/s for the one-pass 128 x 32 kernel)
-        if (total_cells < (1 << 20)) return 0;
-        want = precision == TM_F64 ? "rk_f64_split_32x16_t256" : "rk_f32_split_32x16_t256_q24";
+        // 16 x 16 launch; batches want the split step (each P* sampled once) with
+        // the two-pass Dornic kernel, in FP32 on 128 x 24 tiles (256 x 512^2:
+        // 4.6e10 against 4.3e10 cell-updates/s for the one-pass 128 x 32 kernel).
+        // FP64, fused against split: 22.9 / 26.6 us a step at 384^2, 28.0 / 27.9 at
+        // 512^2, 59.8 / 50.2 at 453,000 cells, 86.4 / 56.3 at 1024^2.
+        if (total_cells < (precision == TM_F64 ? 1 << 18 : 1 << 20)) return 0;
+        want = precision == TM_F64 ? "rk_f64_split_32x16_t256_q16" : "rk_f32_split_32x16_t256_q24";
     }
     const int n = tm_variant_count(model, precision);
     for (int v = 0; v < n; ++v)

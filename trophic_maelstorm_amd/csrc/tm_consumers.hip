@@ -204,7 +204,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
             y[0] = cur;
             if (!(alpha == 0.0 && cur == 0.0)) {
                 Stream s0(di.seed, di.inst_id, cell, c.step);
-                int64_t n;
+                double n;
                 y[0] = dornic_cell(s0, alpha, cur, c.k, c.compat != 0, n);
             }
         }
@@ -271,7 +271,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
             k.lambda = lam;
             k.ll = lam * lexp;
             k.sigma2_1 = sig2_1;
-            int64_t n;
+            double n;
             y[s] = dornic_cell(sc, alpha, is[r], k, c.compat != 0, n);
         }
         dpc_rk4<NS>(p, y);

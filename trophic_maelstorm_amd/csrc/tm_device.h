@@ -237,12 +237,16 @@ TM_HD void dsincos2pi(double u, double& sn, double& cs)
 
 // Acklam's rational approximation of the standard normal quantile (|rel err|
 // < 1.15e-9); one uniform in, one deviate out, no rejection.
+constexpr double kIcdfLow = 0.02425;   // the rational form of the centre covers [kIcdfLow, 1 - kIcdfLow]
+
+TM_HD bool icdf_in_tail(double p) { return p < kIcdfLow || p > 1.0 - kIcdfLow; }
+
 TM_HD double norm_icdf_d(double p)
 {
 #pragma clang fp contract(off)
-    const double plow = 0.02425;
+    const double plow = kIcdfLow;
     double q, num, den;
-    if (p < plow || p > 1.0 - plow) {
+    if (icdf_in_tail(p)) {
         q = dsqrt(-2.0 * dlog(p < plow ? p : 1.0 - p));
         num = ((((-7.784894002430293e-03 * q - 3.223964580411365e-01) * q - 2.400758277161838e+00) * q
                 - 2.549732539343734e+00) * q + 4.374664141464968e+00) * q + 2.938163982698783e+00;
@@ -337,59 +341,173 @@ TM_HD double logfact(int64_t k)
 }
 
 // ---------------------------------------------------------------------------
-// Poisson(z) in FP64 for both storage precisions (z = lambda e^{beta dt} rho is
-// always formed in FP64).  z < 12: sequential-search inversion; z >= 12: PTRS
-// transformed rejection (Hoermann 1993).  compat: the reference's Gaussian
-// shortcut trunc(N sqrt z + z) above 100 (rietkerk_bjork_FKE.cpp:4175-4180).
+// FP32 estimates that settle a logarithmic accept test without its FP64
+// logarithms: 1 = the FP64 test accepts, -1 = it rejects, 0 = too close to call
+// (the caller then evaluates the FP64 test).  Each estimate's margin is above
+// its own rounding error plus the FP64 test's, so a call settled here has the
+// outcome the FP64 test would have, and draws and fields do not change.  A
+// software logarithm costs about 70 FP64 instructions and the PTRS test takes
+// five of them, an estimate about 25 FP32 ones.  Rietkerk 256^2 in one lattice:
+// 15.8 us a step against 20.2, 16 x 512^2 163 us against 185 (two-pass Dornic).
 // ---------------------------------------------------------------------------
-template <class St>
-TM_HD int64_t poisson_d(St& s, double z, bool compat)
+__device__ __forceinline__ float est_log(float x) { return __builtin_amdgcn_logf(x) * 0.693147181f; }
+
+// Poisson (z >= 12): the constants of a PTRS draw, a trial's candidate, and its
+// fast acceptance (Hoermann's box, us >= 0.07 and V <= v_r), which needs no
+// logarithm.
+struct PtrsD {
+    double a, b, vr;
+};
+
+TM_HD PtrsD ptrs_setup_d(double z)
 {
 #pragma clang fp contract(off)
-    if (!(z > 0.0)) return 0;
-    if (compat && z > 100.0) return (int64_t)(norm_icdf_d(s.u64()) * dsqrt(z) + z);
-    if (z < 12.0) {
-        const double u = s.u64();
-        double p = dexp(-z);
-        double F = p;
-        int64_t k = 0;
-        while (u > F && k < 200) {
-            k += 1;
-            p = p * z / (double)k;
-            F = F + p;
-        }
-        return k;
-    }
+    PtrsD p;
     const double slam = dsqrt(z);
-    const double loglam = dlog(z);
-    const double b = 0.931 + 2.53 * slam;
-    const double a = -0.059 + 0.02483 * b;
-    const double invalpha = 1.1239 + 1.1328 / (b - 3.4);
-    const double vr = 0.9277 - 3.6224 / (b - 2.0);
-    const double linv = dlog(invalpha);
+    p.b = 0.931 + 2.53 * slam;
+    p.a = -0.059 + 0.02483 * p.b;
+    p.vr = 0.9277 - 3.6224 / (p.b - 2.0);
+    return p;
+}
+
+TM_HD double ptrs_k_d(const PtrsD& p, double z, double U, double us)
+{
+#pragma clang fp contract(off)
+    return __builtin_floor((2.0 * p.a / us + p.b) * U + z + 0.43);
+}
+
+TM_HD bool ptrs_in_box_d(const PtrsD& p, double us, double V) { return us >= 0.07 && V <= p.vr; }
+
+// The trial's test  log V + log(invalpha) - log(a / us^2 + b) <= -z + k log z - log k!,
+// both sides in FP32: the right one as -stirlerr(k) - bd0(k, z) - log(2 pi k) / 2
+// (Loader 2000), with k - z formed in FP64 and bd0 from its series.  Used for
+// 5 <= k, z < 1e9 and |k - z| < 0.1 (k + z), where every term is below 1e-6 relative
+// and the FP64 sides are good to 1e-5; the margin is 1e-3 + 1e-5 of their size.
+__device__ __forceinline__ int ptrs_estimate(const PtrsD& p, double z, double kd, double us, double V)
+{
+    const float k = (float)kd, zf = (float)z, dk = (float)(kd - z), sum = k + zf;
+    if (!(kd >= 5.0 && z < 1e9 && __builtin_fabsf(dk) < 0.1f * sum)) return 0;
+    const float w = dk * __builtin_amdgcn_rcpf(sum), w2 = w * w;
+    const float bd0 = dk * w + 2.0f * k * w * w2 * (0.333333333f + w2 * (0.2f + w2 * (0.142857143f + w2 * 0.111111111f)));
+    const float r = __builtin_amdgcn_rcpf(k);
+    const float rhs = -r * (0.0833333333f - r * r * 0.00277777778f) - bd0 - 0.5f * est_log(6.28318531f * k);
+    const float usf = (float)us, b = (float)p.b;
+    const float invalpha = 1.1239f + 1.1328f * __builtin_amdgcn_rcpf(b - 3.4f);
+    const float lhs = est_log((float)V * invalpha * __builtin_amdgcn_rcpf((float)p.a * __builtin_amdgcn_rcpf(usf * usf) + b));
+    const float margin = 1e-3f + 1e-5f * (__builtin_fabsf(lhs) + __builtin_fabsf(rhs));
+    return lhs < rhs - margin ? 1 : (lhs > rhs + margin ? -1 : 0);
+}
+
+// Marsaglia-Tsang's test  log u < x^2 / 2 + d (1 - v + log v), v = (1 + y)^3, y = c x:
+// below |y| = 0.1 the right side from its series in y, which does not cancel, and
+// directly above, where d <= 455 keeps its rounding below 1e-4.
+__device__ __forceinline__ int gamma_estimate(double u, double x2, double y, double v, double d)
+{
+    const float yf = (float)y, df = (float)d, vf = (float)v;
+    const float y2 = yf * yf;
+    const float ser = df * y2 * y2 * (-0.75f + yf * (0.6f + yf * (-0.5f + yf * (0.428571429f - 0.375f * yf))));
+    const float dir = 0.5f * (float)x2 + df * (1.0f - vf + est_log(vf));
+    const float rhs = __builtin_fabsf(yf) < 0.1f ? ser : dir;
+    const float lhs = est_log((float)u);
+    return lhs < rhs - 1e-3f ? 1 : (lhs > rhs + 1e-3f ? -1 : 0);
+}
+
+// (double)(int64_t)x of an integer-valued or large x.
+__device__ __forceinline__ double count_of(double x)
+{
+    if (!(__builtin_fabs(x) < 0x1p53)) x = (double)(int64_t)x;   // rare: huge, infinite or NaN
+    return x;
+}
+
+// k and 1/k for the inversion's terms.
+struct KInv {
+    double k, inv;
+};
+template <int N>
+struct KInvTable {
+    KInv v[N];
+};
+template <int N>
+constexpr KInvTable<N> make_kinv()
+{
+    KInvTable<N> t{};
+    for (int i = 0; i < N; ++i) t.v[i] = KInv{(double)(i + 1), 1.0 / (double)(i + 1)};
+    return t;
+}
+static __constant__ const KInvTable<200> kKInv = make_kinv<200>();
+
+// t / k, correctly rounded, for t well above the smallest normals: with r = 1/k
+// rounded, the first fused correction of t r is within one ulp of t / k and the
+// second rounds it correctly (Markstein's theorem).  Five instructions against the
+// division's eleven, on a wave-uniform k.
+__device__ __forceinline__ double div_k(double t, const KInv& c)
+{
+    double q = t * c.inv;
+    q = __builtin_fma(__builtin_fma(-q, c.k, t), c.inv, q);
+    return __builtin_fma(__builtin_fma(-q, c.k, t), c.inv, q);
+}
+
+// Inversion (0 < z < 12): sequential search, every lane of a wave at the same term.
+template <class St>
+__device__ __forceinline__ double poisson_inv_d(St& s, double z)
+{
+#pragma clang fp contract(off)
+    const double u = s.u64();
+    double p = dexp(-z);
+    double F = p, kd = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 200; ++k) {
+        if (!(u > F)) break;
+        const KInv c = kKInv.v[k];
+        kd = c.k;
+        p = div_k(p * z, c);   // p >= 1e-40 while the search goes on: u < 1 - 2^-33
+        F = F + p;
+    }
+    return kd;
+}
+
+// ---------------------------------------------------------------------------
+// Poisson(z) in FP64 for both storage precisions (z = lambda e^{beta dt} rho is
+// always formed in FP64), as an integer-valued double.  z < 12: sequential-search
+// inversion; z >= 12: PTRS transformed rejection (Hoermann 1993).  compat: the
+// reference's Gaussian shortcut trunc(N sqrt z + z) above 100
+// (rietkerk_bjork_FKE.cpp:4175-4180).
+// ---------------------------------------------------------------------------
+template <class St>
+__device__ __forceinline__ double poisson_d(St& s, double z, bool compat)
+{
+#pragma clang fp contract(off)
+    if (!(z > 0.0)) return 0.0;
+    if (compat && z > 100.0) return count_of(__builtin_trunc(norm_icdf_d(s.u64()) * dsqrt(z) + z));
+    if (z < 12.0) return poisson_inv_d(s, z);
+    const PtrsD pt = ptrs_setup_d(z);
     for (int it = 0; it < 64; ++it) {
         const double U = s.u64() - 0.5;
         const double V = s.u64();
         const double us = 0.5 - __builtin_fabs(U);
-        const double kd = __builtin_floor((2.0 * a / us + b) * U + z + 0.43);
-        if (us >= 0.07 && V <= vr) return (int64_t)kd;
+        const double kd = ptrs_k_d(pt, z, U, us);
+        if (ptrs_in_box_d(pt, us, V)) return count_of(kd);
         if (kd < 0.0 || (us < 0.013 && V > us)) continue;
-        const double lhs = dlog(V) + linv - dlog(a / (us * us) + b);
-        const double rhs = -z + kd * loglam - logfact((int64_t)kd);
-        if (lhs <= rhs) return (int64_t)kd;
+        const int est = ptrs_estimate(pt, z, kd, us, V);
+        if (est > 0) return count_of(kd);
+        if (est < 0) continue;
+        const double lhs = dlog(V) + dlog(1.1239 + 1.1328 / (pt.b - 3.4)) - dlog(pt.a / (us * us) + pt.b);
+        const double rhs = -z + kd * dlog(z) - logfact((int64_t)kd);
+        if (lhs <= rhs) return count_of(kd);
     }
-    return (int64_t)__builtin_floor(z);
+    return count_of(__builtin_floor(z));
 }
 
 // Gamma(shape, 1), Marsaglia & Tsang (2000) with the U^(1/shape) boost below
 // shape 1; shape <= 0 gives 0 (the Dornic shape-0 case).  FP64 version, at most
 // TRIALS trials: with TRIALS = 64 it always returns true (64 rejections leave
 // g = d); with fewer it returns false, leaving s and g unspecified, where the
-// sampler would draw one more trial, or (TRIALS = 1) where the squeeze does not
-// settle the trial: the two software logarithms of the test are left to the
-// full sampler, which the caller runs from the transition's first word.
+// sampler would draw one more trial, or (TRIALS = 1) where the normal deviate lies
+// in a tail of the quantile (a software logarithm and a square root) or the
+// squeezes and the estimate leave the trial open: those are left to the full
+// sampler, which the caller runs from the transition's first word.
 template <int TRIALS, class St>
-TM_HD bool gamma_d_try(St& s, double shape, double& g)
+__device__ __forceinline__ bool gamma_d_try(St& s, double shape, double& g)
 {
 #pragma clang fp contract(off)
     if (!(shape > 0.0)) { g = 0.0; return true; }
@@ -399,26 +517,25 @@ TM_HD bool gamma_d_try(St& s, double shape, double& g)
     g = d;
     bool ok = false;
     for (int it = 0; it < TRIALS; ++it) {
-        const double x = norm_icdf_d(s.u64());
-        double v = 1.0 + c * x;
+        const double p = s.u64();
+        if (TRIALS == 1 && icdf_in_tail(p)) return false;
+        const double x = norm_icdf_d(p);
+        const double y = c * x;
+        double v = 1.0 + y;
         if (v <= 0.0) continue;
         v = v * v * v;
         const double u = s.u64();
         const double x2 = x * x;
         if (u < 1.0 - 0.0331 * x2 * x2) { g = d * v; ok = true; break; }
+        const int est = gamma_estimate(u, x2, y, v, d);
+        if (est > 0) { g = d * v; ok = true; break; }
         if (TRIALS == 1) break;
+        if (est < 0) continue;
         if (dlog(u) < 0.5 * x2 + d * (1.0 - v + dlog(v))) { g = d * v; ok = true; break; }
     }
     if (TRIALS < 64 && !ok) return false;
     if (shape < 1.0) g = g * dexp(dlog(s.u64()) / shape);
     return true;
-}
-
-TM_HD double gamma_d(Stream& s, double shape)
-{
-    double g;
-    gamma_d_try<64, Stream>(s, shape, g);
-    return g;
 }
 
 // ---------------------------------------------------------------------------

@@ -245,26 +245,49 @@ template <> struct Arith<float> {
 
 // Dornic Poisson-Gamma transition of one live cell (rietkerk_bjork_FKE.cpp:4168-4196).
 // ONE = true: as the FP32 dornic_cell_f<true> -- false where the transition needs
-// PTRS (mean >= 12), the Gamma trial's logarithmic test (its squeeze failed) or
-// a second Gamma trial, otherwise the same words and value.
+// a software logarithm of an accept test or of the quantile's tail, a second PTRS
+// or Gamma trial, or a fifth word (the boost after a PTRS trial); otherwise the
+// same words and value.
+// n gets the Poisson count as an integer-valued double.
 template <bool ONE, class St>
 __device__ __forceinline__ bool dornic_cell_d(St& s, double alpha_i, double cur, const DornicConst& k,
-                                              bool compat, int64_t& n, double& y)
+                                              bool compat, double& n, double& y)
 {
 #pragma clang fp contract(off)
     const double mu = -1.0 + 2.0 * alpha_i * k.sigma2_1;
     const double ziggy = k.ll * cur;
-    if (ONE && ziggy >= 12.0) return false;
     double gru;
     if (ziggy == 0.0) {
-        n = 0;
+        n = 0.0;
         gru = mu + 1.0;
+    } else if (ONE && ziggy >= 12.0) {
+        if (compat && ziggy > 100.0) {
+            const double p = s.u64();
+            if (icdf_in_tail(p)) return false;
+            n = count_of(__builtin_trunc(norm_icdf_d(p) * dsqrt(ziggy) + ziggy));
+            gru = mu + 1.0 + n;
+        } else {
+            const PtrsD pt = ptrs_setup_d(ziggy);
+            const double U = s.u64() - 0.5;
+            const double V = s.u64();
+            const double us = 0.5 - __builtin_fabs(U);
+            n = ptrs_k_d(pt, ziggy, U, us);
+            if (!ptrs_in_box_d(pt, us, V)) {
+                if (n < 0.0 || (us < 0.013 && V > us)) return false;
+                if (ptrs_estimate(pt, ziggy, n, us, V) <= 0) return false;
+            }
+            n = count_of(n);
+            gru = mu + 1.0 + n;
+            if (gru < 1.0) return false;
+        }
     } else {
         n = poisson_d(s, ziggy, compat);
-        gru = mu + 1.0 + (double)n;
+        gru = mu + 1.0 + n;
     }
     if (compat && gru > 100.0) {
-        y = (norm_icdf_d(s.u64()) * dsqrt(gru) + gru) / k.lambda;
+        const double p = s.u64();
+        if (ONE && icdf_in_tail(p)) return false;
+        y = (norm_icdf_d(p) * dsqrt(gru) + gru) / k.lambda;
         return true;
     }
     double g;
@@ -274,7 +297,7 @@ __device__ __forceinline__ bool dornic_cell_d(St& s, double alpha_i, double cur,
 }
 
 __device__ __forceinline__ double dornic_cell(Stream& s, double alpha_i, double cur, const DornicConst& k,
-                                              bool compat, int64_t& n)
+                                              bool compat, double& n)
 {
     double y;
     dornic_cell_d<false, Stream>(s, alpha_i, cur, k, compat, n, y);
@@ -355,12 +378,16 @@ __device__ __forceinline__ float dornic_cell_f32(Stream& s, float shape0, double
 // four neighbours (old field), in the storage type's arithmetic: FP64 keeps
 // alpha_i and every Dornic quantity in FP64 in the reference's order; FP32 sums
 // the neighbours in FP32 (same order) and forms the Poisson mean in FP64.
-// Returns cur unchanged where alpha_i = 0 and cur = 0 (no draw, n = -1).
+// Returns cur unchanged where alpha_i = 0 and cur = 0 (no draw, n = -1).  The
+// count n stays an integer-valued double in FP64 (Count<T>): an int64 conversion
+// and back costs two dozen instructions, and only recorded draws want integers.
+template <typename T> struct Count { typedef int64_t type; };
+template <> struct Count<double> { typedef double type; };
 template <typename T> struct DornicLive;
 template <> struct DornicLive<double> {
     static __device__ __forceinline__ double step(uint32_t seed, uint32_t inst, uint32_t cell, int64_t step,
                                                   double cur, double up, double dn, double lf, double rt,
-                                                  const DornicConst& k, bool compat, int64_t& n);
+                                                  const DornicConst& k, bool compat, double& n);
 };
 template <> struct DornicLive<float> {
     static __device__ __forceinline__ float step(uint32_t seed, uint32_t inst, uint32_t cell, int64_t step, float cur,
@@ -385,7 +412,7 @@ __device__ __forceinline__ double nbr_alpha(double dc, T up, T dn, T lf, T rt)
 
 __device__ __forceinline__ double DornicLive<double>::step(uint32_t seed, uint32_t inst, uint32_t cell, int64_t step,
                                                            double cur, double up, double dn, double lf, double rt,
-                                                           const DornicConst& k, bool compat, int64_t& n)
+                                                           const DornicConst& k, bool compat, double& n)
 {
     const double alpha_i = nbr_alpha(k.dc, up, dn, lf, rt);
     if (alpha_i == 0.0 && cur == 0.0) return cur;
@@ -642,7 +669,8 @@ struct DPShape {
 // skipped); bad is set when MODE 0 produced a negative or non-finite value.
 template <typename T, int MODE>
 __device__ __forceinline__ T cell_update(const typename StepConst<MODE>::type& c, const DevInst& di,
-                                         uint32_t cell, T cur, T up, T dn, T lf, T rt, int64_t& n, bool& bad)
+                                         uint32_t cell, T cur, T up, T dn, T lf, T rt,
+                                         typename Count<T>::type& n, bool& bad)
 {
     T y = (T)0;
     n = -1;
@@ -663,10 +691,9 @@ __device__ __forceinline__ T cell_update(const typename StepConst<MODE>::type& c
 // has to be computed again by cell_update.
 template <typename T, int MODE>
 __device__ __forceinline__ bool cell_update_first(const typename StepConst<MODE>::type& c, const DevInst& di,
-                                                  uint32_t cell, T cur, T up, T dn, T lf, T rt, T& y, int64_t& n,
-                                                  bool& bad)
+                                                  uint32_t cell, T cur, T up, T dn, T lf, T rt, T& y,
+                                                  typename Count<T>::type& n, bool& bad)
 {
-    static_assert(MODE == 0 || sizeof(T) == 4, "the Rietkerk Dornic first pass is FP32");
     y = (T)0;
     n = -1;
     bad = false;
@@ -789,12 +816,12 @@ __device__ __forceinline__ void dp_tile(const StepArgs& a, int tile, const DevTi
             for (int q = 0; q < nvalid; ++q) {
                 const int rq = r + q;
                 const uint32_t cell = cell0 + q;
-                int64_t n;
+                typename Count<T>::type n;
                 bool bad;
                 const T y = cell_update<T, MODE>(c, di, cell, s_rho[rq], s_rho[rq - RWV], s_rho[rq + RWV],
                                                  s_rho[rq - 1], s_rho[rq + 1], n, bad);
                 if (bad) record_fault(a.state, tl.inst, cell, counter);
-                if (a.draws) a.draws[tl.cell_off + cell] = n;
+                if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 if constexpr (MODE == 0) {
                     sum[0] += (double)y;
                     nlive += y > (T)0 ? 1u : 0u;
@@ -876,7 +903,7 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
                 const int rq = r + q;
                 const uint32_t cell = cell0 + q;
                 T y;
-                int64_t n;
+                typename Count<T>::type n;
                 bool bad;
                 const bool done = cell_update_first<T, MODE>(c, di, cell, s_rho[rq], s_rho[rq - RWV],
                                                              s_rho[rq + RWV], s_rho[rq - 1], s_rho[rq + 1], y, n,
@@ -888,7 +915,7 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
                 } else if (bad) {
                     record_fault(a.state, tl.inst, cell, counter);
                 }
-                if (a.draws) a.draws[tl.cell_off + cell] = n;
+                if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 yq.v[0] = q == 0 ? y : yq.v[0];
                 yq.v[1] = q == 1 ? y : yq.v[1];
                 yq.v[2] = q == 2 ? y : yq.v[2];
@@ -927,12 +954,12 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
         const int ly = (int)(e / TX), lx = (int)(e % TX);
         const int r = (ly + 1) * RWV + V + lx;
         const uint32_t cell = (uint32_t)(tl.y0 + ly) * (uint32_t)L + (uint32_t)(tl.x0 + lx);
-        int64_t n;
+        typename Count<T>::type n;
         bool bad;
         const T y = cell_update<T, MODE>(c, di, cell, s_rho[r], s_rho[r - RWV], s_rho[r + RWV], s_rho[r - 1],
                                          s_rho[r + 1], n, bad);
         if (bad) record_fault(a.state, tl.inst, cell, counter);
-        if (a.draws) a.draws[tl.cell_off + cell] = n;
+        if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
         s_q[i] = y;                                           // the slot's thread read its offset above
     }
     __syncthreads();
@@ -967,8 +994,8 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
 // alone (rietkerk_bjork_FKE.cpp:4154-4211), writing P* to a.aux for the RK4
 // kernel -- same staging, absorbing-group skip and sampler, on its own tiles.
 // Q = 1: the two-pass tile (dp_tile_deferred) with its queue of deferred
-// cells -- the DP step in either precision, the Rietkerk Dornic sub-step in
-// FP32.  One tile per workgroup: its descriptor, instance and constants are
+// cells, for the DP step and the Rietkerk Dornic sub-step in either precision.
+// One tile per workgroup: its descriptor, instance and constants are
 // read before the kernel writes anything, so they are scalar loads issued
 // together, and the image copy follows at once.
 template <typename T, int TX, int TY, int NT, int MODE, int MINW = 1, int Q = 0>
@@ -977,7 +1004,6 @@ __global__ __launch_bounds__(NT, MINW) void dp_step_kernel(StepArgs a)
     typedef DPShape<T, TX, TY, NT> S;
     typedef typename StepConst<MODE>::type Const;
     constexpr int NFIN = MODE == 1 ? 3 : 1;           // fields per instance block of `in`
-    static_assert(Q == 0 || MODE == 0 || sizeof(T) == 4, "deferring Rietkerk Dornic step: FP32 only");
     __shared__ __align__(16) uint32_t s_img[S::NBUF];
     __shared__ uint32_t s_flag[NT / 64];
     __shared__ __align__(8) T s_q[Q ? TX * TY : 1];   // deferred cells: tile offsets, then values
@@ -1121,7 +1147,7 @@ __global__ __launch_bounds__(NT, MINW) void dp_stepk_kernel(StepArgs a)
                     const int rq = r + q;
                     const int lx = 4 * cg + q;
                     const uint32_t cell = (uint32_t)gy * (uint32_t)L + (uint32_t)wrap(tl.x0 + lx, L);
-                    int64_t n;
+                    typename Count<T>::type n;
                     bool bad;
                     const T y = cell_update<T, 0>(c, di, cell, src[rq], src[rq - RW], src[rq + RW], src[rq - 1],
                                                   src[rq + 1], n, bad);
@@ -1142,7 +1168,7 @@ __global__ __launch_bounds__(NT, MINW) void dp_stepk_kernel(StepArgs a)
             const int lx = cc < R ? cc - R : TX + (cc - R);
             const int rq = (ly + srad) * RW + HC + lx;
             const uint32_t cell = (uint32_t)wrap(tl.y0 + ly, L) * (uint32_t)L + (uint32_t)wrap(tl.x0 + lx, L);
-            int64_t n;
+            typename Count<T>::type n;
             bool bad;
             dstf[(ly + R) * RW + HC + lx] = cell_update<T, 0>(c, di, cell, src[rq], src[rq - RW], src[rq + RW],
                                                               src[rq - 1], src[rq + 1], n, bad);
@@ -1189,12 +1215,12 @@ __global__ __launch_bounds__(NT, MINW) void dp_stepk_kernel(StepArgs a)
             for (int q = 0; q < nvalid; ++q) {
                 const int rq = r + q;
                 const uint32_t cell = cell0 + q;
-                int64_t n;
+                typename Count<T>::type n;
                 bool bad;
                 const T y = cell_update<T, 0>(c, di, cell, src[rq], src[rq - RW], src[rq + RW], src[rq - 1],
                                               src[rq + 1], n, bad);
                 if (bad) record_fault(a.state, tl.inst, cell, counter + K - 1, K - 1);
-                if (a.draws) a.draws[tl.cell_off + cell] = n;
+                if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 sum += (double)y;
                 nlive += y > (T)0 ? 1u : 0u;
                 yq.v[0] = q == 0 ? y : yq.v[0];
@@ -1533,10 +1559,10 @@ __global__ __launch_bounds__(NT) void rk_step_kernel(StepArgs a)
 
     // ---- stage 0 (fused step): Dornic P* on the radius-3 frame (FKE:4154-4211) ----
     if constexpr (!SPLIT) {
-        auto dornic_at = [&](int ly, int lx, int64_t* n_out) {
+        auto dornic_at = [&](int ly, int lx, typename Count<T>::type* n_out) {
             const int r = i4(ly, lx);
             const int gy = wrap(tl.y0 + ly, L), gx = wrap(tl.x0 + lx, L);
-            int64_t n = -1;
+            typename Count<T>::type n = -1;
             const T y = DornicLive<T>::step(di.seed, di.inst_id, (uint32_t)((int64_t)gy * L + gx), c.step, sP0[r],
                                             sP0[r - W4], sP0[r + W4], sP0[r - 1], sP0[r + 1], c.k, c.compat != 0, n);
             *n_out = n;
@@ -1545,17 +1571,17 @@ __global__ __launch_bounds__(NT) void rk_step_kernel(StepArgs a)
         for (int j = 0; j < NOWN; ++j) {
             int ly, lx;
             own(j, ly, lx);
-            int64_t n;
+            typename Count<T>::type n;
             dornic_at(ly, lx, &n);
             const int gy = tl.y0 + ly, gx = tl.x0 + lx;
-            if (a.draws && gy < L && gx < L) a.draws[di.cell_off + (int64_t)gy * L + gx] = n;
+            if (a.draws && gy < L && gx < L) a.draws[di.cell_off + (int64_t)gy * L + gx] = (int64_t)n;
         }
         for (int j = 0; j < NR3; ++j) {
             const int k = tid + j * NT;
             if (k < Ring<TX, TY, 3>::N) {
                 int ly, lx;
                 ring_cell<TX, TY, 3>(k, ly, lx);
-                int64_t n;
+                typename Count<T>::type n;
                 dornic_at(ly, lx, &n);
             }
         }

@@ -67,6 +67,11 @@ static const Variant kRK[] = {
      &launch_dp<double, 64, 32, 256, 1>},
     {32, 32, 256, 0, 1, "rk_f64_split_32x32_t256", &launch_rk<double, 32, 32, 256, true>, 64, 32,
      &launch_dp<double, 64, 32, 256, 1>},
+    // _q16: the Dornic kernel in two passes (dp_tile_deferred) on 64 x 16 tiles at 80
+    // VGPRs.  16 x 512^2, Dornic and RK4 together: 163 us a step, one-pass 64 x 32
+    // tiles 202; other tiles (64 x 8, 64 x 32, 128 x 16) and bounds 166 to 178.
+    {32, 16, 256, 0, 1, "rk_f64_split_32x16_t256_q16", &launch_rk<double, 32, 16, 256, true>, 64, 16,
+     &launch_dp<double, 64, 16, 256, 1, 6, 1>},
 };
 
 const Variant* dp_variants_f64(int* n) { *n = (int)(sizeof(kDP) / sizeof(kDP[0])); return kDP; }

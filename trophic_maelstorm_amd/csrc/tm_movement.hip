@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256) void fke_veg_dornic_kernel(tm_rietkerk_params 
     const int y = (int)(i / L), x = (int)(i % L);
     const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
     const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
-    int64_t n;
+    double n;
     bool bad;
     Pstar[i] = tmk::cell_update<double, 1>(c, di, (uint32_t)i, P[i], P[up], P[dn], P[lf], P[rt], n, bad);
 }
@@ -735,7 +735,7 @@ __global__ __launch_bounds__(256) void fke_veg_kernel(StepArgs a)
     const int y = cell / L, x = cell % L;
     const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
     const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
-    int64_t n;
+    double n;
     bool bad;
     fout[cell] = cell_update<double, 1>(c, di, (uint32_t)cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
 #pragma unroll
