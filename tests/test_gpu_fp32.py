@@ -301,3 +301,31 @@ def test_fp32_one_step_dornic_bias(tm):
     print(f"one-step FP32 Dornic bias {rel.mean():.3e} (SE {se:.2e})", flush=True)
     assert se < 2e-8
     assert abs(rel.mean()) < 1e-7
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("prec,n", [("f64", 3), ("f64", 1024), ("f64", 1025), ("f32", 3), ("f32", 256), ("f32", 257),
+                                    ("f32", 1025)])
+def test_small_batch_dp_parts_are_identical(tm, prec, n):
+    """The default DP step takes a workgroup per part of a tile on small batches (one
+    or three cells a thread, by the number of tiles): fields, draws and rho(t) rows
+    equal those of the two-pass tile kernel, at the edges of the rule, on lattices of
+    one tile and (the first) of several partly filled ones."""
+    P = tm.F64 if prec == "f64" else tm.F32
+    names = tm.variant_names(tm.MODEL_DP, P)
+    fixed = "dp_f64_64x32_t256_x8aq" if prec == "f64" else "dp_f32_128x24_t256_w6q"
+    Ls = [130, 61, 17] if n == 3 else [17] * n
+    insts = [tm.Instance(L, 0, 9, k) for k, L in enumerate(Ls)]
+    out = []
+    for v in (-1, names.index(fixed)):
+        with tm.Context() as ctx:
+            ctx.configure(tm.MODEL_DP, P, tm.DPParams(a=0.9), insts)
+            ctx.set_launch(v, 16)
+            ctx.init_uniform([0.0], [1.0])
+            ctx.record_draws(True)
+            rows = ctx.run(5)
+            out.append((rows, [ctx.download(k) for k in range(len(Ls))], [ctx.draws(k) for k in range(len(Ls))]))
+    (r0, f0, d0), (r1, f1, d1) = out
+    assert np.array_equal(r0, r1)
+    for k in range(len(Ls)):
+        assert np.array_equal(f0[k], f1[k]) and np.array_equal(d0[k], d1[k])

@@ -491,18 +491,26 @@ __device__ __forceinline__ void wave_partial(double sum, double cnt, double2* ds
     if ((lane & 31) == 0) ((double*)dst)[lane >> 5] = t;
 }
 
-// Wave partial (sum, count) of one step into its slot; an all-zero wave writes zeros.
-template <int NT>
-__device__ __forceinline__ void step_partial(const StepArgs& a, int tile, int64_t counter, double s,
-                                             uint32_t nlive)
+// Wave partial (sum, count) of one step into its slot (wave w of the tile's NW); an
+// all-zero wave writes zeros.
+template <int NW>
+__device__ __forceinline__ void wave_step_partial(const StepArgs& a, int tile, int w, int64_t counter, double s,
+                                                  uint32_t nlive)
 {
     const int64_t slot = counter & (int64_t)(a.nslots - 1);
-    double2* dst = a.partials + (slot * a.ntiles + tile) * (NT / 64) + (threadIdx.x >> 6);
+    double2* dst = a.partials + (slot * a.ntiles + tile) * NW + w;
     if (__ballot(nlive != 0 || s != 0.0) == 0) {
         if ((threadIdx.x & 63) == 0) *dst = make_double2(0.0, 0.0);
     } else {
         wave_partial(s, (double)nlive, dst);
     }
+}
+
+template <int NT>
+__device__ __forceinline__ void step_partial(const StepArgs& a, int tile, int64_t counter, double s,
+                                             uint32_t nlive)
+{
+    wave_step_partial<NT / 64>(a, tile, threadIdx.x >> 6, counter, s, nlive);
 }
 
 // Asynchronous copy of a tile and its halo into LDS with global_load_lds: each
@@ -1030,6 +1038,71 @@ __global__ __launch_bounds__(NT, MINW) void dp_step_kernel(StepArgs a)
         dp_tile_deferred<T, TX, TY, NT, MODE>(a, tile, tl, di, c, (const T*)s_img, counter, s_q, s_wn);
     else
         dp_tile<T, TX, TY, NT, MODE>(a, tile, tl, di, c, (const T*)s_img, counter, slot);
+}
+
+// The DP step of a batch too small to fill the GPU with tiles: the same tiles, split
+// into the NW parts whose cells one wave of dp_tile owns (part w: tile rows
+// w RP + r + j R4, r < RP, j < G, all columns), a workgroup per part and CPT cells
+// per thread, read straight from global memory (L2 holds such a batch).  The tile
+// kernels give a thread 8 to 12 cells one after another, and 8 lattices of 128^2
+// are 64 tiles on 256 CUs: there the step is the latency of those cells in turn.
+// The part's values go to LDS and its first wave sums them lane by lane in dp_tile's
+// order, so fields, draws and rho(t) partials are dp_tile's bit for bit.
+template <typename T, int TX, int TY, int CPT>
+__global__ __launch_bounds__(TX * TY / 4 / CPT) void dp_part_kernel(StepArgs a)
+{
+    typedef DPShape<T, TX, TY, 256> S;
+    constexpr int RP = 64 / S::CG;                 // rows of one canonical wave
+    constexpr int NC = RP * S::G * TX;             // cells of a part
+    constexpr int NT = NC / CPT;
+    static_assert(S::NW == 4 && NC == TX * TY / 4 && NT % 64 == 0 && NT <= 1024, "part shape");
+    __shared__ T s_y[NC];
+
+    const int tile = blockIdx.x >> 2, w = blockIdx.x & 3;
+    if (tile >= a.ntiles) return;
+    const int64_t counter = a.state->counter + a.k;
+    const DevTile tl = a.tiles[tile];
+    const DevInst di = a.inst[tl.inst];
+    const DPConst c = ((const DPConst*)a.consts)[(int64_t)a.k * a.n_inst + tl.inst];
+    const int L = tl.L;
+    const T* fin = (const T*)a.in + tl.cell_off;
+    T* fout = (T*)a.out + tl.cell_off;
+#pragma unroll 1
+    for (int i = threadIdx.x; i < NC; i += NT) {
+        const int lr = i / TX;
+        const int gy = tl.y0 + w * RP + lr % RP + lr / RP * S::R4, gx = tl.x0 + i % TX;
+        T y = (T)0;
+        if (gy < L && gx < L) {
+            const uint32_t row = (uint32_t)gy * (uint32_t)L, cell = row + (uint32_t)gx;
+            const uint32_t up = (uint32_t)(gy == 0 ? L - 1 : gy - 1) * (uint32_t)L + (uint32_t)gx;
+            const uint32_t dn = (uint32_t)(gy == L - 1 ? 0 : gy + 1) * (uint32_t)L + (uint32_t)gx;
+            const uint32_t lf = row + (uint32_t)(gx == 0 ? L - 1 : gx - 1);
+            const uint32_t rt = row + (uint32_t)(gx == L - 1 ? 0 : gx + 1);
+            typename Count<T>::type n;
+            bool bad;
+            y = cell_update<T, 0>(c, di, cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
+            if (bad) record_fault(a.state, tl.inst, cell, counter);
+            if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
+            fout[cell] = y;
+        }
+        s_y[i] = y;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    // cells past the lattice hold 0, which leaves the sum and the count as they are
+    const int lane = threadIdx.x;
+    double sum = 0.0;
+    uint32_t nlive = 0;
+#pragma unroll
+    for (int j = 0; j < S::G; ++j) {
+        const T* q = s_y + (j * RP + lane / S::CG) * TX + 4 * (lane % S::CG);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            sum += (double)q[k];
+            nlive += q[k] > (T)0 ? 1u : 0u;
+        }
+    }
+    wave_step_partial<4>(a, tile, w, counter, sum, nlive);
 }
 
 // ---------------------------------------------------------------------------

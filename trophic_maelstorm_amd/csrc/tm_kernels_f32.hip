@@ -18,6 +18,21 @@ static void launch_dpk(const StepArgs& a, int grid, hipStream_t s)
     hipLaunchKernelGGL((dp_stepk_kernel<T, TX, TY, NT, K, MINW>), dim3(grid), dim3(NT), 0, s, a);
 }
 
+// The default's single step: a workgroup per part of a tile (dp_part_kernel), one cell
+// a thread up to 256 tiles, three up to 1024, the two-pass tile kernel above.  us a
+// step, one / three cells / tiles: 6.0 / 9.4 / 21.3 at 48 tiles (8 x 128^2), 14.1 / 14.4 /
+// 23.1 at 288, 16.8 / 16.3 / 23.4 at 384, 28.4 / 26.1 / 27.5 at 768, 40.7 / 35.7 / 36.2
+// at 1152.
+static void launch_dp_default(const StepArgs& a, int grid, hipStream_t s)
+{
+    if (a.ntiles <= 256)
+        hipLaunchKernelGGL((dp_part_kernel<float, 128, 24, 1>), dim3(4 * a.ntiles), dim3(768), 0, s, a);
+    else if (a.ntiles <= 1024)
+        hipLaunchKernelGGL((dp_part_kernel<float, 128, 24, 3>), dim3(4 * a.ntiles), dim3(256), 0, s, a);
+    else
+        launch_dp<float, 128, 24, 256, 0, 6, 1>(a, grid, s);
+}
+
 template <typename T, int TX, int TY, int NT, bool SPLIT = false>
 static void launch_rk(const StepArgs& a, int grid, hipStream_t s)
 {
@@ -70,7 +85,7 @@ static const Variant kDP[] = {
     // pass over a queue in LDS (dp_tile_deferred)
     {128, 24, 256, 0, 4, "dp_f32_128x24_t256_w6q", &launch_dp<float, 128, 24, 256, 0, 6, 1>},
     {128, 24, 256, 0, 4, "dp_f32_128x24_t256_x8aq", &launch_dpk<float, 128, 24, 256, 8>, 0, 0, nullptr, 0, 8,
-     &launch_dp<float, 128, 24, 256, 0, 6, 1>, 20},
+     &launch_dp_default, 20},
 };
 
 static const Variant kRK[] = {

@@ -18,6 +18,18 @@ static void launch_dpk(const StepArgs& a, int grid, hipStream_t s)
     hipLaunchKernelGGL((dp_stepk_kernel<T, TX, TY, NT, K, MINW>), dim3(grid), dim3(NT), 0, s, a);
 }
 
+// The default's single step: a workgroup per part of a tile (dp_part_kernel) up to
+// 1024 tiles, the two-pass tile kernel above.  us a step, parts against tiles:
+// 8.8 / 31.1 at 64 tiles (8 x 128^2), 17.2 / 31.1 at 256, 28.4 / 37.9 at 512,
+// 50.3 / 56.9 at 1024 (2.1 M cells); the tiles take 97.3 at 2048, under twice 50.3.
+static void launch_dp_default(const StepArgs& a, int grid, hipStream_t s)
+{
+    if (a.ntiles <= 1024)
+        hipLaunchKernelGGL((dp_part_kernel<double, 64, 32, 1>), dim3(4 * a.ntiles), dim3(512), 0, s, a);
+    else
+        launch_dp<double, 64, 32, 256, 0, 6, 1>(a, grid, s);
+}
+
 template <typename T, int TX, int TY, int NT, bool SPLIT = false>
 static void launch_rk(const StepArgs& a, int grid, hipStream_t s)
 {
@@ -51,9 +63,10 @@ static const Variant kDP[] = {
     // pass over a queue in LDS (dp_tile_deferred)
     {64, 32, 256, 0, 4, "dp_f64_64x32_t256_x8aq", &launch_dpk<double, 64, 32, 256, 8>, 0, 0, nullptr, 0, 8,
      &launch_dp<double, 64, 32, 256, 0, 1, 1>, 20},
-    // _w6: its single step bounded to 80 VGPRs (six waves per SIMD)
+    // _w6 (the default): its single step bounded to 80 VGPRs (six waves per SIMD), and
+    // by parts on small batches
     {64, 32, 256, 0, 4, "dp_f64_64x32_t256_x8aq_w6", &launch_dpk<double, 64, 32, 256, 8>, 0, 0, nullptr, 0, 8,
-     &launch_dp<double, 64, 32, 256, 0, 6, 1>, 20},
+     &launch_dp_default, 20},
 };
 
 static const Variant kRK[] = {
