@@ -465,7 +465,7 @@ typedef struct tm_fke_rk_params {
  * ns = 1 consumer and RK4_Integrate_Stochastic_MultiSp (:2652-2720) for ns = 2.
  * fields [ns + 3][L*L] in the reference's order: P, G, (Pr,) W, O; periodic
  * lattice.  Device arrays (hipMalloc'd), on `stream` (a hipStream_t, or null); the
- * library allocates its scratch (3 (ns + 3) L^2 doubles) and waits for the stream
+ * library allocates its scratch ((ns + 3) L^2 doubles) and waits for the stream
  * before returning.  n_bad (may be null) gets the number of values that ended
  * negative or non-finite, which the reference logs and carries on from
  * (FKE:2511-2529).  Returns 0 or a negative tm_status. */
@@ -477,8 +477,8 @@ int tm_fke_rk4_host(int device, int ns, int L, const tm_fke_rk_params* p, double
 /* tm_fke_rk4 without allocating: no counterpart in the reference.  For callers
  * that cannot allocate device memory (code under HIP graph capture, serving
  * loops, harnesses that forbid hipMalloc).  The same kernels and result as
- * tm_fke_rk4; the stage buffers and the negative-value counter live in a fixed
- * library array on each GPU (3 x 5 x 256^2 doubles, 7.5 MiB, held until the
+ * tm_fke_rk4; the copy of the fields and the negative-value counter live in a fixed
+ * library array on each GPU (5 x 256^2 doubles, 2.5 MiB, held until the
  * process ends), so L <= 256 (ns <= 2), else TM_ERR_TOO_LARGE.  Runs on the
  * current device, whose stream `stream` must be; waits for it before returning.
  * Calls that overlap on one GPU share the array and race. */

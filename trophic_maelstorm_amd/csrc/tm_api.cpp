@@ -117,6 +117,7 @@ struct tm_ctx {
     int dpc_nchunks = 0;
     int dpc_halo = 1;
     int fke_nblocks = 0;           // Rietkerk consumer models: 256-cell blocks (FkeWork in d_dpc)
+    int fke_nrtiles = 0;           // ... and RK4 tiles
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
 };
 
@@ -255,6 +256,7 @@ void release_config(tm_ctx* c)
     c->dpc_nchunks = 0;
     c->dpc_halo = 1;
     c->fke_nblocks = 0;
+    c->fke_nrtiles = 0;
     invalidate_live(c);
     c->series_cap = c->groups_cap = c->stats_cap = c->frame_tab_cap = 0;
     c->series_steps_cap = c->n_series = 0;
@@ -354,6 +356,7 @@ StepArgs step_args(tm_ctx* c, int parity, int k)
     a.nchunks = c->dpc_nchunks;
     a.halo = c->dpc_halo;
     a.nblocks = c->fke_nblocks;
+    a.nrtiles = c->fke_nrtiles;
     return a;
 }
 
@@ -890,7 +893,7 @@ tm_status tm_configure(tm_ctx* c, int model, int precision, const void* params, 
         const char* err = "";
         const int rc = fke_setup(model, (const tm_fke_params*)c->params.data(), n_params, c->inst.data(), n_inst,
                                  c->cell_off.data(), c->total_cells, &c->d_dpc, &c->dpc_nchunks, &c->fke_nblocks,
-                                 &err);
+                                 &c->fke_nrtiles, &err);
         if (rc != TM_OK) {
             const std::string msg = err;
             release_config(c);

@@ -81,7 +81,7 @@ struct StepArgs {
     int32_t nchunks;     // consumer models: statistics chunks of the batch
     int32_t halo;        // consumer models: LDS halo (largest perception radius, >= 1)
     int32_t nblocks;     // Rietkerk consumer models: 256-cell blocks of the batch
-    int32_t pad;
+    int32_t nrtiles;     // Rietkerk consumer models: RK4 tiles of the batch
 };
 
 // Periodic index: v mod L in [0, L).

@@ -384,9 +384,7 @@ struct DevBuf {
 // Trophic RK4 of the Rietkerk consumer model: RK4_Integrate_Stochastic_2Sp /
 // _MultiSp with f_DorFKE_2Sp / f_DorFKE_3Sp (rietkerk_bjork_FKE.cpp:2449-2533,
 // :2611-2720).  Fields in the reference's order: P, G, (Pr,) W, O.  W and O
-// diffuse, so every stage needs its neighbours' stage values: one grid-wide
-// pass per stage.  The K's are folded into one accumulator in the reference's
-// order ((K1 + 2 K2) + 2 K3) + K4, so no K array is kept.
+// diffuse, so every stage needs its neighbours' stage values (fke_rk4_tile).
 // ---------------------------------------------------------------------------
 struct FkeRk {
     int ns, L;                       // consumer species (1 or 2), lattice side
@@ -396,74 +394,133 @@ struct FkeRk {
     double dt, dt2, dt6;             // the RK4's dt; dt2 and dt6 from Dt_Analytic (FKE:206-210)
 };
 
-// f at cell i of the NF fields y (stride L^2), in the reference's operation order.
+// f at a cell from its NS + 3 values y and the sums nW, nO = up + down + left + right
+// of its W and O neighbours, in the reference's operation order.
 template <int NS>
-__device__ __forceinline__ void fke_rhs(const FkeRk& c, const double* y, int64_t L2, int i, int up, int dn, int lf,
-                                        int rt, double (&f)[NS + 3])
+__device__ __forceinline__ void fke_rhs(const FkeRk& c, const double (&y)[NS + 3], double nW, double nO,
+                                        double (&f)[NS + 3])
 {
 #pragma clang fp contract(off)
     constexpr int W = NS + 1, O = NS + 2;
-    const double P = y[i], G = y[L2 + i], Wi = y[W * L2 + i], Oi = y[O * L2 + i];
-    const double* yW = y + W * L2;
-    const double* yO = y + O * L2;
+    const double P = y[0], G = y[1], Wi = y[W], Oi = y[O];
     const double A = c.alpha * (P + c.K2W0) / (P + c.K2) * Oi;
     const double X = c.EA1 * P / (1 + c.A01H01 * P) * G;
     f[0] = c.cgmax * Wi * P / (Wi + c.K1) - (c.A01 * P / (1 + c.A01H01 * P)) * G;
     if constexpr (NS == 1) {
         f[1] = X - c.M1 * G;
     } else {
-        const double Pr = y[2 * L2 + i];
+        const double Pr = y[2];
         f[1] = X - c.M1 * G - c.A12 * G / (1 + c.A12H12 * G) * Pr;
         f[2] = (c.EA2 * G / (1 + c.A12H12 * G)) * Pr - c.M2 * Pr;
     }
-    f[W] = A - c.gmax * Wi * P / (Wi + c.K1) - c.rW * Wi + c.dW * (yW[up] + yW[dn] + yW[lf] + yW[rt] - 4 * Wi);
-    f[O] = c.a - A + c.dO * (yO[up] + yO[dn] + yO[lf] + yO[rt] - 4 * Oi);
+    f[W] = A - c.gmax * Wi * P / (Wi + c.K1) - c.rW * Wi + c.dW * (nW - 4 * Wi);
+    f[O] = c.a - A + c.dO * (nO - 4 * Oi);
 }
 
-// Stage s (1..4) from the stage values src: K_s = f(src).  Stages 1-3 fold K_s
-// into acc and write the next stage's values rho + h K_s to nxt; stage 4 writes
-// rho + dt6 (acc + K4) over rho and counts the cells that turned negative or
+// The four stages of one tile in one workgroup of 1024 threads, a thread per cell of
+// the 32 x 32 frame around a 26 x 26 tile: RK4 widens the W and O stencil by a cell a
+// stage, so stage 1 is evaluated on the whole frame (its neighbours read from global
+// memory), stages 2, 3 and 4 on frames one cell smaller each.  A cell's fields, its
+// stage state and its accumulator ((K1 + 2 K2) + 2 K3) + K4 stay in its thread's
+// registers; only the (W, O) stage states pass through LDS, in two buffers, one
+// barrier a stage.  Four grid-wide passes, with the stage states and the accumulator
+// in memory, moved 20 values a cell and stage and were bound by that; here a field is
+// read and written once and the overlap costs 1.5 times the evaluations.  16 x 256^2
+// with the predator: 44.7 us against 4 x 37; one lattice of 512^2: 17.5 against 4 x 10.4.
+// src0: field 0, src: the base of fields 1 .. NF - 1 (field s at src + s N), out: the
+// base of the results (field s at out + s N); src0 and src must not overlap out.
+// Returns the number of results at this thread's cell that turned negative or
 // non-finite (the reference logs them, FKE:2511-2529, and carries on).
+constexpr int kRkFrame = 32, kRkTile = 26, kRkThreads = kRkFrame * kRkFrame;
+
+struct RkTileLds {
+    double2 wo[2][kRkThreads];
+};
+
 template <int NS>
-__device__ __forceinline__ uint32_t fke_stage_at(const FkeRk& c, int stage, double* rho, const double* src,
-                                                 double* nxt, double* acc, int64_t L2, int i)
+__device__ __forceinline__ uint32_t fke_rk4_tile(const FkeRk& c, const double* __restrict__ src0,
+                                                 const double* __restrict__ src, double* __restrict__ out, int L,
+                                                 int64_t N, int y0, int x0, RkTileLds& sm)
 {
 #pragma clang fp contract(off)
-    constexpr int NF = NS + 3;
-    const int L = c.L;
-    const int y = i / L, x = i % L;
-    const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
-    const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
-    double f[NF];
-    fke_rhs<NS>(c, src, L2, i, up, dn, lf, rt, f);
-    uint32_t bad = 0;
+    constexpr int NF = NS + 3, W = NS + 1, O = NS + 2;
+    const int t = threadIdx.x, ty = t / kRkFrame, tx = t % kRkFrame;
+    const int gy = tmk::wrap(y0 + ty - 3, L), gx = tmk::wrap(x0 + tx - 3, L);
+    const int64_t i = (int64_t)gy * L + gx;
+    auto inner = [&](int r) { return tx >= r && tx < kRkFrame - r && ty >= r && ty < kRkFrame - r; };
+    double y[NF], st[NF], acc[NF], f[NF];
+    y[0] = src0[i];
+#pragma unroll
+    for (int s = 1; s < NF; ++s) y[s] = src[s * N + i];
+    {   // stage 1: neighbours of the old fields
+        const int64_t up = (int64_t)(gy == 0 ? L - 1 : gy - 1) * L + gx, dn = (int64_t)(gy == L - 1 ? 0 : gy + 1) * L + gx;
+        const int64_t lf = (int64_t)gy * L + (gx == 0 ? L - 1 : gx - 1), rt = (int64_t)gy * L + (gx == L - 1 ? 0 : gx + 1);
+        const double* w = src + W * N;
+        const double* o = src + O * N;
+        fke_rhs<NS>(c, y, w[up] + w[dn] + w[lf] + w[rt], o[up] + o[dn] + o[lf] + o[rt], f);
+    }
 #pragma unroll
     for (int s = 0; s < NF; ++s) {
-        const int64_t j = s * L2 + i;
-        if (stage == 1) {
-            acc[j] = f[s];
-            nxt[j] = rho[j] + c.dt2 * f[s];
-        } else if (stage < 4) {
-            acc[j] = acc[j] + 2.0 * f[s];
-            nxt[j] = rho[j] + (stage == 2 ? c.dt2 : c.dt) * f[s];
-        } else {
-            const double r = rho[j] + c.dt6 * (acc[j] + f[s]);
-            rho[j] = r;
+        acc[s] = f[s];
+        st[s] = y[s] + c.dt2 * f[s];
+    }
+    sm.wo[0][t] = make_double2(st[W], st[O]);
+    __syncthreads();
+    auto stage = [&](const double2* b) {
+        const double2 up = b[t - kRkFrame], dn = b[t + kRkFrame], lf = b[t - 1], rt = b[t + 1];
+        fke_rhs<NS>(c, st, up.x + dn.x + lf.x + rt.x, up.y + dn.y + lf.y + rt.y, f);
+    };
+    if (inner(1)) {   // stage 2
+        stage(sm.wo[0]);
+#pragma unroll
+        for (int s = 0; s < NF; ++s) {
+            acc[s] = acc[s] + 2.0 * f[s];
+            st[s] = y[s] + c.dt2 * f[s];
+        }
+        sm.wo[1][t] = make_double2(st[W], st[O]);
+    }
+    __syncthreads();
+    if (inner(2)) {   // stage 3
+        stage(sm.wo[1]);
+#pragma unroll
+        for (int s = 0; s < NF; ++s) {
+            acc[s] = acc[s] + 2.0 * f[s];
+            st[s] = y[s] + c.dt * f[s];
+        }
+        sm.wo[0][t] = make_double2(st[W], st[O]);   // its stage 2 readers are past the barrier
+    }
+    __syncthreads();
+    uint32_t bad = 0;
+    if (inner(3) && y0 + ty - 3 < L && x0 + tx - 3 < L) {   // stage 4: the tile's own cells
+        stage(sm.wo[0]);
+#pragma unroll
+        for (int s = 0; s < NF; ++s) {
+            const double r = y[s] + c.dt6 * (acc[s] + f[s]);
+            out[s * N + i] = r;
             bad += (r < 0 || !__builtin_isfinite(r)) ? 1u : 0u;
         }
     }
     return bad;
 }
 
+// The operator's step, from a copy of the fields (scratch) into the fields.
 template <int NS>
-__global__ __launch_bounds__(256) void fke_rk_stage_kernel(FkeRk c, int stage, double* rho, const double* src,
-                                                           double* nxt, double* acc, unsigned long long* n_bad)
+__global__ __launch_bounds__(kRkThreads) void fke_rk4_kernel(FkeRk c, const double* src, double* out,
+                                                             unsigned long long* n_bad)
 {
-    const int64_t L2 = (int64_t)c.L * c.L;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= L2) return;
-    const uint32_t bad = fke_stage_at<NS>(c, stage, rho, src, nxt, acc, L2, (int)i);
-    if (stage == 4 && bad) atomicAdd(n_bad, (unsigned long long)bad);
+    __shared__ RkTileLds sm;
+    const int64_t N = (int64_t)c.L * c.L;
+    const uint32_t bad = fke_rk4_tile<NS>(c, src, src, out, c.L, N, (int)blockIdx.y * kRkTile, (int)blockIdx.x * kRkTile, sm);
+    if (bad) atomicAdd(n_bad, (unsigned long long)bad);
+}
+
+// Copy n doubles and clear the counter (the RK4 reads its neighbours' old fields,
+// so it cannot run in place).
+__global__ __launch_bounds__(256) void fke_rk4_copy_kernel(const double* __restrict__ src, double* __restrict__ dst,
+                                                           int64_t n, unsigned long long* n_bad)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) *n_bad = 0ull;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) dst[i] = src[i];
 }
 
 bool fke_rk_args(int ns, int L, const tm_fke_rk_params* p, FkeRk* c)
@@ -498,23 +555,17 @@ bool fke_rk_args(int ns, int L, const tm_fke_rk_params* p, FkeRk* c)
     return true;
 }
 
-// The four stage launches on stream st; scratch holds 3 NF L^2 doubles.
+// One step in place on stream st; scratch holds (ns + 3) L^2 doubles.
 void fke_rk_launch(const FkeRk& c, double* fields, double* scratch, unsigned long long* n_bad, hipStream_t st)
 {
-    const int64_t L2 = (int64_t)c.L * c.L;
-    const int64_t nf = (int64_t)(c.ns + 3) * L2;
-    double *sa = scratch, *sb = scratch + nf, *acc = scratch + 2 * nf;
-    const dim3 grid((unsigned)((L2 + 255) / 256));
-    const double* src[4] = {fields, sa, sb, sa};
-    double* nxt[4] = {sa, sb, sa, nullptr};
-    for (int s = 1; s <= 4; ++s) {
-        if (c.ns == 1)
-            hipLaunchKernelGGL(fke_rk_stage_kernel<1>, grid, dim3(256), 0, st, c, s, fields, src[s - 1], nxt[s - 1], acc,
-                               n_bad);
-        else
-            hipLaunchKernelGGL(fke_rk_stage_kernel<2>, grid, dim3(256), 0, st, c, s, fields, src[s - 1], nxt[s - 1], acc,
-                               n_bad);
-    }
+    const int64_t n = (int64_t)(c.ns + 3) * c.L * c.L;
+    hipLaunchKernelGGL(fke_rk4_copy_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)), dim3(256), 0, st,
+                       fields, scratch, n, n_bad);
+    const unsigned t = (unsigned)((c.L + kRkTile - 1) / kRkTile);
+    if (c.ns == 1)
+        hipLaunchKernelGGL(fke_rk4_kernel<1>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad);
+    else
+        hipLaunchKernelGGL(fke_rk4_kernel<2>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad);
 }
 
 // ---------------------------------------------------------------------------
@@ -561,10 +612,9 @@ bool veg_dornic_ok(int L, const tm_rietkerk_params* p)
 //                          factor (fixed-order sums, FKE:4100-4112), per instance
 //   fke_percept            gamma of each consumer from the old densities
 //                          (FKE:4114-4118); velocities are drawn where used
-//   fke_veg                the vegetation's Dornic step P* (FKE:4150-4211), the
-//                          other densities carried into the output buffer
-//   fke_stage x 4          RK4 of the trophic and water terms (FKE:4233-4238),
-//                          one grid-wide pass per stage (W and O diffuse)
+//   fke_veg                the vegetation's Dornic step P* (FKE:4150-4211)
+//   fke_rk4_step           RK4 of the trophic and water terms (FKE:4233-4238) from
+//                          P* and the other old densities, into the output buffer
 //   fke_mprep, fke_move_pass x 3  the consumers' Fokker-Planck movement
 //                          (FKE:4276-4309), in separable form
 //   fke_final              checks and flush of the densities, rho(t) partials of
@@ -592,9 +642,8 @@ struct FkeWork {
     const int2* blocks;        // [nblocks]: (instance, first cell) of 256 cells
     const double* SD;          // movement stencils, offsets in MoveSpecies
     const double* SV;
-    double* sa;                // RK4 stage values, (SP + 2) fields at (SP + 2) cell_off
-    double* sb;
-    double* acc;
+    double* pstar;             // P* of the vegetation's Dornic step, at cell_off
+    const int4* rtiles;        // RK4 tiles: (instance, x0, y0, 0)
     double4* coef;             // movement terms, (SP - 1) fields at (SP - 1) cell_off
     int2* mu;
     double* mv;                // separable movement: planes cx, Y1, Y2, Z of each lattice (4 per
@@ -730,36 +779,29 @@ __global__ __launch_bounds__(256) void fke_veg_kernel(StepArgs a)
     const int L = di.L;
     const int64_t N = (int64_t)L * L;
     const double* fin = (const double*)a.in + (int64_t)NF * di.cell_off;
-    double* fout = (double*)a.out + (int64_t)NF * di.cell_off;
     const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + inst];
     const int y = cell / L, x = cell % L;
     const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
     const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
     double n;
     bool bad;
-    fout[cell] = cell_update<double, 1>(c, di, (uint32_t)cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
-#pragma unroll
-    for (int f = 1; f < SP + 2; ++f) fout[f * N + cell] = fin[f * N + cell];
+    w->pstar[di.cell_off + cell] =
+        cell_update<double, 1>(c, di, (uint32_t)cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
 }
 
+// RK4 of P* (FkeWork::pstar) and the other old densities into the output buffer.
 template <int SP>
-__global__ __launch_bounds__(256) void fke_stage_kernel(StepArgs a, int stage)
+__global__ __launch_bounds__(kRkThreads) void fke_rk4_step_kernel(StepArgs a)
 {
-    constexpr int NF = 2 * SP + 1, ND = SP + 2;
+    constexpr int NF = 2 * SP + 1;
+    __shared__ RkTileLds sm;
     const FkeWork* w = (const FkeWork*)a.work;
-    int inst, cell;
-    DevInst di;
-    if (!fke_cell(a, w, inst, cell, di)) return;
-    FkeRk c = w->mc[di.pidx].rk;
-    c.L = di.L;
+    const int4 tl = w->rtiles[blockIdx.x];   // (instance, x0, y0)
+    const DevInst di = a.inst[tl.x];
+    const FkeRk c = w->mc[di.pidx].rk;
     const int64_t N = (int64_t)di.L * di.L;
-    double* rho = (double*)a.out + (int64_t)NF * di.cell_off;
-    double* sa = w->sa + (int64_t)ND * di.cell_off;
-    double* sb = w->sb + (int64_t)ND * di.cell_off;
-    double* acc = w->acc + (int64_t)ND * di.cell_off;
-    const double* src = stage == 1 ? rho : (stage == 3 ? sb : sa);
-    double* nxt = stage == 2 ? sb : sa;   // unused by stage 4
-    (void)fke_stage_at<SP - 1>(c, stage, rho, src, nxt, acc, N, cell);
+    (void)fke_rk4_tile<SP - 1>(c, w->pstar + di.cell_off, (const double*)a.in + (int64_t)NF * di.cell_off,
+                               (double*)a.out + (int64_t)NF * di.cell_off, di.L, N, tl.z, tl.y, sm);
 }
 
 template <int SP>
@@ -863,7 +905,7 @@ void launch_fke(const StepArgs& a, int grid, hipStream_t s)
     hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL(fke_percept_kernel<SP>, blocks, dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_veg_kernel<SP>, blocks, dim3(256), 0, s, a);
-    for (int st = 1; st <= 4; ++st) hipLaunchKernelGGL(fke_stage_kernel<SP>, blocks, dim3(256), 0, s, a, st);
+    hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
     hipLaunchKernelGGL(fke_mprep_kernel<SP>, moves, dim3(256), 0, s, a);
     hipLaunchKernelGGL((fke_move_pass_kernel<SP, 0>), moves, dim3(256), 0, s, a);
     hipLaunchKernelGGL((fke_move_pass_kernel<SP, 1>), moves, dim3(256), 0, s, a);
@@ -1003,7 +1045,7 @@ void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t
 }
 
 int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance_desc* inst, int n_inst,
-              const int64_t* cell_off, int64_t total_cells, void** work, int* nchunks, int* nblocks,
+              const int64_t* cell_off, int64_t total_cells, void** work, int* nchunks, int* nblocks, int* nrtiles,
               const char** err)
 {
     const int SP = model == TM_MODEL_FKE3 ? 3 : 2, ns = SP - 1;
@@ -1069,6 +1111,7 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     }
     std::vector<DPCInstInfo> info((size_t)n_inst);
     std::vector<int2> chunks, blocks;
+    std::vector<int4> rtiles;
     for (int i = 0; i < n_inst; ++i) {
         const tm_instance_desc& d = inst[i];
         const tm_fke_params& p = P[d.params_index];
@@ -1092,9 +1135,11 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
         in.nchunks = (int)((cells + kFkeChunkCells - 1) / kFkeChunkCells);
         for (int k = 0; k < in.nchunks; ++k) chunks.push_back(make_int2(i, k));
         for (int64_t c0 = 0; c0 < cells; c0 += 256) blocks.push_back(make_int2(i, (int)c0));
+        for (int y0 = 0; y0 < d.L; y0 += kRkTile)
+            for (int x0 = 0; x0 < d.L; x0 += kRkTile) rtiles.push_back(make_int4(i, x0, y0, 0));
     }
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t nd = (size_t)(SP + 2) * total_cells, nm = (size_t)ns * total_cells;
+    const size_t nm = (size_t)ns * total_cells;
     size_t o = up(sizeof(FkeWork));
     const size_t o_mc = o;     o += up(sizeof(FkeModelConst) * mc.size());
     const size_t o_info = o;   o += up(sizeof(DPCInstInfo) * info.size());
@@ -1103,13 +1148,12 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     const size_t o_chunks = o; o += up(sizeof(int2) * chunks.size());
     const size_t o_disk = o;   o += up(sizeof(int2) * disk.size());
     const size_t o_blocks = o; o += up(sizeof(int2) * blocks.size());
+    const size_t o_rtiles = o; o += up(sizeof(int4) * rtiles.size());
     const size_t o_sd = o;     o += up(sizeof(double) * SD.size());
     const size_t o_sv = o;     o += up(sizeof(double) * SV.size());
     const size_t o_mstat = o;  o += up(sizeof(double) * 8 * info.size());
     const size_t o_tables = o;   // everything above is uploaded; the scratch below is not
-    const size_t o_sa = o;     o += up(sizeof(double) * nd);
-    const size_t o_sb = o;     o += up(sizeof(double) * nd);
-    const size_t o_acc = o;    o += up(sizeof(double) * nd);
+    const size_t o_pstar = o;  o += up(sizeof(double) * (size_t)total_cells);
     const size_t o_coef = o;   o += up(sizeof(double4) * nm);
     const size_t o_mu = o;     o += up(sizeof(int2) * nm);
     const size_t o_mv = o;     o += up(sizeof(double) * 4 * nm);
@@ -1131,9 +1175,8 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     w.SD = (const double*)(base + o_sd);
     w.SV = (const double*)(base + o_sv);
     w.mstat = (double*)(base + o_mstat);
-    w.sa = (double*)(base + o_sa);
-    w.sb = (double*)(base + o_sb);
-    w.acc = (double*)(base + o_acc);
+    w.pstar = (double*)(base + o_pstar);
+    w.rtiles = (const int4*)(base + o_rtiles);
     w.coef = (double4*)(base + o_coef);
     w.mu = (int2*)(base + o_mu);
     w.mv = (double*)(base + o_mv);
@@ -1146,6 +1189,7 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     put(o_chunks, chunks.data(), sizeof(int2) * chunks.size());
     put(o_disk, disk.data(), sizeof(int2) * disk.size());
     put(o_blocks, blocks.data(), sizeof(int2) * blocks.size());
+    put(o_rtiles, rtiles.data(), sizeof(int4) * rtiles.size());
     put(o_sd, SD.data(), sizeof(double) * SD.size());
     put(o_sv, SV.data(), sizeof(double) * SV.size());
     if (hipMemcpy(dev, host.data(), o_tables, hipMemcpyHostToDevice) != hipSuccess) {
@@ -1156,6 +1200,7 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     *work = dev;
     *nchunks = (int)chunks.size();
     *nblocks = (int)blocks.size();
+    *nrtiles = (int)rtiles.size();
     return TM_OK;
 }
 
@@ -1336,11 +1381,10 @@ int tm_fke_rk4(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t
     const hipStream_t st = (hipStream_t)stream;
     const size_t nf = (size_t)(ns + 3) * L * L;
     DevBuf d_s, d_bad;
-    if (hipMalloc(&d_s.p, sizeof(double) * 3 * nf) != hipSuccess ||
+    if (hipMalloc(&d_s.p, sizeof(double) * nf) != hipSuccess ||
         hipMalloc(&d_bad.p, sizeof(unsigned long long)) != hipSuccess)
         return TM_ERR_NOMEM;
     unsigned long long bad = 0;
-    if (hipMemcpyAsync(d_bad.p, &bad, sizeof(bad), hipMemcpyHostToDevice, st) != hipSuccess) return TM_ERR_HIP;
     fke_rk_launch(c, fields, (double*)d_s.p, (unsigned long long*)d_bad.p, st);
     if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
     // the scratch is freed on return: wait for the stages that use it
@@ -1352,7 +1396,7 @@ int tm_fke_rk4(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t
 }
 
 // ---------------------------------------------------------------------------
-// tm_fke_rk4_noalloc: tm_fke_rk4 with its stage buffers and its negative-value
+// tm_fke_rk4_noalloc: tm_fke_rk4 with its copy of the fields and its negative-value
 // counter in `scratch`, a file-scope device array, instead of per-call device
 // allocations.  Each GPU the library runs on holds its own copy until the
 // process ends.  In host code the name is only a handle: the array's device
@@ -1362,7 +1406,7 @@ int tm_fke_rk4(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t
 // counter is cleared by a kernel at the start of each call.
 // ---------------------------------------------------------------------------
 constexpr int kRk4NoAllocL = 256;            // largest lattice side (ns <= 2 consumers)
-constexpr size_t kRk4ScratchDoubles = 3 * 5 * (size_t)kRk4NoAllocL * kRk4NoAllocL;   // 3 (ns + 3) L^2
+constexpr size_t kRk4ScratchDoubles = 5 * (size_t)kRk4NoAllocL * kRk4NoAllocL;   // (ns + 3) L^2
 static __device__ __align__(256) double scratch[kRk4ScratchDoubles + 1];             // + the counter
 
 constexpr int kMaxDevices = 64;
@@ -1382,11 +1426,6 @@ static double* rk4_scratch(int dev)
     return g_scratch_ptr[dev];
 }
 
-__global__ void clear_counter_kernel(unsigned long long* n)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *n = 0ull;
-}
-
 int tm_fke_rk4_noalloc(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t* n_bad, void* stream)
 {
     FkeRk c;
@@ -1398,7 +1437,6 @@ int tm_fke_rk4_noalloc(int ns, int L, const tm_fke_rk_params* p, double* fields,
     if (!s) return TM_ERR_HIP;
     unsigned long long* d_bad = (unsigned long long*)(s + kRk4ScratchDoubles);
     const hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(clear_counter_kernel, dim3(1), dim3(64), 0, st, d_bad);
     fke_rk_launch(c, fields, s, d_bad, st);
     if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
     unsigned long long bad = 0;
@@ -1417,13 +1455,11 @@ int tm_fke_rk4_host(int device, int ns, int L, const tm_fke_rk_params* p, double
     const size_t nf = (size_t)(ns + 3) * L * L;
     DevBuf d_f, d_s, d_bad;
     if (hipMalloc(&d_f.p, sizeof(double) * nf) != hipSuccess ||
-        hipMalloc(&d_s.p, sizeof(double) * 3 * nf) != hipSuccess ||
+        hipMalloc(&d_s.p, sizeof(double) * nf) != hipSuccess ||
         hipMalloc(&d_bad.p, sizeof(unsigned long long)) != hipSuccess)
         return TM_ERR_NOMEM;
     unsigned long long bad = 0;
-    if (hipMemcpy(d_f.p, fields, sizeof(double) * nf, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(d_bad.p, &bad, sizeof(bad), hipMemcpyHostToDevice) != hipSuccess)
-        return TM_ERR_HIP;
+    if (hipMemcpy(d_f.p, fields, sizeof(double) * nf, hipMemcpyHostToDevice) != hipSuccess) return TM_ERR_HIP;
     fke_rk_launch(c, (double*)d_f.p, (double*)d_s.p, (unsigned long long*)d_bad.p, nullptr);
     if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
     if (hipMemcpy(fields, d_f.p, sizeof(double) * nf, hipMemcpyDeviceToHost) != hipSuccess ||
