@@ -104,3 +104,24 @@ def test_fke_perception_bit_exact(tm, oracle, ns):
     g1, v1 = tm.fke_perception(rho, gam, veff, pR, dx, v, seed=9, inst=3, step=17)
     g2, v2 = oracle.fke_perception(rho, gam, veff, pR, dx, v, seed=9, inst=3, step=17)
     assert np.array_equal(g1, g2) and np.array_equal(v1, v2)
+
+
+@pytest.mark.parametrize("L,rD,rV,shift", [(5, 1, 0, 0.4), (23, 9, 1, 0.4), (64, 3, 1, 0.9), (65, 9, 2, 2.6), (97, 0, 0, 5.2),
+                                           (129, 30, 1, 0.4), (97, 45, 1, 0.4), (83, 2, 31, 3.0), (70, 1, 1, 30.0)])
+def test_movement_reaches_and_tile_edges(tm, oracle, L, rD, rV, shift):
+    """One lattice at the edges of the 64 x 16 movement tile (one cell past it, smaller
+    than it), with wide diffusion or advection stencils and long shifts: those whose
+    frame fits LDS in two launches, the others (45 sites; shifts of 30) in four passes.
+    Bit for bit the oracle's separable form."""
+    rng = np.random.default_rng(L + rD)
+    rho = rng.uniform(0, 2, (L, L)) * (rng.random((L, L)) < 0.6)
+    gam = rng.random((L, L))
+    th = 2 * np.pi * rng.random((L, L))
+    vx, vy = np.cos(th), np.sin(th)
+    vmax = max(np.abs(vx).max(), np.abs(vy).max())
+    pref = shift / vmax
+    SD, SV = np.exp(-np.arange(rD + 1) / 5.0), np.exp(-np.arange(rV + 1) / 3.0)
+    S = oracle.fke_shift_reach(pref, vmax)
+    print(f"movement L {L} rD {rD} rV {rV} S {S}", flush=True)
+    got = tm.fke_movement(rho[None], gam[None], np.stack([vx, vy], -1)[None], [(rD, rV, pref)], [SD], [SV])
+    assert np.array_equal(got[0], oracle.fke_movement_sep(rho, gam, vx, vy, rD, rV, S, pref, SD, SV))

@@ -116,8 +116,7 @@ struct tm_ctx {
     void* d_dpc = nullptr;
     int dpc_nchunks = 0;
     int dpc_halo = 1;
-    int fke_nblocks = 0;           // Rietkerk consumer models: 256-cell blocks (FkeWork in d_dpc)
-    int fke_nrtiles = 0;           // ... and RK4 tiles
+    FkeGrid fke = {};              // Rietkerk consumer models: launch sizes (FkeWork in d_dpc)
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
 };
 
@@ -255,8 +254,7 @@ void release_config(tm_ctx* c)
     free_dev(c->d_mov);
     c->dpc_nchunks = 0;
     c->dpc_halo = 1;
-    c->fke_nblocks = 0;
-    c->fke_nrtiles = 0;
+    c->fke = FkeGrid{};
     invalidate_live(c);
     c->series_cap = c->groups_cap = c->stats_cap = c->frame_tab_cap = 0;
     c->series_steps_cap = c->n_series = 0;
@@ -355,8 +353,10 @@ StepArgs step_args(tm_ctx* c, int parity, int k)
     a.work = c->d_dpc;
     a.nchunks = c->dpc_nchunks;
     a.halo = c->dpc_halo;
-    a.nblocks = c->fke_nblocks;
-    a.nrtiles = c->fke_nrtiles;
+    a.nblocks = c->fke.blocks;
+    a.nrtiles = c->fke.rtiles;
+    a.nmtiles = c->fke.mtiles;
+    a.move_lds = c->fke.move_lds;
     return a;
 }
 
@@ -794,6 +794,7 @@ void tm_destroy(tm_ctx* c)
     if (!c) return;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
+    workspace_give_back();
     release_config(c);
     free_dev(c->d_state);
     if (c->h_pinned) hipHostFree(c->h_pinned);
@@ -892,8 +893,8 @@ tm_status tm_configure(tm_ctx* c, int model, int precision, const void* params, 
     if (is_fke_model(model)) {
         const char* err = "";
         const int rc = fke_setup(model, (const tm_fke_params*)c->params.data(), n_params, c->inst.data(), n_inst,
-                                 c->cell_off.data(), c->total_cells, &c->d_dpc, &c->dpc_nchunks, &c->fke_nblocks,
-                                 &c->fke_nrtiles, &err);
+                                 c->cell_off.data(), c->total_cells, &c->d_dpc, &c->fke, &err);
+        c->dpc_nchunks = c->fke.chunks;
         if (rc != TM_OK) {
             const std::string msg = err;
             release_config(c);

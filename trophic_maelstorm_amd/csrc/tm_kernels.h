@@ -82,6 +82,8 @@ struct StepArgs {
     int32_t halo;        // consumer models: LDS halo (largest perception radius, >= 1)
     int32_t nblocks;     // Rietkerk consumer models: 256-cell blocks of the batch
     int32_t nrtiles;     // Rietkerk consumer models: RK4 tiles of the batch
+    int32_t nmtiles;     // ... movement tiles
+    int32_t move_lds;    // ... and the movement tile's LDS bytes (0: the four-pass movement)
 };
 
 // Periodic index: v mod L in [0, L).

@@ -75,11 +75,18 @@ inline size_t dpc_lds_bytes(int ns, int tx, int ty, int halo)
 // Returns TM_OK, or a tm_status with *err naming the problem.
 const Variant* fke2_variants_f64(int* n);
 const Variant* fke3_variants_f64(int* n);
+struct FkeGrid {
+    int chunks, blocks;     // statistics chunks; 256-cell blocks
+    int rtiles, mtiles;     // RK4 and movement tiles
+    int move_lds;           // LDS bytes of the movement tile; 0: the four-pass movement
+};
 int fke_setup(int model, const tm_fke_params* params, int n_params, const tm_instance_desc* inst, int n_inst,
-              const int64_t* cell_off, int64_t total_cells, void** work, int* nchunks, int* nblocks, int* nrtiles,
-              const char** err);
+              const int64_t* cell_off, int64_t total_cells, void** work, FkeGrid* grid, const char** err);
 // Movement statistics of the current fields into out [n_inst][4 SpB] (device).
 void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t s);
+
+// Free the device scratch the Rietkerk consumer operators keep between calls.
+void workspace_give_back();
 
 // Default variant index per (model, precision, batch size in cells).
 int default_variant(int model, int precision, int64_t total_cells);

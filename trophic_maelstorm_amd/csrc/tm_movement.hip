@@ -34,6 +34,14 @@ namespace {
 
 constexpr double kMoveEps = 1.0e-10;   // epsilon, rietkerk_bjork_basic.h:119
 
+struct DevBuf {
+    void* p = nullptr;
+    ~DevBuf()
+    {
+        if (p) (void)hipFree(p);
+    }
+};
+
 struct MoveSpecies {
     int rD, rV, W, S, offD, offV;   // S: the largest shift of an advected mean, plus one
     double pref;
@@ -49,10 +57,17 @@ __device__ __forceinline__ int wrapi(int v, int L)
     return v < 0 ? v + L : v;
 }
 
+// v in [-L, 2L) -> v mod L
+__device__ __forceinline__ int wrap1(int v, int L)
+{
+    v += v < 0 ? L : 0;
+    return v >= L ? v - L : v;
+}
+
 // Per source cell: its three term coefficients (gamma^2 rho, (gamma - gamma^2) rho,
 // (1 - gamma)^2 rho, formed as the reference forms them) and its advected mean
 // cell, once per call; mu.x = -1 marks a source below the 1e-10 floor.
-__device__ __forceinline__ void move_prep_at(double pref, int L, int64_t i, double r, double g, double2 v,
+__device__ __forceinline__ void move_prep_at(double pref, int L, int ci, int cj, double r, double g, double2 v,
                                              double4& coef, int2& mu)
 {
 #pragma clang fp contract(off)
@@ -60,9 +75,9 @@ __device__ __forceinline__ void move_prep_at(double pref, int L, int64_t i, doub
         mu = make_int2(-1, -1);
         return;
     }
-    const int ci = (int)(i / L), cj = (int)(i % L);
-    const int mux = (int)(__builtin_round(ci + v.x * (pref)) + L) % L;
-    const int muy = (int)(__builtin_round(cj + v.y * (pref)) + L) % L;
+    // a shift is under L / 2 (2 W + 1 <= L), so one wrap either way is the remainder
+    const int mux = wrap1((int)__builtin_round(ci + v.x * (pref)), L);
+    const int muy = wrap1((int)__builtin_round(cj + v.y * (pref)), L);
     const double g2 = g * g;
     coef = make_double4((g2) * r, (g - g2) * r, (1 - g) * (1 - g) * r, 0.0);
     mu = make_int2(mux, muy);
@@ -79,15 +94,8 @@ __global__ __launch_bounds__(256) void fke_move_prep_kernel(MoveArgs a, const do
     const int64_t L2 = (int64_t)L * L;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= L2) return;
-    move_prep_at(a.sp[s].pref, L, i, rho[s * L2 + i], gamma[s * L2 + i], veff[s * L2 + i], coef[s * L2 + i],
+    move_prep_at(a.sp[s].pref, L, (int)(i / L), (int)(i % L), rho[s * L2 + i], gamma[s * L2 + i], veff[s * L2 + i], coef[s * L2 + i],
                  mu[s * L2 + i]);
-}
-
-// v in [-L, 2L) -> v mod L
-__device__ __forceinline__ int wrap1(int v, int L)
-{
-    v += v < 0 ? L : 0;
-    return v >= L ? v - L : v;
 }
 
 // The separable form, in three passes over one species' lattice.  With each
@@ -170,6 +178,199 @@ __device__ __forceinline__ void put4(double* __restrict__ planes, int64_t N, int
     planes[3 * N + o] = v.w;
 }
 
+// The movement in two launches, for reaches whose tile frame fits LDS
+// (move_tile_lds): the source terms, the shift sums and the row stencils of a
+// kMoveTX x kMoveTY tile in one workgroup (move_rows_tile: the frame of sources in
+// LDS, then the four planes of its rows, then P and Q to memory), and the column
+// stencils with several rows a thread (move_cols_tile).  The four passes moved each
+// source's terms (40 B) and the planes through memory and read every tap through the
+// caches; here a source is read with a 1.5-fold overlap (the frame is S rows and R + S
+// columns wider than the tile, R = max(rD, rV)) and the taps come from LDS or
+// registers.  Every sum keeps its terms and order (move_disp_at, move_row_at,
+// move_col_at), so the result is the passes' bit for bit.
+constexpr int kMoveTX = 64, kMoveTY = 16, kMoveRows = 512, kMoveCols = 256;
+constexpr int kMoveRPT = kMoveTY / (kMoveCols / 64);   // rows a thread of the column pass
+constexpr size_t kMoveLdsMax = 128 * 1024;
+
+__host__ __device__ inline size_t move_tile_lds(const MoveSpecies& sp)
+{
+    const size_t R = (size_t)(sp.rD > sp.rV ? sp.rD : sp.rV), S = (size_t)sp.S;
+    return (kMoveTY + 2 * S) * (kMoveTX + 2 * (R + S)) * (2 * sizeof(double) + sizeof(uint32_t)) + 8 +
+           kMoveTY * (kMoveTX + 2 * R) * 4 * sizeof(double);
+}
+
+// e / w and e % w for e < 2^13 and w <= 2^9 (magic = ceil(2^22 / w), once per workgroup).
+struct FrameDiv {
+    uint32_t w, magic;
+    __device__ __forceinline__ explicit FrameDiv(uint32_t w_) : w(w_), magic((0x400000u + w_ - 1) / w_) {}
+    __device__ __forceinline__ void split(uint32_t e, int& r, int& c) const
+    {
+        const uint32_t q = (e * magic) >> 22;
+        r = (int)q;
+        c = (int)(e - q * w);
+    }
+};
+
+// src(i, r, g, v): the density, gamma and velocity of source cell i.  pq: the planes P
+// and Q of this lattice, N apart.
+template <class Src>
+__device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const double* __restrict__ SD,
+                                               const double* __restrict__ SV, int L, int64_t N, int x0, int y0,
+                                               const Src& src, double* __restrict__ pq, double* lds)
+{
+#pragma clang fp contract(off)
+    const int S = sp.S, R = sp.rD > sp.rV ? sp.rD : sp.rV;
+    const int tw = min(kMoveTX, L - x0), th = min(kMoveTY, L - y0);
+    const int aw = tw + 2 * (R + S), ah = th + 2 * S, mw = tw + 2 * R;
+    const int na = ah * aw, nm = th * mw;
+    double* const cx = lds;                 // planes of the tile's rows, mw wide: c.x of the sources,
+    double* const y1 = cx + nm;             // and the shift sums
+    double* const y2 = y1 + nm;
+    double* const zz = y2 + nm;
+    double* const cy = zz + nm;             // frame of sources, aw wide
+    double* const cz = cy + na;
+    uint32_t* const mu = (uint32_t*)(cz + na);   // (my << 16) | mx, all ones where empty: L <= 46340
+    {
+        const FrameDiv d((uint32_t)aw);
+#pragma unroll 1
+        for (int e = threadIdx.x; e < na; e += kMoveRows) {
+            int r, c;
+            d.split((uint32_t)e, r, c);
+            const int p = tmk::wrap(y0 + r - S, L), q = tmk::wrap(x0 + c - S - R, L);
+            const int64_t i = (int64_t)p * L + q;
+            double rho, g;
+            double2 v;
+            src(i, rho, g, v);
+            double4 coef = make_double4(0.0, 0.0, 0.0, 0.0);
+            int2 m;
+            move_prep_at(sp.pref, L, p, q, rho, g, v, coef, m);
+            cy[e] = coef.y;
+            cz[e] = coef.z;
+            mu[e] = m.x < 0 ? 0xFFFFFFFFu : ((uint32_t)m.y << 16) | (uint32_t)m.x;
+            const int mr = r - S, mc = c - S;
+            if (mr >= 0 && mr < th && mc >= 0 && mc < mw) cx[mr * mw + mc] = m.x < 0 ? 0.0 : coef.x;
+        }
+    }
+    __syncthreads();
+    const FrameDiv dm((uint32_t)mw);
+#pragma unroll 1
+    for (int e = threadIdx.x; e < nm; e += kMoveRows) {
+        int r, c;
+        dm.split((uint32_t)e, r, c);
+        const uint32_t p = (uint32_t)(y0 + r), q = (uint32_t)tmk::wrap(x0 + c - R, L);
+        const uint32_t both = (q << 16) | p;
+        const int o = (r + S) * aw + (c + S);
+        double a1 = 0.0, a2 = 0.0, z = 0.0;
+        auto at = [&](int di, int dj) {              // (an empty source's key matches no cell)
+            const int i = o + di * aw + dj;
+            const uint32_t m = mu[i];
+            if (di == 0 && (m >> 16) == q) a1 += cy[i];       // this row's sources landing on column q,
+            if (dj == 0 && (m & 0xFFFFu) == p) a2 += cy[i];   // this column's landing on row p,
+            if (m == both) z += cz[i];                        // and every source landing on (p, q)
+        };
+        if (S == 1) {   // the usual reach, its nine keys read together
+#pragma unroll
+            for (int di = -1; di <= 1; ++di)
+#pragma unroll
+                for (int dj = -1; dj <= 1; ++dj) at(di, dj);
+        } else {
+            for (int di = -S; di <= S; ++di)
+                for (int dj = -S; dj <= S; ++dj) at(di, dj);
+        }
+        y1[e] = a1;
+        y2[e] = a2;
+        zz[e] = z;
+    }
+    __syncthreads();
+    const FrameDiv dt((uint32_t)tw);
+#pragma unroll 1
+    for (int e = threadIdx.x; e < th * tw; e += kMoveRows) {
+        int r, c;
+        dt.split((uint32_t)e, r, c);
+        const int o = r * mw + c + R;
+        double P = 0.0, Q = 0.0;
+#pragma unroll 4
+        for (int b = -sp.rD; b <= sp.rD; ++b) {
+            const double w = SD[b < 0 ? -b : b];
+            P += w * cx[o - b];
+            Q += w * y2[o - b];
+        }
+        for (int b = -sp.rV; b <= sp.rV; ++b) {
+            const double w = SV[b < 0 ? -b : b];
+            P += w * y1[o - b];
+            Q += w * zz[o - b];
+        }
+        const int64_t i = (int64_t)(y0 + r) * L + (x0 + c);
+        pq[i] = P;
+        pq[N + i] = Q;
+    }
+}
+
+// The column stencils of kMoveRPT consecutive rows x of column y, each output's terms
+// in move_col_at's order (a ascending: source rows descending); a source row is read
+// once for all the outputs it enters.
+__device__ __forceinline__ void move_cols_tile(const MoveSpecies& sp, const double* __restrict__ SD,
+                                               const double* __restrict__ SV, int L, int64_t N, int x, int y,
+                                               const double* __restrict__ pq, double (&acc)[kMoveRPT])
+{
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int j = 0; j < kMoveRPT; ++j) acc[j] = 0.0;
+    auto pass = [&](const double* __restrict__ plane, const double* __restrict__ W, int r) {
+        int row = tmk::wrap(x + kMoveRPT - 1 + r, L);
+        for (int k = kMoveRPT - 1 + r; k >= -r; --k) {
+            const double v = plane[(int64_t)row * L + y];
+            row = row == 0 ? L - 1 : row - 1;
+#pragma unroll
+            for (int j = 0; j < kMoveRPT; ++j) {
+                const int a = j - k;
+                if (a >= -r && a <= r) acc[j] += W[a < 0 ? -a : a] * v;
+            }
+        }
+    };
+    pass(pq, SD, sp.rD);
+    pass(pq + N, SV, sp.rV);
+}
+
+// The device-array operator in two launches; blockIdx.z = species.
+__global__ __launch_bounds__(kMoveRows) void fke_move_rows_kernel(MoveArgs a, const double* __restrict__ rho,
+                                                                  const double* __restrict__ gamma,
+                                                                  const double2* __restrict__ veff,
+                                                                  const double* __restrict__ SDall,
+                                                                  const double* __restrict__ SVall,
+                                                                  double* __restrict__ pq)
+{
+    extern __shared__ __align__(16) double s_move[];
+    const int s = blockIdx.z;
+    const int64_t N = (int64_t)a.L * a.L;
+    const MoveSpecies sp = a.sp[s];
+    auto src = [&](int64_t i, double& r, double& g, double2& v) {
+        r = rho[s * N + i];
+        g = gamma[s * N + i];
+        v = veff[s * N + i];
+    };
+    move_rows_tile(sp, SDall + sp.offD, SVall + sp.offV, a.L, N, (int)blockIdx.x * kMoveTX, (int)blockIdx.y * kMoveTY,
+                   src, pq + 2 * s * N, s_move);
+}
+
+__global__ __launch_bounds__(kMoveCols) void fke_move_cols_kernel(MoveArgs a, const double* __restrict__ pq,
+                                                                  const double* __restrict__ SDall,
+                                                                  const double* __restrict__ SVall,
+                                                                  double* __restrict__ out)
+{
+    const int s = blockIdx.z, L = a.L;
+    const int64_t N = (int64_t)L * L;
+    const MoveSpecies sp = a.sp[s];
+    const int y = (int)blockIdx.x * kMoveTX + (int)(threadIdx.x & 63);
+    const int x = (int)blockIdx.y * kMoveTY + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kMoveRPT;
+    if (x >= L || y >= L) return;
+    double acc[kMoveRPT];
+    move_cols_tile(sp, SDall + sp.offD, SVall + sp.offV, L, N, x, y, pq + 2 * s * N, acc);
+#pragma unroll
+    for (int j = 0; j < kMoveRPT; ++j)
+        if (x + j < L) out[s * N + (int64_t)(x + j) * L + y] = acc[j];
+}
+
 // The three passes of the host-array operator: one thread per (cell, species).
 // mv: 4 planes per species, pq: 2 planes per species.
 __global__ __launch_bounds__(256) void fke_move_disp_kernel(MoveArgs a, const double4* __restrict__ coef,
@@ -213,28 +414,31 @@ __global__ __launch_bounds__(256) void fke_move_col_kernel(MoveArgs a, const dou
                                   (int)(o / L), (int)(o % L));
 }
 
-// The largest |vx|, |vy| of each species (one workgroup per species); a NaN or
-// infinite velocity gives +inf, which the host refuses.
+// The largest |vx|, |vy| of each species, by workgroup: out[s * gridDim.x + block]; a
+// NaN or infinite velocity gives +inf, which the host refuses.  Two species of 1024^2:
+// 9 us with 256 workgroups each, 1573 with one.
 __global__ __launch_bounds__(256) void vmax_kernel(const double2* __restrict__ veff, int64_t L2, double* out)
 {
-    __shared__ double red[256];
-    const int s = blockIdx.x;
+    __shared__ double red[4];
+    const int s = blockIdx.y;
     double m = 0.0;
-    for (int64_t i = threadIdx.x; i < L2; i += 256) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < L2; i += (int64_t)gridDim.x * 256) {
         const double2 v = veff[s * L2 + i];
         const double a = __builtin_fabs(v.x), b = __builtin_fabs(v.y);
         double c = a > b ? a : b;
         if (!(a <= 1e300) || !(b <= 1e300)) c = __builtin_inf();   // NaN or infinite
         m = c > m ? c : m;
     }
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] = red[threadIdx.x] > red[threadIdx.x + o] ? red[threadIdx.x]
-                                                                                         : red[threadIdx.x + o];
-        __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) {
+        const double q = __shfl_xor(m, o);
+        m = q > m ? q : m;
     }
-    if (threadIdx.x == 0) out[s] = red[0];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; ++k) m = red[k] > m ? red[k] : m;
+        out[(int64_t)s * gridDim.x + blockIdx.x] = m;
+    }
 }
 
 // Kernel arguments of ns species from their constants and largest speeds; the
@@ -265,6 +469,47 @@ int move_args(int ns, int L, const tm_fke_move_species* sp, const double* vmax, 
     *nD = offD;
     *nV = offV;
     return TM_OK;
+}
+
+// Buffers of the four-pass movement, for reaches past the tile frame.
+struct MovePassBufs {
+    DevBuf coef, mu, mv;
+    bool get(size_t cells)
+    {
+        return hipMalloc(&coef.p, sizeof(double4) * cells) == hipSuccess &&
+               hipMalloc(&mu.p, sizeof(int2) * cells) == hipSuccess &&
+               hipMalloc(&mv.p, sizeof(double) * 4 * cells) == hipSuccess;
+    }
+};
+
+// The operator's launches on stream st: the two-launch form where every species' tile
+// frame fits LDS, else the four passes.  pq: 2 ns L^2 doubles; b is filled for the
+// passes and must outlive them.
+int move_launch(const MoveArgs& a, int ns, const double* rho, const double* gamma, const double* veff,
+                const double* SD, const double* SV, double* pq, double* out, MovePassBufs& b, hipStream_t st)
+{
+    const int64_t L2 = (int64_t)a.L * a.L;
+    size_t lds = 0;
+    for (int s = 0; s < ns; ++s) lds = std::max(lds, move_tile_lds(a.sp[s]));
+    if (lds <= kMoveLdsMax) {
+        if (lds > 65536 && hipFuncSetAttribute((const void*)fke_move_rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               (int)kMoveLdsMax) != hipSuccess)
+            return TM_ERR_HIP;
+        const dim3 grid((unsigned)((a.L + kMoveTX - 1) / kMoveTX), (unsigned)((a.L + kMoveTY - 1) / kMoveTY), (unsigned)ns);
+        hipLaunchKernelGGL(fke_move_rows_kernel, grid, dim3(kMoveRows), lds, st, a, rho, gamma, (const double2*)veff, SD, SV,
+                           pq);
+        hipLaunchKernelGGL(fke_move_cols_kernel, grid, dim3(kMoveCols), 0, st, a, (const double*)pq, SD, SV, out);
+    } else {
+        if (!b.get((size_t)ns * L2)) return TM_ERR_NOMEM;
+        const dim3 grid((unsigned)((L2 + 255) / 256), (unsigned)ns);
+        hipLaunchKernelGGL(fke_move_prep_kernel, grid, dim3(256), 0, st, a, rho, gamma, (const double2*)veff,
+                           (double4*)b.coef.p, (int2*)b.mu.p);
+        hipLaunchKernelGGL(fke_move_disp_kernel, grid, dim3(256), 0, st, a, (const double4*)b.coef.p,
+                           (const int2*)b.mu.p, (double*)b.mv.p);
+        hipLaunchKernelGGL(fke_move_row_kernel, grid, dim3(256), 0, st, a, (const double*)b.mv.p, SD, SV, pq);
+        hipLaunchKernelGGL(fke_move_col_kernel, grid, dim3(256), 0, st, a, (const double*)pq, SD, SV, out);
+    }
+    return hipGetLastError() == hipSuccess ? TM_OK : TM_ERR_HIP;
 }
 
 // Perception gamma and velocities (calc_gamma_vel_2Sp/3Sp_NonRefugia,
@@ -372,12 +617,91 @@ void gauss_stencil(double sigma, int R, double* st)
     for (int x = 0; x <= R; ++x) st[x] /= sum;
 }
 
-struct DevBuf {
-    void* p = nullptr;
-    ~DevBuf()
+// Device scratch of the operators, kept between calls: allocating and freeing it cost
+// tm_fke_movement 1.1 ms a call at 2 x 1024^2.  A call holds its block alone from
+// get() until it has waited for the kernels that use it (idle), so calls of several
+// threads and streams never share one; a block that is not known to be idle is freed,
+// which waits for the device.  At most kKeepTotal bytes in kKeepBlocks blocks stay,
+// the oldest going first; tm_destroy and a failed allocation give all of them back.
+class Workspace {
+public:
+    bool idle = true;
+    Workspace() = default;
+    Workspace(const Workspace&) = delete;
+    Workspace& operator=(const Workspace&) = delete;
+    ~Workspace()
     {
-        if (p) (void)hipFree(p);
+        if (!b_.p) return;
+        if (!idle || b_.bytes > kKeepTotal) {
+            (void)hipFree(b_.p);
+            return;
+        }
+        Pool& k = pool();
+        std::lock_guard<std::mutex> lock(k.mu);
+        k.v[k.n++] = b_;
+        size_t total = 0;
+        for (int i = 0; i < k.n; ++i) total += k.v[i].bytes;
+        while (total > kKeepTotal || k.n > kKeepBlocks) {
+            total -= k.v[0].bytes;
+            (void)hipFree(k.v[0].p);
+            k.erase(0);
+        }
     }
+    // A block of at least `bytes` on the current device.
+    bool get(size_t bytes)
+    {
+        int dev;
+        if (hipGetDevice(&dev) != hipSuccess) return false;
+        {
+            Pool& k = pool();
+            std::lock_guard<std::mutex> lock(k.mu);
+            for (int i = 0; i < k.n; ++i)
+                if (k.v[i].dev == dev && k.v[i].bytes >= bytes && k.v[i].bytes / 4 <= bytes) {
+                    b_ = k.v[i];
+                    k.erase(i);
+                    return true;
+                }
+        }
+        b_ = Block{nullptr, bytes, dev};
+        if (hipMalloc(&b_.p, bytes) == hipSuccess) return true;
+        (void)hipGetLastError();
+        give_back();
+        if (hipMalloc(&b_.p, bytes) == hipSuccess) return true;
+        b_.p = nullptr;
+        return false;
+    }
+    template <typename T> T* at(size_t offset) const { return (T*)((char*)b_.p + offset); }
+    static void give_back()
+    {
+        Pool& k = pool();
+        std::lock_guard<std::mutex> lock(k.mu);
+        for (int i = 0; i < k.n; ++i) (void)hipFree(k.v[i].p);
+        k.n = 0;
+    }
+
+private:
+    static constexpr size_t kKeepTotal = (size_t)128 << 20;
+    static constexpr int kKeepBlocks = 8;
+    struct Block {
+        void* p;
+        size_t bytes;
+        int dev;
+    };
+    struct Pool {
+        std::mutex mu;
+        Block v[kKeepBlocks + 1];
+        int n = 0;
+        void erase(int i)
+        {
+            for (--n; i < n; ++i) v[i] = v[i + 1];
+        }
+    };
+    static Pool& pool()
+    {
+        static Pool* p = new Pool();   // never destroyed: the process ends with its blocks
+        return *p;
+    }
+    Block b_ = {nullptr, 0, 0};
 };
 
 // ---------------------------------------------------------------------------
@@ -615,8 +939,9 @@ bool veg_dornic_ok(int L, const tm_rietkerk_params* p)
 //   fke_veg                the vegetation's Dornic step P* (FKE:4150-4211)
 //   fke_rk4_step           RK4 of the trophic and water terms (FKE:4233-4238) from
 //                          P* and the other old densities, into the output buffer
-//   fke_mprep, fke_move_pass x 3  the consumers' Fokker-Planck movement
-//                          (FKE:4276-4309), in separable form
+//   fke_move_rows_step, fke_move_cols_step  the consumers' Fokker-Planck movement
+//                          (FKE:4276-4309), in separable form; reaches past the tile
+//                          frame take fke_mprep and fke_move_pass x 3
 //   fke_final              checks and flush of the densities, rho(t) partials of
 //                          every field (FKE:4352-4462)
 // Every operation is the one the per-operator entry points (tm_fke_perception,
@@ -644,10 +969,11 @@ struct FkeWork {
     const double* SV;
     double* pstar;             // P* of the vegetation's Dornic step, at cell_off
     const int4* rtiles;        // RK4 tiles: (instance, x0, y0, 0)
-    double4* coef;             // movement terms, (SP - 1) fields at (SP - 1) cell_off
-    int2* mu;
-    double* mv;                // separable movement: planes cx, Y1, Y2, Z of each lattice (4 per
-    double* pq;                // coef entry, at 4 x its offset), then planes P, Q (2, at 2 x)
+    const int4* mtiles;        // movement tiles, the same
+    double* pq;                // movement: planes P, Q of each consumer's lattice, at 2 (SP - 1) cell_off
+    double4* coef;             // the four-pass movement's terms, (SP - 1) fields at (SP - 1) cell_off,
+    int2* mu;                  // and planes cx, Y1, Y2, Z of each lattice (4 per coef entry); null
+    double* mv;                // where the tile form runs
     double* mstat;             // [n_inst][8] means of the movement statistics
 };
 
@@ -823,7 +1149,7 @@ __global__ __launch_bounds__(256) void fke_mprep_kernel(StepArgs a)
         v = fke_velocity(di.seed, di.inst_id, (uint32_t)cell, step, s, mc.v[s]);
     }
     const int64_t j = (int64_t)(SP - 1) * di.cell_off + (s - 1) * N + cell;
-    move_prep_at(mc.ms[s - 1].pref, L, cell, f[s * N + cell], f[(SP + 1 + s) * N + cell], v, w->coef[j], w->mu[j]);
+    move_prep_at(mc.ms[s - 1].pref, L, cell / L, cell % L, f[s * N + cell], f[(SP + 1 + s) * N + cell], v, w->coef[j], w->mu[j]);
 }
 
 // The separable movement's passes (move_disp_at, move_row_at, move_col_at) on
@@ -852,6 +1178,55 @@ __global__ __launch_bounds__(256) void fke_move_pass_kernel(StepArgs a)
         double* f = (double*)a.out + (int64_t)NF * di.cell_off;
         f[s * N + cell] = move_col_at(w->pq + 2 * base, N, w->SD + sp.offD, w->SV + sp.offV, sp.rD, sp.rV, L, p, q);
     }
+}
+
+// The movement in two launches (move_rows_tile, move_cols_tile) on the batch's movement
+// tiles; blockIdx.y = consumer - 1.
+template <int SP>
+__global__ __launch_bounds__(kMoveRows) void fke_move_rows_step_kernel(StepArgs a)
+{
+    constexpr int NF = 2 * SP + 1;
+    extern __shared__ __align__(16) double s_move[];
+    const FkeWork* w = (const FkeWork*)a.work;
+    const int4 tl = w->mtiles[blockIdx.x];   // (instance, x0, y0)
+    const DevInst di = a.inst[tl.x];
+    const int s = blockIdx.y + 1, L = di.L;
+    const int64_t N = (int64_t)L * L;
+    const double* f = (const double*)a.out + (int64_t)NF * di.cell_off;
+    const FkeModelConst& mc = w->mc[di.pidx];
+    const MoveSpecies sp = mc.ms[s - 1];
+    const double vs = mc.v[s];
+    const int64_t step = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.x].step;
+    auto src = [&](int64_t i, double& r, double& g, double2& v) {
+        r = f[s * N + i];
+        g = f[(SP + 1 + s) * N + i];
+        v = make_double2(0.0, 0.0);   // the two-species step draws no velocity
+        if (SP == 3) v = fke_velocity(di.seed, di.inst_id, (uint32_t)i, step, s, vs);
+    };
+    move_rows_tile(sp, w->SD + sp.offD, w->SV + sp.offV, L, N, tl.y, tl.z, src,
+                   w->pq + 2 * ((int64_t)(SP - 1) * di.cell_off + (s - 1) * N), s_move);
+}
+
+template <int SP>
+__global__ __launch_bounds__(kMoveCols) void fke_move_cols_step_kernel(StepArgs a)
+{
+    constexpr int NF = 2 * SP + 1;
+    const FkeWork* w = (const FkeWork*)a.work;
+    const int4 tl = w->mtiles[blockIdx.x];
+    const DevInst di = a.inst[tl.x];
+    const int s = blockIdx.y + 1, L = di.L;
+    const int64_t N = (int64_t)L * L;
+    const MoveSpecies sp = w->mc[di.pidx].ms[s - 1];
+    const int y = tl.y + (int)(threadIdx.x & 63);
+    const int x = tl.z + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) * kMoveRPT;
+    if (x >= L || y >= L) return;
+    double acc[kMoveRPT];
+    move_cols_tile(sp, w->SD + sp.offD, w->SV + sp.offV, L, N, x, y,
+                   w->pq + 2 * ((int64_t)(SP - 1) * di.cell_off + (s - 1) * N), acc);
+    double* f = (double*)a.out + (int64_t)NF * di.cell_off + s * N;
+#pragma unroll
+    for (int j = 0; j < kMoveRPT; ++j)
+        if (x + j < L) f[(int64_t)(x + j) * L + y] = acc[j];
 }
 
 // Checks and flush of the densities (the perception fields are left as they
@@ -900,16 +1275,23 @@ __global__ __launch_bounds__(NT) void fke_final_kernel(StepArgs a)
 template <int SP, int TX, int TY, int NT>
 void launch_fke(const StepArgs& a, int grid, hipStream_t s)
 {
-    const dim3 blocks((unsigned)a.nblocks), moves((unsigned)a.nblocks, SP - 1);
+    const dim3 blocks((unsigned)a.nblocks);
     hipLaunchKernelGGL(fke_chunk_kernel<SP>, dim3(a.nchunks), dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL(fke_percept_kernel<SP>, blocks, dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_veg_kernel<SP>, blocks, dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
-    hipLaunchKernelGGL(fke_mprep_kernel<SP>, moves, dim3(256), 0, s, a);
-    hipLaunchKernelGGL((fke_move_pass_kernel<SP, 0>), moves, dim3(256), 0, s, a);
-    hipLaunchKernelGGL((fke_move_pass_kernel<SP, 1>), moves, dim3(256), 0, s, a);
-    hipLaunchKernelGGL((fke_move_pass_kernel<SP, 2>), moves, dim3(256), 0, s, a);
+    if (a.move_lds > 0) {
+        const dim3 tiles((unsigned)a.nmtiles, SP - 1);
+        hipLaunchKernelGGL(fke_move_rows_step_kernel<SP>, tiles, dim3(kMoveRows), (size_t)a.move_lds, s, a);
+        hipLaunchKernelGGL(fke_move_cols_step_kernel<SP>, tiles, dim3(kMoveCols), 0, s, a);
+    } else {   // a reach too wide for the tile frame
+        const dim3 moves((unsigned)a.nblocks, SP - 1);
+        hipLaunchKernelGGL(fke_mprep_kernel<SP>, moves, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((fke_move_pass_kernel<SP, 0>), moves, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((fke_move_pass_kernel<SP, 1>), moves, dim3(256), 0, s, a);
+        hipLaunchKernelGGL((fke_move_pass_kernel<SP, 2>), moves, dim3(256), 0, s, a);
+    }
     hipLaunchKernelGGL((fke_final_kernel<SP, TX, TY, NT>), dim3(grid), dim3(NT), 0, s, a);
 }
 
@@ -1045,8 +1427,7 @@ void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t
 }
 
 int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance_desc* inst, int n_inst,
-              const int64_t* cell_off, int64_t total_cells, void** work, int* nchunks, int* nblocks, int* nrtiles,
-              const char** err)
+              const int64_t* cell_off, int64_t total_cells, void** work, FkeGrid* grid, const char** err)
 {
     const int SP = model == TM_MODEL_FKE3 ? 3 : 2, ns = SP - 1;
     *work = nullptr;
@@ -1111,7 +1492,8 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     }
     std::vector<DPCInstInfo> info((size_t)n_inst);
     std::vector<int2> chunks, blocks;
-    std::vector<int4> rtiles;
+    std::vector<int4> rtiles, mtiles;
+    size_t lds = 0;   // of the movement tile, over every consumer of every point
     for (int i = 0; i < n_inst; ++i) {
         const tm_instance_desc& d = inst[i];
         const tm_fke_params& p = P[d.params_index];
@@ -1137,6 +1519,9 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
         for (int64_t c0 = 0; c0 < cells; c0 += 256) blocks.push_back(make_int2(i, (int)c0));
         for (int y0 = 0; y0 < d.L; y0 += kRkTile)
             for (int x0 = 0; x0 < d.L; x0 += kRkTile) rtiles.push_back(make_int4(i, x0, y0, 0));
+        for (int y0 = 0; y0 < d.L; y0 += kMoveTY)
+            for (int x0 = 0; x0 < d.L; x0 += kMoveTX) mtiles.push_back(make_int4(i, x0, y0, 0));
+        for (int s = 0; s < ns; ++s) lds = std::max(lds, move_tile_lds(m.ms[s]));
     }
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t nm = (size_t)ns * total_cells;
@@ -1149,15 +1534,23 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     const size_t o_disk = o;   o += up(sizeof(int2) * disk.size());
     const size_t o_blocks = o; o += up(sizeof(int2) * blocks.size());
     const size_t o_rtiles = o; o += up(sizeof(int4) * rtiles.size());
+    const size_t o_mtiles = o; o += up(sizeof(int4) * mtiles.size());
     const size_t o_sd = o;     o += up(sizeof(double) * SD.size());
     const size_t o_sv = o;     o += up(sizeof(double) * SV.size());
     const size_t o_mstat = o;  o += up(sizeof(double) * 8 * info.size());
     const size_t o_tables = o;   // everything above is uploaded; the scratch below is not
     const size_t o_pstar = o;  o += up(sizeof(double) * (size_t)total_cells);
-    const size_t o_coef = o;   o += up(sizeof(double4) * nm);
-    const size_t o_mu = o;     o += up(sizeof(int2) * nm);
-    const size_t o_mv = o;     o += up(sizeof(double) * 4 * nm);
     const size_t o_pq = o;     o += up(sizeof(double) * 2 * nm);
+    const bool passes = lds > kMoveLdsMax;
+    const size_t o_coef = o;   o += passes ? up(sizeof(double4) * nm) : 0;
+    const size_t o_mu = o;     o += passes ? up(sizeof(int2) * nm) : 0;
+    const size_t o_mv = o;     o += passes ? up(sizeof(double) * 4 * nm) : 0;
+    const void* rows = SP == 3 ? (const void*)fke_move_rows_step_kernel<3> : (const void*)fke_move_rows_step_kernel<2>;
+    if (!passes && lds > 65536 &&
+        hipFuncSetAttribute(rows, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMoveLdsMax) != hipSuccess) {
+        *err = "Rietkerk consumer movement: no LDS for its tile";
+        return TM_ERR_HIP;
+    }
     void* dev = nullptr;
     if (hipMalloc(&dev, o) != hipSuccess) {
         *err = "Rietkerk consumer tables and scratch: allocation failed";
@@ -1177,10 +1570,13 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     w.mstat = (double*)(base + o_mstat);
     w.pstar = (double*)(base + o_pstar);
     w.rtiles = (const int4*)(base + o_rtiles);
-    w.coef = (double4*)(base + o_coef);
-    w.mu = (int2*)(base + o_mu);
-    w.mv = (double*)(base + o_mv);
+    w.mtiles = (const int4*)(base + o_mtiles);
     w.pq = (double*)(base + o_pq);
+    if (passes) {
+        w.coef = (double4*)(base + o_coef);
+        w.mu = (int2*)(base + o_mu);
+        w.mv = (double*)(base + o_mv);
+    }
     std::vector<char> host(o_tables, 0);
     auto put = [&](size_t off, const void* src, size_t n) { if (n) std::memcpy(host.data() + off, src, n); };
     put(0, &w, sizeof(w));
@@ -1190,6 +1586,7 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     put(o_disk, disk.data(), sizeof(int2) * disk.size());
     put(o_blocks, blocks.data(), sizeof(int2) * blocks.size());
     put(o_rtiles, rtiles.data(), sizeof(int4) * rtiles.size());
+    put(o_mtiles, mtiles.data(), sizeof(int4) * mtiles.size());
     put(o_sd, SD.data(), sizeof(double) * SD.size());
     put(o_sv, SV.data(), sizeof(double) * SV.size());
     if (hipMemcpy(dev, host.data(), o_tables, hipMemcpyHostToDevice) != hipSuccess) {
@@ -1198,11 +1595,12 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
         return TM_ERR_HIP;
     }
     *work = dev;
-    *nchunks = (int)chunks.size();
-    *nblocks = (int)blocks.size();
-    *nrtiles = (int)rtiles.size();
+    *grid = FkeGrid{(int)chunks.size(), (int)blocks.size(), (int)rtiles.size(), (int)mtiles.size(),
+                    passes ? 0 : (int)lds};
     return TM_OK;
 }
+
+void workspace_give_back() { Workspace::give_back(); }
 
 }  // namespace tmk
 
@@ -1240,35 +1638,33 @@ int tm_fke_movement(int ns, int L, const tm_fke_move_species* sp, const double* 
     const int64_t L2 = (int64_t)L * L;
     if (L2 > 0x7FFFFFFFll) return TM_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
-    DevBuf d_vmax;
-    if (hipMalloc(&d_vmax.p, sizeof(double) * ns) != hipSuccess) return TM_ERR_NOMEM;
-    hipLaunchKernelGGL(vmax_kernel, dim3(ns), dim3(256), 0, st, (const double2*)v_eff, L2, (double*)d_vmax.p);
-    double vmax[3] = {0.0, 0.0, 0.0};
-    if (hipMemcpyAsync(vmax, d_vmax.p, sizeof(double) * ns, hipMemcpyDeviceToHost, st) != hipSuccess ||
+    const unsigned nb = (unsigned)std::min<int64_t>(256, (L2 + 1023) / 1024);
+    const size_t pq_bytes = sizeof(double) * 2 * (size_t)ns * L2;
+    double bmax[3 * 256];
+    const size_t nmax = (size_t)ns * nb;
+    MovePassBufs b;   // outlives ws: freed after the wait below
+    Workspace ws;
+    if (!ws.get(pq_bytes + sizeof(double) * nmax)) return TM_ERR_NOMEM;
+    double* const pq = ws.at<double>(0);
+    double* const d_vmax = ws.at<double>(pq_bytes);
+    ws.idle = false;
+    hipLaunchKernelGGL(vmax_kernel, dim3(nb, (unsigned)ns), dim3(256), 0, st, (const double2*)v_eff, L2, d_vmax);
+    if (hipMemcpyAsync(bmax, d_vmax, sizeof(double) * nmax, hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return TM_ERR_HIP;
+    ws.idle = true;
+    double vmax[3] = {0.0, 0.0, 0.0};
+    for (int s = 0; s < ns; ++s) vmax[s] = *std::max_element(bmax + (size_t)s * nb, bmax + (size_t)(s + 1) * nb);
     MoveArgs a;
     int nD, nV;
-    const int rc = move_args(ns, L, sp, vmax, &a, &nD, &nV);
+    int rc = move_args(ns, L, sp, vmax, &a, &nD, &nV);
     if (rc != TM_OK) return rc;
-    DevBuf d_coef, d_mu, d_mv, d_pq;
-    if (hipMalloc(&d_coef.p, sizeof(double4) * (size_t)ns * L2) != hipSuccess ||
-        hipMalloc(&d_mu.p, sizeof(int2) * (size_t)ns * L2) != hipSuccess ||
-        hipMalloc(&d_mv.p, sizeof(double) * 4 * (size_t)ns * L2) != hipSuccess ||
-        hipMalloc(&d_pq.p, sizeof(double) * 2 * (size_t)ns * L2) != hipSuccess)
-        return TM_ERR_NOMEM;
-    const dim3 grid((unsigned)((L2 + 255) / 256), (unsigned)ns);
-    hipLaunchKernelGGL(fke_move_prep_kernel, grid, dim3(256), 0, st, a, rho, gamma, (const double2*)v_eff,
-                       (double4*)d_coef.p, (int2*)d_mu.p);
-    hipLaunchKernelGGL(fke_move_disp_kernel, grid, dim3(256), 0, st, a, (const double4*)d_coef.p,
-                       (const int2*)d_mu.p, (double*)d_mv.p);
-    hipLaunchKernelGGL(fke_move_row_kernel, grid, dim3(256), 0, st, a, (const double*)d_mv.p, stencil_D, stencil_V,
-                       (double*)d_pq.p);
-    hipLaunchKernelGGL(fke_move_col_kernel, grid, dim3(256), 0, st, a, (const double*)d_pq.p, stencil_D, stencil_V,
-                       out);
-    if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
-    // the scratch is released when this returns: wait for the kernels that use it
-    return hipStreamSynchronize(st) == hipSuccess ? TM_OK : TM_ERR_HIP;
+    ws.idle = false;
+    rc = move_launch(a, ns, rho, gamma, v_eff, stencil_D, stencil_V, pq, out, b, st);
+    // the scratch is handed on when this returns: wait for the kernels that use it
+    if (hipStreamSynchronize(st) != hipSuccess) return rc != TM_OK ? rc : TM_ERR_HIP;
+    ws.idle = true;
+    return rc;
 }
 
 int tm_fke_movement_host(int device, int ns, int L, const tm_fke_move_species* sp, const double* stencil_D,
@@ -1291,13 +1687,13 @@ int tm_fke_movement_host(int device, int ns, int L, const tm_fke_move_species* s
     int rc = move_args(ns, L, sp, vmax, &a, &nD, &nV);
     if (rc != TM_OK) return rc;
     if (hipSetDevice(device) != hipSuccess) return TM_ERR_NODEV;
-    DevBuf d_rho, d_gam, d_v, d_out, d_sd, d_sv, d_coef, d_mu, d_mv, d_pq;
+    DevBuf d_rho, d_gam, d_v, d_out, d_sd, d_sv, d_pq;
+    MovePassBufs b;
     const size_t fb = sizeof(double) * (size_t)ns * L2;
     if (hipMalloc(&d_rho.p, fb) != hipSuccess || hipMalloc(&d_gam.p, fb) != hipSuccess ||
         hipMalloc(&d_v.p, 2 * fb) != hipSuccess || hipMalloc(&d_out.p, fb) != hipSuccess ||
         hipMalloc(&d_sd.p, sizeof(double) * nD) != hipSuccess || hipMalloc(&d_sv.p, sizeof(double) * nV) != hipSuccess ||
-        hipMalloc(&d_coef.p, 4 * fb) != hipSuccess || hipMalloc(&d_mu.p, sizeof(int2) * (size_t)ns * L2) != hipSuccess ||
-        hipMalloc(&d_mv.p, 4 * fb) != hipSuccess || hipMalloc(&d_pq.p, 2 * fb) != hipSuccess)
+        hipMalloc(&d_pq.p, 2 * fb) != hipSuccess)
         return TM_ERR_NOMEM;
     if (hipMemcpy(d_rho.p, rho, fb, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(d_gam.p, gamma, fb, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1305,16 +1701,9 @@ int tm_fke_movement_host(int device, int ns, int L, const tm_fke_move_species* s
         hipMemcpy(d_sd.p, stencil_D, sizeof(double) * nD, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(d_sv.p, stencil_V, sizeof(double) * nV, hipMemcpyHostToDevice) != hipSuccess)
         return TM_ERR_HIP;
-    const dim3 grid((unsigned)((L2 + 255) / 256), (unsigned)ns);
-    hipLaunchKernelGGL(fke_move_prep_kernel, grid, dim3(256), 0, nullptr, a, (const double*)d_rho.p,
-                       (const double*)d_gam.p, (const double2*)d_v.p, (double4*)d_coef.p, (int2*)d_mu.p);
-    hipLaunchKernelGGL(fke_move_disp_kernel, grid, dim3(256), 0, nullptr, a, (const double4*)d_coef.p,
-                       (const int2*)d_mu.p, (double*)d_mv.p);
-    hipLaunchKernelGGL(fke_move_row_kernel, grid, dim3(256), 0, nullptr, a, (const double*)d_mv.p,
-                       (const double*)d_sd.p, (const double*)d_sv.p, (double*)d_pq.p);
-    hipLaunchKernelGGL(fke_move_col_kernel, grid, dim3(256), 0, nullptr, a, (const double*)d_pq.p,
-                       (const double*)d_sd.p, (const double*)d_sv.p, (double*)d_out.p);
-    if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
+    rc = move_launch(a, ns, (const double*)d_rho.p, (const double*)d_gam.p, (const double*)d_v.p,
+                     (const double*)d_sd.p, (const double*)d_sv.p, (double*)d_pq.p, (double*)d_out.p, b, nullptr);
+    if (rc != TM_OK) return rc;
     if (hipMemcpy(out, d_out.p, fb, hipMemcpyDeviceToHost) != hipSuccess) return TM_ERR_HIP;
     return TM_OK;
 }
@@ -1380,17 +1769,18 @@ int tm_fke_rk4(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t
     if (!fields || !fke_rk_args(ns, L, p, &c)) return TM_ERR_ARG;
     const hipStream_t st = (hipStream_t)stream;
     const size_t nf = (size_t)(ns + 3) * L * L;
-    DevBuf d_s, d_bad;
-    if (hipMalloc(&d_s.p, sizeof(double) * nf) != hipSuccess ||
-        hipMalloc(&d_bad.p, sizeof(unsigned long long)) != hipSuccess)
-        return TM_ERR_NOMEM;
+    Workspace ws;
+    if (!ws.get(sizeof(double) * nf + sizeof(unsigned long long))) return TM_ERR_NOMEM;
+    unsigned long long* const d_bad = ws.at<unsigned long long>(sizeof(double) * nf);
     unsigned long long bad = 0;
-    fke_rk_launch(c, fields, (double*)d_s.p, (unsigned long long*)d_bad.p, st);
+    ws.idle = false;
+    fke_rk_launch(c, fields, ws.at<double>(0), d_bad, st);
     if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
-    // the scratch is freed on return: wait for the stages that use it
-    if (hipMemcpyAsync(&bad, d_bad.p, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
+    // the scratch is handed on when this returns: wait for the kernels that use it
+    if (hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
         hipStreamSynchronize(st) != hipSuccess)
         return TM_ERR_HIP;
+    ws.idle = true;
     if (n_bad) *n_bad = (int64_t)bad;
     return TM_OK;
 }
