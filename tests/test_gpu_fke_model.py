@@ -100,3 +100,24 @@ def test_fke_model_rejects_movement_wider_than_lattice(tm):
             ctx.configure(tm.MODEL_FKE3, tm.F64, tm.FKEParams(), [tm.Instance(16, 0, 1, 0)])   # predator W = 9
         with pytest.raises(tm.TMError, match="TM_ERR_ARG"):
             ctx.configure(tm.MODEL_FKE2, tm.F32, tm.FKEParams(), [tm.Instance(32, 0, 1, 0)])   # FP64 only
+
+
+@pytest.mark.parametrize("sp", [2, 3])
+def test_fke_large_batch_equals_small_batches(tm, sp):
+    """The vegetation's Dornic step runs in two passes on 64 x 16 tiles on large batches
+    and one cell a thread on small ones: 360 lattices of 23^2 and 65^2 (2520 tiles of
+    64 x 4) against the same instances three at a time, bit for bit."""
+    model = tm.MODEL_FKE3 if sp == 3 else tm.MODEL_FKE2
+    hi = [60.0, 3.0, 0.5, 2.0, 2.0, 0.0, 0.0] if sp == 3 else [60.0, 3.0, 2.0, 2.0, 0.0]
+    insts = [tm.Instance(65 if k % 36 == 0 else 23, 0, 5, k) for k in range(360)]
+    out = []
+    for batch in (insts, [insts[0], insts[7], insts[359]]):
+        with tm.Context() as ctx:
+            ctx.configure(model, tm.F64, tm.FKEParams(), batch)
+            ctx.init_uniform([0.0] * len(hi), hi)
+            rows = ctx.run(3)
+            pick = [0, 7, 359] if len(batch) == 360 else [0, 1, 2]
+            out.append([(ctx.download(k), rows[k]) for k in pick])
+    for (f0, r0), (f1, r1) in zip(*out):
+        assert np.array_equal(f0, f1)
+        assert np.array_equal(r0, r1)

@@ -51,12 +51,6 @@ struct MoveArgs {
     int L;
 };
 
-__device__ __forceinline__ int wrapi(int v, int L)
-{
-    v %= L;
-    return v < 0 ? v + L : v;
-}
-
 // v in [-L, 2L) -> v mod L
 __device__ __forceinline__ int wrap1(int v, int L)
 {
@@ -309,24 +303,71 @@ __device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const doub
 // The column stencils of kMoveRPT consecutive rows x of column y, each output's terms
 // in move_col_at's order (a ascending: source rows descending); a source row is read
 // once for all the outputs it enters.
+// R >= 0: a half-width known at compile time, every row loaded before the sums (one
+// wait for memory instead of one a row).  R < 0: any r >= 2, the rows every output
+// takes four at a time, the three at either end apart.
+template <int R>
+__device__ __forceinline__ void move_cols_pass(const double* __restrict__ plane, const double* __restrict__ W, int r,
+                                               int L, int x, int y, double (&acc)[kMoveRPT])
+{
+#pragma clang fp contract(off)
+    if constexpr (R >= 0) {
+        constexpr int K = kMoveRPT + 2 * R;
+        double v[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) v[i] = plane[(int64_t)tmk::wrap(x + kMoveRPT - 1 + R - i, L) * L + y];
+#pragma unroll
+        for (int i = 0; i < K; ++i)
+#pragma unroll
+            for (int j = 0; j < kMoveRPT; ++j) {
+                const int a = j - (kMoveRPT - 1 + R - i);
+                if (a >= -R && a <= R) acc[j] += W[a < 0 ? -a : a] * v[i];
+            }
+    } else {
+        int row = tmk::wrap(x + kMoveRPT - 1 + r, L);
+        auto next = [&]() {
+            const double v = plane[(int64_t)row * L + y];
+            row = row == 0 ? L - 1 : row - 1;
+            return v;
+        };
+        double e[kMoveRPT - 1];
+#pragma unroll
+        for (int t = 0; t < kMoveRPT - 1; ++t) e[t] = next();          // row x + RPT - 1 + r - t: the last t + 1 outputs
+#pragma unroll
+        for (int t = 0; t < kMoveRPT - 1; ++t)
+#pragma unroll
+            for (int j = kMoveRPT - 1 - t; j < kMoveRPT; ++j) {
+                const int a = j - (kMoveRPT - 1 + r - t);
+                acc[j] += W[a < 0 ? -a : a] * e[t];
+            }
+#pragma unroll 4
+        for (int k = r; k >= kMoveRPT - 1 - r; --k) {                   // row x + k: every output
+            const double v = next();
+#pragma unroll
+            for (int j = 0; j < kMoveRPT; ++j) acc[j] += W[j - k < 0 ? k - j : j - k] * v;
+        }
+#pragma unroll
+        for (int t = 0; t < kMoveRPT - 1; ++t) e[t] = next();          // row x + RPT - 2 - r - t: the first outputs
+#pragma unroll
+        for (int t = 0; t < kMoveRPT - 1; ++t)
+#pragma unroll
+            for (int j = 0; j < kMoveRPT - 1 - t; ++j) {
+                const int a = j - (kMoveRPT - 2 - r - t);
+                acc[j] += W[a < 0 ? -a : a] * e[t];
+            }
+    }
+}
+
 __device__ __forceinline__ void move_cols_tile(const MoveSpecies& sp, const double* __restrict__ SD,
                                                const double* __restrict__ SV, int L, int64_t N, int x, int y,
                                                const double* __restrict__ pq, double (&acc)[kMoveRPT])
 {
-#pragma clang fp contract(off)
 #pragma unroll
     for (int j = 0; j < kMoveRPT; ++j) acc[j] = 0.0;
     auto pass = [&](const double* __restrict__ plane, const double* __restrict__ W, int r) {
-        int row = tmk::wrap(x + kMoveRPT - 1 + r, L);
-        for (int k = kMoveRPT - 1 + r; k >= -r; --k) {
-            const double v = plane[(int64_t)row * L + y];
-            row = row == 0 ? L - 1 : row - 1;
-#pragma unroll
-            for (int j = 0; j < kMoveRPT; ++j) {
-                const int a = j - k;
-                if (a >= -r && a <= r) acc[j] += W[a < 0 ? -a : a] * v;
-            }
-        }
+        if (r == 0) move_cols_pass<0>(plane, W, r, L, x, y, acc);
+        else if (r == 1) move_cols_pass<1>(plane, W, r, L, x, y, acc);
+        else move_cols_pass<-1>(plane, W, r, L, x, y, acc);
     };
     pass(pq, SD, sp.rD);
     pass(pq + N, SV, sp.rV);
@@ -517,7 +558,7 @@ int move_launch(const MoveArgs& a, int ns, const double* rho, const double* gamm
 // gathered from the old densities.  Per-species numbers of the step (means,
 // inverses, neighbour counts) come from the host.
 struct PerceptArgs {
-    int ns, L;
+    int ns, L, R;
     double v[3], mean[3], inv[3], fr[3];
     int eff[3];
     uint32_t seed, inst;
@@ -537,13 +578,34 @@ __device__ __forceinline__ double2 fke_velocity(uint32_t seed, uint32_t inst, ui
     return make_double2(v * cs, v * sn);
 }
 
+// acc + the sum of src (WEIGH: src (1 - pred inv)) over the first n perception offsets
+// around (p, q), in table order.  NEAR: every offset is within L of its cell, so one
+// wrap either way is enough; loads of four offsets are in flight at a time.
+template <bool WEIGH, bool NEAR>
+__device__ __forceinline__ double fke_disk_sum(const int2* __restrict__ disk, int n, const double* __restrict__ src,
+                                               const double* __restrict__ pred, double inv, int L, int p, int q,
+                                               double acc)
+{
+#pragma clang fp contract(off)
+#pragma unroll 4
+    for (int k = 0; k < n; ++k) {
+        const int2 o = disk[k];
+        const int64_t j = NEAR ? (int64_t)wrap1(p + o.x, L) * L + wrap1(q + o.y, L)
+                               : (int64_t)tmk::wrap(p + o.x, L) * L + tmk::wrap(q + o.y, L);
+        if (WEIGH) acc += src[j] * (1 - pred[j] * inv);
+        else acc += src[j];
+    }
+    return acc;
+}
+
 // Perception gamma of consumer s (1 .. ns-1) at cell (p, q) from its previous
 // value g: the old densities rho [ns][N] summed over the first eff[s] perception
 // offsets (weighed down by the predators for the grazer of the three-species
 // form), scaled by the prey's inverse mean and clamped to [0, 1]; 1 when the
 // consumer is extinct, 0 when its prey is; unchanged when it perceives nothing.
+// R: the table's radius.
 __device__ __forceinline__ double fke_gamma_at(int ns, int s, const double* mean, const double* inv, const double* fr,
-                                               const int* eff, const int2* __restrict__ disk,
+                                               const int* eff, const int2* __restrict__ disk, int R,
                                                const double* __restrict__ rho, int64_t N, int L, int p, int q,
                                                double g)
 {
@@ -552,13 +614,15 @@ __device__ __forceinline__ double fke_gamma_at(int ns, int s, const double* mean
     if (mean[s] < 1.0e-12) return 1.0;
     if (mean[s - 1] < 1.0e-12) return 0.0;
     const double* src = rho + (s - 1) * N;
+    const double* pred = rho + 2 * N;
     const bool weigh = ns == 3 && s == 1 && !(mean[2] < 1.0e-12);
-    double acc = g;
-    for (int k = 0; k < eff[s]; ++k) {
-        const int2 o = disk[k];
-        const int64_t j = (int64_t)wrapi(p + o.x, L) * L + wrapi(q + o.y, L);
-        if (weigh) acc += src[j] * (1 - rho[2 * N + j] * inv[2]);
-        else acc += src[j];
+    double acc;
+    if (R <= L) {
+        acc = weigh ? fke_disk_sum<true, true>(disk, eff[s], src, pred, inv[2], L, p, q, g)
+                    : fke_disk_sum<false, true>(disk, eff[s], src, src, 0.0, L, p, q, g);
+    } else {
+        acc = weigh ? fke_disk_sum<true, false>(disk, eff[s], src, pred, inv[2], L, p, q, g)
+                    : fke_disk_sum<false, false>(disk, eff[s], src, src, 0.0, L, p, q, g);
     }
     if (ns == 2 || s == 1) acc = (acc * inv[s - 1]) / (double)eff[s];
     else acc = (acc / (double)eff[s]) * inv[s - 1];
@@ -580,7 +644,7 @@ __global__ __launch_bounds__(256) void fke_perception_kernel(PerceptArgs a, cons
         for (int s = 0; s < 3; ++s) veff[s * N + i] = fke_velocity(a.seed, a.inst, (uint32_t)i, a.step, s, a.v[s]);
     for (int s = 1; s < a.ns; ++s) {
         double* g = gamma + (s - 1) * N + i;
-        *g = fke_gamma_at(a.ns, s, a.mean, a.inv, a.fr, a.eff, disk, rho, N, L, p, q, *g);
+        *g = fke_gamma_at(a.ns, s, a.mean, a.inv, a.fr, a.eff, disk, a.R, rho, N, L, p, q, *g);
     }
 }
 
@@ -899,23 +963,87 @@ void fke_rk_launch(const FkeRk& c, double* fields, double* scratch, unsigned lon
 // d (beta_0 = -M[0] - 4 D_0 / dx^2, FKE:3847-3849).  No flush: the reference
 // flushes after the movement step.
 // ---------------------------------------------------------------------------
+// One kVegTX x kVegTY tile by 256 threads (a wave per row, four rows each), in two
+// passes as dp_tile_deferred: the cells whose first trial does not settle go to a queue
+// in LDS and are finished densely packed.  The cells' neighbours come from the caches.
+// A wave used to run every path its 64 cells took between them: 16 x 256^2 in 36 us.
+constexpr int kVegTX = 64, kVegTY = 16;
+// Up to this many 64 x 4 tiles the model runs one cell a thread instead: us a step of the
+// three-species model, direct / two passes: 45 / 54 on 4 x 64^2, 54 / 61 on 2 x 256^2, 106 /
+// 107 on 8 x 256^2 (2048 tiles), 175 / 171 on 16 x 256^2.
+constexpr int kVegDirectTiles = 2048;
+
+// A cell and its four neighbours (value, up, down, left, right), periodic.
+__device__ __forceinline__ uint32_t veg_stencil(const double* __restrict__ P, int L, int y, int x, double (&v)[5])
+{
+    const uint32_t row = (uint32_t)y * (uint32_t)L, cell = row + (uint32_t)x;
+    v[0] = P[cell];
+    v[1] = P[(uint32_t)(y == 0 ? L - 1 : y - 1) * (uint32_t)L + (uint32_t)x];
+    v[2] = P[(uint32_t)(y == L - 1 ? 0 : y + 1) * (uint32_t)L + (uint32_t)x];
+    v[3] = P[row + (uint32_t)(x == 0 ? L - 1 : x - 1)];
+    v[4] = P[row + (uint32_t)(x == L - 1 ? 0 : x + 1)];
+    return cell;
+}
+
+__device__ __forceinline__ void veg_cell(const tmk::RKConstD& c, const tmk::DevInst& di, int L, int y, int x,
+                                         const double* __restrict__ P, double* __restrict__ Pstar)
+{
+    double v[5], n;
+    bool bad;
+    const uint32_t cell = veg_stencil(P, L, y, x, v);
+    Pstar[cell] = tmk::cell_update<double, 1>(c, di, cell, v[0], v[1], v[2], v[3], v[4], n, bad);
+}
+
+struct VegLds {
+    uint32_t n;
+    uint16_t q[kVegTX * kVegTY];
+};
+
+__device__ __forceinline__ void veg_tile(const tmk::RKConstD& c, const tmk::DevInst& di, int L, int x0, int y0,
+                                         const double* __restrict__ P, double* __restrict__ Pstar, VegLds& sm)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (threadIdx.x == 0) sm.n = 0u;
+    __syncthreads();
+#pragma unroll 1
+    for (int j = 0; j < kVegTY / 4; ++j) {
+        const int ly = 4 * j + w, y = y0 + ly, x = x0 + lane;
+        const bool in = y < L && x < L;
+        bool done = true;
+        if (in) {
+            double v[5], r, n;
+            bool bad;
+            const uint32_t cell = veg_stencil(P, L, y, x, v);
+            done = tmk::cell_update_first<double, 1>(c, di, cell, v[0], v[1], v[2], v[3], v[4], r, n, bad);
+            if (done) Pstar[cell] = r;
+        }
+        const uint64_t m = __ballot(!done);
+        if (m) {
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&sm.n, (uint32_t)__popcll(m));   // the queue's order does not matter
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            if (!done) sm.q[base + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = (uint16_t)(ly * kVegTX + lane);
+        }
+    }
+    __syncthreads();
+    const uint32_t nq = sm.n;
+#pragma unroll 1
+    for (uint32_t i = threadIdx.x; i < nq; i += 256) {
+        const uint32_t e = sm.q[i];
+        veg_cell(c, di, L, y0 + (int)(e / kVegTX), x0 + (int)(e % kVegTX), P, Pstar);
+    }
+}
+
 __global__ __launch_bounds__(256) void fke_veg_dornic_kernel(tm_rietkerk_params p, int L, uint32_t seed,
                                                              uint32_t inst, int64_t step, const double* P,
                                                              double* Pstar)
 {
-    const int64_t L2 = (int64_t)L * L;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= L2) return;
+    __shared__ VegLds sm;
     const tmk::RKConstD c = tmk::rk_constants(p, step);
     tmk::DevInst di = {};
     di.seed = seed;
     di.inst_id = inst;
-    const int y = (int)(i / L), x = (int)(i % L);
-    const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
-    const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
-    double n;
-    bool bad;
-    Pstar[i] = tmk::cell_update<double, 1>(c, di, (uint32_t)i, P[i], P[up], P[dn], P[lf], P[rt], n, bad);
+    veg_tile(c, di, L, (int)blockIdx.x * kVegTX, (int)blockIdx.y * kVegTY, P, Pstar, sm);
 }
 
 bool veg_dornic_ok(int L, const tm_rietkerk_params* p)
@@ -932,11 +1060,12 @@ bool veg_dornic_ok(int L, const tm_rietkerk_params* p)
 // [NF][L*L] at NF cell_off: P, G, (Pr,) W, O, then gamma_1 (, gamma_2);
 // NF = 2 SP + 1 for SP = 2 or 3 biota species.  One step, every launch over the
 // whole batch:
-//   fke_chunk / fke_state  spatial means of the old densities and the cover
-//                          factor (fixed-order sums, FKE:4100-4112), per instance
+//   fke_head               the vegetation's Dornic step P* (FKE:4150-4211) and the
+//                          chunk sums of the old densities, beside each other
+//   fke_state              spatial means and the cover factor (fixed-order sums,
+//                          FKE:4100-4112), per instance
 //   fke_percept            gamma of each consumer from the old densities
 //                          (FKE:4114-4118); velocities are drawn where used
-//   fke_veg                the vegetation's Dornic step P* (FKE:4150-4211)
 //   fke_rk4_step           RK4 of the trophic and water terms (FKE:4233-4238) from
 //                          P* and the other old densities, into the output buffer
 //   fke_move_rows_step, fke_move_cols_step  the consumers' Fokker-Planck movement
@@ -1003,13 +1132,11 @@ __device__ __forceinline__ void chunk_fold(double (&v)[NV], double (&red)[NV][25
 }
 
 template <int SP>
-__global__ __launch_bounds__(256) void fke_chunk_kernel(StepArgs a)
+__device__ __forceinline__ void fke_chunk(const StepArgs& a, const FkeWork* w, int block, double (&red)[SP + 1][256])
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * SP + 1;
-    __shared__ double red[SP + 1][256];
-    const FkeWork* w = (const FkeWork*)a.work;
-    const int2 ch = w->chunks[blockIdx.x];
+    const int2 ch = w->chunks[block];
     const DevInst di = a.inst[ch.x];
     const int64_t N = (int64_t)di.L * di.L;
     const double* f0 = (const double*)a.in + (int64_t)NF * di.cell_off;
@@ -1022,7 +1149,40 @@ __global__ __launch_bounds__(256) void fke_chunk_kernel(StepArgs a)
         for (int f = 0; f < SP; ++f) s[f] += f0[f * N + i];
         s[SP] += f0[i] > 0 ? 1.0 : 0.0;
     }
-    chunk_fold<SP + 1>(s, red, w->chunk + (int64_t)blockIdx.x * 8);
+    chunk_fold<SP + 1>(s, red, w->chunk + (int64_t)block * 8);
+}
+
+// The vegetation's Dornic step P* (workgroups 0 .. nveg - 1) and the chunk sums of the
+// old densities (the rest): both read the old fields only, so one launch runs the
+// short sums beside the samplers.  DIRECT: one cell a thread on the final kernel's
+// 64 x 4 tiles, in one pass, for batches whose 64 x 16 tiles leave CUs idle.
+template <int SP, bool DIRECT>
+__global__ __launch_bounds__(256) void fke_head_kernel(StepArgs a, int nveg)
+{
+    constexpr int NF = 2 * SP + 1;
+    static_assert(kMoveTX == kVegTX && kMoveTY == kVegTY, "the movement's tile table");
+    __shared__ union {
+        VegLds veg;
+        double red[SP + 1][256];
+    } sm;
+    const FkeWork* w = (const FkeWork*)a.work;
+    if ((int)blockIdx.x >= nveg) {
+        fke_chunk<SP>(a, w, (int)blockIdx.x - nveg, sm.red);
+        return;
+    }
+    if constexpr (DIRECT) {
+        const DevTile tl = a.tiles[blockIdx.x];
+        const DevInst di = a.inst[tl.inst];
+        const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.inst];
+        const int y = tl.y0 + (int)(threadIdx.x >> 6), x = tl.x0 + (int)(threadIdx.x & 63);
+        if (y >= tl.L || x >= tl.L) return;
+        veg_cell(c, di, tl.L, y, x, (const double*)a.in + (int64_t)NF * tl.cell_off, w->pstar + tl.cell_off);
+    } else {
+        const int4 tl = w->mtiles[blockIdx.x];
+        const DevInst di = a.inst[tl.x];
+        const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
+        veg_tile(c, di, di.L, tl.y, tl.z, (const double*)a.in + (int64_t)NF * di.cell_off, w->pstar + di.cell_off, sm.veg);
+    }
 }
 
 // The per-instance numbers of the perception step, as tm_fke_perception_host
@@ -1071,48 +1231,30 @@ __device__ __forceinline__ bool fke_cell(const StepArgs& a, const FkeWork* w, in
     return (int64_t)cell < (int64_t)di.L * di.L;
 }
 
+// Perception gamma of every consumer, a wave per row of the final kernel's 64 x 4
+// tiles, so that a row's wrap is scalar and a column's two selects: an index division
+// per offset and one offset in flight at a time took 45 us on 16 x 256^2.
 template <int SP>
 __global__ __launch_bounds__(256) void fke_percept_kernel(StepArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     const FkeWork* w = (const FkeWork*)a.work;
-    int inst, cell;
-    DevInst di;
-    if (!fke_cell(a, w, inst, cell, di)) return;
-    const int L = di.L;
-    const int64_t N = (int64_t)L * L;
-    const double* fin = (const double*)a.in + (int64_t)NF * di.cell_off;
-    double* fout = (double*)a.out + (int64_t)NF * di.cell_off;
-    const DPCStepState st = w->st[inst];
-    const DPCInstInfo info = w->info[inst];
-    const int p = cell / L, q = cell % L;
+    if ((int)blockIdx.x >= a.ntiles) return;
+    const DevTile tl = a.tiles[blockIdx.x];
+    const int L = tl.L;
+    const int p = tl.y0 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), q = tl.x0 + (int)(threadIdx.x & 63);
+    if (p >= L || q >= L) return;
+    const int64_t N = (int64_t)L * L, cell = (int64_t)p * L + q;
+    const double* fin = (const double*)a.in + (int64_t)NF * tl.cell_off;
+    double* fout = (double*)a.out + (int64_t)NF * tl.cell_off;
+    const DPCStepState st = w->st[tl.inst];
+    const DPCInstInfo info = w->info[tl.inst];
 #pragma unroll
     for (int s = 1; s < SP; ++s) {
         const int64_t j = (int64_t)(SP + 1 + s) * N + cell;
-        fout[j] = fke_gamma_at(SP, s, st.mean, st.inv, info.fr, st.eff, w->disk + info.disk_off, fin, N, L, p, q,
+        fout[j] = fke_gamma_at(SP, s, st.mean, st.inv, info.fr, st.eff, w->disk + info.disk_off, info.R, fin, N, L, p, q,
                                fin[j]);
     }
-}
-
-template <int SP>
-__global__ __launch_bounds__(256) void fke_veg_kernel(StepArgs a)
-{
-    constexpr int NF = 2 * SP + 1;
-    const FkeWork* w = (const FkeWork*)a.work;
-    int inst, cell;
-    DevInst di;
-    if (!fke_cell(a, w, inst, cell, di)) return;
-    const int L = di.L;
-    const int64_t N = (int64_t)L * L;
-    const double* fin = (const double*)a.in + (int64_t)NF * di.cell_off;
-    const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + inst];
-    const int y = cell / L, x = cell % L;
-    const int up = (y == 0 ? L - 1 : y - 1) * L + x, dn = (y == L - 1 ? 0 : y + 1) * L + x;
-    const int lf = y * L + (x == 0 ? L - 1 : x - 1), rt = y * L + (x == L - 1 ? 0 : x + 1);
-    double n;
-    bool bad;
-    w->pstar[di.cell_off + cell] =
-        cell_update<double, 1>(c, di, (uint32_t)cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
 }
 
 // RK4 of P* (FkeWork::pstar) and the other old densities into the output buffer.
@@ -1275,16 +1417,18 @@ __global__ __launch_bounds__(NT) void fke_final_kernel(StepArgs a)
 template <int SP, int TX, int TY, int NT>
 void launch_fke(const StepArgs& a, int grid, hipStream_t s)
 {
-    const dim3 blocks((unsigned)a.nblocks);
-    hipLaunchKernelGGL(fke_chunk_kernel<SP>, dim3(a.nchunks), dim3(256), 0, s, a);
+    if (a.ntiles <= kVegDirectTiles)
+        hipLaunchKernelGGL((fke_head_kernel<SP, true>), dim3((unsigned)(grid + a.nchunks)), dim3(256), 0, s, a, grid);
+    else
+        hipLaunchKernelGGL((fke_head_kernel<SP, false>), dim3((unsigned)(a.nmtiles + a.nchunks)), dim3(256), 0, s, a,
+                           a.nmtiles);
     hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
-    hipLaunchKernelGGL(fke_percept_kernel<SP>, blocks, dim3(256), 0, s, a);
-    hipLaunchKernelGGL(fke_veg_kernel<SP>, blocks, dim3(256), 0, s, a);
+    hipLaunchKernelGGL(fke_percept_kernel<SP>, dim3(grid), dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
     if (a.move_lds > 0) {
-        const dim3 tiles((unsigned)a.nmtiles, SP - 1);
-        hipLaunchKernelGGL(fke_move_rows_step_kernel<SP>, tiles, dim3(kMoveRows), (size_t)a.move_lds, s, a);
-        hipLaunchKernelGGL(fke_move_cols_step_kernel<SP>, tiles, dim3(kMoveCols), 0, s, a);
+        hipLaunchKernelGGL(fke_move_rows_step_kernel<SP>, dim3((unsigned)a.nmtiles, SP - 1), dim3(kMoveRows),
+                           (size_t)a.move_lds, s, a);
+        hipLaunchKernelGGL(fke_move_cols_step_kernel<SP>, dim3((unsigned)a.nmtiles, SP - 1), dim3(kMoveCols), 0, s, a);
     } else {   // a reach too wide for the tile frame
         const dim3 moves((unsigned)a.nblocks, SP - 1);
         hipLaunchKernelGGL(fke_mprep_kernel<SP>, moves, dim3(256), 0, s, a);
@@ -1725,6 +1869,7 @@ int tm_fke_perception_host(int device, int ns, int L, const double* pR, double d
     PerceptArgs a{};
     a.ns = ns;
     a.L = L;
+    a.R = R;
     a.seed = seed;
     a.inst = inst;
     a.step = step;
@@ -1863,9 +2008,8 @@ int tm_fke_veg_dornic(int L, const tm_rietkerk_params* p, uint32_t seed, uint32_
                       const double* P, double* Pstar, void* stream)
 {
     if (!P || !Pstar || P == Pstar || !veg_dornic_ok(L, p)) return TM_ERR_ARG;
-    const int64_t L2 = (int64_t)L * L;
-    hipLaunchKernelGGL(fke_veg_dornic_kernel, dim3((unsigned)((L2 + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
-                       *p, L, seed, inst, step, P, Pstar);
+    hipLaunchKernelGGL(fke_veg_dornic_kernel, dim3((unsigned)((L + kVegTX - 1) / kVegTX), (unsigned)((L + kVegTY - 1) / kVegTY)),
+                       dim3(256), 0, (hipStream_t)stream, *p, L, seed, inst, step, P, Pstar);
     return hipGetLastError() == hipSuccess ? TM_OK : TM_ERR_HIP;
 }
 
