@@ -146,3 +146,24 @@ def test_consumer_species_statistics(tm, oracle, model):
             got = ctx.replicate_stats(flags)
             assert got.shape == (2, 6, 4 * ns)
             assert np.array_equal(got, oracle.species_stats(series, pidx, 2, ns, flags)), flags
+
+
+@pytest.mark.parametrize("ns", [2, 3])
+def test_consumers_large_batch_equals_small_batches(tm, ns):
+    """The vegetation's Dornic step runs in two passes on 64 x 16 tiles on large batches
+    and one cell a thread on small ones: 360 lattices of 23^2 and 65^2 (2520 tiles of
+    64 x 4) against the same instances three at a time, bit for bit."""
+    model = tm.MODEL_DP3 if ns == 3 else tm.MODEL_DP2
+    hi = [20.0, 2.0, 0.5, 0.0, 0.0] if ns == 3 else [20.0, 2.0, 0.0]
+    insts = [tm.Instance(65 if k % 36 == 0 else 23, 0, 5, k) for k in range(360)]
+    out = []
+    for batch in (insts, [insts[0], insts[7], insts[359]]):
+        with tm.Context() as ctx:
+            ctx.configure(model, tm.F64, tm.DPCParams(a=1e-5), batch)
+            ctx.init_uniform([0.0] * len(hi), hi)
+            rows = ctx.run(3)
+            pick = [0, 7, 359] if len(batch) == 360 else [0, 1, 2]
+            out.append([(ctx.download(k), rows[k]) for k in pick])
+    for (f0, r0), (f1, r1) in zip(*out):
+        assert np.array_equal(f0, f1)
+        assert np.array_equal(r0, r1)

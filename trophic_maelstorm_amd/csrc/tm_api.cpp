@@ -28,6 +28,7 @@
 #include "tm/tm.h"
 #include "tm_io.h"
 #include "tm_launch.h"
+#include "tm_veg.h"
 
 using namespace tmk;
 
@@ -116,6 +117,7 @@ struct tm_ctx {
     void* d_dpc = nullptr;
     int dpc_nchunks = 0;
     int dpc_halo = 1;
+    int dpc_vtiles = 0, dpc_vdirect = 0;   // DP consumers: the vegetation's Dornic tiles
     FkeGrid fke = {};              // Rietkerk consumer models: launch sizes (FkeWork in d_dpc)
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
 };
@@ -353,6 +355,8 @@ StepArgs step_args(tm_ctx* c, int parity, int k)
     a.work = c->d_dpc;
     a.nchunks = c->dpc_nchunks;
     a.halo = c->dpc_halo;
+    a.nvtiles = c->dpc_vtiles;
+    a.vdirect = c->dpc_vdirect;
     a.nblocks = c->fke.blocks;
     a.nrtiles = c->fke.rtiles;
     a.nmtiles = c->fke.mtiles;
@@ -656,7 +660,6 @@ tm_status fault_status(tm_ctx* c)
     return TM_OK;
 }
 
-// Zero state with no fault recorded.
 // Consumer models: perception tables per parameter point, statistics chunks
 // and per-instance tables, in one device allocation behind a DPCWork header.
 tm_status setup_dpc(tm_ctx* c)
@@ -694,15 +697,29 @@ tm_status setup_dpc(tm_ctx* c)
         in.nchunks = nch;
         for (int k = 0; k < nch; ++k) chunks.push_back(make_int2((int)i, k));
     }
+    // The vegetation's Dornic step: 64 x 16 tiles in two passes, or 64 x 4 tiles with one
+    // cell a thread where those are at most kVegDirectTiles and the larger would leave
+    // CUs idle.
+    std::vector<int4> vtiles;
+    for (const int ty : {4, 16}) {
+        vtiles.clear();
+        for (size_t i = 0; i < c->inst.size(); ++i)
+            for (int y0 = 0; y0 < c->inst[i].L; y0 += ty)
+                for (int x0 = 0; x0 < c->inst[i].L; x0 += 64) vtiles.push_back(make_int4((int)i, x0, y0, 0));
+        c->dpc_vdirect = ty == 4;
+        if (vtiles.size() <= (size_t)kVegDirectTiles) break;
+    }
+    c->dpc_vtiles = (int)vtiles.size();
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t o_info = up(sizeof(DPCWork));
     const size_t o_st = o_info + up(sizeof(DPCInstInfo) * info.size());
     const size_t o_chunk = o_st + up(sizeof(DPCStepState) * info.size());
     const size_t o_chunks = o_chunk + up(sizeof(double) * 4 * chunks.size());
     const size_t o_disk = o_chunks + up(sizeof(int2) * chunks.size());
-    const size_t total = o_disk + up(sizeof(int2) * disk.size());
+    const size_t o_vtiles = o_disk + up(sizeof(int2) * disk.size());
+    const size_t total = o_vtiles + up(sizeof(int4) * vtiles.size());   // of the tables; P* and lambda follow
     free_dev(c->d_dpc);
-    if (hipMalloc(&c->d_dpc, total) != hipSuccess) return fail(c, TM_ERR_NOMEM, "consumer tables allocation failed");
+    if (hipMalloc(&c->d_dpc, total + sizeof(double) * (size_t)ns * (size_t)c->total_cells) != hipSuccess) return fail(c, TM_ERR_NOMEM, "consumer tables allocation failed");
     char* base = (char*)c->d_dpc;
     DPCWork w{};
     w.params = (const tm_dpc_params*)c->d_params;
@@ -711,17 +728,22 @@ tm_status setup_dpc(tm_ctx* c)
     w.chunk = (double*)(base + o_chunk);
     w.chunks = (const int2*)(base + o_chunks);
     w.disk = (const int2*)(base + o_disk);
+    w.vtiles = (const int4*)(base + o_vtiles);
+    w.pstar = (double*)(base + total);
+    w.lambda = w.pstar + c->total_cells;
     std::vector<char> host(total, 0);
     std::memcpy(host.data(), &w, sizeof(w));
     std::memcpy(host.data() + o_info, info.data(), sizeof(DPCInstInfo) * info.size());
     std::memcpy(host.data() + o_chunks, chunks.data(), sizeof(int2) * chunks.size());
     std::memcpy(host.data() + o_disk, disk.data(), sizeof(int2) * disk.size());
+    std::memcpy(host.data() + o_vtiles, vtiles.data(), sizeof(int4) * vtiles.size());
     HIPCHK(c, hipMemcpy(c->d_dpc, host.data(), total, hipMemcpyHostToDevice));
     c->dpc_nchunks = (int)chunks.size();
     c->dpc_halo = halo;
     return TM_OK;
 }
 
+// Zero state with no fault recorded.
 tm_status reset_state(tm_ctx* c)
 {
     DevState st{};

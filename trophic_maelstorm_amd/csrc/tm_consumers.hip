@@ -6,25 +6,27 @@
 // gamma_1 .. gamma_{NS-1} (NF = 2 NS - 1), species-major [NF][L*L].
 //
 // A step is three launches:
-//   dpc_chunk_kernel  one workgroup per 4096-cell chunk: the chunk's sums of
-//                     every density and the occupied count of the vegetation,
-//                     in a fixed order (lane strides, then a pairwise fold);
+//   dpc_head_kernel   the vegetation's Dornic step P* (:2901-2945), and beside it one
+//                     workgroup per 4096-cell chunk: the chunk's sums of every
+//                     density and the occupied count of the vegetation, in a
+//                     fixed order (lane strides, then a pairwise fold);
 //   dpc_state_kernel  one thread per instance: the chunk sums in chunk order ->
 //                     spatial means, the cover factor and the number of
 //                     perception neighbours each consumer uses this step
 //                     (multiSPDP.cpp:2962-2975, :1705-1730);
 //   dpc_step_kernel   one workgroup per tile: the tile and a halo of the
-//                     perception radius of every density in LDS, then per cell
-//                     the vegetation's Dornic step (:2901-2945), each consumer's
-//                     perception gamma (:1699-1786, :2166-2284) and its Dornic
-//                     step with upwind advection in a random direction
-//                     (:3041-3190), the RK4 of the trophic terms (:1821-1898),
-//                     checks and flush (:3228-3262), and rho(t) partials.
+//                     perception radius of every density in LDS, then each
+//                     consumer's perception gamma (:1699-1786, :2166-2284) and
+//                     its Dornic step with upwind advection in a random direction
+//                     (:3041-3190), and per cell the RK4 of the trophic terms from
+//                     P* (:1821-1898), checks and flush (:3228-3262), and rho(t)
+//                     partials.
 // The means steer the step (they scale gamma and switch consumers off), so they
 // come from the fixed-order reduction rather than from the compensated rho(t)
 // rows; the rows stay the reporting path.
 #include <hip/hip_runtime.h>
 #include "tm_launch.h"
+#include "tm_veg.h"
 
 namespace tmk {
 
@@ -34,13 +36,11 @@ constexpr int kChunk = kDpcChunkCells;
 constexpr double kGammaEps = 1.0e-12;   // calc_gamma's eps (multiSPDP.cpp:1715, :2182)
 
 template <int NS>
-__global__ __launch_bounds__(256) void dpc_chunk_kernel(StepArgs a)
+__device__ __forceinline__ void dpc_chunk(const StepArgs& a, const DPCWork* w, int block, double (&red)[NS + 1][256])
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * NS - 1;
-    __shared__ double red[NS + 1][256];
-    const DPCWork* w = (const DPCWork*)a.work;
-    const int2 ch = w->chunks[blockIdx.x];
+    const int2 ch = w->chunks[block];
     const DevInst di = a.inst[ch.x];
     const int64_t N = (int64_t)di.L * di.L;
     const double* f0 = (const double*)a.in + (int64_t)NF * di.cell_off;
@@ -66,7 +66,35 @@ __global__ __launch_bounds__(256) void dpc_chunk_kernel(StepArgs a)
     }
     if (t == 0) {
 #pragma unroll
-        for (int f = 0; f <= NS; ++f) w->chunk[(int64_t)blockIdx.x * 4 + f] = red[f][0];
+        for (int f = 0; f <= NS; ++f) w->chunk[(int64_t)block * 4 + f] = red[f][0];
+    }
+}
+
+// The vegetation's Dornic step (workgroups 0 .. nvtiles - 1) and the chunk sums (the
+// rest): both read the old fields only, so the short sums run beside the samplers.
+template <int NS>
+__global__ __launch_bounds__(256, 5) void dpc_head_kernel(StepArgs a)
+{
+    constexpr int NF = 2 * NS - 1;
+    __shared__ union {
+        VegLds veg;
+        double red[NS + 1][256];
+    } sm;
+    const DPCWork* w = (const DPCWork*)a.work;
+    if ((int)blockIdx.x >= a.nvtiles) {
+        dpc_chunk<NS>(a, w, (int)blockIdx.x - a.nvtiles, sm.red);
+        return;
+    }
+    const int4 tl = w->vtiles[blockIdx.x];   // (instance, x0, y0)
+    const DevInst di = a.inst[tl.x];
+    const DPCConst c = ((const DPCConst*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
+    const VegConst vc = {c.k, di.seed, di.inst_id, c.compat, c.step};
+    const double* P = (const double*)a.in + (int64_t)NF * di.cell_off;
+    if (a.vdirect) {   // 64 x 4 tiles, one cell a thread
+        const int y = tl.z + (int)(threadIdx.x >> 6), x = tl.y + (int)(threadIdx.x & 63);
+        if (y < di.L && x < di.L) veg_cell(vc, di.L, y, x, P, w->pstar + di.cell_off);
+    } else {
+        veg_tile(vc, di.L, tl.y, tl.z, P, w->pstar + di.cell_off, sm.veg);
     }
 }
 
@@ -142,13 +170,69 @@ __device__ __forceinline__ void dpc_rk4(const tm_dpc_params& p, double* y)
     for (int s = 0; s < NS; ++s) y[s] += (dt6) * (k1[s] + 2.0 * k2[s] + 2.0 * k3[s] + k4[s]);
 }
 
+// One consumer's Dornic transition with upwind advection in a random direction
+// (multiSPDP.cpp:3041-3190) at image index r of its density is, from its perception
+// gamma.  FIRST: as dornic_cell_d's first pass; lambda and words (of the direction and
+// the count) are for its kDornicGamma.
+template <bool FIRST>
+__device__ __forceinline__ int dpc_consumer(const tm_dpc_params& p, int s, const DevInst& di, uint32_t cell,
+                                            int64_t step, bool compat, double gam, const double* is, int r, int RW,
+                                            double& y, double& lambda, int& words)
+{
+#pragma clang fp contract(off)
+    const double dx = p.dx, dt = p.dt;
+    const double dx2 = dx * dx, dx1 = 1 / dx, dx1_2 = 1 / (dx2), dxb2 = dx / 2.0;
+    const double Dc0 = p.D[0] / (dx2);
+    y = is[r];
+    Stream sc(di.seed, di.inst_id, cell, step);
+    sc.blk = (uint32_t)s << 24;
+    double sn, cs;
+    dsincos2pi(sc.u64(), sn, cs);
+    const double vx = p.v[s] * cs, vy = p.v[s] * sn;
+    const double vxa = vx * (double)((0 < vx) - (vx < 0));
+    const double vya = vy * (double)((0 < vy) - (vy < 0));
+    const double gp = (1 - gam);
+    double Dx = (p.D[s] - (dxb2) * (gp * vxa * (1 - dt * dx1 * gp * vxa))) * dx1_2;
+    double Dy = (p.D[s] - (dxb2) * (gp * vya * (1 - dt * dx1 * gp * vya))) * dx1_2;
+    if (Dx < Dc0) Dx = Dc0;
+    if (Dy < Dc0) Dy = Dc0;
+    const double ux = vx > 0 ? is[r - 1] : is[r + 1];
+    const double uy = vy > 0 ? is[r - RW] : is[r + RW];
+    const double alpha = gam * (Dy * (is[r - RW] + is[r + RW]) + Dx * (is[r - 1] + is[r + 1]))
+                         + dx1 * (gp) * (vxa * ux + vya * uy);
+    if (alpha == 0 && is[r] == 0) return kDornicDone;
+    const double beta = -p.M[s] - 2 * gam * (Dx + Dy) - (1 - gam) * (vxa + vya) * dx1;
+    const double lexp = dexp((beta) * dt);
+    const double sig2_1 = 1 / (p.sigma[s] * p.sigma[s]);
+    const double lam = 2 * (beta) * (sig2_1) / (lexp - 1.0);
+    DornicConst k{};
+    k.lambda = lam;
+    k.ll = lam * lexp;
+    k.sigma2_1 = sig2_1;
+    double n;
+    const int st = dornic_cell_d<FIRST, Stream>(sc, alpha, is[r], k, compat, n, y);
+    lambda = lam;
+    words = 1 + dornic_words(k.ll * is[r], compat);
+    return st;
+}
+
+// One tile, in phases with a barrier between them: the consumers' perception gamma and
+// first trials per cell (the vegetation's P* is in DPCWork::pstar), the transitions
+// those leave open from two queues per consumer, densely packed, then the RK4, checks,
+// flush and partials per cell.  Between phases a cell's new densities and gamma wait in
+// the output fields.  In one pass every wave ran every sampler path of its 64 cells and
+// held the samplers', the perception's and the RK4's registers at once (146 VGPRs): 16 x
+// 256^2, two species, 139 us for the step kernel alone, 32 + 77 here.
 template <int NS, int TX, int TY, int NT, int MINW>
 __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
 {
 #pragma clang fp contract(off)
-    constexpr int NF = 2 * NS - 1;
+    constexpr int NF = 2 * NS - 1, NC = TX * TY;
+    static_assert(NC <= 512, "a queue entry holds a cell in 9 bits, then its words");
     extern __shared__ __align__(16) double s_lds[];
     __shared__ double s_red[2 * NF * (NT / 64)];
+    __shared__ uint16_t s_q[NS - 1][NC];        // restarts from the front, Gamma deviates from the back
+    __shared__ uint32_t s_n[NS - 1][2];
 
     const int64_t counter = a.state->counter + a.k;
     const int64_t slot = counter & (int64_t)(a.nslots - 1);
@@ -169,111 +253,121 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
     const int64_t N = (int64_t)L * L;
     const double* fin = (const double*)a.in + (int64_t)NF * tl.cell_off;
     double* fout = (double*)a.out + (int64_t)NF * tl.cell_off;
+    const double* pstar = w->pstar + tl.cell_off;
 
-    for (int e = threadIdx.x; e < IMG; e += NT) {
-        const int ry = e / RW, rx = e - (e / RW) * RW;
-        const int gy = wrap(tl.y0 + ry - H, L), gx = wrap(tl.x0 + rx - H, L);
-        const int64_t g = (int64_t)gy * L + gx;
+    // 32 lanes along a row, NT / 32 rows at a time: no index division
+    for (int ry = threadIdx.x >> 5; ry < RH; ry += NT / 32) {
+        const int64_t row = (int64_t)wrap(tl.y0 + ry - H, L) * L;
+        for (int rx = threadIdx.x & 31; rx < RW; rx += 32) {
+            const int64_t g = row + wrap(tl.x0 + rx - H, L);
 #pragma unroll
-        for (int s = 0; s < NS; ++s) img[s * IMG + e] = fin[s * N + g];
+            for (int s = 0; s < NS; ++s) img[s * IMG + ry * RW + rx] = fin[s * N + g];
+        }
     }
     for (int k = threadIdx.x; k < info.disk_len; k += NT) {
         const int2 o = w->disk[info.disk_off + k];
         offs[k] = o.x * RW + o.y;
     }
+    if (threadIdx.x < 2 * (NS - 1)) (&s_n[0][0])[threadIdx.x] = 0u;
     __syncthreads();
 
-    const double dx = p.dx, dt = p.dt;
-    const double dx2 = dx * dx, dx1 = 1 / dx, dx1_2 = 1 / (dx2), dxb2 = dx / 2.0;
-    const double Dc0 = p.D[0] / (dx2);
+    // perception gamma of each consumer from the old fields, and its first trials
+#pragma unroll
+    for (int s = 1; s < NS; ++s) {
+        const bool live = !(st.mean[s] == 0.0);
+        const double* is = img + s * IMG;
+        const int eff = st.eff[s];
+#pragma unroll 1
+        for (int e = threadIdx.x; e < NC; e += NT) {
+            const int ly = e / TX, lx = e % TX;
+            const int gy = tl.y0 + ly, gx = tl.x0 + lx;
+            const int r = (ly + H) * RW + (lx + H);
+            const double* src = img + (s - 1) * IMG + r;
+            int res = kDornicDone, words = 0;
+            if (gy < L && gx < L) {
+                const uint32_t cell = (uint32_t)gy * (uint32_t)L + (uint32_t)gx;
+                double g = fin[(NS + s - 1) * N + cell];
+                if (info.fr[s] == 0.0) {
+                } else if (st.mean[s] < kGammaEps || st.mean[s - 1] < kGammaEps) {
+                    g = 0.0;
+                } else {
+                    if constexpr (NS == 2) {            // accumulates onto the previous value (:1756-1760)
+#pragma unroll 4
+                        for (int k = 0; k < eff; ++k) g += src[offs[k]];
+                        g = (g * st.inv[s - 1]) / (double)eff;
+                    } else if (s == 1) {                // grazers, weighed down by predators (:2228-2249)
+                        double acc = 0.0;
+                        if (st.mean[2] < kGammaEps) {
+#pragma unroll 4
+                            for (int k = 0; k < eff; ++k) acc += src[offs[k]];
+                        } else {
+                            const double* pr = img + 2 * IMG + r;
+#pragma unroll 4
+                            for (int k = 0; k < eff; ++k) acc += src[offs[k]] * (1 - pr[offs[k]] * st.inv[2]);
+                        }
+                        g = (acc * st.inv[s - 1]) / (double)eff;
+                    } else {                            // predators (:2251-2258)
+                        double acc = 0.0;
+#pragma unroll 4
+                        for (int k = 0; k < eff; ++k) acc += src[offs[k]];
+                        g = (acc / (double)eff) * st.inv[s - 1];
+                    }
+                    if (g > 1) g = 1.0;
+                    else if (g < 0) g = 0.0;
+                }
+                double y = is[r];
+                if (live) {
+                    if (g > 1) g = 1;
+                    double lambda;
+                    res = dpc_consumer<true>(p, s, di, cell, c.step, c.compat != 0, g, is, r, RW, y, lambda, words);
+                    if (res == kDornicGamma) w->lambda[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell] = lambda;
+                }
+                fout[(NS + s - 1) * N + cell] = g;
+                fout[s * N + cell] = y;
+            }
+            queue_push<false>(res == kDornicRestart, (uint16_t)e, s_q[s - 1], &s_n[s - 1][0]);
+            queue_push<true>(res == kDornicGamma, (uint16_t)(e | words << 9), s_q[s - 1] + NC, &s_n[s - 1][1]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 1; s < NS; ++s) {
+        // one list, restarts first: its waves run beside each other, nearly each on one kind
+        const uint32_t n0 = s_n[s - 1][0], n1 = s_n[s - 1][1];
+#pragma unroll 1
+        for (uint32_t i = threadIdx.x; i < n0 + n1; i += NT) {
+            const int q = i < n0 ? s_q[s - 1][i] : s_q[s - 1][NC - 1 - (i - n0)], e = q & 511;
+            const int ly = e / TX, lx = e % TX;
+            const uint32_t cell = (uint32_t)(tl.y0 + ly) * (uint32_t)L + (uint32_t)(tl.x0 + lx);
+            double y, lambda;
+            if (i < n0) {
+                int words;
+                dpc_consumer<false>(p, s, di, cell, c.step, c.compat != 0, fout[(NS + s - 1) * N + cell],
+                                    img + s * IMG, (ly + H) * RW + (lx + H), RW, y, lambda, words);
+            } else {
+                Stream sc(di.seed, di.inst_id, cell, c.step);
+                sc.blk = (uint32_t)s << 24;
+                sc.skip(q >> 9);
+                lambda = w->lambda[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell];
+                y = dornic_gamma_d(sc, fout[s * N + cell], lambda, c.compat != 0);
+            }
+            fout[s * N + cell] = y;
+        }
+    }
+    __syncthreads();
+
     double sum[NF], cnt[NF];
 #pragma unroll
     for (int f = 0; f < NF; ++f) { sum[f] = 0.0; cnt[f] = 0.0; }
-
-    for (int e = threadIdx.x; e < TX * TY; e += NT) {
+    for (int e = threadIdx.x; e < NC; e += NT) {
         const int ly = e / TX, lx = e % TX;
         const int gy = tl.y0 + ly, gx = tl.x0 + lx;
         if (gy >= L || gx >= L) continue;
         const uint32_t cell = (uint32_t)gy * (uint32_t)L + (uint32_t)gx;
-        const int r = (ly + H) * RW + (lx + H);
         double y[NS];
-        // vegetation: Dornic (multiSPDP.cpp:2901-2945)
-        {
-            const double cur = img[r];
-            const double alpha = Dc0 * (img[r - RW] + img[r + RW] + img[r - 1] + img[r + 1]);
-            y[0] = cur;
-            if (!(alpha == 0.0 && cur == 0.0)) {
-                Stream s0(di.seed, di.inst_id, cell, c.step);
-                double n;
-                y[0] = dornic_cell(s0, alpha, cur, c.k, c.compat != 0, n);
-            }
-        }
-        // perception gamma of each consumer, from the old fields
-        double gam[NS];
-        gam[0] = 0.0;
+        y[0] = pstar[cell];
 #pragma unroll
-        for (int s = 1; s < NS; ++s) {
-            double g = fin[(NS + s - 1) * N + cell];
-            if (info.fr[s] == 0.0) { gam[s] = g; continue; }
-            if (st.mean[s] < kGammaEps || st.mean[s - 1] < kGammaEps) { gam[s] = 0.0; continue; }
-            const double* src = img + (s - 1) * IMG + r;
-            const int eff = st.eff[s];
-            if constexpr (NS == 2) {            // accumulates onto the previous value (:1756-1760)
-                for (int k = 0; k < eff; ++k) g += src[offs[k]];
-                g = (g * st.inv[s - 1]) / (double)eff;
-            } else if (s == 1) {                // grazers, weighed down by predators (:2228-2249)
-                double acc = 0.0;
-                if (st.mean[2] < kGammaEps) {
-                    for (int k = 0; k < eff; ++k) acc += src[offs[k]];
-                } else {
-                    const double* pr = img + 2 * IMG + r;
-                    for (int k = 0; k < eff; ++k) acc += src[offs[k]] * (1 - pr[offs[k]] * st.inv[2]);
-                }
-                g = (acc * st.inv[s - 1]) / (double)eff;
-            } else {                            // predators (:2251-2258)
-                double acc = 0.0;
-                for (int k = 0; k < eff; ++k) acc += src[offs[k]];
-                g = (acc / (double)eff) * st.inv[s - 1];
-            }
-            if (g > 1) g = 1.0;
-            else if (g < 0) g = 0.0;
-            gam[s] = g;
-        }
-        // consumers: Dornic with upwind advection in a random direction (:3041-3190)
-#pragma unroll
-        for (int s = 1; s < NS; ++s) {
-            const double* is = img + s * IMG;
-            y[s] = is[r];
-            if (st.mean[s] == 0.0) continue;
-            if (gam[s] > 1) gam[s] = 1;
-            Stream sc(di.seed, di.inst_id, cell, c.step);
-            sc.blk = (uint32_t)s << 24;
-            double sn, cs;
-            dsincos2pi(sc.u64(), sn, cs);
-            const double vx = p.v[s] * cs, vy = p.v[s] * sn;
-            const double vxa = vx * (double)((0 < vx) - (vx < 0));
-            const double vya = vy * (double)((0 < vy) - (vy < 0));
-            const double gp = (1 - gam[s]);
-            double Dx = (p.D[s] - (dxb2) * (gp * vxa * (1 - dt * dx1 * gp * vxa))) * dx1_2;
-            double Dy = (p.D[s] - (dxb2) * (gp * vya * (1 - dt * dx1 * gp * vya))) * dx1_2;
-            if (Dx < Dc0) Dx = Dc0;
-            if (Dy < Dc0) Dy = Dc0;
-            const double ux = vx > 0 ? is[r - 1] : is[r + 1];
-            const double uy = vy > 0 ? is[r - RW] : is[r + RW];
-            const double alpha = gam[s] * (Dy * (is[r - RW] + is[r + RW]) + Dx * (is[r - 1] + is[r + 1]))
-                                 + dx1 * (gp) * (vxa * ux + vya * uy);
-            if (alpha == 0 && is[r] == 0) continue;
-            const double beta = -p.M[s] - 2 * gam[s] * (Dx + Dy) - (1 - gam[s]) * (vxa + vya) * dx1;
-            const double lexp = dexp((beta) * dt);
-            const double sig2_1 = 1 / (p.sigma[s] * p.sigma[s]);
-            const double lam = 2 * (beta) * (sig2_1) / (lexp - 1.0);
-            DornicConst k{};
-            k.lambda = lam;
-            k.ll = lam * lexp;
-            k.sigma2_1 = sig2_1;
-            double n;
-            y[s] = dornic_cell(sc, alpha, is[r], k, c.compat != 0, n);
-        }
+        for (int s = 1; s < NS; ++s) y[s] = fout[s * N + cell];
         dpc_rk4<NS>(p, y);
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -286,9 +380,9 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
         }
 #pragma unroll
         for (int s = 1; s < NS; ++s) {
-            fout[(NS + s - 1) * N + cell] = gam[s];
-            sum[NS + s - 1] += gam[s];
-            cnt[NS + s - 1] += gam[s] > 0.0 ? 1.0 : 0.0;
+            const double g = fout[(NS + s - 1) * N + cell];
+            sum[NS + s - 1] += g;
+            cnt[NS + s - 1] += g > 0.0 ? 1.0 : 0.0;
         }
     }
     block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ntiles + tile) * NF, s_red);
@@ -298,14 +392,14 @@ template <int NS, int TX, int TY, int NT, int MINW = 1>
 void launch_dpc(const StepArgs& a, int grid, hipStream_t s)
 {
     const size_t lds = dpc_lds_bytes(NS, TX, TY, a.halo);
-    if (lds > 65536) {   // above the default dynamic-LDS limit (CDNA4 has 160 KiB per CU)
+    if (lds > 57344) {   // above the default LDS limit with the static arrays (CDNA4 has 160 KiB per CU)
         static size_t granted = 0;
         if (lds > granted &&
             hipFuncSetAttribute((const void*)dpc_step_kernel<NS, TX, TY, NT, MINW>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess)
             granted = lds;
     }
-    hipLaunchKernelGGL(dpc_chunk_kernel<NS>, dim3(a.nchunks), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(dpc_head_kernel<NS>, dim3(a.nvtiles + a.nchunks), dim3(256), 0, s, a);
     hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL((dpc_step_kernel<NS, TX, TY, NT, MINW>), dim3(grid), dim3(NT), lds, s, a);
 }

@@ -86,6 +86,10 @@ struct Stream {
         left -= 1;
         return w;
     }
+    __device__ void skip(int n)
+    {
+        for (int i = 0; i < n; ++i) (void)word();
+    }
     // (w + 1/2) 2^-32: exact in double, never 0 or 1.
     __device__ double u64() { return ((double)word() + 0.5) * 0x1p-32; }
     // FP32 uniform ((w >> 9) + 1/2) 2^-23: exact, never 0 or 1.
@@ -380,15 +384,19 @@ TM_HD bool ptrs_in_box_d(const PtrsD& p, double us, double V) { return us >= 0.0
 
 // The trial's test  log V + log(invalpha) - log(a / us^2 + b) <= -z + k log z - log k!,
 // both sides in FP32: the right one as -stirlerr(k) - bd0(k, z) - log(2 pi k) / 2
-// (Loader 2000), with k - z formed in FP64 and bd0 from its series.  Used for
-// 5 <= k, z < 1e9 and |k - z| < 0.1 (k + z), where every term is below 1e-6 relative
-// and the FP64 sides are good to 1e-5; the margin is 1e-3 + 1e-5 of their size.
+// (Loader 2000), with k - z formed in FP64 and bd0 from its series where |k - z| <
+// 0.1 (k + z), else as k log(k / z) + z - k for k < 1000 (its rounding, 3e-7 k, is
+// then below 3e-4).  Used for 5 <= k, z < 1e9, where every other term is below 1e-6
+// relative and the FP64 sides are good to 1e-5; the margin is 1e-3 + 1e-5 of their size.
 __device__ __forceinline__ int ptrs_estimate(const PtrsD& p, double z, double kd, double us, double V)
 {
     const float k = (float)kd, zf = (float)z, dk = (float)(kd - z), sum = k + zf;
-    if (!(kd >= 5.0 && z < 1e9 && __builtin_fabsf(dk) < 0.1f * sum)) return 0;
+    const bool near = __builtin_fabsf(dk) < 0.1f * sum;
+    if (!(kd >= 5.0 && z < 1e9 && (near || kd < 1000.0))) return 0;
     const float w = dk * __builtin_amdgcn_rcpf(sum), w2 = w * w;
-    const float bd0 = dk * w + 2.0f * k * w * w2 * (0.333333333f + w2 * (0.2f + w2 * (0.142857143f + w2 * 0.111111111f)));
+    const float ser = dk * w + 2.0f * k * w * w2 * (0.333333333f + w2 * (0.2f + w2 * (0.142857143f + w2 * 0.111111111f)));
+    const float dir = k * est_log(k * __builtin_amdgcn_rcpf(zf)) - dk;
+    const float bd0 = near ? ser : dir;
     const float r = __builtin_amdgcn_rcpf(k);
     const float rhs = -r * (0.0833333333f - r * r * 0.00277777778f) - bd0 - 0.5f * est_log(6.28318531f * k);
     const float usf = (float)us, b = (float)p.b;

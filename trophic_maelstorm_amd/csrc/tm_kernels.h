@@ -81,6 +81,8 @@ struct StepArgs {
     int32_t nchunks;     // consumer models: statistics chunks of the batch
     int32_t halo;        // consumer models: LDS halo (largest perception radius, >= 1)
     int32_t nblocks;     // Rietkerk consumer models: 256-cell blocks of the batch
+    int32_t nvtiles;     // DP consumer models: the vegetation's Dornic tiles,
+    int32_t vdirect;     // ... 64 x 4 with one cell a thread (else 64 x 16 in two passes)
     int32_t nrtiles;     // Rietkerk consumer models: RK4 tiles of the batch
     int32_t nmtiles;     // ... movement tiles
     int32_t move_lds;    // ... and the movement tile's LDS bytes (0: the four-pass movement)
@@ -246,28 +248,49 @@ template <> struct Arith<float> {
 };
 
 // Dornic Poisson-Gamma transition of one live cell (rietkerk_bjork_FKE.cpp:4168-4196).
-// ONE = true: as the FP32 dornic_cell_f<true> -- false where the transition needs
-// a software logarithm of an accept test or of the quantile's tail, a second PTRS
-// or Gamma trial, or a fifth word (the boost after a PTRS trial); otherwise the
-// same words and value.
 // n gets the Poisson count as an integer-valued double.
+// ONE = true is the first pass of a deferring step: where the transition needs a software
+// logarithm of an accept test or of the quantile's tail, a second PTRS or Gamma trial, or
+// a fifth word (the boost after a PTRS trial) it stops.  kDornicRestart: before the count
+// is settled; kDornicGamma: n is the count and y the Gamma shape mu + 1 + n, for
+// dornic_gamma_d on the stream past dornic_words words.  Otherwise (kDornicDone) it
+// draws the same words and computes the same value as ONE = false.
+enum { kDornicDone = 0, kDornicRestart = 1, kDornicGamma = 2 };
+
+// Words the count takes from the stream where kDornicGamma is returned.
+__device__ __forceinline__ int dornic_words(double z, bool compat)
+{
+    if (!(z > 0.0)) return 0;
+    return z < 12.0 || (compat && z > 100.0) ? 1 : 2;
+}
+
+// The Gamma deviate of shape gru over lambda.
+__device__ __forceinline__ double dornic_gamma_d(Stream& s, double gru, double lambda, bool compat)
+{
+#pragma clang fp contract(off)
+    if (compat && gru > 100.0) return (norm_icdf_d(s.u64()) * dsqrt(gru) + gru) / lambda;
+    double g;
+    gamma_d_try<64, Stream>(s, gru, g);
+    return g / lambda;
+}
+
 template <bool ONE, class St>
-__device__ __forceinline__ bool dornic_cell_d(St& s, double alpha_i, double cur, const DornicConst& k,
-                                              bool compat, double& n, double& y)
+__device__ __forceinline__ int dornic_cell_d(St& s, double alpha_i, double cur, const DornicConst& k,
+                                             bool compat, double& n, double& y)
 {
 #pragma clang fp contract(off)
     const double mu = -1.0 + 2.0 * alpha_i * k.sigma2_1;
     const double ziggy = k.ll * cur;
     double gru;
+    bool big = false;   // the count took a PTRS trial's two words
     if (ziggy == 0.0) {
         n = 0.0;
         gru = mu + 1.0;
     } else if (ONE && ziggy >= 12.0) {
         if (compat && ziggy > 100.0) {
             const double p = s.u64();
-            if (icdf_in_tail(p)) return false;
+            if (icdf_in_tail(p)) return kDornicRestart;
             n = count_of(__builtin_trunc(norm_icdf_d(p) * dsqrt(ziggy) + ziggy));
-            gru = mu + 1.0 + n;
         } else {
             const PtrsD pt = ptrs_setup_d(ziggy);
             const double U = s.u64() - 0.5;
@@ -275,27 +298,30 @@ __device__ __forceinline__ bool dornic_cell_d(St& s, double alpha_i, double cur,
             const double us = 0.5 - __builtin_fabs(U);
             n = ptrs_k_d(pt, ziggy, U, us);
             if (!ptrs_in_box_d(pt, us, V)) {
-                if (n < 0.0 || (us < 0.013 && V > us)) return false;
-                if (ptrs_estimate(pt, ziggy, n, us, V) <= 0) return false;
+                if (n < 0.0 || (us < 0.013 && V > us)) return kDornicRestart;
+                if (ptrs_estimate(pt, ziggy, n, us, V) <= 0) return kDornicRestart;
             }
             n = count_of(n);
-            gru = mu + 1.0 + n;
-            if (gru < 1.0) return false;
+            big = true;
         }
+        gru = mu + 1.0 + n;
     } else {
         n = poisson_d(s, ziggy, compat);
         gru = mu + 1.0 + n;
     }
     if (compat && gru > 100.0) {
         const double p = s.u64();
-        if (ONE && icdf_in_tail(p)) return false;
+        y = gru;
+        if (ONE && icdf_in_tail(p)) return kDornicGamma;
         y = (norm_icdf_d(p) * dsqrt(gru) + gru) / k.lambda;
-        return true;
+        return kDornicDone;
     }
     double g;
-    if (!gamma_d_try<ONE ? 1 : 64, St>(s, gru, g)) return false;
+    y = gru;
+    if (ONE && big && gru < 1.0) return kDornicGamma;
+    if (!gamma_d_try<ONE ? 1 : 64, St>(s, gru, g)) return kDornicGamma;
     y = g / k.lambda;
-    return true;
+    return kDornicDone;
 }
 
 __device__ __forceinline__ double dornic_cell(Stream& s, double alpha_i, double cur, const DornicConst& k,
@@ -721,7 +747,8 @@ __device__ __forceinline__ bool cell_update_first(const typename StepConst<MODE>
             const double alpha_i = nbr_alpha(c.k.dc, up, dn, lf, rt);
             if (!(alpha_i == 0.0 && cur == (T)0)) {
                 Stream4 st(di.seed, di.inst_id, cell, c.step);
-                if (!dornic_cell_d<true, Stream4>(st, alpha_i, cur, c.k, c.compat != 0, n, y)) return false;
+                if (dornic_cell_d<true, Stream4>(st, alpha_i, cur, c.k, c.compat != 0, n, y) != kDornicDone)
+                    return false;
             }
         }
         if constexpr (MODE == 0) {

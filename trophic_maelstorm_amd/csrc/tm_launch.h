@@ -59,6 +59,9 @@ struct DPCWork {
     double* chunk;        // [nchunks][4]: density sums, vegetation occupied count
     const int2* chunks;   // [nchunks]: (instance, chunk index within it)
     const int2* disk;     // perception offsets (row, column) of every table
+    const int4* vtiles;   // the vegetation's Dornic tiles: (instance, x0, y0, 0)
+    double* pstar;        // ... and its result P*, at cell_off
+    double* lambda;       // lambda of the consumers' cells whose Gamma deviate is deferred, (ns - 1) fields
 };
 // LDS of the consumer step kernel: NS density images with the halo, plus the
 // perception offsets of the largest radius.

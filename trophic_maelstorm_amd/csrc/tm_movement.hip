@@ -29,6 +29,7 @@
 #include "tm_device.h"
 #include "tm_kernels.h"
 #include "tm_launch.h"
+#include "tm_veg.h"
 
 namespace {
 
@@ -963,87 +964,13 @@ void fke_rk_launch(const FkeRk& c, double* fields, double* scratch, unsigned lon
 // d (beta_0 = -M[0] - 4 D_0 / dx^2, FKE:3847-3849).  No flush: the reference
 // flushes after the movement step.
 // ---------------------------------------------------------------------------
-// One kVegTX x kVegTY tile by 256 threads (a wave per row, four rows each), in two
-// passes as dp_tile_deferred: the cells whose first trial does not settle go to a queue
-// in LDS and are finished densely packed.  The cells' neighbours come from the caches.
-// A wave used to run every path its 64 cells took between them: 16 x 256^2 in 36 us.
-constexpr int kVegTX = 64, kVegTY = 16;
-// Up to this many 64 x 4 tiles the model runs one cell a thread instead: us a step of the
-// three-species model, direct / two passes: 45 / 54 on 4 x 64^2, 54 / 61 on 2 x 256^2, 106 /
-// 107 on 8 x 256^2 (2048 tiles), 175 / 171 on 16 x 256^2.
-constexpr int kVegDirectTiles = 2048;
-
-// A cell and its four neighbours (value, up, down, left, right), periodic.
-__device__ __forceinline__ uint32_t veg_stencil(const double* __restrict__ P, int L, int y, int x, double (&v)[5])
-{
-    const uint32_t row = (uint32_t)y * (uint32_t)L, cell = row + (uint32_t)x;
-    v[0] = P[cell];
-    v[1] = P[(uint32_t)(y == 0 ? L - 1 : y - 1) * (uint32_t)L + (uint32_t)x];
-    v[2] = P[(uint32_t)(y == L - 1 ? 0 : y + 1) * (uint32_t)L + (uint32_t)x];
-    v[3] = P[row + (uint32_t)(x == 0 ? L - 1 : x - 1)];
-    v[4] = P[row + (uint32_t)(x == L - 1 ? 0 : x + 1)];
-    return cell;
-}
-
-__device__ __forceinline__ void veg_cell(const tmk::RKConstD& c, const tmk::DevInst& di, int L, int y, int x,
-                                         const double* __restrict__ P, double* __restrict__ Pstar)
-{
-    double v[5], n;
-    bool bad;
-    const uint32_t cell = veg_stencil(P, L, y, x, v);
-    Pstar[cell] = tmk::cell_update<double, 1>(c, di, cell, v[0], v[1], v[2], v[3], v[4], n, bad);
-}
-
-struct VegLds {
-    uint32_t n;
-    uint16_t q[kVegTX * kVegTY];
-};
-
-__device__ __forceinline__ void veg_tile(const tmk::RKConstD& c, const tmk::DevInst& di, int L, int x0, int y0,
-                                         const double* __restrict__ P, double* __restrict__ Pstar, VegLds& sm)
-{
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (threadIdx.x == 0) sm.n = 0u;
-    __syncthreads();
-#pragma unroll 1
-    for (int j = 0; j < kVegTY / 4; ++j) {
-        const int ly = 4 * j + w, y = y0 + ly, x = x0 + lane;
-        const bool in = y < L && x < L;
-        bool done = true;
-        if (in) {
-            double v[5], r, n;
-            bool bad;
-            const uint32_t cell = veg_stencil(P, L, y, x, v);
-            done = tmk::cell_update_first<double, 1>(c, di, cell, v[0], v[1], v[2], v[3], v[4], r, n, bad);
-            if (done) Pstar[cell] = r;
-        }
-        const uint64_t m = __ballot(!done);
-        if (m) {
-            uint32_t base = 0;
-            if (lane == 0) base = atomicAdd(&sm.n, (uint32_t)__popcll(m));   // the queue's order does not matter
-            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-            if (!done) sm.q[base + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = (uint16_t)(ly * kVegTX + lane);
-        }
-    }
-    __syncthreads();
-    const uint32_t nq = sm.n;
-#pragma unroll 1
-    for (uint32_t i = threadIdx.x; i < nq; i += 256) {
-        const uint32_t e = sm.q[i];
-        veg_cell(c, di, L, y0 + (int)(e / kVegTX), x0 + (int)(e % kVegTX), P, Pstar);
-    }
-}
-
 __global__ __launch_bounds__(256) void fke_veg_dornic_kernel(tm_rietkerk_params p, int L, uint32_t seed,
                                                              uint32_t inst, int64_t step, const double* P,
                                                              double* Pstar)
 {
-    __shared__ VegLds sm;
+    __shared__ tmk::VegLds sm;
     const tmk::RKConstD c = tmk::rk_constants(p, step);
-    tmk::DevInst di = {};
-    di.seed = seed;
-    di.inst_id = inst;
-    veg_tile(c, di, L, (int)blockIdx.x * kVegTX, (int)blockIdx.y * kVegTY, P, Pstar, sm);
+    tmk::veg_tile({c.k, seed, inst, c.compat, c.step}, L, (int)blockIdx.x * tmk::kVegTX, (int)blockIdx.y * tmk::kVegTY, P, Pstar, sm);
 }
 
 bool veg_dornic_ok(int L, const tm_rietkerk_params* p)
@@ -1157,7 +1084,7 @@ __device__ __forceinline__ void fke_chunk(const StepArgs& a, const FkeWork* w, i
 // short sums beside the samplers.  DIRECT: one cell a thread on the final kernel's
 // 64 x 4 tiles, in one pass, for batches whose 64 x 16 tiles leave CUs idle.
 template <int SP, bool DIRECT>
-__global__ __launch_bounds__(256) void fke_head_kernel(StepArgs a, int nveg)
+__global__ __launch_bounds__(256, 5) void fke_head_kernel(StepArgs a, int nveg)
 {
     constexpr int NF = 2 * SP + 1;
     static_assert(kMoveTX == kVegTX && kMoveTY == kVegTY, "the movement's tile table");
@@ -1176,12 +1103,13 @@ __global__ __launch_bounds__(256) void fke_head_kernel(StepArgs a, int nveg)
         const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.inst];
         const int y = tl.y0 + (int)(threadIdx.x >> 6), x = tl.x0 + (int)(threadIdx.x & 63);
         if (y >= tl.L || x >= tl.L) return;
-        veg_cell(c, di, tl.L, y, x, (const double*)a.in + (int64_t)NF * tl.cell_off, w->pstar + tl.cell_off);
+        veg_cell({c.k, di.seed, di.inst_id, c.compat, c.step}, tl.L, y, x, (const double*)a.in + (int64_t)NF * tl.cell_off, w->pstar + tl.cell_off);
     } else {
         const int4 tl = w->mtiles[blockIdx.x];
         const DevInst di = a.inst[tl.x];
         const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
-        veg_tile(c, di, di.L, tl.y, tl.z, (const double*)a.in + (int64_t)NF * di.cell_off, w->pstar + di.cell_off, sm.veg);
+        veg_tile({c.k, di.seed, di.inst_id, c.compat, c.step}, di.L, tl.y, tl.z,
+                 (const double*)a.in + (int64_t)NF * di.cell_off, w->pstar + di.cell_off, sm.veg);
     }
 }
 
@@ -2008,7 +1936,7 @@ int tm_fke_veg_dornic(int L, const tm_rietkerk_params* p, uint32_t seed, uint32_
                       const double* P, double* Pstar, void* stream)
 {
     if (!P || !Pstar || P == Pstar || !veg_dornic_ok(L, p)) return TM_ERR_ARG;
-    hipLaunchKernelGGL(fke_veg_dornic_kernel, dim3((unsigned)((L + kVegTX - 1) / kVegTX), (unsigned)((L + kVegTY - 1) / kVegTY)),
+    hipLaunchKernelGGL(fke_veg_dornic_kernel, dim3((unsigned)((L + tmk::kVegTX - 1) / tmk::kVegTX), (unsigned)((L + tmk::kVegTY - 1) / tmk::kVegTY)),
                        dim3(256), 0, (hipStream_t)stream, *p, L, seed, inst, step, P, Pstar);
     return hipGetLastError() == hipSuccess ? TM_OK : TM_ERR_HIP;
 }
