@@ -49,3 +49,42 @@ def test_snapshot_resume_is_exact(tm, tmp_path):
         ctx.run(3)
         resumed = ctx.download(0)
     assert np.array_equal(straight, resumed)
+
+
+@pytest.mark.parametrize("prec,L", [("f64", 181), ("f64", 182), ("f64", 601), ("f32", 257), ("f32", 1023)])
+def test_large_downloads_through_staging(tm, prec, L):
+    """Downloads from 256 KiB on go through pinned staging in 32 KiB pieces and 2 MiB
+    halves: sides that leave ragged pieces and start an instance at any dword, one and
+    several halves, equal to the snapshot of the same fields (a plain copy), from two
+    contexts in turn and from two threads at once."""
+    import threading
+    P = tm.F64 if prec == "f64" else tm.F32
+    insts = [tm.Instance(7, 0, 3, 0), tm.Instance(L, 0, 3, 1), tm.Instance(L, 0, 3, 2)]
+
+    def fields(ctx, k, path):
+        ctx.save_snapshot(k, path)
+        raw = open(path, "rb").read()
+        return np.frombuffer(raw, np.float64 if prec == "f64" else np.float32, offset=64).astype(np.float64).reshape(1, L, L)
+
+    import tempfile
+    with tempfile.TemporaryDirectory() as d, tm.Context() as a, tm.Context() as b:
+        for c in (a, b):
+            c.configure(tm.MODEL_DP, P, tm.DPParams(), insts)
+            c.init_uniform([0.0], [1.0])
+            c.run(2)
+        want = [fields(a, k, f"{d}/s{k}") for k in (1, 2)]
+        for c in (a, b, a):
+            for k in (1, 2):
+                assert np.array_equal(c.download(k), want[k - 1])
+        got = {}
+
+        def many(name, c):
+            got[name] = [c.download(k) for _ in range(6) for k in (1, 2)]
+
+        ts = [threading.Thread(target=many, args=(n, c)) for n, c in (("a", a), ("b", b))]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for r in got.values():
+            assert len(r) == 12 and all(np.array_equal(x, want[i % 2]) for i, x in enumerate(r))

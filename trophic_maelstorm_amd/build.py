@@ -38,6 +38,7 @@ UNITS = {
     "tm_movement.hip": ["-ffp-contract=off", *NO_LICM],
     "tm_api.cpp": ["-ffp-contract=off"],
     "tm_io.cpp": ["-ffp-contract=off"],
+    "tm_hostcopy.hip": [],
 }
 
 

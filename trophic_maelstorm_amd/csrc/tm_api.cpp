@@ -20,12 +20,14 @@
 #include <cstring>
 #include <fstream>
 #include <map>
+#include <memory>
 #include <sstream>
 #include <string>
 #include <sys/stat.h>
 #include <vector>
 
 #include "tm/tm.h"
+#include "tm_hostcopy.h"
 #include "tm_io.h"
 #include "tm_launch.h"
 #include "tm_veg.h"
@@ -120,6 +122,9 @@ struct tm_ctx {
     int dpc_vtiles = 0, dpc_vdirect = 0;   // DP consumers: the vegetation's Dornic tiles
     FkeGrid fke = {};              // Rietkerk consumer models: launch sizes (FkeWork in d_dpc)
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
+
+    std::shared_ptr<HostCopier> copier;   // large downloads; taken at the first one
+    bool copier_tried = false;
 };
 
 namespace {
@@ -945,6 +950,10 @@ tm_status tm_upload_fields(tm_ctx* c, int i, const double* host)
     return TM_OK;
 }
 
+// Instances of this many bytes on are downloaded through the HostCopier: 23 us against 31
+// at 512 KiB of FP64, 18 against 26 at 256 KiB of FP32; at 128 KiB the two are within 2 us.
+constexpr size_t kStagedCopyMin = (size_t)256 << 10;
+
 tm_status tm_download_fields(tm_ctx* c, int i, double* host)
 {
     tm_status s = check_ready(c);
@@ -953,6 +962,17 @@ tm_status tm_download_fields(tm_ctx* c, int i, double* host)
     const int64_t n = (int64_t)c->nf * c->inst[i].L * c->inst[i].L;
     const char* src = (const char*)c->d_fields[c->parity] + c->esize * c->nf * c->cell_off[i];
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    if ((size_t)n * c->esize >= kStagedCopyMin) {
+        if (!c->copier_tried) {
+            c->copier_tried = true;
+            c->copier = HostCopier::get(c->device);
+        }
+        if (c->copier) {
+            const HostCopier::Result r = c->copier->copy(host, src, (size_t)n, c->prec == TM_F32);
+            if (r == HostCopier::kOk) return TM_OK;
+            if (r == HostCopier::kFailed) return fail(c, TM_ERR_HIP, "tm_download_fields: copy failed");
+        }   // else another thread's copy runs: straight into the caller's memory
+    }
     if (c->prec == TM_F64) {
         HIPCHK(c, hipMemcpy(host, src, sizeof(double) * n, hipMemcpyDeviceToHost));
     } else {
