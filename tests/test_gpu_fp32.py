@@ -329,3 +329,27 @@ def test_small_batch_dp_parts_are_identical(tm, prec, n):
     assert np.array_equal(r0, r1)
     for k in range(len(Ls)):
         assert np.array_equal(f0[k], f1[k]) and np.array_equal(d0[k], d1[k])
+
+
+@pytest.mark.parametrize("want", ["rk_f32_frame_16x16", "rk_f32_frame_32x16", "rk_f32_frame_32x24", "rk_f32_frame_32x32"])
+def test_fp32_rietkerk_frames_are_identical(tm, want):
+    """The frame form of the fused FP32 Rietkerk step gives the tile form's draws and
+    fields bit for bit, on lattices smaller than a tile, one cell past it and larger;
+    the rows (sums of other tiles) to FP64 rounding."""
+    names = tm.variant_names(tm.MODEL_RIETKERK, tm.F32)
+    insts = [tm.Instance(L, k % 2, 8, k) for k, L in enumerate([5, 10, 11, 27, 53, 130])]
+    ps = [tm.RietkerkParams(R=0.9), tm.RietkerkParams(R=1.2, sampler=tm.SAMPLER_COMPAT)]
+    out = []
+    for v in ("rk_f32_16x16_t256", want):
+        with tm.Context() as ctx:
+            ctx.configure(tm.MODEL_RIETKERK, tm.F32, ps, insts)
+            ctx.set_launch(names.index(v), 5)
+            ctx.init_uniform([0, 0, 0], [90, 1, 1])
+            ctx.record_draws(True)
+            rows = ctx.run(8)
+            out.append((np.concatenate([ctx.download(k).ravel() for k in range(len(insts))]),
+                        np.concatenate([ctx.draws(k).ravel() for k in range(len(insts))]), rows))
+    (f0, d0, r0), (f1, d1, r1) = out
+    assert np.array_equal(d0, d1)
+    assert np.array_equal(f0, f1)
+    assert np.allclose(r0, r1, rtol=1e-12, atol=0)

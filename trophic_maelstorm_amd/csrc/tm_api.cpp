@@ -893,7 +893,7 @@ tm_status tm_configure(tm_ctx* c, int model, int precision, const void* params, 
         c->cell_off[i] = c->total_cells;
         c->total_cells += (int64_t)instances[i].L * instances[i].L;
     }
-    c->variant = default_variant(model, precision, c->total_cells);
+    c->variant = default_variant(model, precision, c->inst.data(), (int)c->inst.size(), c->n_cu);
     {   // whole multi-step launches per graph block, as tm_set_launch makes them
         const int spl = cur_variant(c).spl;
         if (spl > 1 && c->graph_steps > 0) c->graph_steps = (c->graph_steps + spl - 1) / spl * spl;
@@ -1304,7 +1304,7 @@ tm_status tm_set_launch(tm_ctx* c, int variant, int graph_steps)
     const int n = tm_variant_count(c->model, c->prec);
     if (variant < -1 || variant >= n) return fail(c, TM_ERR_ARG, "variant out of range");
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    c->variant = variant < 0 ? default_variant(c->model, c->prec, c->total_cells) : variant;
+    c->variant = variant < 0 ? default_variant(c->model, c->prec, c->inst.data(), (int)c->inst.size(), c->n_cu) : variant;
     // A graph block of a multi-step variant is a whole number of its launches:
     // a remainder would run as single steps in every block.
     const int spl = cur_variant(c).spl;
@@ -1622,7 +1622,51 @@ tm_status tm_replicate_stats(tm_ctx* c, int flags, double* stats)
 }  // extern "C"
 
 namespace tmk {
-int default_variant(int model, int precision, int64_t total_cells)
+// Tiles of tx x ty the batch's lattices take; those of odd sides count `odd` times.
+static double batch_tiles(const tm_instance_desc* inst, int n_inst, int tx, int ty, double odd = 1.0)
+{
+    double n = 0.0;
+    for (int i = 0; i < n_inst; ++i)
+        n += (double)((inst[i].L + tx - 1) / tx) * ((inst[i].L + ty - 1) / ty) * (inst[i].L % 2 ? odd : 1.0);
+    return n;
+}
+
+// Rietkerk.  Small batches are latency-bound and take the fused step on the frame that
+// puts the fewest waves on the busiest CU (a 1024-thread frame only at one workgroup a CU:
+// in two rounds its barriers cost more).  FP64, us a step at 4 / 8 / 12 / 16 / 24 waves: 10.0
+// (64^2, 128^2), 12.0 (181^2), 14.6 (256^2), 17.4 (384^2), 26.1 (450^2); the split step from
+// there (512^2: 28.2, 30 fused; 600^2: 34, 39).  FP32: 8.3 at 12 waves (256^2), 22.0 at 60
+// (725^2), 35.5 at 108 (1024^2, split 39.1), 37.9 at 120 (16 x 257^2, split 48); at 216
+// (1448^2) 66 against 52.
+// The split step samples each P* once; its RK4 runs on 32 x 16 tiles staged in LDS, or in
+// FP64 on frames of 26 x 10 tiles, whichever has the less to do: a frame tile costs 0.55
+// of the other, odd sides 1.3 times more to stage.  32 x 16 against frames: 57.0 / 59.2 on
+// 16 x 250^2, 163 / 182 on 16 x 512^2, 52 / 49 on 64 x 100^2, 119 / 107 on 8 x 513^2, 83 / 68 on
+// 64 x 129^2, 48 / 45 on 16 x 187^2.
+static const char* rietkerk_default(int precision, const tm_instance_desc* inst, int n_inst, int n_cu)
+{
+    struct Frame { int fx, fy; const char* f64; const char* f32; };
+    static const Frame frames[] = {{16, 16, "rk_f64_frame_16x16", "rk_f32_frame_16x16"},
+                                   {32, 16, "rk_f64_frame_32x16", "rk_f32_frame_32x16"},
+                                   {32, 24, "rk_f64_frame_32x24", "rk_f32_frame_32x24"},
+                                   {32, 32, "rk_f64_frame_32x32", "rk_f32_frame_32x32"}};
+    double best = 1e300;
+    const Frame* pick = nullptr;
+    for (const Frame& f : frames) {
+        const double per_cu = std::ceil(batch_tiles(inst, n_inst, f.fx - 6, f.fy - 6) / std::max(1, n_cu));
+        const double waves = per_cu * (f.fx * f.fy / 64);
+        if (waves < best && (f.fy < 32 || per_cu <= 1.0)) {
+            best = waves;
+            pick = &f;
+        }
+    }
+    if (best <= (precision == TM_F64 ? 24.0 : 120.0)) return precision == TM_F64 ? pick->f64 : pick->f32;
+    if (precision == TM_F32) return "rk_f32_split_32x16_t256_q24";
+    return batch_tiles(inst, n_inst, 32, 16, 1.3) > 0.55 * batch_tiles(inst, n_inst, 26, 10) ? "rk_f64_split_frame_32x16"
+                                                                                            : "rk_f64_split_32x16_t256_q16";
+}
+
+int default_variant(int model, int precision, const tm_instance_desc* inst, int n_inst, int n_cu)
 {
     const char* want;
     if (model == TM_MODEL_FKE2 || model == TM_MODEL_FKE3) {
@@ -1637,14 +1681,7 @@ int default_variant(int model, int precision, int64_t total_cells)
         // trials), eight steps per launch once the field is mostly absorbing
         want = precision == TM_F64 ? "dp_f64_64x32_t256_x8aq_w6" : "dp_f32_128x24_t256_x8aq";
     } else {
-        // Rietkerk: small lattices are latency-bound and want the single fused
-        // 16 x 16 launch; batches want the split step (each P* sampled once) with
-        // the two-pass Dornic kernel, in FP32 on 128 x 24 tiles (256 x 512^2:
-        // 4.6e10 against 4.3e10 cell-updates/s for the one-pass 128 x 32 kernel).
-        // FP64, fused against split: 22.9 / 26.6 us a step at 384^2, 28.0 / 27.9 at
-        // 512^2, 59.8 / 50.2 at 453,000 cells, 86.4 / 56.3 at 1024^2.
-        if (total_cells < (precision == TM_F64 ? 1 << 18 : 1 << 20)) return 0;
-        want = precision == TM_F64 ? "rk_f64_split_32x16_t256_q16" : "rk_f32_split_32x16_t256_q24";
+        want = rietkerk_default(precision, inst, n_inst, n_cu);
     }
     const int n = tm_variant_count(model, precision);
     for (int v = 0; v < n; ++v)

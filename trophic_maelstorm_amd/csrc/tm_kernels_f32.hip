@@ -88,6 +88,12 @@ static const Variant kDP[] = {
      &launch_dp_default, 20},
 };
 
+template <typename T, int FX, int FY, bool SPLIT>
+static void launch_frame(const StepArgs& a, int grid, hipStream_t s)
+{
+    hipLaunchKernelGGL((rk_frame_kernel<T, FX, FY, SPLIT>), dim3(grid), dim3(FX * FY), 0, s, a);
+}
+
 static const Variant kRK[] = {
     {16, 16, 256, 0, 1, "rk_f32_16x16_t256", &launch_rk<float, 16, 16, 256>},
     {32, 16, 256, 0, 1, "rk_f32_32x16_t256", &launch_rk<float, 32, 16, 256>},
@@ -106,6 +112,12 @@ static const Variant kRK[] = {
      &launch_dp<float, 128, 32, 256, 1, 1, 1>},
     {32, 16, 256, 0, 1, "rk_f32_split_32x16_t256_q24", &launch_rk<float, 32, 16, 256, true>, 128, 24,
      &launch_dp<float, 128, 24, 256, 1, 1, 1>},
+    // frame_FXxFY: a thread per cell of the frame around a tile 6 narrower and shorter
+    // (rk_frame_kernel), fused for small batches
+    {26, 26, 1024, 0, 1, "rk_f32_frame_32x32", &launch_frame<float, 32, 32, false>},
+    {26, 10, 512, 0, 1, "rk_f32_frame_32x16", &launch_frame<float, 32, 16, false>},
+    {10, 10, 256, 0, 1, "rk_f32_frame_16x16", &launch_frame<float, 16, 16, false>},
+    {26, 18, 768, 0, 1, "rk_f32_frame_32x24", &launch_frame<float, 32, 24, false>},
 };
 
 const Variant* dp_variants_f32(int* n) { *n = (int)(sizeof(kDP) / sizeof(kDP[0])); return kDP; }

@@ -69,6 +69,12 @@ static const Variant kDP[] = {
      &launch_dp_default, 20},
 };
 
+template <typename T, int FX, int FY, bool SPLIT>
+static void launch_frame(const StepArgs& a, int grid, hipStream_t s)
+{
+    hipLaunchKernelGGL((rk_frame_kernel<T, FX, FY, SPLIT>), dim3(grid), dim3(FX * FY), 0, s, a);
+}
+
 static const Variant kRK[] = {
     {16, 16, 256, 0, 1, "rk_f64_16x16_t256", &launch_rk<double, 16, 16, 256>},
     {32, 16, 256, 0, 1, "rk_f64_32x16_t256", &launch_rk<double, 32, 16, 256>},
@@ -85,6 +91,14 @@ static const Variant kRK[] = {
     // tiles 202; other tiles (64 x 8, 64 x 32, 128 x 16) and bounds 166 to 178.
     {32, 16, 256, 0, 1, "rk_f64_split_32x16_t256_q16", &launch_rk<double, 32, 16, 256, true>, 64, 16,
      &launch_dp<double, 64, 16, 256, 1, 6, 1>},
+    // frame_FXxFY: a thread per cell of the frame around a tile 6 narrower and shorter
+    // (rk_frame_kernel), fused for small batches, split with the two-pass Dornic kernel
+    {26, 26, 1024, 0, 1, "rk_f64_frame_32x32", &launch_frame<double, 32, 32, false>},
+    {26, 10, 512, 0, 1, "rk_f64_frame_32x16", &launch_frame<double, 32, 16, false>},
+    {26, 10, 512, 0, 1, "rk_f64_split_frame_32x16", &launch_frame<double, 32, 16, true>, 64, 16,
+     &launch_dp<double, 64, 16, 256, 1, 6, 1>},
+    {10, 10, 256, 0, 1, "rk_f64_frame_16x16", &launch_frame<double, 16, 16, false>},
+    {26, 18, 768, 0, 1, "rk_f64_frame_32x24", &launch_frame<double, 32, 24, false>},
 };
 
 const Variant* dp_variants_f64(int* n) { *n = (int)(sizeof(kDP) / sizeof(kDP[0])); return kDP; }

@@ -91,8 +91,8 @@ void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t
 // Free the device scratch the Rietkerk consumer operators keep between calls.
 void workspace_give_back();
 
-// Default variant index per (model, precision, batch size in cells).
-int default_variant(int model, int precision, int64_t total_cells);
+// Default variant index of a batch.
+int default_variant(int model, int precision, const tm_instance_desc* inst, int n_inst, int n_cu);
 
 void launch_measure_f64(int nf, const DevInst* inst, const DevTile* tiles, int ntiles, int tx, int ty,
                         const void* fields, double2* partials, hipStream_t s);
