@@ -39,6 +39,7 @@ UNITS = {
     "tm_api.cpp": ["-ffp-contract=off"],
     "tm_io.cpp": ["-ffp-contract=off"],
     "tm_hostcopy.hip": [],
+    "tm_groups.hip": [],
 }
 
 

@@ -27,12 +27,19 @@
 #include <vector>
 
 #include "tm/tm.h"
+#include "tm_groups.h"
 #include "tm_hostcopy.h"
 #include "tm_io.h"
 #include "tm_launch.h"
 #include "tm_veg.h"
 
 using namespace tmk;
+
+// A place in the batch's instances and in the launch tables that follow their order.
+struct GroupPos {
+    int inst, tile, tile_a;                          // step tiles, the split step's Dornic tiles
+    int chunk, vtile, rtile, mtile, block;           // consumer models
+};
 
 struct tm_ctx {
     int device = 0;
@@ -77,6 +84,13 @@ struct tm_ctx {
     bool record_draws = false;
     double* h_pinned = nullptr;   // small pinned staging for state writes
 
+    // Instance groups (group_cut): where the second begins and the batch ends.  A run of
+    // such a batch takes a lane and, while it is alone, a second one for the second group.
+    GroupPos cut = {}, end = {};
+    std::shared_ptr<RunLanes> lanes;
+    int lane[2] = {-1, -1};
+    hipStream_t q = nullptr;   // where launches go: `stream`, or during a run its lane
+
     int parity = 0;
     int64_t counter = 0;
 
@@ -117,10 +131,9 @@ struct tm_ctx {
 
     // consumer models: DPCWork, per-instance tables, chunk sums, perception offsets
     void* d_dpc = nullptr;
-    int dpc_nchunks = 0;
     int dpc_halo = 1;
-    int dpc_vtiles = 0, dpc_vdirect = 0;   // DP consumers: the vegetation's Dornic tiles
-    FkeGrid fke = {};              // Rietkerk consumer models: launch sizes (FkeWork in d_dpc)
+    int dpc_vdirect = 0;           // DP consumers: the vegetation's Dornic tiles, one cell a thread
+    int move_lds = 0;              // Rietkerk consumers: LDS of the movement tile
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
 
     std::shared_ptr<HostCopier> copier;   // large downloads; taken at the first one
@@ -259,9 +272,9 @@ void release_config(tm_ctx* c)
     free_dev(c->d_live);
     free_dev(c->d_dpc);
     free_dev(c->d_mov);
-    c->dpc_nchunks = 0;
     c->dpc_halo = 1;
-    c->fke = FkeGrid{};
+    c->move_lds = 0;
+    c->cut = c->end = GroupPos{};
     invalidate_live(c);
     c->series_cap = c->groups_cap = c->stats_cap = c->frame_tab_cap = 0;
     c->series_steps_cap = c->n_series = 0;
@@ -275,6 +288,33 @@ const Variant& cur_variant(tm_ctx* c)
     int n;
     const Variant* v = variant_table(c->model, c->prec, &n);
     return v[c->variant];
+}
+
+// Where the second of two instance groups begins, or 0 for one group.  The cut makes the
+// larger group smallest.  Below kGroupCells the second chain of launches costs more than
+// it fills (us a step, one group / two): 8 x 128^2 FP64 DP 8.7 / 8.9, two-species DP
+// consumers 42.2 / 42.7, three-species Rietkerk consumers 53.2 / 54.5, FP32 Rietkerk at
+// 10 x 128^2 9.4 / 9.8; 12 x 128^2: FP64 DP 11.2 / 9.1, FP64 and FP32 Rietkerk 25.9 / 21.7
+// and 11.0 / 9.0, consumers 47.6 / 45.1 and 64.6 / 57.6.  A cell of FP32 DP costs least:
+// 16 x 128^2 6.7 / 7.6, 24 x 128^2 8.5 / 7.4.  A group of under a twentieth of the cells
+// has nothing to fill the other's gaps with (1024^2 + 64^2 of FP32 Rietkerk 35.8 / 36.7;
+// 1024^2 + 4 x 128^2 of FP64 61.9 / 58.5).
+constexpr int64_t kGroupCells = 12 * 128 * 128;
+
+int group_cut(tm_ctx* c)
+{
+    if (c->total_cells < (c->model == TM_MODEL_DP && c->prec == TM_F32 ? 2 : 1) * kGroupCells) return 0;
+    int cut = 0;
+    int64_t larger = c->total_cells;
+    for (size_t i = 1; i < c->inst.size(); ++i) {
+        const int64_t m = std::max(c->cell_off[i], c->total_cells - c->cell_off[i]);
+        if (m < larger) {
+            larger = m;
+            cut = (int)i;
+        }
+    }
+    if (20 * (c->total_cells - larger) < c->total_cells) return 0;
+    return c->lanes && c->lanes->prepare() ? cut : 0;
 }
 
 // (Re)build the tile table for the current variant and upload it with the
@@ -295,6 +335,7 @@ tm_status build_tiles(tm_ctx* c)
         di.step0 = d.step0;
         di.cell_off = c->cell_off[i];
         di.tile0 = (int32_t)c->tiles.size();
+        if ((int)i == c->cut.inst) c->cut.tile = di.tile0;
         // Vertical strips: consecutive tiles share a halo row, but the
         // workgroups in flight then read the same columns a row stride apart.
         // Along rows: the workgroups in flight read contiguous addresses.
@@ -310,23 +351,29 @@ tm_status build_tiles(tm_ctx* c)
         di.ntiles = (int32_t)c->tiles.size() - di.tile0;
         c->dinst.push_back(di);
     }
+    c->end.inst = (int)c->inst.size();
+    c->end.tile = (int)c->tiles.size();
     free_dev(c->d_tiles);
     free_dev(c->d_partials);
     HIPCHK(c, hipMalloc((void**)&c->d_tiles, sizeof(DevTile) * c->tiles.size()));
     HIPCHK(c, hipMemcpy(c->d_tiles, c->tiles.data(), sizeof(DevTile) * c->tiles.size(), hipMemcpyHostToDevice));
     free_dev(c->d_tiles_a);
     c->tiles_a.clear();
+    c->cut.tile_a = 0;
     if (v.fn_a) {   // split step: the Dornic kernel's own tiles, and the P* field
-        for (size_t i = 0; i < c->inst.size(); ++i)
+        for (size_t i = 0; i < c->inst.size(); ++i) {
+            if ((int)i == c->cut.inst) c->cut.tile_a = (int)c->tiles_a.size();
             for (int x0 = 0; x0 < c->inst[i].L; x0 += v.ax)
                 for (int y0 = 0; y0 < c->inst[i].L; y0 += v.ay)
                     c->tiles_a.push_back(DevTile{(int32_t)i, x0, y0, c->inst[i].L, c->cell_off[i]});
+        }
         HIPCHK(c, hipMalloc((void**)&c->d_tiles_a, sizeof(DevTile) * c->tiles_a.size()));
         HIPCHK(c, hipMemcpy(c->d_tiles_a, c->tiles_a.data(), sizeof(DevTile) * c->tiles_a.size(),
                             hipMemcpyHostToDevice));
         if (!c->d_aux && hipMalloc(&c->d_aux, c->esize * (size_t)c->total_cells) != hipSuccess)
             return fail(c, TM_ERR_NOMEM, "P* field allocation failed");
     }
+    c->end.tile_a = (int)c->tiles_a.size();
     if (!c->d_inst) HIPCHK(c, hipMalloc((void**)&c->d_inst, sizeof(DevInst) * c->dinst.size()));
     HIPCHK(c, hipMemcpy(c->d_inst, c->dinst.data(), sizeof(DevInst) * c->dinst.size(), hipMemcpyHostToDevice));
     c->nslots = 64;   // a power of two >= the graph block (kernels mask the slot index)
@@ -338,43 +385,55 @@ tm_status build_tiles(tm_ctx* c)
     return TM_OK;
 }
 
-StepArgs step_args(tm_ctx* c, int parity, int k)
+// The launch of instance group g (0: up to the cut, 1: from it), or of the whole batch
+// (kWholeBatch).
+constexpr int kWholeBatch = -1;
+ConsumerArgs step_args(tm_ctx* c, int parity, int k, int g = kWholeBatch)
 {
-    StepArgs a{};
+    const GroupPos lo = g == 1 ? c->cut : GroupPos{}, hi = g == 0 ? c->cut : c->end;
+    ConsumerArgs a{};
     a.inst = c->d_inst;
-    a.tiles = c->d_tiles;
+    a.tiles = c->d_tiles + lo.tile;
     a.consts = c->d_consts;
     a.in = c->d_fields[parity];
     a.out = c->d_fields[parity ^ 1];
-    a.partials = c->d_partials;
+    a.partials = c->d_partials + (size_t)lo.tile * cur_variant(c).pw * c->nf;
     a.state = c->d_state;
+    a.fault = c->d_state->fault + (g == 1 ? 1 : 0);
     a.draws = c->record_draws ? c->d_draws : nullptr;
-    a.tiles_a = c->d_tiles_a;
+    a.tiles_a = c->d_tiles_a + lo.tile_a;
     a.aux = c->d_aux;
-    a.ntiles_a = (int32_t)c->tiles_a.size();
-    a.ntiles = (int32_t)c->tiles.size();
+    a.ntiles_a = hi.tile_a - lo.tile_a;
+    a.ntiles = hi.tile - lo.tile;
+    a.ptiles = c->end.tile;
     a.nslots = c->nslots;
     a.k = k;
     a.n_inst = (int32_t)c->inst.size();
     a.xcd = c->xcd;
     a.work = c->d_dpc;
-    a.nchunks = c->dpc_nchunks;
+    a.nchunks = hi.chunk - lo.chunk;
     a.halo = c->dpc_halo;
-    a.nvtiles = c->dpc_vtiles;
+    a.nvtiles = hi.vtile - lo.vtile;
     a.vdirect = c->dpc_vdirect;
-    a.nblocks = c->fke.blocks;
-    a.nrtiles = c->fke.rtiles;
-    a.nmtiles = c->fke.mtiles;
-    a.move_lds = c->fke.move_lds;
+    a.nblocks = hi.block - lo.block;
+    a.nrtiles = hi.rtile - lo.rtile;
+    a.nmtiles = hi.mtile - lo.mtile;
+    a.move_lds = c->move_lds;
+    a.inst0 = lo.inst;
+    a.inst1 = hi.inst;
+    a.chunk0 = lo.chunk;
+    a.vtile0 = lo.vtile;
+    a.rtile0 = lo.rtile;
+    a.mtile0 = lo.mtile;
+    a.block0 = lo.block;
     return a;
 }
 
 // Persistent variants launch wg_per_cu workgroups per CU, each walking a
 // contiguous tile range; the others launch one workgroup per tile.
-int grid_of(tm_ctx* c)
+int grid_of(tm_ctx* c, int n)
 {
     const Variant& v = cur_variant(c);
-    const int n = (int)c->tiles.size();
     if (v.wg_per_cu <= 0) return n;
     return std::max(1, std::min(n, c->n_cu * v.wg_per_cu));
 }
@@ -382,13 +441,14 @@ int grid_of(tm_ctx* c)
 // One launch advancing steps k .. k + m - 1: m = the variant's steps per launch,
 // or 1 (a multi-step variant's single-step kernel: single-step mode, or a
 // block's last steps).
-void launch_step(tm_ctx* c, int parity, int k, int m = 1)
+void launch_step(tm_ctx* c, int parity, int k, int m = 1, int g = kWholeBatch)
 {
-    const StepArgs a = step_args(c, parity, k);
+    const ConsumerArgs a = step_args(c, parity, k, g);
     const Variant& v = cur_variant(c);
-    if (v.fn_a) v.fn_a(a, (int)c->tiles_a.size(), c->stream);   // split: P* first
+    const hipStream_t s = g == 1 ? c->lanes->stream(c->lane[1]) : c->q;
+    if (v.fn_a) v.fn_a(a, a.ntiles_a, s);   // split: P* first
     const StepLaunch fn = (v.spl > 1 && m == 1) ? v.fn_one : v.fn;
-    fn(a, grid_of(c), c->stream);
+    fn(a, grid_of(c, a.ntiles), s);
 }
 
 // Bookkeeping of tm_mode_steps: n steps of one block in the current mode.
@@ -428,23 +488,83 @@ void launch_fold(tm_ctx* c, int nsteps)
     a.rows_cap = c->rows_cap;
     a.measure = 0;
     a.pw = cur_variant(c).pw;
-    launch_combine(a, (int)c->inst.size(), nsteps, c->stream);
+    launch_combine(a, (int)c->inst.size(), nsteps, c->q);
+}
+
+// A run, from before its first launch to after its last wait: counted, and, with `lanes`,
+// a grouped batch's launches in a lane of its own, after what is on the context's stream.
+class Run {
+public:
+    Run(tm_ctx* c, bool lanes) : c_(c)
+    {
+        if (!c->lanes) return;
+        c->lanes->begin();
+        if (!lanes || c->cut.inst == 0 || (c->lane[0] = c->lanes->take()) < 0) return;
+        c->q = c->lanes->stream(c->lane[0]);
+        if (!c->lanes->order(c->lane[0], c->stream, c->q)) c->q = c->stream;
+    }
+    ~Run()
+    {
+        c_->q = c_->stream;
+        if (!c_->lanes) return;
+        for (int& l : c_->lane) {
+            if (l < 0) continue;
+            (void)hipStreamSynchronize(c_->lanes->stream(l));   // done already unless the run failed
+            c_->lanes->give(l);
+            l = -1;
+        }
+        c_->lanes->end();
+    }
+    Run(const Run&) = delete;
+    Run& operator=(const Run&) = delete;
+
+private:
+    tm_ctx* c_;
+};
+
+// The second group's lane for the next block: while the run is in a lane and alone.
+bool take_second_lane(tm_ctx* c)
+{
+    if (c->lane[0] < 0 || c->q == c->stream || !c->lanes->alone()) return false;
+    if (c->lane[1] < 0) c->lane[1] = c->lanes->take();
+    return c->lane[1] >= 0;
+}
+
+void join_second_lane(tm_ctx* c)
+{
+    const hipStream_t side = c->lanes->stream(c->lane[1]);
+    if (!c->lanes->order(c->lane[1], side, c->q)) (void)hipStreamSynchronize(side);
 }
 
 // One block of n <= nslots steps starting from buffer `parity`: constants,
 // n step launches, the rows fold (optional) and the counter bump.
-void enqueue_block(tm_ctx* c, int parity, int n, bool fold)
+// grouped: the step launches by instance group on two lanes, while the run has both;
+// never under capture (a graph's branches would pick their own queues).
+void enqueue_block(tm_ctx* c, int parity, int n, bool fold, bool grouped)
 {
-    launch_prep(c->model, c->d_inst, c->d_params, c->d_state, (int)c->inst.size(), n, c->d_consts, c->stream);
+    launch_prep(c->model, c->d_inst, c->d_params, c->d_state, (int)c->inst.size(), n, c->d_consts, c->q);
     const int spl = steps_per_launch(c);
+    if (grouped) grouped = take_second_lane(c);
+    const hipStream_t side = grouped ? c->lanes->stream(c->lane[1]) : nullptr;
+    if (grouped) grouped = c->lanes->order(c->lane[1], c->q, side);
     for (int k = 0; k < n;) {
         const int m = k + spl <= n ? spl : 1;
-        launch_step(c, parity, k, m);
+        if (grouped && !c->lanes->alone()) {   // another run began since: one chain each
+            join_second_lane(c);
+            grouped = false;
+        }
+        if (grouped) {
+            launch_step(c, parity, k, m, 0);
+            launch_step(c, parity, k, m, 1);
+        } else {
+            launch_step(c, parity, k, m);
+        }
         parity ^= 1;
         k += m;
     }
+    if (grouped) join_second_lane(c);
     if (fold) launch_fold(c, n);
-    launch_bump(c->d_state, n, c->stream);
+    launch_bump(c->d_state, n, c->q);
 }
 
 // Capture one block of n steps (with or without the rows fold) for a parity:
@@ -453,7 +573,7 @@ tm_status capture_block(tm_ctx* c, int parity, int n, bool fold, hipGraphExec_t*
 {
     hipGraph_t g = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_block(c, parity, n, fold);
+    enqueue_block(c, parity, n, fold, false);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (e != hipSuccess) return fail(c, TM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
@@ -492,7 +612,7 @@ tm_status set_run_base(tm_ctx* c)
     // run_base <- counter, ordered on the stream before the step launches.
     *(int64_t*)c->h_pinned = c->counter;
     HIPCHK(c, hipMemcpyAsync((char*)c->d_state + offsetof(DevState, run_base), c->h_pinned, sizeof(int64_t),
-                             hipMemcpyHostToDevice, c->stream));
+                             hipMemcpyHostToDevice, c->q));
     return TM_OK;
 }
 
@@ -503,10 +623,10 @@ void enqueue_measure(tm_ctx* c, double* out, int64_t stride)
     const Variant& v = cur_variant(c);
     if (c->prec == TM_F64)
         launch_measure_f64(c->nf, c->d_inst, c->d_tiles, (int)c->tiles.size(), v.tx, v.ty, c->d_fields[c->parity],
-                           c->d_partials, c->stream);
+                           c->d_partials, c->q);
     else
         launch_measure_f32(c->nf, c->d_inst, c->d_tiles, (int)c->tiles.size(), v.tx, v.ty, c->d_fields[c->parity],
-                           c->d_partials, c->stream);
+                           c->d_partials, c->q);
     CombineArgs a{};
     a.inst = c->d_inst;
     a.partials = c->d_partials;
@@ -519,7 +639,7 @@ void enqueue_measure(tm_ctx* c, double* out, int64_t stride)
     a.rows_cap = stride;
     a.measure = 1;
     a.pw = 1;
-    launch_combine(a, (int)c->inst.size(), 1, c->stream);
+    launch_combine(a, (int)c->inst.size(), 1, c->q);
 }
 
 tm_status ensure_live(tm_ctx* c)
@@ -540,10 +660,10 @@ tm_status live_fraction_now(tm_ctx* c, double* frac)
     const int n = (int)c->inst.size();
     double* sums = c->d_live + 2 * c->nf * n;
     enqueue_measure(c, c->d_live, 1);
-    launch_live_count(c->d_live, 1, 2 * c->nf, 0, n, sums, c->stream);
+    launch_live_count(c->d_live, 1, 2 * c->nf, 0, n, sums, c->q);
     double occ = 0.0;
-    HIPCHK(c, hipMemcpyAsync(&occ, sums, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, hipMemcpyAsync(&occ, sums, sizeof(double), hipMemcpyDeviceToHost, c->q));
+    HIPCHK(c, hipStreamSynchronize(c->q));
     *frac = occ / (double)c->total_cells;
     return TM_OK;
 }
@@ -604,15 +724,15 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
         }
         double* sums = c->d_live + 2 * c->nf * c->inst.size();
         launch_live_count(c->d_rows, c->rows_cap, 2 * c->nf, n_steps - left - 1, (int)c->inst.size(), sums + j,
-                          c->stream);
-        HIPCHK(c, hipMemcpyAsync((void*)(h_sum + j), sums + j, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipEventRecord(c->live_ev[j], c->stream));
+                          c->q);
+        HIPCHK(c, hipMemcpyAsync((void*)(h_sum + j), sums + j, sizeof(double), hipMemcpyDeviceToHost, c->q));
+        HIPCHK(c, hipEventRecord(c->live_ev[j], c->q));
         c->live_pending[j] = true;
         c->live_block += 1;
         return update_mode(c);
     };
     while (B > 0 && left >= B) {
-        enqueue_block(c, c->parity, B, true);
+        enqueue_block(c, c->parity, B, true, true);
         HIPCHK(c, hipGetLastError());
         count_steps(c, B);
         c->counter += B;
@@ -622,7 +742,7 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
     }
     while (left > 0) {
         const int chunk = (int)std::min<int64_t>(left, c->nslots);
-        enqueue_block(c, c->parity, chunk, true);
+        enqueue_block(c, c->parity, chunk, true, true);
         HIPCHK(c, hipGetLastError());
         count_steps(c, chunk);
         c->parity ^= (launches_of(c, chunk) & 1);
@@ -641,10 +761,13 @@ tm_status read_fault(tm_ctx* c, int32_t* inst, int64_t* cell, int64_t* step)
     *inst = -1;
     *cell = -1;
     *step = -1;
-    if (st.fault_counter != ~0ull) {
-        *inst = (int32_t)((st.fault_key >> 40) & 0xFFFFF);   // bits 60..63: the step's place in its launch
-        *cell = (int64_t)(st.fault_key & ((1ull << 40) - 1));
-        *step = (*inst >= 0 && *inst < (int)c->inst.size() ? c->inst[*inst].step0 : 0) + (int64_t)st.fault_counter;
+    Fault f = st.fault[0];   // the groups' earliest
+    for (const Fault& o : st.fault)
+        if (o.counter < f.counter || (o.counter == f.counter && o.key < f.key)) f = o;
+    if (f.counter != ~0ull) {
+        *inst = (int32_t)((f.key >> 40) & 0xFFFFF);   // bits 60..63: the step's place in its launch
+        *cell = (int64_t)(f.key & ((1ull << 40) - 1));
+        *step = (*inst >= 0 && *inst < (int)c->inst.size() ? c->inst[*inst].step0 : 0) + (int64_t)f.counter;
     }
     return TM_OK;
 }
@@ -690,6 +813,7 @@ tm_status setup_dpc(tm_ctx* c)
         const tm_instance_desc& d = c->inst[i];
         const tm_dpc_params& p = P[d.params_index];
         const double rmax = perception_rmax(p, ns);
+        if ((int)i == c->cut.inst) c->cut.chunk = (int)chunks.size();
         DPCInstInfo& in = info[i];
         in = DPCInstInfo{};
         in.R = p_R[(size_t)d.params_index];
@@ -708,13 +832,16 @@ tm_status setup_dpc(tm_ctx* c)
     std::vector<int4> vtiles;
     for (const int ty : {4, 16}) {
         vtiles.clear();
-        for (size_t i = 0; i < c->inst.size(); ++i)
+        for (size_t i = 0; i < c->inst.size(); ++i) {
+            if ((int)i == c->cut.inst) c->cut.vtile = (int)vtiles.size();
             for (int y0 = 0; y0 < c->inst[i].L; y0 += ty)
                 for (int x0 = 0; x0 < c->inst[i].L; x0 += 64) vtiles.push_back(make_int4((int)i, x0, y0, 0));
+        }
         c->dpc_vdirect = ty == 4;
         if (vtiles.size() <= (size_t)kVegDirectTiles) break;
     }
-    c->dpc_vtiles = (int)vtiles.size();
+    c->end.vtile = (int)vtiles.size();
+    c->end.chunk = (int)chunks.size();
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
     const size_t o_info = up(sizeof(DPCWork));
     const size_t o_st = o_info + up(sizeof(DPCInstInfo) * info.size());
@@ -743,7 +870,6 @@ tm_status setup_dpc(tm_ctx* c)
     std::memcpy(host.data() + o_disk, disk.data(), sizeof(int2) * disk.size());
     std::memcpy(host.data() + o_vtiles, vtiles.data(), sizeof(int4) * vtiles.size());
     HIPCHK(c, hipMemcpy(c->d_dpc, host.data(), total, hipMemcpyHostToDevice));
-    c->dpc_nchunks = (int)chunks.size();
     c->dpc_halo = halo;
     return TM_OK;
 }
@@ -752,8 +878,7 @@ tm_status setup_dpc(tm_ctx* c)
 tm_status reset_state(tm_ctx* c)
 {
     DevState st{};
-    st.fault_counter = ~0ull;
-    st.fault_key = ~0ull;
+    for (Fault& f : st.fault) f = Fault{~0ull, ~0ull};
     HIPCHK(c, hipMemcpy(c->d_state, &st, sizeof(st), hipMemcpyHostToDevice));
     return TM_OK;
 }
@@ -800,6 +925,7 @@ tm_status tm_create(tm_ctx** out, int device)
         return TM_ERR_NODEV;
     }
     c->arch = prop.gcnArchName;
+    c->lanes = RunLanes::get(device);
     c->n_cu = prop.multiProcessorCount;
     if (c->arch.rfind("gfx950", 0) != 0) {
         delete c;
@@ -812,6 +938,7 @@ tm_status tm_create(tm_ctx** out, int device)
         tm_destroy(c);
         return TM_ERR_HIP;
     }
+    c->q = c->stream;
     *out = c;
     return TM_OK;
 }
@@ -893,6 +1020,7 @@ tm_status tm_configure(tm_ctx* c, int model, int precision, const void* params, 
         c->cell_off[i] = c->total_cells;
         c->total_cells += (int64_t)instances[i].L * instances[i].L;
     }
+    c->cut.inst = group_cut(c);
     c->variant = default_variant(model, precision, c->inst.data(), (int)c->inst.size(), c->n_cu);
     {   // whole multi-step launches per graph block, as tm_set_launch makes them
         const int spl = cur_variant(c).spl;
@@ -919,9 +1047,18 @@ tm_status tm_configure(tm_ctx* c, int model, int precision, const void* params, 
     if (is_consumer_model(model) && (s = setup_dpc(c)) != TM_OK) return s;
     if (is_fke_model(model)) {
         const char* err = "";
+        FkeGrid cut = {}, all = {};
         const int rc = fke_setup(model, (const tm_fke_params*)c->params.data(), n_params, c->inst.data(), n_inst,
-                                 c->cell_off.data(), c->total_cells, &c->d_dpc, &c->fke, &err);
-        c->dpc_nchunks = c->fke.chunks;
+                                 c->cell_off.data(), c->total_cells, c->cut.inst, &c->d_dpc, &cut, &all, &err);
+        auto place = [](GroupPos& p, const FkeGrid& g) {
+            p.chunk = g.chunks;
+            p.block = g.blocks;
+            p.rtile = g.rtiles;
+            p.mtile = g.mtiles;
+        };
+        place(c->cut, cut);
+        place(c->end, all);
+        c->move_lds = all.move_lds;
         if (rc != TM_OK) {
             const std::string msg = err;
             release_config(c);
@@ -1165,9 +1302,10 @@ tm_status tm_run(tm_ctx* c, int64_t n_steps, double* rows)
     if (s != TM_OK) return s;
     if (n_steps < 0) return fail(c, TM_ERR_ARG, "negative n_steps");
     if (n_steps == 0) return TM_OK;
-    HIPCHK(c, hipEventRecord(c->run_ev[0], c->stream));
+    const Run run(c, true);
+    HIPCHK(c, hipEventRecord(c->run_ev[0], c->q));
     if ((s = advance(c, n_steps)) != TM_OK) return s;
-    HIPCHK(c, hipEventRecord(c->run_ev[1], c->stream));
+    HIPCHK(c, hipEventRecord(c->run_ev[1], c->q));
     if (rows) {
         // The run's rows are strided on the device (rows_cap steps per instance):
         // packed there first, then one contiguous copy.  A strided copy into
@@ -1176,12 +1314,12 @@ tm_status tm_run(tm_ctx* c, int64_t n_steps, double* rows)
         const double* src = c->d_rows;
         if (n_steps < c->rows_cap && c->inst.size() > 1) {
             HIPCHK(c, hipMemcpy2DAsync(c->d_rows_pack, w * n_steps, c->d_rows, w * c->rows_cap, w * n_steps,
-                                       c->inst.size(), hipMemcpyDeviceToDevice, c->stream));
+                                       c->inst.size(), hipMemcpyDeviceToDevice, c->q));
             src = c->d_rows_pack;
         }
-        HIPCHK(c, hipMemcpyAsync(rows, src, w * n_steps * c->inst.size(), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(rows, src, w * n_steps * c->inst.size(), hipMemcpyDeviceToHost, c->q));
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->q));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->run_ev[0], c->run_ev[1]));
     c->last_run_ms = ms;
@@ -1337,6 +1475,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
     // Step kernels only (no rows fold): graphs of up to 100 steps, one per
     // starting parity, captured once per context and launch shape and kept with
     // the run graphs, replayed between two events on the context stream.
+    const Run run(c, false);
     const int B = (int)std::min<int64_t>(std::min<int64_t>(n_steps, 100), c->nslots);
     const int flip = launches_of(c, B) & 1;
     if (c->time_graph_steps != B) {
@@ -1360,7 +1499,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
     }
     int64_t nlaunch = (n_steps / B) * launches_of(c, B);
     if (left > 0) {
-        enqueue_block(c, c->parity, (int)left, false);
+        enqueue_block(c, c->parity, (int)left, false, false);
         c->parity ^= (launches_of(c, left) & 1);
         nlaunch += launches_of(c, left);
     }
@@ -1407,6 +1546,7 @@ tm_status tm_autotune(tm_ctx* c, const char* cache_path, int* out_variant, int* 
     }
     // Dry timing: launches read the current buffer and write the other one
     // without advancing the step counter, so the batch state is unchanged.
+    const Run run(c, false);
     const int nv = tm_variant_count(c->model, c->prec);
     const int graph_steps = c->graph_steps;
     hipEvent_t e0, e1;
@@ -1539,9 +1679,10 @@ tm_status tm_run_series(tm_ctx* c, const int64_t* steps, int n_meas, double* ser
         HIPCHK(c, hipMalloc((void**)&c->d_series_steps, sizeof(int64_t) * (size_t)n_meas));
         c->series_steps_cap = n_meas;
     }
+    const Run run(c, true);
     HIPCHK(c, hipMemcpyAsync(c->d_series_steps, steps, sizeof(int64_t) * (size_t)n_meas, hipMemcpyHostToDevice,
-                             c->stream));
-    HIPCHK(c, hipEventRecord(c->run_ev[0], c->stream));
+                             c->q));
+    HIPCHK(c, hipEventRecord(c->run_ev[0], c->q));
     int m = 0;
     for (; m < n_meas && steps[m] == 0; ++m) enqueue_measure(c, c->d_series + (int64_t)m * w, n_meas);
     // Advance in chunks of whole graph blocks whose rows fit a ~32 MiB rows
@@ -1557,18 +1698,18 @@ tm_status tm_run_series(tm_ctx* c, const int64_t* steps, int n_meas, double* ser
         int m1 = m;
         while (m1 < n_meas && steps[m1] <= s0 + len) ++m1;
         launch_gather_series(c->d_rows, c->rows_cap, w, c->d_series_steps, m, m1, s0, n_meas, n_inst, c->d_series,
-                             c->stream);
+                             c->q);
         m = m1;
         s0 += len;
         // the next advance() rewrites the pinned staging its first copy reads
-        if (s0 < total) HIPCHK(c, hipStreamSynchronize(c->stream));
+        if (s0 < total) HIPCHK(c, hipStreamSynchronize(c->q));
     }
     HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipEventRecord(c->run_ev[1], c->stream));
+    HIPCHK(c, hipEventRecord(c->run_ev[1], c->q));
     if (series)
         HIPCHK(c, hipMemcpyAsync(series, c->d_series, sizeof(double) * (size_t)need, hipMemcpyDeviceToHost,
-                                 c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+                                 c->q));
+    HIPCHK(c, hipStreamSynchronize(c->q));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->run_ev[0], c->run_ev[1]));
     c->last_run_ms = ms;

@@ -36,7 +36,7 @@ constexpr int kChunk = kDpcChunkCells;
 constexpr double kGammaEps = 1.0e-12;   // calc_gamma's eps (multiSPDP.cpp:1715, :2182)
 
 template <int NS>
-__device__ __forceinline__ void dpc_chunk(const StepArgs& a, const DPCWork* w, int block, double (&red)[NS + 1][256])
+__device__ __forceinline__ void dpc_chunk(const ConsumerArgs& a, const DPCWork* w, int block, double (&red)[NS + 1][256])
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * NS - 1;
@@ -73,7 +73,7 @@ __device__ __forceinline__ void dpc_chunk(const StepArgs& a, const DPCWork* w, i
 // The vegetation's Dornic step (workgroups 0 .. nvtiles - 1) and the chunk sums (the
 // rest): both read the old fields only, so the short sums run beside the samplers.
 template <int NS>
-__global__ __launch_bounds__(256, 5) void dpc_head_kernel(StepArgs a)
+__global__ __launch_bounds__(256, 5) void dpc_head_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * NS - 1;
     __shared__ union {
@@ -82,10 +82,10 @@ __global__ __launch_bounds__(256, 5) void dpc_head_kernel(StepArgs a)
     } sm;
     const DPCWork* w = (const DPCWork*)a.work;
     if ((int)blockIdx.x >= a.nvtiles) {
-        dpc_chunk<NS>(a, w, (int)blockIdx.x - a.nvtiles, sm.red);
+        dpc_chunk<NS>(a, w, a.chunk0 + (int)blockIdx.x - a.nvtiles, sm.red);
         return;
     }
-    const int4 tl = w->vtiles[blockIdx.x];   // (instance, x0, y0)
+    const int4 tl = w->vtiles[a.vtile0 + blockIdx.x];   // (instance, x0, y0)
     const DevInst di = a.inst[tl.x];
     const DPCConst c = ((const DPCConst*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
     const VegConst vc = {c.k, di.seed, di.inst_id, c.compat, c.step};
@@ -99,11 +99,11 @@ __global__ __launch_bounds__(256, 5) void dpc_head_kernel(StepArgs a)
 }
 
 template <int NS>
-__global__ __launch_bounds__(64) void dpc_state_kernel(StepArgs a)
+__global__ __launch_bounds__(64) void dpc_state_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    if (i >= a.n_inst) return;
+    const int i = a.inst0 + blockIdx.x * 64 + threadIdx.x;
+    if (i >= a.inst1) return;
     const DPCWork* w = (const DPCWork*)a.work;
     const DPCInstInfo in = w->info[i];
     const DevInst di = a.inst[i];
@@ -224,7 +224,7 @@ __device__ __forceinline__ int dpc_consumer(const tm_dpc_params& p, int s, const
 // held the samplers', the perception's and the RK4's registers at once (146 VGPRs): 16 x
 // 256^2, two species, 139 us for the step kernel alone, 32 + 77 here.
 template <int NS, int TX, int TY, int NT, int MINW>
-__global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
+__global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * NS - 1, NC = TX * TY;
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             double v = y[s];
-            if (v < 0 || !__builtin_isfinite(v)) record_fault(a.state, tl.inst, s * N + cell, counter);
+            if (v < 0 || !__builtin_isfinite(v)) record_fault(a.fault, tl.inst, s * N + cell, counter);
             if (v < c.eps && v >= c.neg) v = 0.0;
             fout[s * N + cell] = v;
             sum[s] += v;
@@ -385,12 +385,13 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(StepArgs a)
             cnt[NS + s - 1] += g > 0.0 ? 1.0 : 0.0;
         }
     }
-    block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ntiles + tile) * NF, s_red);
+    block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ptiles + tile) * NF, s_red);
 }
 
 template <int NS, int TX, int TY, int NT, int MINW = 1>
-void launch_dpc(const StepArgs& a, int grid, hipStream_t s)
+void launch_dpc(const StepArgs& step, int grid, hipStream_t s)
 {
+    const ConsumerArgs& a = static_cast<const ConsumerArgs&>(step);
     const size_t lds = dpc_lds_bytes(NS, TX, TY, a.halo);
     if (lds > 57344) {   // above the default LDS limit with the static arrays (CDNA4 has 160 KiB per CU)
         static size_t granted = 0;
@@ -400,7 +401,7 @@ void launch_dpc(const StepArgs& a, int grid, hipStream_t s)
             granted = lds;
     }
     hipLaunchKernelGGL(dpc_head_kernel<NS>, dim3(a.nvtiles + a.nchunks), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3((a.inst1 - a.inst0 + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL((dpc_step_kernel<NS, TX, TY, NT, MINW>), dim3(grid), dim3(NT), lds, s, a);
 }
 

@@ -47,26 +47,34 @@ struct DevTile {
     int64_t cell_off;
 };
 
+// A batch's launches are split over at most this many instance groups.
+constexpr int kMaxGroups = 2;
+
+struct Fault {
+    uint64_t counter;
+    uint64_t key;  // (instance << 40) | cell
+};
+
 struct DevState {
     int64_t counter;     // steps taken since configure
     int64_t run_base;    // counter at the start of the current tm_run (row index base)
     uint32_t done;       // workgroups finished in the current launch
     uint32_t pad;
-    // First numeric fault, as the minimum over (launch counter, instance, cell);
-    // all ones while none.  Launches run in stream order, so a later launch only
-    // records when no earlier one did, and within a launch atomicMin picks the
-    // same cell the reference's sequential sweep reports first.
-    uint64_t fault_counter;
-    uint64_t fault_key;  // (instance << 40) | cell
+    // First numeric fault of each instance group, as the minimum over (launch
+    // counter, instance, cell); all ones while none.  A group's launches run in
+    // stream order, so a later launch only records when no earlier one did, and
+    // within a launch atomicMin picks the same cell the reference's sequential
+    // sweep reports first; the host takes the smallest (counter, key) of the groups.
+    Fault fault[kMaxGroups];
 };
 
 struct StepArgs {
     const DevInst* inst;
-    const DevTile* tiles;
+    const DevTile* tiles;  // this launch's (partials: from the first of them)
     const void* consts;  // [B][n_inst] DPConst / RKConstD of this block (prep_consts)
     const void* in;      // T*: fields, instance block [nf][L*L] at cell_off * nf
     void* out;
-    double2* partials;   // [nslots][ntiles][nf]: (FP64 sum, count)
+    double2* partials;   // [nslots][ptiles][nf]: (FP64 sum, count)
     DevState* state;
     int64_t* draws;      // nullable: Poisson integer per cell of the last step
     const DevTile* tiles_a;  // split Rietkerk step: tiles of the Dornic kernel
@@ -77,15 +85,26 @@ struct StepArgs {
     int32_t n_inst;
     int32_t xcd;         // XCD-aware tile order
     int32_t ntiles_a;
-    const void* work;    // consumer models: DPCWork / FkeWork (device) of the batch
-    int32_t nchunks;     // consumer models: statistics chunks of the batch
-    int32_t halo;        // consumer models: LDS halo (largest perception radius, >= 1)
-    int32_t nblocks;     // Rietkerk consumer models: 256-cell blocks of the batch
-    int32_t nvtiles;     // DP consumer models: the vegetation's Dornic tiles,
-    int32_t vdirect;     // ... 64 x 4 with one cell a thread (else 64 x 16 in two passes)
-    int32_t nrtiles;     // Rietkerk consumer models: RK4 tiles of the batch
-    int32_t nmtiles;     // ... movement tiles
-    int32_t move_lds;    // ... and the movement tile's LDS bytes (0: the four-pass movement)
+    // Last, because these two ahead of the counts cost 0.1 us of a 14.6 us launch.
+    Fault* fault;        // of the launch's instance group
+    int32_t ptiles;      // tiles of the whole batch (stride of the partials)
+};
+
+// The consumer models' kernels take these too.
+struct ConsumerArgs : StepArgs {
+    const void* work;    // DPCWork / FkeWork (device) of the batch
+    // The launch's instances, and how many of each table's entries it takes from where:
+    // statistics chunks; the DP consumers' vegetation tiles; the Rietkerk consumers' RK4
+    // tiles, movement tiles and 256-cell blocks.
+    int32_t inst0, inst1;
+    int32_t nchunks, chunk0;
+    int32_t nvtiles, vtile0;
+    int32_t nrtiles, rtile0;
+    int32_t nmtiles, mtile0;
+    int32_t nblocks, block0;
+    int32_t halo;        // LDS halo (largest perception radius, >= 1)
+    int32_t vdirect;     // vegetation tiles of 64 x 4 with one cell a thread (else 64 x 16 in two passes)
+    int32_t move_lds;    // LDS bytes of the movement tile (0: the four-pass movement)
 };
 
 // Periodic index: v mod L in [0, L).
@@ -112,12 +131,12 @@ __device__ __forceinline__ int tile_of(int t, int ntiles, int xcd)
 // an earlier step of the launch, recorded in any order, always has the smaller
 // key, as it has the smaller counter.  The host drops the phase when it decodes
 // the key.
-__device__ __forceinline__ void record_fault(DevState* st, int inst, int64_t cell, int64_t counter,
+__device__ __forceinline__ void record_fault(Fault* st, int inst, int64_t cell, int64_t counter,
                                              int phase = 0)
 {
-    if (st->fault_counter < (uint64_t)counter) return;
-    atomicMin((unsigned long long*)&st->fault_counter, (unsigned long long)counter);
-    atomicMin((unsigned long long*)&st->fault_key, ((unsigned long long)phase << 60) |
+    if (st->counter < (uint64_t)counter) return;
+    atomicMin((unsigned long long*)&st->counter, (unsigned long long)counter);
+    atomicMin((unsigned long long*)&st->key, ((unsigned long long)phase << 60) |
                                                        ((unsigned long long)inst << 40) | (unsigned long long)cell);
 }
 
@@ -526,7 +545,7 @@ __device__ __forceinline__ void wave_step_partial(const StepArgs& a, int tile, i
                                                   uint32_t nlive)
 {
     const int64_t slot = counter & (int64_t)(a.nslots - 1);
-    double2* dst = a.partials + (slot * a.ntiles + tile) * NW + w;
+    double2* dst = a.partials + (slot * a.ptiles + tile) * NW + w;
     if (__ballot(nlive != 0 || s != 0.0) == 0) {
         if ((threadIdx.x & 63) == 0) *dst = make_double2(0.0, 0.0);
     } else {
@@ -806,7 +825,7 @@ __device__ __forceinline__ void zero_tile(const StepArgs& a, int tile, const Dev
     }
     if ((threadIdx.x & 63) == 0)
         for (int k = 0; k < nsl; ++k)
-            a.partials[(slots[k] * a.ntiles + tile) * (NT / 64) + (threadIdx.x >> 6)] = make_double2(0.0, 0.0);
+            a.partials[(slots[k] * a.ptiles + tile) * (NT / 64) + (threadIdx.x >> 6)] = make_double2(0.0, 0.0);
 }
 
 // One tile from its LDS image: the per-cell step on each of this thread's G
@@ -857,7 +876,7 @@ __device__ __forceinline__ void dp_tile(const StepArgs& a, int tile, const DevTi
                 bool bad;
                 const T y = cell_update<T, MODE>(c, di, cell, s_rho[rq], s_rho[rq - RWV], s_rho[rq + RWV],
                                                  s_rho[rq - 1], s_rho[rq + 1], n, bad);
-                if (bad) record_fault(a.state, tl.inst, cell, counter);
+                if (bad) record_fault(a.fault, tl.inst, cell, counter);
                 if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 if constexpr (MODE == 0) {
                     sum[0] += (double)y;
@@ -872,7 +891,7 @@ __device__ __forceinline__ void dp_tile(const StepArgs& a, int tile, const DevTi
         store_quad(fout + (int64_t)gy * L, gx0, nvalid, vec, yq);
     }
     if constexpr (MODE == 0) {
-        double2* dst = a.partials + (slot * a.ntiles + tile) * S::NW + (tid >> 6);
+        double2* dst = a.partials + (slot * a.ptiles + tile) * S::NW + (tid >> 6);
         if (__ballot(nlive != 0 || sum[0] != 0.0) == 0) {   // an all-zero wave: no reduction
             if ((tid & 63) == 0) *dst = make_double2(0.0, 0.0);
         } else {
@@ -950,7 +969,7 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
                     y = (T)0;
                     n = -1;
                 } else if (bad) {
-                    record_fault(a.state, tl.inst, cell, counter);
+                    record_fault(a.fault, tl.inst, cell, counter);
                 }
                 if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 yq.v[0] = q == 0 ? y : yq.v[0];
@@ -995,7 +1014,7 @@ __device__ __forceinline__ void dp_tile_deferred(const StepArgs& a, int tile, co
         bool bad;
         const T y = cell_update<T, MODE>(c, di, cell, s_rho[r], s_rho[r - RWV], s_rho[r + RWV], s_rho[r - 1],
                                          s_rho[r + 1], n, bad);
-        if (bad) record_fault(a.state, tl.inst, cell, counter);
+        if (bad) record_fault(a.fault, tl.inst, cell, counter);
         if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
         s_q[i] = y;                                           // the slot's thread read its offset above
     }
@@ -1110,7 +1129,7 @@ __global__ __launch_bounds__(TX * TY / 4 / CPT) void dp_part_kernel(StepArgs a)
             typename Count<T>::type n;
             bool bad;
             y = cell_update<T, 0>(c, di, cell, fin[cell], fin[up], fin[dn], fin[lf], fin[rt], n, bad);
-            if (bad) record_fault(a.state, tl.inst, cell, counter);
+            if (bad) record_fault(a.fault, tl.inst, cell, counter);
             if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
             fout[cell] = y;
         }
@@ -1253,7 +1272,7 @@ __global__ __launch_bounds__(NT, MINW) void dp_stepk_kernel(StepArgs a)
                     bool bad;
                     const T y = cell_update<T, 0>(c, di, cell, src[rq], src[rq - RW], src[rq + RW], src[rq - 1],
                                                   src[rq + 1], n, bad);
-                    if (bad && own_row && tl.x0 + lx < L) record_fault(a.state, tl.inst, cell, counter + j - 1, j - 1);
+                    if (bad && own_row && tl.x0 + lx < L) record_fault(a.fault, tl.inst, cell, counter + j - 1, j - 1);
                     yq.v[0] = q == 0 ? y : yq.v[0];
                     yq.v[1] = q == 1 ? y : yq.v[1];
                     yq.v[2] = q == 2 ? y : yq.v[2];
@@ -1321,7 +1340,7 @@ __global__ __launch_bounds__(NT, MINW) void dp_stepk_kernel(StepArgs a)
                 bool bad;
                 const T y = cell_update<T, 0>(c, di, cell, src[rq], src[rq - RW], src[rq + RW], src[rq - 1],
                                               src[rq + 1], n, bad);
-                if (bad) record_fault(a.state, tl.inst, cell, counter + K - 1, K - 1);
+                if (bad) record_fault(a.fault, tl.inst, cell, counter + K - 1, K - 1);
                 if (a.draws) a.draws[tl.cell_off + cell] = (int64_t)n;
                 sum += (double)y;
                 nlive += y > (T)0 ? 1u : 0u;
@@ -1823,14 +1842,14 @@ __global__ __launch_bounds__(NT) void rk_step_kernel(StepArgs a)
             const bool ok = y[f] >= (T)0 && y[f] <= Arith<T>::largest();
             const T v = ok && y[f] < c.eps ? (T)0 : y[f];
             if (in) {
-                if (!ok) record_fault(a.state, tl.inst, f * N + cell, counter);
+                if (!ok) record_fault(a.fault, tl.inst, f * N + cell, counter);
                 fout[f * N + cell] = v;
             }
             sum[f] += (double)(in ? v : (T)0);       // + 0 for cells past the lattice
             wcnt[f] += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(in && v > (T)0));
         }
     }
-    double2* dst = a.partials + (slot * a.ntiles + tile) * 3;
+    double2* dst = a.partials + (slot * a.ptiles + tile) * 3;
     block_partials3<NT>(sum, wcnt, dst, sm.red);
 }
 
@@ -1927,7 +1946,7 @@ __global__ __launch_bounds__(FX * FY) void rk_frame_kernel(StepArgs a)
             const T r = y[f] + c.dt6 * (acc[f] + k[f]);
             const bool ok = r >= (T)0 && r <= Arith<T>::largest();   // fails for negative, NaN or infinite values
             v[f] = ok && r < c.eps ? (T)0 : r;
-            if (!ok) record_fault(a.state, tl.inst, (int64_t)f * N + i, counter);
+            if (!ok) record_fault(a.fault, tl.inst, (int64_t)f * N + i, counter);
             fout[f * N + i] = v[f];
         }
     }
@@ -1936,7 +1955,7 @@ __global__ __launch_bounds__(FX * FY) void rk_frame_kernel(StepArgs a)
         sum[f] = (double)v[f];
         wcnt[f] = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(v[f] > (T)0));
     }
-    block_partials3<NT>(sum, wcnt, a.partials + (slot * a.ntiles + tile) * 3, s_red);
+    block_partials3<NT>(sum, wcnt, a.partials + (slot * a.ptiles + tile) * 3, s_red);
 }
 
 // ---------------------------------------------------------------------------

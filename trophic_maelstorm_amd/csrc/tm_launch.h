@@ -84,9 +84,10 @@ struct FkeGrid {
     int move_lds;           // LDS bytes of the movement tile; 0: the four-pass movement
 };
 int fke_setup(int model, const tm_fke_params* params, int n_params, const tm_instance_desc* inst, int n_inst,
-              const int64_t* cell_off, int64_t total_cells, void** work, FkeGrid* grid, const char** err);
+              const int64_t* cell_off, int64_t total_cells, int cut_inst, void** work, FkeGrid* cut, FkeGrid* grid,
+              const char** err);   // cut: the sizes of the instances before cut_inst
 // Movement statistics of the current fields into out [n_inst][4 SpB] (device).
-void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t s);
+void launch_fke_mov_stats(int model, const ConsumerArgs& a, double* out, hipStream_t s);
 
 // Free the device scratch the Rietkerk consumer operators keep between calls.
 void workspace_give_back();

@@ -1059,7 +1059,7 @@ __device__ __forceinline__ void chunk_fold(double (&v)[NV], double (&red)[NV][25
 }
 
 template <int SP>
-__device__ __forceinline__ void fke_chunk(const StepArgs& a, const FkeWork* w, int block, double (&red)[SP + 1][256])
+__device__ __forceinline__ void fke_chunk(const ConsumerArgs& a, const FkeWork* w, int block, double (&red)[SP + 1][256])
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * SP + 1;
@@ -1084,7 +1084,7 @@ __device__ __forceinline__ void fke_chunk(const StepArgs& a, const FkeWork* w, i
 // short sums beside the samplers.  DIRECT: one cell a thread on the final kernel's
 // 64 x 4 tiles, in one pass, for batches whose 64 x 16 tiles leave CUs idle.
 template <int SP, bool DIRECT>
-__global__ __launch_bounds__(256, 5) void fke_head_kernel(StepArgs a, int nveg)
+__global__ __launch_bounds__(256, 5) void fke_head_kernel(ConsumerArgs a, int nveg)
 {
     constexpr int NF = 2 * SP + 1;
     static_assert(kMoveTX == kVegTX && kMoveTY == kVegTY, "the movement's tile table");
@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(256, 5) void fke_head_kernel(StepArgs a, int nveg)
     } sm;
     const FkeWork* w = (const FkeWork*)a.work;
     if ((int)blockIdx.x >= nveg) {
-        fke_chunk<SP>(a, w, (int)blockIdx.x - nveg, sm.red);
+        fke_chunk<SP>(a, w, a.chunk0 + (int)blockIdx.x - nveg, sm.red);
         return;
     }
     if constexpr (DIRECT) {
@@ -1105,7 +1105,7 @@ __global__ __launch_bounds__(256, 5) void fke_head_kernel(StepArgs a, int nveg)
         if (y >= tl.L || x >= tl.L) return;
         veg_cell({c.k, di.seed, di.inst_id, c.compat, c.step}, tl.L, y, x, (const double*)a.in + (int64_t)NF * tl.cell_off, w->pstar + tl.cell_off);
     } else {
-        const int4 tl = w->mtiles[blockIdx.x];
+        const int4 tl = w->mtiles[a.mtile0 + blockIdx.x];
         const DevInst di = a.inst[tl.x];
         const RKConstD c = ((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
         veg_tile({c.k, di.seed, di.inst_id, c.compat, c.step}, di.L, tl.y, tl.z,
@@ -1116,11 +1116,11 @@ __global__ __launch_bounds__(256, 5) void fke_head_kernel(StepArgs a, int nveg)
 // The per-instance numbers of the perception step, as tm_fke_perception_host
 // forms them (FKE:4100-4112, :2534-2606, :3371-3482).
 template <int SP>
-__global__ __launch_bounds__(64) void fke_state_kernel(StepArgs a)
+__global__ __launch_bounds__(64) void fke_state_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
-    const int i = blockIdx.x * 64 + threadIdx.x;
-    if (i >= a.n_inst) return;
+    const int i = a.inst0 + blockIdx.x * 64 + threadIdx.x;
+    if (i >= a.inst1) return;
     const FkeWork* w = (const FkeWork*)a.work;
     const DPCInstInfo in = w->info[i];
     const DevInst di = a.inst[i];
@@ -1150,9 +1150,9 @@ __global__ __launch_bounds__(64) void fke_state_kernel(StepArgs a)
 }
 
 // The cell of the thread in the block table; false past its instance's end.
-__device__ __forceinline__ bool fke_cell(const StepArgs& a, const FkeWork* w, int& inst, int& cell, DevInst& di)
+__device__ __forceinline__ bool fke_cell(const ConsumerArgs& a, const FkeWork* w, int& inst, int& cell, DevInst& di)
 {
-    const int2 b = w->blocks[blockIdx.x];
+    const int2 b = w->blocks[a.block0 + blockIdx.x];
     inst = b.x;
     cell = b.y + (int)threadIdx.x;
     di = a.inst[inst];
@@ -1163,7 +1163,7 @@ __device__ __forceinline__ bool fke_cell(const StepArgs& a, const FkeWork* w, in
 // tiles, so that a row's wrap is scalar and a column's two selects: an index division
 // per offset and one offset in flight at a time took 45 us on 16 x 256^2.
 template <int SP>
-__global__ __launch_bounds__(256) void fke_percept_kernel(StepArgs a)
+__global__ __launch_bounds__(256) void fke_percept_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     const FkeWork* w = (const FkeWork*)a.work;
@@ -1187,12 +1187,12 @@ __global__ __launch_bounds__(256) void fke_percept_kernel(StepArgs a)
 
 // RK4 of P* (FkeWork::pstar) and the other old densities into the output buffer.
 template <int SP>
-__global__ __launch_bounds__(kRkThreads) void fke_rk4_step_kernel(StepArgs a)
+__global__ __launch_bounds__(kRkThreads) void fke_rk4_step_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     __shared__ RkTileLds sm;
     const FkeWork* w = (const FkeWork*)a.work;
-    const int4 tl = w->rtiles[blockIdx.x];   // (instance, x0, y0)
+    const int4 tl = w->rtiles[a.rtile0 + blockIdx.x];   // (instance, x0, y0)
     const DevInst di = a.inst[tl.x];
     const FkeRk c = w->mc[di.pidx].rk;
     const int64_t N = (int64_t)di.L * di.L;
@@ -1201,7 +1201,7 @@ __global__ __launch_bounds__(kRkThreads) void fke_rk4_step_kernel(StepArgs a)
 }
 
 template <int SP>
-__global__ __launch_bounds__(256) void fke_mprep_kernel(StepArgs a)
+__global__ __launch_bounds__(256) void fke_mprep_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     const FkeWork* w = (const FkeWork*)a.work;
@@ -1225,7 +1225,7 @@ __global__ __launch_bounds__(256) void fke_mprep_kernel(StepArgs a)
 // The separable movement's passes (move_disp_at, move_row_at, move_col_at) on
 // each consumer's lattice; the last writes the moved density.
 template <int SP, int PASS>
-__global__ __launch_bounds__(256) void fke_move_pass_kernel(StepArgs a)
+__global__ __launch_bounds__(256) void fke_move_pass_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     const FkeWork* w = (const FkeWork*)a.work;
@@ -1253,12 +1253,12 @@ __global__ __launch_bounds__(256) void fke_move_pass_kernel(StepArgs a)
 // The movement in two launches (move_rows_tile, move_cols_tile) on the batch's movement
 // tiles; blockIdx.y = consumer - 1.
 template <int SP>
-__global__ __launch_bounds__(kMoveRows) void fke_move_rows_step_kernel(StepArgs a)
+__global__ __launch_bounds__(kMoveRows) void fke_move_rows_step_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     extern __shared__ __align__(16) double s_move[];
     const FkeWork* w = (const FkeWork*)a.work;
-    const int4 tl = w->mtiles[blockIdx.x];   // (instance, x0, y0)
+    const int4 tl = w->mtiles[a.mtile0 + blockIdx.x];   // (instance, x0, y0)
     const DevInst di = a.inst[tl.x];
     const int s = blockIdx.y + 1, L = di.L;
     const int64_t N = (int64_t)L * L;
@@ -1278,11 +1278,11 @@ __global__ __launch_bounds__(kMoveRows) void fke_move_rows_step_kernel(StepArgs 
 }
 
 template <int SP>
-__global__ __launch_bounds__(kMoveCols) void fke_move_cols_step_kernel(StepArgs a)
+__global__ __launch_bounds__(kMoveCols) void fke_move_cols_step_kernel(ConsumerArgs a)
 {
     constexpr int NF = 2 * SP + 1;
     const FkeWork* w = (const FkeWork*)a.work;
-    const int4 tl = w->mtiles[blockIdx.x];
+    const int4 tl = w->mtiles[a.mtile0 + blockIdx.x];
     const DevInst di = a.inst[tl.x];
     const int s = blockIdx.y + 1, L = di.L;
     const int64_t N = (int64_t)L * L;
@@ -1302,7 +1302,7 @@ __global__ __launch_bounds__(kMoveCols) void fke_move_cols_step_kernel(StepArgs 
 // Checks and flush of the densities (the perception fields are left as they
 // are), then the (sum, occupied count) partials of every field of the tile.
 template <int SP, int TX, int TY, int NT>
-__global__ __launch_bounds__(NT) void fke_final_kernel(StepArgs a)
+__global__ __launch_bounds__(NT) void fke_final_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * SP + 1, ND = SP + 2;
@@ -1329,7 +1329,7 @@ __global__ __launch_bounds__(NT) void fke_final_kernel(StepArgs a)
         for (int k = 0; k < NF; ++k) {
             double v = f[k * N + cell];
             if (k < ND) {
-                if (v < 0 || !__builtin_isfinite(v)) record_fault(a.state, tl.inst, k * N + cell, counter);
+                if (v < 0 || !__builtin_isfinite(v)) record_fault(a.fault, tl.inst, k * N + cell, counter);
                 if (v < eps && v >= 0.0) {   // FKE:4459-4461
                     v = 0.0;
                     f[k * N + cell] = v;
@@ -1339,18 +1339,19 @@ __global__ __launch_bounds__(NT) void fke_final_kernel(StepArgs a)
             cnt[k] += v > 0.0 ? 1.0 : 0.0;
         }
     }
-    block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ntiles + tile) * NF, s_red);
+    block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ptiles + tile) * NF, s_red);
 }
 
 template <int SP, int TX, int TY, int NT>
-void launch_fke(const StepArgs& a, int grid, hipStream_t s)
+void launch_fke(const StepArgs& step, int grid, hipStream_t s)
 {
+    const ConsumerArgs& a = static_cast<const ConsumerArgs&>(step);
     if (a.ntiles <= kVegDirectTiles)
         hipLaunchKernelGGL((fke_head_kernel<SP, true>), dim3((unsigned)(grid + a.nchunks)), dim3(256), 0, s, a, grid);
     else
         hipLaunchKernelGGL((fke_head_kernel<SP, false>), dim3((unsigned)(a.nmtiles + a.nchunks)), dim3(256), 0, s, a,
                            a.nmtiles);
-    hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.n_inst + 63) / 64), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.inst1 - a.inst0 + 63) / 64), dim3(64), 0, s, a);
     hipLaunchKernelGGL(fke_percept_kernel<SP>, dim3(grid), dim3(256), 0, s, a);
     hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
     if (a.move_lds > 0) {
@@ -1370,7 +1371,7 @@ void launch_fke(const StepArgs& a, int grid, hipStream_t s)
 // ---- movement statistics (Rho_Mov, FKE:4034-4060) ---------------------------
 // pass 0: chunk sums of gamma, vx, vy of each consumer; pass 1: of (gamma - mean)^2.
 template <int SP>
-__global__ __launch_bounds__(256) void fke_mstat_chunk_kernel(StepArgs a, int pass)
+__global__ __launch_bounds__(256) void fke_mstat_chunk_kernel(ConsumerArgs a, int pass)
 {
 #pragma clang fp contract(off)
     constexpr int NF = 2 * SP + 1, NV = 3 * (SP - 1);
@@ -1409,7 +1410,7 @@ __global__ __launch_bounds__(256) void fke_mstat_chunk_kernel(StepArgs a, int pa
 }
 
 template <int SP>
-__global__ __launch_bounds__(64) void fke_mstat_fold_kernel(StepArgs a, int pass, double* out)
+__global__ __launch_bounds__(64) void fke_mstat_fold_kernel(ConsumerArgs a, int pass, double* out)
 {
 #pragma clang fp contract(off)
     constexpr int NV = 3 * (SP - 1);
@@ -1443,7 +1444,7 @@ __global__ __launch_bounds__(64) void fke_mstat_fold_kernel(StepArgs a, int pass
 }
 
 template <int SP>
-void launch_mstat(const StepArgs& a, double* out, hipStream_t s)
+void launch_mstat(const ConsumerArgs& a, double* out, hipStream_t s)
 {
     for (int pass = 0; pass < 2; ++pass) {
         hipLaunchKernelGGL(fke_mstat_chunk_kernel<SP>, dim3(a.nchunks), dim3(256), 0, s, a, pass);
@@ -1492,14 +1493,15 @@ int fke_move_of(const tm_fke_params& p, int s, bool drawn, std::vector<double>& 
 const Variant* fke2_variants_f64(int* n) { *n = (int)(sizeof(kFKE2) / sizeof(kFKE2[0])); return kFKE2; }
 const Variant* fke3_variants_f64(int* n) { *n = (int)(sizeof(kFKE3) / sizeof(kFKE3[0])); return kFKE3; }
 
-void launch_fke_mov_stats(int model, const StepArgs& a, double* out, hipStream_t s)
+void launch_fke_mov_stats(int model, const ConsumerArgs& a, double* out, hipStream_t s)
 {
     if (model == TM_MODEL_FKE3) launch_mstat<3>(a, out, s);
     else launch_mstat<2>(a, out, s);
 }
 
 int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance_desc* inst, int n_inst,
-              const int64_t* cell_off, int64_t total_cells, void** work, FkeGrid* grid, const char** err)
+              const int64_t* cell_off, int64_t total_cells, int cut_inst, void** work, FkeGrid* cut, FkeGrid* grid,
+              const char** err)
 {
     const int SP = model == TM_MODEL_FKE3 ? 3 : 2, ns = SP - 1;
     *work = nullptr;
@@ -1566,7 +1568,9 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     std::vector<int2> chunks, blocks;
     std::vector<int4> rtiles, mtiles;
     size_t lds = 0;   // of the movement tile, over every consumer of every point
+    *cut = FkeGrid{};
     for (int i = 0; i < n_inst; ++i) {
+        if (i == cut_inst) *cut = FkeGrid{(int)chunks.size(), (int)blocks.size(), (int)rtiles.size(), (int)mtiles.size(), 0};
         const tm_instance_desc& d = inst[i];
         const tm_fke_params& p = P[d.params_index];
         const FkeModelConst& m = mc[(size_t)d.params_index];
