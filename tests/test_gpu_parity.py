@@ -287,3 +287,51 @@ def test_multistep_variant_through_extinction_bit_exact(tm, oracle, variant):
         assert_rows_close(rows[k], ref["rows"])
     occupied = rows[:, :, 0].sum(axis=0) / sum(L * L for L in Ls)
     assert occupied[0] > 0.9 and occupied[-1] <= 0.02     # both modes were used
+
+
+@pytest.mark.parametrize("model", ["DP", "RIETKERK"])
+def test_rows_around_the_staging_size(tm, model):
+    """Rows of up to 256 KiB reach the host through pinned memory, larger ones by copies
+    (64 lattices: 256 steps of DP are the last staged run): the same rows, in one run, in
+    runs of other lengths and as the oracle of the final state has them."""
+    m = getattr(tm, "MODEL_" + model)
+    nf = 1 if model == "DP" else 3
+    params = tm.DPParams() if model == "DP" else tm.RietkerkParams()
+    last = 256 // nf
+    insts = [tm.Instance(5 + k % 3, 0, 3, k) for k in range(64)]
+    got = {}
+    for split in ([last], [last + 1], [1, last - 1], [last // 2, 3, last + 1 - last // 2 - 3]):
+        with tm.Context() as ctx:
+            ctx.configure(m, tm.F64, params, insts)
+            ctx.init_uniform([0.0] * nf, [3.0, 5.0, 8.0][:nf])
+            rows = np.concatenate([ctx.run(n) for n in split], axis=1)
+            assert rows.shape == (64, sum(split), 2 * nf)
+            f = ctx.download(63)
+            assert np.array_equal(rows[63, -1, ::2], [np.count_nonzero(x > 0) for x in f])
+            assert np.allclose(rows[63, -1, 1::2], [x.mean() for x in f], rtol=1e-14, atol=0)
+            got[tuple(split)] = rows
+    ref = got[(last + 1,)]
+    for rows in got.values():
+        assert np.array_equal(rows, ref[:, :rows.shape[1]])
+
+
+def test_reset_clears_a_fault(tm):
+    """tm_fault_info after a faulting run, after tm_reset, and after a clean run."""
+    L = 40
+    bad = np.zeros((1, L, L))
+    bad[0, 5, 7] = 100.0
+    with tm.Context() as ctx:
+        ctx.configure(tm.MODEL_DP, tm.F64, tm.DPParams(), [tm.Instance(L, 0, 1, 0)])
+        ctx.upload(0, bad)
+        with pytest.raises(tm.NumericFault):
+            ctx.run(1)
+        first = ctx.fault_info()
+        assert first[0] == 0 and first[2] == 0
+        ctx.upload(0, np.zeros((1, L, L)))
+        with pytest.raises(tm.NumericFault):   # the record stays until a reset
+            ctx.run(2)
+        assert ctx.fault_info() == first
+        ctx.reset()
+        assert ctx.fault_info() == (-1, -1, -1)
+        ctx.run(2)
+        assert ctx.fault_info() == (-1, -1, -1)

@@ -35,6 +35,18 @@
 
 using namespace tmk;
 
+// Rows of up to this many bytes go to the host through pinned memory that a kernel writes:
+// 64 lattices' rows in 7 us of 20 KiB and 28 of 250, where a strided device copy and a copy
+// into pageable memory took 44 and 57.
+constexpr size_t kRowsStage = (size_t)256 << 10;
+
+// The context's pinned host memory.
+struct HostBlock {
+    double live[2];            // occupied counts of the newest blocks
+    Fault fault[kMaxGroups];   // the fault records as the last rows fold saw them
+    double rows[kRowsStage / sizeof(double)];
+};
+
 // A place in the batch's instances and in the launch tables that follow their order.
 struct GroupPos {
     int inst, tile, tile_a;                          // step tiles, the split step's Dornic tiles
@@ -82,7 +94,7 @@ struct tm_ctx {
     int64_t rows_cap = 0;
     int64_t* d_draws = nullptr;
     bool record_draws = false;
-    double* h_pinned = nullptr;   // small pinned staging for state writes
+    HostBlock* h_pinned = nullptr;
 
     // Instance groups (group_cut): where the second begins and the batch ends.  A run of
     // such a batch takes a lane and, while it is alone, a second one for the second group.
@@ -104,7 +116,7 @@ struct tm_ctx {
     bool blocked = true;
     double live_frac = -1.0;
     double* d_live = nullptr;   // [n_inst][2 nf] rows of a measure of the current state, then 2 sums
-    hipEvent_t live_ev[2] = {nullptr, nullptr};   // per-block live counts copied to h_pinned[2 + j]
+    hipEvent_t live_ev[2] = {nullptr, nullptr};   // per-block live counts copied to h_pinned->live[j]
     bool live_pending[2] = {false, false};
     int64_t live_block = 0;
     int64_t steps_single = 0, steps_blocked = 0;   // steps tm_run advanced by each kind of launch
@@ -474,7 +486,7 @@ int launches_of(tm_ctx* c, int64_t n)
     return (int)(n / spl + n % spl);
 }
 
-void launch_fold(tm_ctx* c, int nsteps)
+void launch_fold(tm_ctx* c, int nsteps, int64_t row0)
 {
     CombineArgs a{};
     a.inst = c->d_inst;
@@ -488,6 +500,9 @@ void launch_fold(tm_ctx* c, int nsteps)
     a.rows_cap = c->rows_cap;
     a.measure = 0;
     a.pw = cur_variant(c).pw;
+    a.fault = c->h_pinned->fault;
+    a.counter = c->counter;
+    a.row0 = row0;
     launch_combine(a, (int)c->inst.size(), nsteps, c->q);
 }
 
@@ -537,10 +552,11 @@ void join_second_lane(tm_ctx* c)
 }
 
 // One block of n <= nslots steps starting from buffer `parity`: constants,
-// n step launches, the rows fold (optional) and the counter bump.
+// n step launches, and the rows fold (into the run's rows from row0 on), which also sets
+// the step counter; row0 < 0: no fold, a counter bump.
 // grouped: the step launches by instance group on two lanes, while the run has both;
 // never under capture (a graph's branches would pick their own queues).
-void enqueue_block(tm_ctx* c, int parity, int n, bool fold, bool grouped)
+void enqueue_block(tm_ctx* c, int parity, int n, int64_t row0, bool grouped)
 {
     launch_prep(c->model, c->d_inst, c->d_params, c->d_state, (int)c->inst.size(), n, c->d_consts, c->q);
     const int spl = steps_per_launch(c);
@@ -563,17 +579,17 @@ void enqueue_block(tm_ctx* c, int parity, int n, bool fold, bool grouped)
         k += m;
     }
     if (grouped) join_second_lane(c);
-    if (fold) launch_fold(c, n);
-    launch_bump(c->d_state, n, c->q);
+    if (row0 >= 0) launch_fold(c, n, row0);
+    else launch_bump(c->d_state, n, c->q);
 }
 
-// Capture one block of n steps (with or without the rows fold) for a parity:
+// Capture one block of n steps (without a rows fold) for a parity:
 // the graphs tm_time_steps replays.
-tm_status capture_block(tm_ctx* c, int parity, int n, bool fold, hipGraphExec_t* out)
+tm_status capture_block(tm_ctx* c, int parity, int n, hipGraphExec_t* out)
 {
     hipGraph_t g = nullptr;
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_block(c, parity, n, fold, false);
+    enqueue_block(c, parity, n, -1, false);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (e != hipSuccess) return fail(c, TM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
@@ -604,15 +620,6 @@ tm_status check_ready(tm_ctx* c)
 {
     if (!c) return TM_ERR_ARG;
     if (!c->model) return fail(c, TM_ERR_STATE, "tm_configure has not been called");
-    return TM_OK;
-}
-
-tm_status set_run_base(tm_ctx* c)
-{
-    // run_base <- counter, ordered on the stream before the step launches.
-    *(int64_t*)c->h_pinned = c->counter;
-    HIPCHK(c, hipMemcpyAsync((char*)c->d_state + offsetof(DevState, run_base), c->h_pinned, sizeof(int64_t),
-                             hipMemcpyHostToDevice, c->q));
     return TM_OK;
 }
 
@@ -700,12 +707,11 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
     tm_status s = ensure_rows(c, n_steps);
     if (s != TM_OK) return s;
     if ((s = update_mode(c)) != TM_OK) return s;
-    if ((s = set_run_base(c)) != TM_OK) return s;
     const bool adaptive = cur_variant(c).spl > 1 && cur_variant(c).adaptive;
     if (adaptive && (s = ensure_live(c)) != TM_OK) return s;
     int64_t left = n_steps;
     const int B = c->graph_steps;
-    volatile double* h_sum = (volatile double*)c->h_pinned + 2;   // [2], after the run-base staging word
+    volatile double* h_sum = c->h_pinned->live;
     auto after_block = [&]() -> tm_status {
         if (!adaptive) return TM_OK;
         // The sum of two blocks back, waited for: the host stays at most two
@@ -732,7 +738,7 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
         return update_mode(c);
     };
     while (B > 0 && left >= B) {
-        enqueue_block(c, c->parity, B, true, true);
+        enqueue_block(c, c->parity, B, n_steps - left, true);
         HIPCHK(c, hipGetLastError());
         count_steps(c, B);
         c->counter += B;
@@ -742,7 +748,7 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
     }
     while (left > 0) {
         const int chunk = (int)std::min<int64_t>(left, c->nslots);
-        enqueue_block(c, c->parity, chunk, true, true);
+        enqueue_block(c, c->parity, chunk, n_steps - left, true);
         HIPCHK(c, hipGetLastError());
         count_steps(c, chunk);
         c->parity ^= (launches_of(c, chunk) & 1);
@@ -754,15 +760,21 @@ tm_status advance(tm_ctx* c, int64_t n_steps)
 }
 
 // First fault recorded by the kernels: (instance, cell, instance step), or all -1.
-tm_status read_fault(tm_ctx* c, int32_t* inst, int64_t* cell, int64_t* step)
+// folded: of a run that ended with a rows fold and has been waited for.
+tm_status read_fault(tm_ctx* c, bool folded, int32_t* inst, int64_t* cell, int64_t* step)
 {
-    DevState st;
-    HIPCHK(c, hipMemcpy(&st, c->d_state, sizeof(st), hipMemcpyDeviceToHost));
+    Fault rec[kMaxGroups];
+    if (folded) {
+        std::memcpy(rec, c->h_pinned->fault, sizeof(rec));
+    } else {
+        HIPCHK(c, hipStreamSynchronize(c->stream));   // tm_reset's kernel
+        HIPCHK(c, hipMemcpy(rec, c->d_state->fault, sizeof(rec), hipMemcpyDeviceToHost));
+    }
     *inst = -1;
     *cell = -1;
     *step = -1;
-    Fault f = st.fault[0];   // the groups' earliest
-    for (const Fault& o : st.fault)
+    Fault f = rec[0];   // the groups' earliest
+    for (const Fault& o : rec)
         if (o.counter < f.counter || (o.counter == f.counter && o.key < f.key)) f = o;
     if (f.counter != ~0ull) {
         *inst = (int32_t)((f.key >> 40) & 0xFFFFF);   // bits 60..63: the step's place in its launch
@@ -772,11 +784,11 @@ tm_status read_fault(tm_ctx* c, int32_t* inst, int64_t* cell, int64_t* step)
     return TM_OK;
 }
 
-tm_status fault_status(tm_ctx* c)
+tm_status fault_status(tm_ctx* c, bool folded)
 {
     int32_t inst;
     int64_t cell, step;
-    tm_status s = read_fault(c, &inst, &cell, &step);
+    tm_status s = read_fault(c, folded, &inst, &cell, &step);
     if (s != TM_OK) return s;
     if (inst >= 0) {
         char buf[160];
@@ -877,9 +889,8 @@ tm_status setup_dpc(tm_ctx* c)
 // Zero state with no fault recorded.
 tm_status reset_state(tm_ctx* c)
 {
-    DevState st{};
-    for (Fault& f : st.fault) f = Fault{~0ull, ~0ull};
-    HIPCHK(c, hipMemcpy(c->d_state, &st, sizeof(st), hipMemcpyHostToDevice));
+    launch_reset(c->d_state, c->stream);
+    HIPCHK(c, hipGetLastError());
     return TM_OK;
 }
 
@@ -933,7 +944,7 @@ tm_status tm_create(tm_ctx** out, int device)
     }
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void**)&c->d_state, sizeof(DevState)) != hipSuccess ||
-        hipHostMalloc((void**)&c->h_pinned, 64, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void**)&c->h_pinned, sizeof(HostBlock), hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->run_ev[0]) != hipSuccess || hipEventCreate(&c->run_ev[1]) != hipSuccess) {
         tm_destroy(c);
         return TM_ERR_HIP;
@@ -1306,25 +1317,30 @@ tm_status tm_run(tm_ctx* c, int64_t n_steps, double* rows)
     HIPCHK(c, hipEventRecord(c->run_ev[0], c->q));
     if ((s = advance(c, n_steps)) != TM_OK) return s;
     HIPCHK(c, hipEventRecord(c->run_ev[1], c->q));
-    if (rows) {
+    const size_t w = sizeof(double) * 2 * c->nf;
+    const size_t bytes = w * n_steps * c->inst.size();
+    if (rows && bytes <= kRowsStage) {
+        launch_pack_rows(c->d_rows, c->rows_cap, 2 * c->nf, n_steps, (int)c->inst.size(), c->h_pinned->rows, c->q);
+    } else if (rows) {
         // The run's rows are strided on the device (rows_cap steps per instance):
         // packed there first, then one contiguous copy.  A strided copy into
         // pageable host memory goes one instance row at a time (about 7 us each).
-        const size_t w = sizeof(double) * 2 * c->nf;
         const double* src = c->d_rows;
         if (n_steps < c->rows_cap && c->inst.size() > 1) {
             HIPCHK(c, hipMemcpy2DAsync(c->d_rows_pack, w * n_steps, c->d_rows, w * c->rows_cap, w * n_steps,
                                        c->inst.size(), hipMemcpyDeviceToDevice, c->q));
             src = c->d_rows_pack;
         }
-        HIPCHK(c, hipMemcpyAsync(rows, src, w * n_steps * c->inst.size(), hipMemcpyDeviceToHost, c->q));
+        HIPCHK(c, hipMemcpyAsync(rows, src, bytes, hipMemcpyDeviceToHost, c->q));
     }
+    HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->q));
+    if (rows && bytes <= kRowsStage) std::memcpy(rows, c->h_pinned->rows, bytes);
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->run_ev[0], c->run_ev[1]));
     c->last_run_ms = ms;
     c->last_run_steps = n_steps;
-    return fault_status(c);
+    return fault_status(c, true);
 }
 
 tm_status tm_mode_steps(const tm_ctx* c, int64_t* single_steps, int64_t* blocked_steps)
@@ -1403,7 +1419,7 @@ tm_status tm_fault_info(tm_ctx* c, int32_t* inst, int64_t* cell, int64_t* step)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     int32_t i;
     int64_t ce, st;
-    if ((s = read_fault(c, &i, &ce, &st)) != TM_OK) return s;
+    if ((s = read_fault(c, false, &i, &ce, &st)) != TM_OK) return s;
     if (inst) *inst = i;
     if (cell) *cell = ce;
     if (step) *step = st;
@@ -1485,7 +1501,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
         }
         c->time_graph_steps = 0;
         for (int par = 0; par < 2; ++par)   // a block from either parity
-            if ((s = capture_block(c, par, B, false, &c->time_graph[par])) != TM_OK) return s;
+            if ((s = capture_block(c, par, B, &c->time_graph[par])) != TM_OK) return s;
         c->time_graph_steps = B;
     }
     for (auto& e : c->time_ev)
@@ -1499,7 +1515,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
     }
     int64_t nlaunch = (n_steps / B) * launches_of(c, B);
     if (left > 0) {
-        enqueue_block(c, c->parity, (int)left, false, false);
+        enqueue_block(c, c->parity, (int)left, -1, false);
         c->parity ^= (launches_of(c, left) & 1);
         nlaunch += launches_of(c, left);
     }
@@ -1511,7 +1527,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
     c->counter += n_steps;
     *ms_total = ms;
     if (launches) *launches = nlaunch;
-    return fault_status(c);
+    return fault_status(c, false);
 }
 
 tm_status tm_reset(tm_ctx* c)
@@ -1701,8 +1717,6 @@ tm_status tm_run_series(tm_ctx* c, const int64_t* steps, int n_meas, double* ser
                              c->q);
         m = m1;
         s0 += len;
-        // the next advance() rewrites the pinned staging its first copy reads
-        if (s0 < total) HIPCHK(c, hipStreamSynchronize(c->q));
     }
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->run_ev[1], c->q));
@@ -1715,7 +1729,7 @@ tm_status tm_run_series(tm_ctx* c, const int64_t* steps, int n_meas, double* ser
     c->last_run_ms = ms;
     c->last_run_steps = total;
     c->n_series = n_meas;
-    return fault_status(c);
+    return fault_status(c, total > 0);
 }
 
 tm_status tm_replicate_stats(tm_ctx* c, int flags, double* stats)

@@ -57,7 +57,6 @@ struct Fault {
 
 struct DevState {
     int64_t counter;     // steps taken since configure
-    int64_t run_base;    // counter at the start of the current tm_run (row index base)
     uint32_t done;       // workgroups finished in the current launch
     uint32_t pad;
     // First numeric fault of each instance group, as the minimum over (launch
@@ -2039,9 +2038,29 @@ __global__ __launch_bounds__(256) void prep_consts_kernel(const DevInst* inst, c
 }
 
 #ifdef TM_DEFINE_COMBINE   // defined by exactly one translation unit
+// After a block of steps without a rows fold.
 __global__ void bump_counter_kernel(DevState* state, int n)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) state->counter += n;
+}
+
+// No steps taken, no fault recorded.
+__global__ void reset_state_kernel(DevState* state)
+{
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        *state = DevState{};
+        for (int g = 0; g < kMaxGroups; ++g) state->fault[g] = Fault{~0ull, ~0ull};
+    }
+}
+
+// The n steps' rows of every instance from the rows buffer, one after another: w doubles
+// a row, rows_cap rows an instance.
+__global__ __launch_bounds__(256) void pack_rows_kernel(const double* rows, int64_t rows_cap, int w, int64_t n,
+                                                        int64_t total, double* out)
+{
+    const int64_t per = n * w;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256)
+        out[t] = rows[t / per * rows_cap * w + t % per];
 }
 #endif
 
@@ -2080,13 +2099,19 @@ __global__ __launch_bounds__(256) void measure_kernel(const DevInst* inst, const
 // Fold tile partials into rho(t) rows: one workgroup per (instance, step).
 // Per-thread Kahan sums over a fixed tile stride, then a fixed pairwise tree
 // of compensated (TwoSum) additions -- deterministic run to run.
-// rows: [n_inst][rows_cap][2 nf]; row = step counter - run_base.
+// rows: [n_inst][rows_cap][2 nf].  The launch ends its block of steps: it also sets
+// the step counter, which the block's other kernels read and this one is given, and
+// leaves the fault records in host memory.  With a kernel for the counter and copies of
+// the base of the rows before and the records after it, a run of one step of one small
+// lattice was 69 us, 47 without them.
 // ---------------------------------------------------------------------------
 struct CombineArgs {
     const DevInst* inst;
     const double2* partials;
-    const DevState* state;
+    DevState* state;
     double* rows;
+    Fault* fault;                        // pinned host memory [kMaxGroups]
+    int64_t counter, row0;               // at the block's start: step counter, steps of the run
     int32_t ntiles, nslots, nf, nsteps;  // nsteps: steps folded by this launch
     int64_t rows_cap;
     int32_t measure;                     // 1: slot 0, row 0 (tm_measure)
@@ -2110,9 +2135,12 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(CombineArgs a)
     const DevInst di = a.inst[i];
     int64_t slot = 0, row = 0;
     if (!a.measure) {
-        const int64_t c = a.state->counter + j;   // step counter of this row (before the bump)
-        slot = c & (int64_t)(a.nslots - 1);
-        row = c - a.state->run_base;
+        slot = (a.counter + j) & (int64_t)(a.nslots - 1);
+        row = a.row0 + j;
+        if (i == 0 && j == 0 && threadIdx.x == 0) {
+            a.state->counter = a.counter + a.nsteps;
+            for (int g = 0; g < kMaxGroups; ++g) a.fault[g] = a.state->fault[g];
+        }
     }
     const double2* p = a.partials + ((slot * a.ntiles + di.tile0) * a.pw) * a.nf;
     const int nsub = di.ntiles * a.pw;

@@ -4,6 +4,8 @@
 #define TM_DEFINE_COMBINE
 #include "tm_launch.h"
 
+#include <algorithm>
+
 namespace tmk {
 
 template <typename T, int TX, int TY, int NT, int MODE = 0, int MINW = 1, int Q = 0>
@@ -148,6 +150,18 @@ void launch_prep(int model, const DevInst* inst, const void* params, const DevSt
 void launch_bump(DevState* state, int n, hipStream_t s)
 {
     hipLaunchKernelGGL(bump_counter_kernel, dim3(1), dim3(64), 0, s, state, n);
+}
+
+void launch_reset(DevState* state, hipStream_t s)
+{
+    hipLaunchKernelGGL(reset_state_kernel, dim3(1), dim3(64), 0, s, state);
+}
+
+void launch_pack_rows(const double* rows, int64_t rows_cap, int w, int64_t n, int n_inst, double* out, hipStream_t s)
+{
+    const int64_t total = n * w * n_inst;
+    hipLaunchKernelGGL(pack_rows_kernel, dim3((unsigned)std::min<int64_t>(256, (total + 255) / 256)), dim3(256), 0, s,
+                       rows, rows_cap, w, n, total, out);
 }
 
 size_t const_size(int model)

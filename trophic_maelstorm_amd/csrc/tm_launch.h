@@ -103,6 +103,8 @@ void launch_combine(const CombineArgs& a, int n_inst, int nsteps, hipStream_t s)
 void launch_prep(int model, const DevInst* inst, const void* params, const DevState* state, int n_inst,
                  int nsteps, void* table, hipStream_t s);
 void launch_bump(DevState* state, int n, hipStream_t s);
+void launch_reset(DevState* state, hipStream_t s);
+void launch_pack_rows(const double* rows, int64_t rows_cap, int w, int64_t n, int n_inst, double* out, hipStream_t s);
 size_t const_size(int model);
 
 // Initial frames (tm_frames.hip), one launch for the whole batch.  Values per
