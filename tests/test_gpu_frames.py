@@ -78,3 +78,32 @@ def test_dp_from_speckle_frame_bit_exact(tm, oracle):
     ref = oracle.dp_run(oracle.dp_params(a=1.0), rho0, L, 4, 77, 0, steps)
     assert np.array_equal(got, ref["fields"])
     np.testing.assert_allclose(rows[0], ref["rows"], rtol=1e-12)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65])
+def test_frames_do_not_depend_on_the_batch(tm, n):
+    """Frame tables go to the kernel as arguments for up to 64 instances and 16 points and
+    by a copy above, with 256 or 4096 cells a workgroup: an instance's frame is the same
+    in a batch of any size, for each kind of frame."""
+    print(f"frames n={n}", flush=True)
+    points = [tm.DPParams(a=0.6 + 0.01 * k) for k in range(17)]
+    target = tm.Instance(70, 3, 9, 5)
+    batches = [([target], points[:4], 0),
+               ([tm.Instance(33, k % 4, 9, 100 + k) for k in range(n - 1)] + [target], points[:4], n - 1),
+               ([target] + [tm.Instance(17, k % 17, 9, 100 + k) for k in range(n - 1)], points, 0),
+               ([tm.Instance(1025, 0, 9, 99), target], points[:16], 1)]
+    out = []
+    for insts, pts, at in batches:
+        with tm.Context() as ctx:
+            ctx.configure(tm.MODEL_DP, tm.F64, pts, insts)
+            got = []
+            ctx.init_uniform([0.25], [2.0])
+            got.append(ctx.download(at))
+            ctx.init_speckle([0.3] * len(pts), [[2.0]] * len(pts), [[0.5]] * len(pts))
+            got.append(ctx.download(at))
+            ctx.init_gauss([[3.0]] * len(pts), 1, (8.0,))
+            got.append(ctx.download(at))
+            out.append(got)
+    for got in out[1:]:
+        for x, y in zip(out[0], got):
+            assert np.array_equal(x, y)

@@ -15,7 +15,7 @@
 // library's own exp, and stored in the field precision.
 // * Uniform frames (tm_init_uniform): word f % 4 of Philox(seed, instance_id;
 //   cell, 0xFFFFFFFF, 0xFFFFFFFF, f / 4) gives field f = lo_f + (hi_f - lo_f) u.
-// Workgroup b covers kFrameCellsPerBlock consecutive cells of the instance k
+// Workgroup b covers block_cells consecutive cells of the instance k
 // with blk0[k] <= b < blk0[k+1] (its 256 threads stride through them, so every
 // store is a contiguous wave); the values of the instance's parameter point
 // come from vals[params_index].
@@ -26,11 +26,9 @@ namespace tmk {
 namespace {
 
 template <typename T>
-__global__ __launch_bounds__(256) void init_frames_kernel(int mode, const DevInst* __restrict__ inst,
-                                                          const int64_t* __restrict__ blk0, int n_inst, int nf,
-                                                          int n_gauss, FrameSd sd_div,
-                                                          const FrameVals* __restrict__ vals,
-                                                          T* __restrict__ fields)
+__device__ __forceinline__ void init_frame_block(int mode, const DevInst* __restrict__ inst, const int64_t* blk0,
+                                                 int n_inst, int block_cells, int nf, int n_gauss,
+                                                 const FrameSd& sd_div, const FrameVals* vals, T* __restrict__ fields)
 {
 #pragma clang fp contract(off)
     const int64_t b = blockIdx.x;
@@ -45,8 +43,8 @@ __global__ __launch_bounds__(256) void init_frames_kernel(int mode, const DevIns
     const int64_t N = (int64_t)L * L;
     T* f0 = fields + (int64_t)nf * d.cell_off;
     const FrameVals v = vals[d.pidx];
-    const int64_t base = (b - blk0[lo]) * kFrameCellsPerBlock;
-    for (int r = 0; r < kFrameCellsPerBlock / 256; ++r) {
+    const int64_t base = (b - blk0[lo]) * block_cells;
+    for (int r = 0; r < block_cells / 256; ++r) {
         const int64_t i = base + r * 256 + threadIdx.x;
         if (i >= N) return;
         if (mode != 1) {
@@ -85,21 +83,54 @@ __global__ __launch_bounds__(256) void init_frames_kernel(int mode, const DevIns
     }
 }
 
+template <typename T>
+__global__ __launch_bounds__(256) void init_frames_kernel(int mode, const DevInst* __restrict__ inst,
+                                                          const int64_t* __restrict__ blk0, int n_inst,
+                                                          int block_cells, int nf, int n_gauss, FrameSd sd_div,
+                                                          const FrameVals* __restrict__ vals,
+                                                          T* __restrict__ fields)
+{
+    init_frame_block<T>(mode, inst, blk0, n_inst, block_cells, nf, n_gauss, sd_div, vals, fields);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void init_frames_args_kernel(int mode, const DevInst* __restrict__ inst,
+                                                               FrameArgTab tab, int n_inst, int block_cells, int nf,
+                                                               int n_gauss, FrameSd sd_div, T* __restrict__ fields)
+{
+    init_frame_block<T>(mode, inst, tab.blk0, n_inst, block_cells, nf, n_gauss, sd_div, tab.vals, fields);
+}
+
 }  // namespace
 
 void launch_init_frames(int prec, int mode, const DevInst* inst, const int64_t* blk0, int n_inst, int64_t nblocks,
-                        int nf, int n_gauss, const double* sd_div, const FrameVals* vals, void* fields,
-                        hipStream_t s)
+                        int block_cells, int nf, int n_gauss, const double* sd_div, const FrameVals* vals,
+                        void* fields, hipStream_t s)
 {
     if (nblocks <= 0) return;
     FrameSd sd;
     for (int f = 0; f < kMaxFields; ++f) sd.v[f] = sd_div[f];
     if (prec == TM_F64)
         hipLaunchKernelGGL(init_frames_kernel<double>, dim3((unsigned)nblocks), dim3(256), 0, s, mode, inst, blk0,
-                           n_inst, nf, n_gauss, sd, vals, (double*)fields);
+                           n_inst, block_cells, nf, n_gauss, sd, vals, (double*)fields);
     else
         hipLaunchKernelGGL(init_frames_kernel<float>, dim3((unsigned)nblocks), dim3(256), 0, s, mode, inst, blk0,
-                           n_inst, nf, n_gauss, sd, vals, (float*)fields);
+                           n_inst, block_cells, nf, n_gauss, sd, vals, (float*)fields);
+}
+
+void launch_init_frames_args(int prec, int mode, const DevInst* inst, const FrameArgTab& tab, int n_inst,
+                             int64_t nblocks, int block_cells, int nf, int n_gauss, const double* sd_div,
+                             void* fields, hipStream_t s)
+{
+    if (nblocks <= 0) return;
+    FrameSd sd;
+    for (int f = 0; f < kMaxFields; ++f) sd.v[f] = sd_div[f];
+    if (prec == TM_F64)
+        hipLaunchKernelGGL(init_frames_args_kernel<double>, dim3((unsigned)nblocks), dim3(256), 0, s, mode, inst, tab,
+                           n_inst, block_cells, nf, n_gauss, sd, (double*)fields);
+    else
+        hipLaunchKernelGGL(init_frames_args_kernel<float>, dim3((unsigned)nblocks), dim3(256), 0, s, mode, inst, tab,
+                           n_inst, block_cells, nf, n_gauss, sd, (float*)fields);
 }
 
 }  // namespace tmk

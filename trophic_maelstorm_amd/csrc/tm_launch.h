@@ -110,9 +110,8 @@ size_t const_size(int model);
 // Initial frames (tm_frames.hip), one launch for the whole batch.  Values per
 // parameter point: speckle frames use perc, a = high, b = low; Gaussian frames
 // use a = amp; uniform frames a = lo, b = hi.  mode 0 = speckle, 1 = Gaussian,
-// 2 = uniform; blk0[n_inst + 1] = first workgroup of each instance
-// (kFrameCellsPerBlock cells per workgroup).
-constexpr int kFrameCellsPerBlock = 4096;
+// 2 = uniform; blk0[n_inst + 1] = first workgroup of each instance (block_cells cells
+// per workgroup, a multiple of 256).
 struct FrameVals {
     double perc;
     double a[kMaxFields], b[kMaxFields];
@@ -121,8 +120,18 @@ struct FrameSd {   // Gaussian widths L / v[f], per field (sd_div[kMaxFields] at
     double v[kMaxFields];
 };
 void launch_init_frames(int prec, int mode, const DevInst* inst, const int64_t* blk0, int n_inst, int64_t nblocks,
-                        int nf, int n_gauss, const double* sd_div, const FrameVals* vals, void* fields,
-                        hipStream_t s);
+                        int block_cells, int nf, int n_gauss, const double* sd_div, const FrameVals* vals,
+                        void* fields, hipStream_t s);
+// ... with blk0 and vals as kernel arguments, for batches whose tables fit them: no copy
+// of the tables in front of the frame.
+constexpr int kFrameArgInst = 64, kFrameArgPoints = 16;
+struct FrameArgTab {
+    int64_t blk0[kFrameArgInst + 1];
+    FrameVals vals[kFrameArgPoints];
+};
+void launch_init_frames_args(int prec, int mode, const DevInst* inst, const FrameArgTab& tab, int n_inst,
+                             int64_t nblocks, int block_cells, int nf, int n_gauss, const double* sd_div,
+                             void* fields, hipStream_t s);
 
 // Sum of field 0's occupied counts over the instances in one row (tm_ensemble.hip).
 void launch_live_count(const double* rows, int64_t rows_cap, int w, int64_t row, int n_inst, double* out,
