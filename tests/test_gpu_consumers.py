@@ -167,3 +167,15 @@ def test_consumers_large_batch_equals_small_batches(tm, ns):
     for (f0, r0), (f1, r1) in zip(*out):
         assert np.array_equal(f0, f1)
         assert np.array_equal(r0, r1)
+
+
+@pytest.mark.parametrize("model", ["DP2", "DP3"])
+def test_consumers_many_chunks_bit_exact(tm, oracle, model):
+    """The sums of a lattice's chunks go through a wave 64 chunks at a time: 67, 64, 1
+    and 2 chunks in one batch."""
+    m = getattr(tm, "MODEL_" + model)
+    ns = tm.NSPECIES[m]
+    Ls = [521, 512, 33, 67]
+    insts = [tm.Instance(L, 0, 7, 40 + k, 3 * k) for k, L in enumerate(Ls)]
+    rng = np.random.default_rng(21)
+    _run_both(tm, oracle, m, [params()], insts, [_initial(rng, ns, L) for L in Ls], 2)

@@ -121,3 +121,22 @@ def test_fke_large_batch_equals_small_batches(tm, sp):
     for (f0, r0), (f1, r1) in zip(*out):
         assert np.array_equal(f0, f1)
         assert np.array_equal(r0, r1)
+
+
+@pytest.mark.parametrize("SP", [2, 3])
+def test_fke_model_many_chunks_matches_oracle(tm, oracle, SP):
+    """The sums of a lattice's chunks go through a wave 64 chunks at a time: 67, 64 and 1
+    chunks in one batch; its second group takes the RK4 before the perception."""
+    p = [tm.FKEParams()]
+    insts = [tm.Instance(521, 0, 5, 0), tm.Instance(512, 0, 5, 1), tm.Instance(48, 0, 6, 2)]
+    f0 = [model_fields(SP, d.L, 100 + d.L) for d in insts]
+    print(f"fke chunks SP={SP}", flush=True)
+    with tm.Context() as ctx:
+        ctx.configure(tm.MODEL_FKE2 if SP == 2 else tm.MODEL_FKE3, tm.F64, p, insts)
+        for k, f in enumerate(f0):
+            ctx.upload(k, f)
+        ctx.run(2)
+        got = [ctx.download(k) for k in range(len(insts))]
+    for k, d in enumerate(insts):
+        ref, _, _ = _oracle_run(oracle, p[0], SP, f0[k], d, 2)
+        assert np.array_equal(got[k], ref), (SP, d.L, np.argwhere(got[k] != ref)[:5])

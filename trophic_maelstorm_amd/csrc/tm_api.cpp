@@ -431,6 +431,10 @@ ConsumerArgs step_args(tm_ctx* c, int parity, int k, int g = kWholeBatch)
     a.nrtiles = hi.rtile - lo.rtile;
     a.nmtiles = hi.mtile - lo.mtile;
     a.move_lds = c->move_lds;
+    // Two chains settle into step with each other: in the other order, the second group's
+    // kernels are not the first's beside them (16 x 256^2, three-species Rietkerk consumers:
+    // 154 us, 165 in one order; 7 x 256^2 84 and 88; 16 x 128^2 64 and 62).
+    a.rk_first = g == 1 && c->total_cells >= 2 * kGroupCells;
     a.inst0 = lo.inst;
     a.inst1 = hi.inst;
     a.chunk0 = lo.chunk;

@@ -98,37 +98,30 @@ __global__ __launch_bounds__(256, 5) void dpc_head_kernel(ConsumerArgs a)
     }
 }
 
+// The per-instance numbers of the perception step, a wave per instance.
 template <int NS>
 __global__ __launch_bounds__(64) void dpc_state_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
-    const int i = a.inst0 + blockIdx.x * 64 + threadIdx.x;
-    if (i >= a.inst1) return;
+    __shared__ double s_sum[64 * (NS + 1)];
+    const int i = a.inst0 + blockIdx.x, f = threadIdx.x;
     const DPCWork* w = (const DPCWork*)a.work;
-    const DPCInstInfo in = w->info[i];
+    const DPCInstInfo& in = w->info[i];
     const DevInst di = a.inst[i];
     const double N = (double)((int64_t)di.L * di.L);
-    double tot[NS], occ = 0.0;
-#pragma unroll
-    for (int f = 0; f < NS; ++f) tot[f] = 0.0;
-    for (int c = 0; c < in.nchunks; ++c) {
-        const double* p = w->chunk + (int64_t)(in.chunk0 + c) * 4;
-#pragma unroll
-        for (int f = 0; f < NS; ++f) tot[f] += p[f];
-        occ += p[NS];
-    }
-    DPCStepState st{};
-    for (int f = 0; f < NS; ++f) st.mean[f] = tot[f] / N;
-    double nfac = 1 - occ / N;                       // multiSPDP.cpp:2972-2974
+    const double tot = chunk_totals<NS + 1, 4>(w->chunk + (int64_t)in.chunk0 * 4, in.nchunks, s_sum);
+    if (f >= NS) return;
+    const double fr = in.fr[f];
+    double nfac = 1 - s_sum[NS] / N;                 // multiSPDP.cpp:2972-2974
     if (nfac < 0.35) nfac = 0.35;
     const int new_len = (int)(nfac * nfac * (double)in.disk_len);
-    for (int f = 0; f < NS; ++f) st.inv[f] = st.mean[f] >= kGammaEps ? 1 / st.mean[f] : 1 / kGammaEps;
-    for (int f = 0; f < NS; ++f) {
-        int e = (int)(in.fr[f] * in.fr[f] * (double)new_len);
-        if (NS == 3 && e < 1 && in.fr[f] > 0) e = 1;     // multiSPDP.cpp:2215-2216
-        st.eff[f] = e;
-    }
-    w->st[i] = st;
+    const double mean = tot / N;
+    int e = (int)(fr * fr * (double)new_len);
+    if (NS == 3 && e < 1 && fr > 0) e = 1;     // multiSPDP.cpp:2215-2216
+    DPCStepState& st = w->st[i];
+    st.mean[f] = mean;
+    st.inv[f] = mean >= kGammaEps ? 1 / mean : 1 / kGammaEps;
+    st.eff[f] = e;
 }
 
 // f_DP_Dor_2Sp / f_DP_Dor_3Sp (multiSPDP.cpp:1670-1697, :1789-1819) at one cell.
@@ -401,7 +394,7 @@ void launch_dpc(const StepArgs& step, int grid, hipStream_t s)
             granted = lds;
     }
     hipLaunchKernelGGL(dpc_head_kernel<NS>, dim3(a.nvtiles + a.nchunks), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3((a.inst1 - a.inst0 + 63) / 64), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3(a.inst1 - a.inst0), dim3(64), 0, s, a);
     hipLaunchKernelGGL((dpc_step_kernel<NS, TX, TY, NT, MINW>), dim3(grid), dim3(NT), lds, s, a);
 }
 

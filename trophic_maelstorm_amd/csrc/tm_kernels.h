@@ -104,6 +104,7 @@ struct ConsumerArgs : StepArgs {
     int32_t halo;        // LDS halo (largest perception radius, >= 1)
     int32_t vdirect;     // vegetation tiles of 64 x 4 with one cell a thread (else 64 x 16 in two passes)
     int32_t move_lds;    // LDS bytes of the movement tile (0: the four-pass movement)
+    int32_t rk_first;    // Rietkerk consumers: the RK4 before the perception
 };
 
 // Periodic index: v mod L in [0, L).

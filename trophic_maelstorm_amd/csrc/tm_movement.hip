@@ -1119,34 +1119,26 @@ template <int SP>
 __global__ __launch_bounds__(64) void fke_state_kernel(ConsumerArgs a)
 {
 #pragma clang fp contract(off)
-    const int i = a.inst0 + blockIdx.x * 64 + threadIdx.x;
-    if (i >= a.inst1) return;
+    __shared__ double s_sum[64 * (SP + 1)];
+    const int i = a.inst0 + blockIdx.x, f = threadIdx.x;
     const FkeWork* w = (const FkeWork*)a.work;
-    const DPCInstInfo in = w->info[i];
+    const DPCInstInfo& in = w->info[i];
     const DevInst di = a.inst[i];
     const double N = (double)((int64_t)di.L * di.L);
-    double tot[SP], occ = 0.0;
-#pragma unroll
-    for (int f = 0; f < SP; ++f) tot[f] = 0.0;
-    for (int c = 0; c < in.nchunks; ++c) {
-        const double* p = w->chunk + (int64_t)(in.chunk0 + c) * 8;
-#pragma unroll
-        for (int f = 0; f < SP; ++f) tot[f] += p[f];
-        occ += p[SP];
-    }
-    DPCStepState st{};
-    double nfac = 1 - occ / N;                       // FKE:4109-4112
+    const double tot = tmk::chunk_totals<SP + 1, 8>(w->chunk + (int64_t)in.chunk0 * 8, in.nchunks, s_sum);
+    if (f >= SP) return;
+    const double fr = in.fr[f];
+    double nfac = 1 - s_sum[SP] / N;                 // FKE:4109-4112
     if (nfac < 0.35) nfac = 0.35;
     int new_len = (int)(nfac * nfac * (double)in.disk_len);
     if (SP == 3 && new_len < 1) new_len = 1;         // FKE:3386
-    for (int f = 0; f < SP; ++f) {
-        st.mean[f] = tot[f] / N;
-        st.inv[f] = st.mean[f] >= 1.0e-12 ? 1 / st.mean[f] : 1 / 1.0e-12;
-        int e = (int)(in.fr[f] * in.fr[f] * (double)new_len);
-        if (SP == 3 && e < 1 && in.fr[f] > 0) e = 1;     // FKE:3415-3416
-        st.eff[f] = e;
-    }
-    w->st[i] = st;
+    const double mean = tot / N;
+    int e = (int)(fr * fr * (double)new_len);
+    if (SP == 3 && e < 1 && fr > 0) e = 1;     // FKE:3415-3416
+    DPCStepState& st = w->st[i];
+    st.mean[f] = mean;
+    st.inv[f] = mean >= 1.0e-12 ? 1 / mean : 1 / 1.0e-12;
+    st.eff[f] = e;
 }
 
 // The cell of the thread in the block table; false past its instance's end.
@@ -1351,9 +1343,11 @@ void launch_fke(const StepArgs& step, int grid, hipStream_t s)
     else
         hipLaunchKernelGGL((fke_head_kernel<SP, false>), dim3((unsigned)(a.nmtiles + a.nchunks)), dim3(256), 0, s, a,
                            a.nmtiles);
-    hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((a.inst1 - a.inst0 + 63) / 64), dim3(64), 0, s, a);
+    // The RK4 needs P* only, the perception the sums only: either order will do.
+    if (a.rk_first) hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
+    hipLaunchKernelGGL(fke_state_kernel<SP>, dim3((unsigned)(a.inst1 - a.inst0)), dim3(64), 0, s, a);
     hipLaunchKernelGGL(fke_percept_kernel<SP>, dim3(grid), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
+    if (!a.rk_first) hipLaunchKernelGGL(fke_rk4_step_kernel<SP>, dim3((unsigned)a.nrtiles), dim3(kRkThreads), 0, s, a);
     if (a.move_lds > 0) {
         hipLaunchKernelGGL(fke_move_rows_step_kernel<SP>, dim3((unsigned)a.nmtiles, SP - 1), dim3(kMoveRows),
                            (size_t)a.move_lds, s, a);
