@@ -97,3 +97,32 @@ def test_vegetation_dornic_matches_oracle(tm, oracle, sampler, L):
     got = np.where((got < 1e-10) & (got >= 0.0), 0.0, got)
     assert np.array_equal(got, ref["fields"][0])
     assert np.all(got[4:8, 5:11] == 0.0)
+
+
+def test_device_entry_counts_negative_values_call_by_call(tm, oracle):
+    """tm_fke_rk4 fetches its count only when a value was negative, and keeps its scratch:
+    calls with and without negative values in turn return each its own count."""
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+    hip.hipMemcpy.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int]
+    hip.hipFree.argtypes = [C.c_void_p]
+    y = np.ascontiguousarray(fields(1, 33, 3))
+    calls = []
+    for kw in (dict(a=-50.0, D_O=0.1, dt=0.05), dict(dt=0.004), dict(a=-50.0, D_O=0.1, dt=0.05), dict(dt=0.004)):
+        pg, po = _params(tm, oracle, **kw)
+        calls.append((pg, oracle.fke_rk4(po, y)))
+    p = C.c_void_p()
+    assert hip.hipMalloc(C.byref(p), y.nbytes) == 0
+    try:
+        for pg, (ref, rbad) in calls:
+            assert hip.hipMemcpy(p, y.ctypes.data, y.nbytes, 1) == 0
+            par = pg._c()
+            bad = C.c_int64(-1)
+            assert tm.lib().tm_fke_rk4(1, 33, C.cast(C.byref(par), C.c_void_p), p, C.byref(bad), None) == 0
+            got = np.empty_like(y)
+            assert hip.hipMemcpy(got.ctypes.data, p, got.nbytes, 2) == 0
+            assert np.array_equal(got, ref)
+            assert bad.value == rbad
+    finally:
+        hip.hipFree(p)
+    assert calls[0][1][1] > 0 and calls[1][1][1] == 0

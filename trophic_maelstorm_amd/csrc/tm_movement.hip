@@ -698,7 +698,7 @@ public:
     {
         if (!b_.p) return;
         if (!idle || b_.bytes > kKeepTotal) {
-            (void)hipFree(b_.p);
+            release(b_);
             return;
         }
         Pool& k = pool();
@@ -708,7 +708,7 @@ public:
         for (int i = 0; i < k.n; ++i) total += k.v[i].bytes;
         while (total > kKeepTotal || k.n > kKeepBlocks) {
             total -= k.v[0].bytes;
-            (void)hipFree(k.v[0].p);
+            release(k.v[0]);
             k.erase(0);
         }
     }
@@ -727,20 +727,21 @@ public:
                     return true;
                 }
         }
-        b_ = Block{nullptr, bytes, dev};
-        if (hipMalloc(&b_.p, bytes) == hipSuccess) return true;
+        b_ = Block{nullptr, nullptr, bytes, dev};
+        if (make(b_)) return true;
         (void)hipGetLastError();
         give_back();
-        if (hipMalloc(&b_.p, bytes) == hipSuccess) return true;
-        b_.p = nullptr;
-        return false;
+        return make(b_);
     }
+    // Pinned host memory that goes with the block, kHostDoubles long.
+    double* host() const { return b_.h; }
+    static constexpr int kHostDoubles = 3 * 256;
     template <typename T> T* at(size_t offset) const { return (T*)((char*)b_.p + offset); }
     static void give_back()
     {
         Pool& k = pool();
         std::lock_guard<std::mutex> lock(k.mu);
-        for (int i = 0; i < k.n; ++i) (void)hipFree(k.v[i].p);
+        for (int i = 0; i < k.n; ++i) release(k.v[i]);
         k.n = 0;
     }
 
@@ -749,9 +750,24 @@ private:
     static constexpr int kKeepBlocks = 8;
     struct Block {
         void* p;
+        double* h;
         size_t bytes;
         int dev;
     };
+    static bool make(Block& b)
+    {
+        if (hipMalloc(&b.p, b.bytes) != hipSuccess) b.p = nullptr;
+        else if (hipHostMalloc((void**)&b.h, sizeof(double) * kHostDoubles, hipHostMallocDefault) == hipSuccess) return true;
+        if (b.p) (void)hipFree(b.p);
+        b.p = nullptr;
+        b.h = nullptr;
+        return false;
+    }
+    static void release(Block& b)
+    {
+        (void)hipFree(b.p);
+        (void)hipHostFree(b.h);
+    }
     struct Pool {
         std::mutex mu;
         Block v[kKeepBlocks + 1];
@@ -895,12 +911,15 @@ __device__ __forceinline__ uint32_t fke_rk4_tile(const FkeRk& c, const double* _
 // The operator's step, from a copy of the fields (scratch) into the fields.
 template <int NS>
 __global__ __launch_bounds__(kRkThreads) void fke_rk4_kernel(FkeRk c, const double* src, double* out,
-                                                             unsigned long long* n_bad)
+                                                             unsigned long long* n_bad, uint32_t* any_bad)
 {
     __shared__ RkTileLds sm;
     const int64_t N = (int64_t)c.L * c.L;
     const uint32_t bad = fke_rk4_tile<NS>(c, src, src, out, c.L, N, (int)blockIdx.y * kRkTile, (int)blockIdx.x * kRkTile, sm);
-    if (bad) atomicAdd(n_bad, (unsigned long long)bad);
+    if (bad) {
+        atomicAdd(n_bad, (unsigned long long)bad);
+        if (any_bad) *any_bad = 1u;
+    }
 }
 
 // Copy n doubles and clear the counter (the RK4 reads its neighbours' old fields,
@@ -944,17 +963,21 @@ bool fke_rk_args(int ns, int L, const tm_fke_rk_params* p, FkeRk* c)
     return true;
 }
 
-// One step in place on stream st; scratch holds (ns + 3) L^2 doubles.
-void fke_rk_launch(const FkeRk& c, double* fields, double* scratch, unsigned long long* n_bad, hipStream_t st)
+// One step in place on stream st; scratch holds (ns + 3) L^2 doubles.  any_bad (pinned
+// host memory, cleared by the caller, or null) is set if n_bad is not zero.
+void fke_rk_launch(const FkeRk& c, double* fields, double* scratch, unsigned long long* n_bad, hipStream_t st,
+                   uint32_t* any_bad = nullptr)
 {
     const int64_t n = (int64_t)(c.ns + 3) * c.L * c.L;
     hipLaunchKernelGGL(fke_rk4_copy_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 4096)), dim3(256), 0, st,
                        fields, scratch, n, n_bad);
     const unsigned t = (unsigned)((c.L + kRkTile - 1) / kRkTile);
     if (c.ns == 1)
-        hipLaunchKernelGGL(fke_rk4_kernel<1>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad);
+        hipLaunchKernelGGL(fke_rk4_kernel<1>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad,
+                           any_bad);
     else
-        hipLaunchKernelGGL(fke_rk4_kernel<2>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad);
+        hipLaunchKernelGGL(fke_rk4_kernel<2>, dim3(t, t), dim3(kRkThreads), 0, st, c, scratch, fields, n_bad,
+                           any_bad);
 }
 
 // ---------------------------------------------------------------------------
@@ -1710,18 +1733,14 @@ int tm_fke_movement(int ns, int L, const tm_fke_move_species* sp, const double* 
     hipStream_t st = (hipStream_t)stream;
     const unsigned nb = (unsigned)std::min<int64_t>(256, (L2 + 1023) / 1024);
     const size_t pq_bytes = sizeof(double) * 2 * (size_t)ns * L2;
-    double bmax[3 * 256];
-    const size_t nmax = (size_t)ns * nb;
     MovePassBufs b;   // outlives ws: freed after the wait below
     Workspace ws;
-    if (!ws.get(pq_bytes + sizeof(double) * nmax)) return TM_ERR_NOMEM;
+    if (!ws.get(pq_bytes)) return TM_ERR_NOMEM;
     double* const pq = ws.at<double>(0);
-    double* const d_vmax = ws.at<double>(pq_bytes);
+    double* const bmax = ws.host();   // written by the kernel: a copy took 8 us more
     ws.idle = false;
-    hipLaunchKernelGGL(vmax_kernel, dim3(nb, (unsigned)ns), dim3(256), 0, st, (const double2*)v_eff, L2, d_vmax);
-    if (hipMemcpyAsync(bmax, d_vmax, sizeof(double) * nmax, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-        return TM_ERR_HIP;
+    hipLaunchKernelGGL(vmax_kernel, dim3(nb, (unsigned)ns), dim3(256), 0, st, (const double2*)v_eff, L2, bmax);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return TM_ERR_HIP;
     ws.idle = true;
     double vmax[3] = {0.0, 0.0, 0.0};
     for (int s = 0; s < ns; ++s) vmax[s] = *std::max_element(bmax + (size_t)s * nb, bmax + (size_t)(s + 1) * nb);
@@ -1843,13 +1862,16 @@ int tm_fke_rk4(int ns, int L, const tm_fke_rk_params* p, double* fields, int64_t
     Workspace ws;
     if (!ws.get(sizeof(double) * nf + sizeof(unsigned long long))) return TM_ERR_NOMEM;
     unsigned long long* const d_bad = ws.at<unsigned long long>(sizeof(double) * nf);
+    volatile uint32_t* const any_bad = (uint32_t*)ws.host();   // usually none, and no copy of the count (9 us)
+    *any_bad = 0;
     unsigned long long bad = 0;
     ws.idle = false;
-    fke_rk_launch(c, fields, ws.at<double>(0), d_bad, st);
+    fke_rk_launch(c, fields, ws.at<double>(0), d_bad, st, (uint32_t*)any_bad);
     if (hipGetLastError() != hipSuccess) return TM_ERR_HIP;
     // the scratch is handed on when this returns: wait for the kernels that use it
-    if (hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
+    if (hipStreamSynchronize(st) != hipSuccess) return TM_ERR_HIP;
+    if (*any_bad && (hipMemcpyAsync(&bad, d_bad, sizeof(bad), hipMemcpyDeviceToHost, st) != hipSuccess ||
+                     hipStreamSynchronize(st) != hipSuccess))
         return TM_ERR_HIP;
     ws.idle = true;
     if (n_bad) *n_bad = (int64_t)bad;
