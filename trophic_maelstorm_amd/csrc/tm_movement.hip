@@ -183,7 +183,11 @@ __device__ __forceinline__ void put4(double* __restrict__ planes, int64_t N, int
 // columns wider than the tile, R = max(rD, rV)) and the taps come from LDS or
 // registers.  Every sum keeps its terms and order (move_disp_at, move_row_at,
 // move_col_at), so the result is the passes' bit for bit.
-constexpr int kMoveTX = 64, kMoveTY = 16, kMoveRows = 512, kMoveCols = 256;
+constexpr int kMoveTX = 64, kMoveTY = 16, kMoveCols = 256;
+// Threads of a rows tile: the operator waits for its sources' loads, which more waves
+// hide (two consumers of 1024^2: 512 threads 44.6 us, 768 and 1024 39.6); the model step
+// draws its velocities (three species, 16 x 256^2: 155, 157 and 166 us a step).
+constexpr int kMoveRows = 512, kMoveOpRows = 768;
 constexpr int kMoveRPT = kMoveTY / (kMoveCols / 64);   // rows a thread of the column pass
 constexpr size_t kMoveLdsMax = 128 * 1024;
 
@@ -208,7 +212,7 @@ struct FrameDiv {
 
 // src(i, r, g, v): the density, gamma and velocity of source cell i.  pq: the planes P
 // and Q of this lattice, N apart.
-template <class Src>
+template <int NT, class Src>
 __device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const double* __restrict__ SD,
                                                const double* __restrict__ SV, int L, int64_t N, int x0, int y0,
                                                const Src& src, double* __restrict__ pq, double* lds)
@@ -228,7 +232,7 @@ __device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const doub
     {
         const FrameDiv d((uint32_t)aw);
 #pragma unroll 1
-        for (int e = threadIdx.x; e < na; e += kMoveRows) {
+        for (int e = threadIdx.x; e < na; e += NT) {
             int r, c;
             d.split((uint32_t)e, r, c);
             const int p = tmk::wrap(y0 + r - S, L), q = tmk::wrap(x0 + c - S - R, L);
@@ -249,7 +253,7 @@ __device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const doub
     __syncthreads();
     const FrameDiv dm((uint32_t)mw);
 #pragma unroll 1
-    for (int e = threadIdx.x; e < nm; e += kMoveRows) {
+    for (int e = threadIdx.x; e < nm; e += NT) {
         int r, c;
         dm.split((uint32_t)e, r, c);
         const uint32_t p = (uint32_t)(y0 + r), q = (uint32_t)tmk::wrap(x0 + c - R, L);
@@ -279,7 +283,7 @@ __device__ __forceinline__ void move_rows_tile(const MoveSpecies& sp, const doub
     __syncthreads();
     const FrameDiv dt((uint32_t)tw);
 #pragma unroll 1
-    for (int e = threadIdx.x; e < th * tw; e += kMoveRows) {
+    for (int e = threadIdx.x; e < th * tw; e += NT) {
         int r, c;
         dt.split((uint32_t)e, r, c);
         const int o = r * mw + c + R;
@@ -375,7 +379,7 @@ __device__ __forceinline__ void move_cols_tile(const MoveSpecies& sp, const doub
 }
 
 // The device-array operator in two launches; blockIdx.z = species.
-__global__ __launch_bounds__(kMoveRows) void fke_move_rows_kernel(MoveArgs a, const double* __restrict__ rho,
+__global__ __launch_bounds__(kMoveOpRows) void fke_move_rows_kernel(MoveArgs a, const double* __restrict__ rho,
                                                                   const double* __restrict__ gamma,
                                                                   const double2* __restrict__ veff,
                                                                   const double* __restrict__ SDall,
@@ -391,7 +395,7 @@ __global__ __launch_bounds__(kMoveRows) void fke_move_rows_kernel(MoveArgs a, co
         g = gamma[s * N + i];
         v = veff[s * N + i];
     };
-    move_rows_tile(sp, SDall + sp.offD, SVall + sp.offV, a.L, N, (int)blockIdx.x * kMoveTX, (int)blockIdx.y * kMoveTY,
+    move_rows_tile<kMoveOpRows>(sp, SDall + sp.offD, SVall + sp.offV, a.L, N, (int)blockIdx.x * kMoveTX, (int)blockIdx.y * kMoveTY,
                    src, pq + 2 * s * N, s_move);
 }
 
@@ -538,7 +542,7 @@ int move_launch(const MoveArgs& a, int ns, const double* rho, const double* gamm
                                                (int)kMoveLdsMax) != hipSuccess)
             return TM_ERR_HIP;
         const dim3 grid((unsigned)((a.L + kMoveTX - 1) / kMoveTX), (unsigned)((a.L + kMoveTY - 1) / kMoveTY), (unsigned)ns);
-        hipLaunchKernelGGL(fke_move_rows_kernel, grid, dim3(kMoveRows), lds, st, a, rho, gamma, (const double2*)veff, SD, SV,
+        hipLaunchKernelGGL(fke_move_rows_kernel, grid, dim3(kMoveOpRows), lds, st, a, rho, gamma, (const double2*)veff, SD, SV,
                            pq);
         hipLaunchKernelGGL(fke_move_cols_kernel, grid, dim3(kMoveCols), 0, st, a, (const double*)pq, SD, SV, out);
     } else {
@@ -1288,7 +1292,7 @@ __global__ __launch_bounds__(kMoveRows) void fke_move_rows_step_kernel(ConsumerA
         v = make_double2(0.0, 0.0);   // the two-species step draws no velocity
         if (SP == 3) v = fke_velocity(di.seed, di.inst_id, (uint32_t)i, step, s, vs);
     };
-    move_rows_tile(sp, w->SD + sp.offD, w->SV + sp.offV, L, N, tl.y, tl.z, src,
+    move_rows_tile<kMoveRows>(sp, w->SD + sp.offD, w->SV + sp.offV, L, N, tl.y, tl.z, src,
                    w->pq + 2 * ((int64_t)(SP - 1) * di.cell_off + (s - 1) * N), s_move);
 }
 
