@@ -179,3 +179,25 @@ def test_consumers_many_chunks_bit_exact(tm, oracle, model):
     insts = [tm.Instance(L, 0, 7, 40 + k, 3 * k) for k, L in enumerate(Ls)]
     rng = np.random.default_rng(21)
     _run_both(tm, oracle, m, [params()], insts, [_initial(rng, ns, L) for L in Ls], 2)
+
+
+@pytest.mark.parametrize("model", ["DP2", "DP3"])
+@pytest.mark.parametrize("ntiles", [2, 640, 642])
+def test_consumers_default_threads_are_identical(tm, model, ntiles):
+    """The default step takes a thread per cell up to 640 tiles of 32 x 16 and two cells a
+    thread above: fields and rows are those of the plain variant with two, bit for bit."""
+    m = getattr(tm, "MODEL_" + model)
+    hi = [20.0, 2.0, 0.5, 0.0, 0.0] if model == "DP3" else [20.0, 2.0, 0.0]
+    insts = [tm.Instance(30, 0, 5, k) for k in range(ntiles // 2)]   # 1 x 2 tiles each
+    out = []
+    for want in (None, f"dpc{model[2]}_f64_32x16_t256"):
+        with tm.Context() as ctx:
+            ctx.configure(m, tm.F64, tm.DPCParams(a=1e-5), insts)
+            if want:
+                ctx.set_launch(tm.variant_names(m, tm.F64).index(want), 100)
+            ctx.init_uniform([0.0] * len(hi), hi)
+            rows = ctx.run(3)
+            out.append((rows, [ctx.download(k) for k in (0, len(insts) - 1)]))
+    assert np.array_equal(out[0][0], out[1][0])
+    for a, b in zip(out[0][1], out[1][1]):
+        assert np.array_equal(a, b)

@@ -222,6 +222,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
 #pragma clang fp contract(off)
     constexpr int NF = 2 * NS - 1, NC = TX * TY;
     static_assert(NC <= 512, "a queue entry holds a cell in 9 bits, then its words");
+    static_assert(NT == 256 || (NT == 512 && NC == 512), "one or two cells a thread");
     extern __shared__ __align__(16) double s_lds[];
     __shared__ double s_red[2 * NF * (NT / 64)];
     __shared__ uint16_t s_q[NS - 1][NC];        // restarts from the front, Gamma deviates from the back
@@ -378,7 +379,25 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
             cnt[NS + s - 1] += g > 0.0 ? 1.0 : 0.0;
         }
     }
-    block_partials<NT, NF>(sum, cnt, a.partials + (slot * a.ptiles + tile) * NF, s_red);
+    if constexpr (NT > 256) {   // the sums of 256 threads with two cells each, for the same rows
+        __shared__ double s_x[2 * NF][256];
+        const int t = threadIdx.x - 256;
+        if (t >= 0) {
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                s_x[2 * f][t] = sum[f];
+                s_x[2 * f + 1][t] = cnt[f];
+            }
+        }
+        __syncthreads();
+        if (t >= 0) return;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            sum[f] += s_x[2 * f][threadIdx.x];
+            cnt[f] += s_x[2 * f + 1][threadIdx.x];
+        }
+    }
+    block_partials<256, NF>(sum, cnt, a.partials + (slot * a.ptiles + tile) * NF, s_red);
 }
 
 template <int NS, int TX, int TY, int NT, int MINW = 1>
@@ -398,18 +417,33 @@ void launch_dpc(const StepArgs& step, int grid, hipStream_t s)
     hipLaunchKernelGGL((dpc_step_kernel<NS, TX, TY, NT, MINW>), dim3(grid), dim3(NT), lds, s, a);
 }
 
+// The defaults: batches of at most kWideTiles tiles (two and a half a CU) take a thread per
+// cell, which halves the chain of each thread's cells; above, 512-thread workgroups leave
+// fewer of them in flight.  us a step, 256 / 512 threads: two species 64^2 38.1 / 32.0, 8 x
+// 128^2 (256 tiles) 41.7 / 36.0, 512^2 (512) 49.7 / 45.6, 24 x 128^2 (768) 54.2 / 54.3, 1024^2
+// 112 / 137; three species 8 x 128^2 55.3 / 46.3, 20 x 128^2 (640) 74.8 / 65.6, 988 tiles of
+// odd lattices 82.3 / 87.7.
+constexpr int kWideTiles = 640;
+
+template <int NS, int MINW>
+void launch_dpc_default(const StepArgs& a, int grid, hipStream_t s)
+{
+    if (a.ptiles <= kWideTiles) launch_dpc<NS, 32, 16, 512>(a, grid, s);
+    else launch_dpc<NS, 32, 16, 256, MINW>(a, grid, s);
+}
+
 // _wN: at most 512/N VGPRs, N waves per SIMD
 const Variant kDPC2[] = {
     {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256", &launch_dpc<2, 32, 16, 256>, 0, 0, nullptr, 1},
     {64, 8, 256, 0, 1, "dpc2_f64_64x8_t256", &launch_dpc<2, 64, 8, 256>, 0, 0, nullptr, 1},
     {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256_w4", &launch_dpc<2, 32, 16, 256, 4>, 0, 0, nullptr, 1},
-    {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256_w5", &launch_dpc<2, 32, 16, 256, 5>, 0, 0, nullptr, 1},
+    {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256_w5", &launch_dpc_default<2, 5>, 0, 0, nullptr, 1},
     {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256_w6", &launch_dpc<2, 32, 16, 256, 6>, 0, 0, nullptr, 1},
 };
 const Variant kDPC3[] = {
     {32, 16, 256, 0, 1, "dpc3_f64_32x16_t256", &launch_dpc<3, 32, 16, 256>, 0, 0, nullptr, 1},
     {64, 8, 256, 0, 1, "dpc3_f64_64x8_t256", &launch_dpc<3, 64, 8, 256>, 0, 0, nullptr, 1},
-    {32, 16, 256, 0, 1, "dpc3_f64_32x16_t256_w4", &launch_dpc<3, 32, 16, 256, 4>, 0, 0, nullptr, 1},
+    {32, 16, 256, 0, 1, "dpc3_f64_32x16_t256_w4", &launch_dpc_default<3, 4>, 0, 0, nullptr, 1},
     {32, 16, 256, 0, 1, "dpc3_f64_32x16_t256_w5", &launch_dpc<3, 32, 16, 256, 5>, 0, 0, nullptr, 1},
 };
 
