@@ -1,0 +1,36 @@
+"""Index arithmetic of the per-tile step kernels on lattices of any side up to 65535, by
+running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
+and the last tile is written, nothing else is, and nothing outside the fields is read.
+No GPU needed."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CPP = os.path.join(ROOT, "tests", "cpp")
+CLANG = "/opt/rocm/llvm/bin/clang++"
+
+
+def compile_cpu(src, exe, *extra):
+    """Compile a source of the library, or of tests/cpp, for the CPU through cpu_hip."""
+    r = subprocess.run([CLANG, "-std=c++17", "-O1", "-ffp-contract=off", "-w", "-I", os.path.join(CPP, "cpu_hip"),
+                        "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "trophic_maelstorm_amd", "csrc"),
+                        os.path.join(CPP, src), "-pthread", "-o", str(exe), *extra], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return str(exe)
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    return compile_cpu("kernel_indices.cpp", tmp_path_factory.mktemp("cpu") / "kernel_indices")
+
+
+# 37837 and 37839 lie on either side of 3 L^2 = 2^32, 46339 below 2 L^2 = 2^32
+SIDES = [1, 5, 33, 64, 4097, 37837, 37839, 46339, 65534]
+
+
+@pytest.mark.parametrize("kernel", ["frame", "part", "tile", "veg"])
+def test_tiles_read_and_write_their_cells_only(exe, kernel):
+    r = subprocess.run([exe, kernel, *map(str, SIDES)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

@@ -1878,7 +1878,7 @@ __global__ __launch_bounds__(FX * FY) void rk_frame_kernel(StepArgs a)
     const DevInst di = a.inst[tl.inst];
     const RKConst<T> c = rk_cast<T>(((const RKConstD*)a.consts)[(int64_t)a.k * a.n_inst + tl.inst]);
     const int L = tl.L;
-    const uint32_t N = (uint32_t)L * (uint32_t)L;
+    const int64_t N = (int64_t)L * L;   // three fields pass 2^32 cells from a side of 37838
     const T* fin = (const T*)a.in + 3 * tl.cell_off;
     T* fout = (T*)a.out + 3 * tl.cell_off;
     const int t = threadIdx.x, ty = t / FX, tx = t % FX;
@@ -1946,7 +1946,7 @@ __global__ __launch_bounds__(FX * FY) void rk_frame_kernel(StepArgs a)
             const T r = y[f] + c.dt6 * (acc[f] + k[f]);
             const bool ok = r >= (T)0 && r <= Arith<T>::largest();   // fails for negative, NaN or infinite values
             v[f] = ok && r < c.eps ? (T)0 : r;
-            if (!ok) record_fault(a.fault, tl.inst, (int64_t)f * N + i, counter);
+            if (!ok) record_fault(a.fault, tl.inst, f * N + i, counter);
             fout[f * N + i] = v[f];
         }
     }
