@@ -26,8 +26,8 @@ def exe(tmp_path_factory):
     return compile_cpu("kernel_indices.cpp", tmp_path_factory.mktemp("cpu") / "kernel_indices")
 
 
-# 37837 and 37839 lie on either side of 3 L^2 = 2^32, 46339 below 2 L^2 = 2^32
-SIDES = [1, 5, 33, 64, 4097, 37837, 37839, 46339, 65534]
+# 37837 and 37839 lie on either side of 3 L^2 = 2^32, 46339 and 46343 of 2 L^2 = 2^32
+SIDES = [1, 5, 33, 64, 4097, 37837, 37839, 46339, 46343, 65534, 65535]
 
 
 @pytest.mark.parametrize("kernel", ["frame", "part", "tile", "veg"])

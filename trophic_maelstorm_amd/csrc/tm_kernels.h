@@ -609,15 +609,15 @@ __device__ __forceinline__ void tile_to_lds(const T* fin, int L, int x0, int y0,
     } else {
         // a wave per row (its wrap scalar), 64 dwords an instruction
         constexpr int DW = sizeof(T) / 4;             // dwords per element
-        const uint32_t* src0 = (const uint32_t*)fin;
         for (int ry = __builtin_amdgcn_readfirstlane(tid >> 6); ry < RH; ry += NT / 64) {
             const uint32_t row = (uint32_t)wrap(y0 + ry - H, L) * (uint32_t)L;
 #pragma unroll
             for (int c0 = 0; c0 < RWV * DW; c0 += 64) {
                 const int d = c0 + (tid & 63);
                 if (d < RWV * DW) {
-                    const uint32_t off = (row + (uint32_t)wrap(x0 - HC + d / DW, L)) * DW + (uint32_t)(d % DW);
-                    __builtin_amdgcn_global_load_lds(src0 + off, lds + ry * RWV * DW + c0, 4, 0, 0);
+                    // cells in 32 bits, dwords in 64: an FP64 field has 2^32 of them at a side of 46341
+                    const T* cell = fin + (row + (uint32_t)wrap(x0 - HC + d / DW, L));
+                    __builtin_amdgcn_global_load_lds((const uint32_t*)cell + d % DW, lds + ry * RWV * DW + c0, 4, 0, 0);
                 }
             }
         }
