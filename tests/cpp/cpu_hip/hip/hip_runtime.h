@@ -21,7 +21,7 @@
 #define __device__
 #define __global__
 #define __constant__
-#define __shared__ static
+#define __shared__ thread_local   /* static storage, shared by the fibers; `extern` ones are the test's to define */
 #define __forceinline__ inline
 #define __launch_bounds__(...)
 #define __align__(n) __attribute__((aligned(n)))
@@ -186,17 +186,26 @@ inline void run_workgroup(dim3 grid, dim3 block, dim3 at, std::function<void()> 
     munmap(stacks, kStack * n);
 }
 
-// Set by a test to see launches: (name, grid, block, dynamic LDS bytes, stream, run).
-inline std::function<void(const char*, dim3, dim3, size_t, void*, std::function<void()>)> on_launch;
+// Set by a test to see launches, and to run them or not.
+struct Launch {
+    const char* name;
+    const void* kernel;
+    dim3 grid, block;
+    size_t lds;      // dynamic
+    void* stream;
+    std::function<void()> run;
+};
+inline std::function<void(const Launch&)> on_launch;
 
-inline void launch(const char* name, dim3 grid, dim3 block, size_t lds, void* stream, std::function<void()> body)
+inline void launch(const char* name, const void* kernel, dim3 grid, dim3 block, size_t lds, void* stream,
+                   std::function<void()> body)
 {
     auto run = [=]() {
         for (unsigned z = 0; z < grid.z; ++z)
             for (unsigned y = 0; y < grid.y; ++y)
                 for (unsigned x = 0; x < grid.x; ++x) run_workgroup(grid, block, dim3(x, y, z), body);
     };
-    if (on_launch) on_launch(name, grid, block, lds, stream, run);
+    if (on_launch) on_launch(Launch{name, kernel, grid, block, lds, stream, run});
     else run();
 }
 
@@ -267,10 +276,14 @@ enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999, hipErrorNotReady = 600 
 enum { hipMemcpyHostToDevice, hipMemcpyDeviceToHost };
 enum { hipHostMallocDefault = 0, hipStreamNonBlocking = 1, hipEventDisableTiming = 2 };
 enum hipDeviceAttribute_t { hipDeviceAttributeWallClockRate };
+enum hipFuncAttribute { hipFuncAttributeMaxDynamicSharedMemorySize };
+struct hipFuncAttributes { size_t sharedSizeBytes; };
 
 namespace cpu_hip {
 inline std::function<void(const char*, const void*)> on_call;   // (function, pointer it is about)
 inline std::function<hipError_t(hipStream_t)> on_query;          // hipStreamQuery, hipStreamSynchronize
+inline std::function<size_t(const void*)> static_lds;            // of a kernel
+inline std::function<hipError_t(const void*, int)> on_opt_in;    // to dynamic LDS above the default limit
 inline int device = 0;
 inline void called(const char* f, const void* p = nullptr) { if (on_call) on_call(f, p); }
 }  // namespace cpu_hip
@@ -291,7 +304,16 @@ inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = malloc(1); return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+inline hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void* f)
+{
+    a->sharedSizeBytes = cpu_hip::static_lds ? cpu_hip::static_lds(f) : 0;
+    return hipSuccess;
+}
+inline hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int v)
+{
+    return cpu_hip::on_opt_in ? cpu_hip::on_opt_in(f, v) : hipSuccess;
+}
 inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 100000; return hipSuccess; }
 
 #define hipLaunchKernelGGL(kernel, grid, block, lds, stream, ...) \
-    cpu_hip::launch(#kernel, (grid), (block), (lds), (stream), [=]() mutable { (kernel)(__VA_ARGS__); })
+    cpu_hip::launch(#kernel, (const void*)(kernel), (grid), (block), (lds), (stream), [=]() mutable { (kernel)(__VA_ARGS__); })

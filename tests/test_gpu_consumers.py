@@ -201,3 +201,22 @@ def test_consumers_default_threads_are_identical(tm, model, ntiles):
     assert np.array_equal(out[0][0], out[1][0])
     for a, b in zip(out[0][1], out[1][1]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("model", ["DP2", "DP3"])
+@pytest.mark.parametrize("R", [9, 10, 12])
+def test_consumers_wide_radii_bit_exact(tm, oracle, model, R):
+    """The widest accepted perception radii, whose images take the step kernels past 64 KiB
+    of LDS: a thread per cell (small batches) and two cells a thread (the variants)."""
+    m = getattr(tm, "MODEL_" + model)
+    ns = tm.NSPECIES[m]
+    p = params(pR=(0.0, 0.1 * R + 0.05, 0.06 * R), dx=0.1)
+    insts = [tm.Instance(L, 0, 9, k) for k, L in enumerate([31, 50])]
+    rng = np.random.default_rng(R)
+    init = [_initial(rng, ns, d.L, sparse=0.7) for d in insts]
+    print(f"wide radii {model} R={R}", flush=True)
+    base, _ = _run_both(tm, oracle, m, [p], insts, init, 3)
+    for v in (f"dpc{model[2]}_f64_64x8_t256", f"dpc{model[2]}_f64_32x16_t256"):
+        got, _ = _run_both(tm, oracle, m, [p], insts, init, 3, variant=v)
+        for a, b in zip(base, got):
+            assert np.array_equal(a, b)

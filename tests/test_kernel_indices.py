@@ -1,7 +1,7 @@
 """Index arithmetic of the per-tile step kernels on lattices of any side up to 65535, by
 running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
 and the last tile is written, nothing else is, and nothing outside the fields is read.
-No GPU needed."""
+And the LDS that the consumers' launches take.  No GPU needed."""
 import os
 import subprocess
 
@@ -33,4 +33,10 @@ SIDES = [1, 5, 33, 64, 4097, 37837, 37839, 46339, 46343, 65534, 65535]
 @pytest.mark.parametrize("kernel", ["frame", "part", "tile", "veg"])
 def test_tiles_read_and_write_their_cells_only(exe, kernel):
     r = subprocess.run([exe, kernel, *map(str, SIDES)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+def test_consumer_launches_opt_in_to_their_lds(tmp_path):
+    exe = compile_cpu("consumer_lds.cpp", tmp_path / "consumer_lds")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

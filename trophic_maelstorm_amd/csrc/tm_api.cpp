@@ -819,6 +819,7 @@ tm_status setup_dpc(tm_ctx* c)
         for (const auto& q : o) disk.push_back(make_int2(q.first, q.second));
         halo = std::max(halo, R);
     }
+    if (!dpc_lds_ready(ns, halo)) return fail(c, TM_ERR_HIP, "no LDS for the perception radius");
     std::vector<DPCInstInfo> info(c->inst.size());
     std::vector<int2> chunks;
     for (size_t i = 0; i < c->inst.size(); ++i) {

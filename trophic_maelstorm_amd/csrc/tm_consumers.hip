@@ -404,17 +404,24 @@ template <int NS, int TX, int TY, int NT, int MINW = 1>
 void launch_dpc(const StepArgs& step, int grid, hipStream_t s)
 {
     const ConsumerArgs& a = static_cast<const ConsumerArgs&>(step);
-    const size_t lds = dpc_lds_bytes(NS, TX, TY, a.halo);
-    if (lds > 57344) {   // above the default LDS limit with the static arrays (CDNA4 has 160 KiB per CU)
-        static size_t granted = 0;
-        if (lds > granted &&
-            hipFuncSetAttribute((const void*)dpc_step_kernel<NS, TX, TY, NT, MINW>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess)
-            granted = lds;
-    }
+    const size_t lds = dpc_lds_bytes(NS, TX, TY, a.halo);   // opted in to by dpc_lds_ready
     hipLaunchKernelGGL(dpc_head_kernel<NS>, dim3(a.nvtiles + a.nchunks), dim3(256), 0, s, a);
     hipLaunchKernelGGL(dpc_state_kernel<NS>, dim3(a.inst1 - a.inst0), dim3(64), 0, s, a);
     hipLaunchKernelGGL((dpc_step_kernel<NS, TX, TY, NT, MINW>), dim3(grid), dim3(NT), lds, s, a);
+}
+
+// A workgroup takes 64 KiB of LDS by default, its static arrays among them; CDNA4 has 160.
+// The opt-in is always to the widest radius, so that no context lowers another's.
+template <int NS, int TX, int TY, int NT, int MINW = 1>
+bool dpc_opt_in(int halo)
+{
+    constexpr size_t kDefaultLds = 64 << 10;
+    const void* const f = (const void*)dpc_step_kernel<NS, TX, TY, NT, MINW>;
+    hipFuncAttributes at;
+    if (hipFuncGetAttributes(&at, f) != hipSuccess) return false;
+    return at.sharedSizeBytes + dpc_lds_bytes(NS, TX, TY, halo) <= kDefaultLds ||
+           hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)dpc_lds_bytes(NS, TX, TY, TM_DPC_MAX_RADIUS)) == hipSuccess;
 }
 
 // The defaults: batches of at most kWideTiles tiles (two and a half a CU) take a thread per
@@ -432,7 +439,7 @@ void launch_dpc_default(const StepArgs& a, int grid, hipStream_t s)
     else launch_dpc<NS, 32, 16, 256, MINW>(a, grid, s);
 }
 
-// _wN: at most 512/N VGPRs, N waves per SIMD
+// _wN: at most 512/N VGPRs, N waves per SIMD.  dpc_lds_ready has these kernels too.
 const Variant kDPC2[] = {
     {32, 16, 256, 0, 1, "dpc2_f64_32x16_t256", &launch_dpc<2, 32, 16, 256>, 0, 0, nullptr, 1},
     {64, 8, 256, 0, 1, "dpc2_f64_64x8_t256", &launch_dpc<2, 64, 8, 256>, 0, 0, nullptr, 1},
@@ -448,6 +455,15 @@ const Variant kDPC3[] = {
 };
 
 }  // namespace
+
+bool dpc_lds_ready(int ns, int halo)
+{
+    if (ns == 2)
+        return dpc_opt_in<2, 32, 16, 256>(halo) && dpc_opt_in<2, 64, 8, 256>(halo) && dpc_opt_in<2, 32, 16, 256, 4>(halo) &&
+               dpc_opt_in<2, 32, 16, 256, 5>(halo) && dpc_opt_in<2, 32, 16, 256, 6>(halo) && dpc_opt_in<2, 32, 16, 512>(halo);
+    return dpc_opt_in<3, 32, 16, 256>(halo) && dpc_opt_in<3, 64, 8, 256>(halo) && dpc_opt_in<3, 32, 16, 256, 4>(halo) &&
+           dpc_opt_in<3, 32, 16, 256, 5>(halo) && dpc_opt_in<3, 32, 16, 512>(halo);
+}
 
 const Variant* dpc2_variants_f64(int* n) { *n = (int)(sizeof(kDPC2) / sizeof(kDPC2[0])); return kDPC2; }
 const Variant* dpc3_variants_f64(int* n) { *n = (int)(sizeof(kDPC3) / sizeof(kDPC3[0])); return kDPC3; }

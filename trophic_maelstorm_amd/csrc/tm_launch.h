@@ -63,7 +63,10 @@ struct DPCWork {
     double* pstar;        // ... and its result P*, at cell_off
     double* lambda;       // lambda of the consumers' cells whose Gamma deviate is deferred, (ns - 1) fields
 };
-// LDS of the consumer step kernel: NS density images with the halo, plus the
+// Opts the consumer step kernels in to the LDS they need at this halo on the current
+// device; false where that is refused.
+bool dpc_lds_ready(int ns, int halo);
+// Dynamic LDS of the consumer step kernel: NS density images with the halo, plus the
 // perception offsets of the largest radius.
 inline size_t dpc_lds_bytes(int ns, int tx, int ty, int halo)
 {
