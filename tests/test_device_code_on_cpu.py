@@ -1,7 +1,8 @@
 """Index arithmetic of the per-tile step kernels on lattices of any side up to 65535, by
 running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
 and the last tile is written, nothing else is, and nothing outside the fields is read.
-And the LDS that the consumers' launches take.  No GPU needed."""
+And, the same way, the LDS that the consumers' launches take and the accept estimates of
+the FP64 samplers.  No GPU needed."""
 import os
 import subprocess
 
@@ -39,4 +40,12 @@ def test_tiles_read_and_write_their_cells_only(exe, kernel):
 def test_consumer_launches_opt_in_to_their_lds(tmp_path):
     exe = compile_cpu("consumer_lds.cpp", tmp_path / "consumer_lds")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+def test_accept_estimates_as_compiled(tmp_path):
+    """ptrs_estimate and gamma_estimate from the source the kernels are built of, with
+    v_log_f32 and v_rcp_f32 an ulp off either way, near equality and far from it."""
+    exe = compile_cpu("accept_estimates.cpp", tmp_path / "accept_estimates")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
