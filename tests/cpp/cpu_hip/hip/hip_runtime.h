@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <tuple>
 #include <vector>
 
 #define __HIP_DEVICE_COMPILE__ 1
@@ -197,15 +198,17 @@ struct Launch {
 };
 inline std::function<void(const Launch&)> on_launch;
 
-inline void launch(const char* name, const void* kernel, dim3 grid, dim3 block, size_t lds, void* stream,
-                   std::function<void()> body)
+template <class... P, class... A>
+void launch(const char* name, void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, void* stream, A&&... args)
 {
+    const std::tuple<std::decay_t<P>...> values(std::forward<A>(args)...);   // as they are now
+    const std::function<void()> body = [=]() { std::apply(kernel, values); };
     auto run = [=]() {
         for (unsigned z = 0; z < grid.z; ++z)
             for (unsigned y = 0; y < grid.y; ++y)
                 for (unsigned x = 0; x < grid.x; ++x) run_workgroup(grid, block, dim3(x, y, z), body);
     };
-    if (on_launch) on_launch(Launch{name, kernel, grid, block, lds, stream, run});
+    if (on_launch) on_launch(Launch{name, (const void*)kernel, grid, block, lds, stream, run});
     else run();
 }
 
@@ -316,4 +319,4 @@ inline hipError_t hipFuncSetAttribute(const void* f, hipFuncAttribute, int v)
 inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 100000; return hipSuccess; }
 
 #define hipLaunchKernelGGL(kernel, grid, block, lds, stream, ...) \
-    cpu_hip::launch(#kernel, (const void*)(kernel), (grid), (block), (lds), (stream), [=]() mutable { (kernel)(__VA_ARGS__); })
+    cpu_hip::launch(#kernel, (kernel), (grid), (block), (lds), (stream), __VA_ARGS__)

@@ -1,8 +1,8 @@
 """Index arithmetic of the per-tile step kernels on lattices of any side up to 65535, by
 running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
 and the last tile is written, nothing else is, and nothing outside the fields is read.
-And, the same way, the LDS that the consumers' launches take and the accept estimates of
-the FP64 samplers.  No GPU needed."""
+And, the same way, the LDS that the consumers' launches take, the accept estimates of the
+FP64 samplers and the staged downloads' failures.  No GPU needed."""
 import os
 import subprocess
 
@@ -47,5 +47,13 @@ def test_accept_estimates_as_compiled(tmp_path):
     """ptrs_estimate and gamma_estimate from the source the kernels are built of, with
     v_log_f32 and v_rcp_f32 an ulp off either way, near equality and far from it."""
     exe = compile_cpu("accept_estimates.cpp", tmp_path / "accept_estimates")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+def test_staged_download_reports_failures(tmp_path):
+    """A device copy that never lands is an error, not an endless wait; the caller's
+    current device stays."""
+    exe = compile_cpu("hostcopy.cpp", tmp_path / "hostcopy")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

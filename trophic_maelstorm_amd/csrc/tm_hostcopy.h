@@ -27,7 +27,8 @@ public:
     enum Result { kOk, kBusy, kFailed };
     // n elements at src (device, complete: the caller has waited for its writers) to dst
     // (host): floats widened to doubles, or doubles as they are.  kBusy, with nothing
-    // done, while another thread's copy runs; kFailed on a HIP error.
+    // done, while another thread's copy runs; kFailed on a HIP error, of the device's copy
+    // too.  The caller's current device stays what it is.
     Result copy(double* dst, const void* src, size_t n, bool widen);
 
 private:

@@ -36,10 +36,30 @@ __global__ __launch_bounds__(256) void to_pinned_kernel(const char* __restrict__
     if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x, mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// Makes a device current, and the one before it again.
+class OnDevice {
+public:
+    explicit OnDevice(int device)
+    {
+        if (hipGetDevice(&before_) != hipSuccess) before_ = device;
+        ok_ = before_ == device || hipSetDevice(device) == hipSuccess;
+        if (before_ == device || !ok_) before_ = -1;
+    }
+    ~OnDevice() { if (before_ >= 0) (void)hipSetDevice(before_); }
+    OnDevice(const OnDevice&) = delete;
+    OnDevice& operator=(const OnDevice&) = delete;
+    bool ok() const { return ok_; }
+
+private:
+    int before_ = -1;
+    bool ok_ = false;
+};
+
 }  // namespace
 
 struct HostCopier::Impl {
     static constexpr size_t kPer = kHalf / kPiece;   // pieces of a half
+    int device = 0;
     hipStream_t stream = nullptr;
     char* half[2] = {nullptr, nullptr};       // pinned
     uint64_t* flags = nullptr;                // pinned, kPer per half
@@ -49,7 +69,7 @@ struct HostCopier::Impl {
     // the copy in hand, set before `job` is raised: segment g (kHalf bytes of the source)
     // passes through half g % 2 in pieces of kPiece, marked mark0 + g
     double* dst = nullptr;
-    size_t bytes = 0, pieces = 0;
+    size_t bytes = 0, pieces = 0, queued = 0;        // queued: segments, the calling thread's
     uint64_t mark0 = 0;
     bool widen = false;
     std::atomic<size_t> next{0};              // piece to take
@@ -63,9 +83,31 @@ struct HostCopier::Impl {
     std::atomic<uint64_t> job{0};
     std::atomic<bool> stop{false};
 
+    // The calling thread, now and then while it waits: a stream that failed, or is done
+    // and left a flag as it was, ends the copy for all threads.
+    void look()
+    {
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();
+            return;
+        }
+        bool all = e == hipSuccess;
+        for (size_t g = queued < 2 ? 0 : queued - 2; g < queued; ++g)   // the segments in the halves
+            for (size_t i = 0; i < kPer && g * kPer + i < pieces; ++i)
+                all = all && __atomic_load_n(flags + (g & 1) * kPer + i, __ATOMIC_ACQUIRE) == mark0 + g;
+        if (!all) failed = true;
+    }
+    static constexpr unsigned kLookEvery = 4096;     // waits; a wait is a yield, under a microsecond
+    void wait(unsigned& waits, bool caller)
+    {
+        if (caller && ++waits % kLookEvery == 0) look();
+        std::this_thread::yield();
+    }
+
     // One piece below `limit` off the common counter, once it has landed; false when none
     // is left.
-    bool piece(size_t limit)
+    bool piece(size_t limit, bool caller)
     {
         size_t p = next.load();
         do {
@@ -74,9 +116,10 @@ struct HostCopier::Impl {
         const size_t g = p / kPer, i = p % kPer;
         const uint64_t* f = flags + (g & 1) * kPer + i;
         const uint64_t want = mark0 + g;
+        unsigned waits = 0;
         while (__atomic_load_n(f, __ATOMIC_ACQUIRE) != want) {
             if (failed.load()) return false;
-            std::this_thread::yield();
+            wait(waits, caller);
         }
         const size_t b0 = p * kPiece, m = std::min(kPiece, bytes - b0);
         const char* from = half[g & 1] + i * kPiece;
@@ -106,7 +149,7 @@ struct HostCopier::Impl {
             }
             if (stop.load()) return;
             seen = job.load(std::memory_order_acquire);
-            while (piece(pieces)) {}
+            while (piece(pieces, false)) {}
             busy.fetch_sub(1, std::memory_order_release);
         }
     }
@@ -139,7 +182,9 @@ std::shared_ptr<HostCopier> HostCopier::get(int device) noexcept
         if (std::shared_ptr<HostCopier> c = of[device].lock()) return c;
         std::shared_ptr<HostCopier> c(new HostCopier());
         Impl* m = c->impl_ = new Impl();
-        const bool ok = hipSetDevice(device) == hipSuccess &&
+        m->device = device;
+        const OnDevice on(device);
+        const bool ok = on.ok() &&
                         hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking) == hipSuccess &&
                         hipHostMalloc((void**)&m->half[0], kHalf, hipHostMallocDefault) == hipSuccess &&
                         hipHostMalloc((void**)&m->half[1], kHalf, hipHostMallocDefault) == hipSuccess &&
@@ -164,6 +209,8 @@ HostCopier::Result HostCopier::copy(double* dst, const void* src, size_t n, bool
     Impl& m = *impl_;
     std::unique_lock<std::mutex> use(m.use, std::try_to_lock);
     if (!use.owns_lock()) return kBusy;
+    const OnDevice on(m.device);
+    if (!on.ok()) return kFailed;
     m.dst = dst;
     m.bytes = n * (widen ? sizeof(float) : sizeof(double));
     m.pieces = (m.bytes + kPiece - 1) / kPiece;
@@ -175,7 +222,9 @@ HostCopier::Result HostCopier::copy(double* dst, const void* src, size_t n, bool
     m.out[0] = m.out[1] = 0;
     m.failed = false;
     m.busy = kThreads - 1;
-    size_t queued = 0;
+    m.queued = 0;
+    size_t& queued = m.queued;
+    unsigned waits = 0;
     auto queue = [&]() {
         const size_t b0 = queued * kHalf, b = std::min(kHalf, m.bytes - b0);
         hipLaunchKernelGGL(to_pinned_kernel, dim3((unsigned)((b + kPiece - 1) / kPiece)), dim3(256), 0, m.stream,
@@ -194,10 +243,10 @@ HostCopier::Result HostCopier::copy(double* dst, const void* src, size_t n, bool
     // this thread copies pieces of the queued segments only: a later one would wait for it.
     while (queued < segs && !m.failed) {
         if (m.out[queued & 1].load(std::memory_order_acquire) >= queued / 2 * Impl::kPer) queue();
-        else if (!m.piece(queued * Impl::kPer)) std::this_thread::yield();
+        else if (!m.piece(queued * Impl::kPer, true)) m.wait(waits, true);
     }
-    while (m.piece(m.pieces)) {}
-    while (m.busy.load(std::memory_order_acquire) != 0) std::this_thread::yield();
+    while (m.piece(m.pieces, true)) {}
+    while (m.busy.load(std::memory_order_acquire) != 0) m.wait(waits, true);
     if (m.failed) (void)hipStreamSynchronize(m.stream);
     return m.failed ? kFailed : kOk;
 }
