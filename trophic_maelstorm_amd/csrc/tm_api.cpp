@@ -960,7 +960,7 @@ void tm_destroy(tm_ctx* c)
     if (!c) return;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
-    workspace_give_back();
+    workspace_give_back(c->device);
     release_config(c);
     free_dev(c->d_state);
     if (c->h_pinned) hipHostFree(c->h_pinned);

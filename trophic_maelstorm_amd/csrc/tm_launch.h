@@ -92,8 +92,8 @@ int fke_setup(int model, const tm_fke_params* params, int n_params, const tm_ins
 // Movement statistics of the current fields into out [n_inst][4 SpB] (device).
 void launch_fke_mov_stats(int model, const ConsumerArgs& a, double* out, hipStream_t s);
 
-// Free the device scratch the Rietkerk consumer operators keep between calls.
-void workspace_give_back();
+// Free the scratch on a device that the Rietkerk consumer operators keep between calls.
+void workspace_give_back(int device);
 
 // Default variant index of a batch.
 int default_variant(int model, int precision, const tm_instance_desc* inst, int n_inst, int n_cu);

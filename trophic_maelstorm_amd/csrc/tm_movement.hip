@@ -691,7 +691,7 @@ void gauss_stencil(double sigma, int R, double* st)
 // get() until it has waited for the kernels that use it (idle), so calls of several
 // threads and streams never share one; a block that is not known to be idle is freed,
 // which waits for the device.  At most kKeepTotal bytes in kKeepBlocks blocks stay,
-// the oldest going first; tm_destroy and a failed allocation give all of them back.
+// the oldest going first; tm_destroy and a failed allocation give their device's back.
 class Workspace {
 public:
     bool idle = true;
@@ -706,15 +706,20 @@ public:
             return;
         }
         Pool& k = pool();
-        std::lock_guard<std::mutex> lock(k.mu);
-        k.v[k.n++] = b_;
-        size_t total = 0;
-        for (int i = 0; i < k.n; ++i) total += k.v[i].bytes;
-        while (total > kKeepTotal || k.n > kKeepBlocks) {
-            total -= k.v[0].bytes;
-            release(k.v[0]);
-            k.erase(0);
+        Block out[kKeepBlocks + 1];   // freed past the lock: a free waits for its device
+        int n = 0;
+        {
+            std::lock_guard<std::mutex> lock(k.mu);
+            k.v[k.n++] = b_;
+            size_t total = 0;
+            for (int i = 0; i < k.n; ++i) total += k.v[i].bytes;
+            while (total > kKeepTotal || k.n > kKeepBlocks) {
+                total -= k.v[0].bytes;
+                out[n++] = k.v[0];
+                k.erase(0);
+            }
         }
+        while (n > 0) release(out[--n]);
     }
     // A block of at least `bytes` on the current device.
     bool get(size_t bytes)
@@ -734,19 +739,30 @@ public:
         b_ = Block{nullptr, nullptr, bytes, dev};
         if (make(b_)) return true;
         (void)hipGetLastError();
-        give_back();
+        give_back(dev);
         return make(b_);
     }
     // Pinned host memory that goes with the block, kHostDoubles long.
     double* host() const { return b_.h; }
     static constexpr int kHostDoubles = 3 * 256;
     template <typename T> T* at(size_t offset) const { return (T*)((char*)b_.p + offset); }
-    static void give_back()
+    static void give_back(int dev)
     {
         Pool& k = pool();
-        std::lock_guard<std::mutex> lock(k.mu);
-        for (int i = 0; i < k.n; ++i) release(k.v[i]);
-        k.n = 0;
+        Block out[kKeepBlocks + 1];
+        int n = 0;
+        {
+            std::lock_guard<std::mutex> lock(k.mu);
+            for (int i = 0; i < k.n;) {
+                if (k.v[i].dev == dev) {
+                    out[n++] = k.v[i];
+                    k.erase(i);
+                } else {
+                    ++i;
+                }
+            }
+        }
+        while (n > 0) release(out[--n]);
     }
 
 private:
@@ -1697,7 +1713,7 @@ int fke_setup(int model, const tm_fke_params* P, int n_params, const tm_instance
     return TM_OK;
 }
 
-void workspace_give_back() { Workspace::give_back(); }
+void workspace_give_back(int device) { Workspace::give_back(device); }
 
 }  // namespace tmk
 
