@@ -2,8 +2,8 @@
 running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
 and the last tile is written, nothing else is, and nothing outside the fields is read.
 And, the same way, the LDS that the consumers' launches take, the accept estimates of the
-FP64 samplers, the staged downloads' failures and the operators' kept scratch.  No GPU
-needed."""
+FP64 samplers, the staged downloads' failures, the operators' kept scratch and the lanes
+of runs.  No GPU needed."""
 import os
 import subprocess
 
@@ -64,3 +64,9 @@ def test_operators_scratch_is_given_back_by_device(tmp_path):
     exe = compile_cpu("workspace.cpp", tmp_path / "workspace")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stderr)
+
+
+def test_lanes_are_measured_again_after_a_busy_start(tmp_path):
+    exe = compile_cpu("run_lanes.cpp", tmp_path / "run_lanes")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

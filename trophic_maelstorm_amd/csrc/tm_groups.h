@@ -29,7 +29,8 @@ public:
     static std::shared_ptr<RunLanes> get(int device) noexcept;
     ~RunLanes();
     // Makes and measures the lanes at the first call (1 to 2 ms); false where fewer than
-    // two run side by side.
+    // two ran side by side.  Work of others on the GPU can make two queues look like one,
+    // so up to kAttempts calls measure until two are found.
     bool prepare();
     // A free lane of its own, or -1; to be given back when what it was given is done.
     int take();
@@ -47,11 +48,11 @@ public:
     bool alone() const { return runs_.load() == 1; }
 
 private:
-    static constexpr int kLanes = 4, kTries = 8;
+    static constexpr int kLanes = 4, kTries = 8, kAttempts = 4;
     bool side_by_side(int n);   // streams 0 .. n
     std::mutex mu_;
     std::atomic<int> runs_{0};
-    bool made_ = false;
+    int attempts_ = 0;
     int n_ = 0;
     hipStream_t s_[kLanes] = {};
     hipEvent_t ev_[kLanes] = {};

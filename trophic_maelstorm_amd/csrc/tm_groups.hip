@@ -99,8 +99,8 @@ bool RunLanes::side_by_side(int n)
 bool RunLanes::prepare()
 {
     std::lock_guard<std::mutex> lock(mu_);
-    if (made_) return n_ >= 2;
-    made_ = true;
+    if (n_ >= 2 || attempts_ == kAttempts) return n_ >= 2;
+    ++attempts_;
     // New streams take the least used queues, so those passed over are kept meanwhile.
     hipStream_t passed_over[kTries];
     int np = 0;
@@ -128,6 +128,7 @@ bool RunLanes::prepare()
 int RunLanes::take()
 {
     std::lock_guard<std::mutex> lock(mu_);
+    if (n_ < 2) return -1;
     for (int k = 0; k < n_; ++k)
         if (!taken_[k]) {
             taken_[k] = true;
