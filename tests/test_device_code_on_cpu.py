@@ -2,8 +2,8 @@
 running them on the CPU (tests/cpp/cpu_hip) over sparse memory: every cell of the first
 and the last tile is written, nothing else is, and nothing outside the fields is read.
 And, the same way, the LDS that the consumers' launches take, the accept estimates of the
-FP64 samplers, the staged downloads' failures, the operators' kept scratch and the lanes
-of runs.  No GPU needed."""
+FP64 samplers, the staged downloads' failures, the operators' kept scratch, the lanes of
+runs and the default steps' choice of kernel.  No GPU needed."""
 import os
 import subprocess
 
@@ -70,3 +70,28 @@ def test_lanes_are_measured_again_after_a_busy_start(tmp_path):
     exe = compile_cpu("run_lanes.cpp", tmp_path / "run_lanes")
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+RULES = [
+    ("tm_kernels_f64.hip", "dp_variants_f64", "dp_f64_64x32_t256_x8aq_w6",
+     [(1280, "dp_part_kernel<double, 64, 32, 1>"), (1281, "dp_step_kernel")]),
+    ("tm_kernels_f32.hip", "dp_variants_f32", "dp_f32_128x24_t256_x8aq",
+     [(384, "dp_part_kernel<float, 128, 24, 1>"), (385, "dp_part_kernel<float, 128, 24, 3>"),
+      (1152, "dp_part_kernel<float, 128, 24, 3>"), (1153, "dp_step_kernel")]),
+    ("tm_movement.hip", "fke2_variants_f64", "fke2_f64_t256",
+     [(3072, "fke_head_kernel<SP, true>"), (3073, "fke_head_kernel<SP, false>")]),
+    ("tm_movement.hip", "fke3_variants_f64", "fke3_f64_t256",
+     [(3072, "fke_head_kernel<SP, true>"), (3073, "fke_head_kernel<SP, false>")]),
+]
+
+
+@pytest.mark.parametrize("unit,table,variant,edges", RULES, ids=[r[1] for r in RULES])
+def test_size_rules_hold_for_the_batch(tmp_path, unit, table, variant, edges):
+    """A batch in two instance groups takes the kernel of the whole batch's size."""
+    exe = compile_cpu("size_rules.cpp", tmp_path / "size_rules", f'-DUNIT="{unit}"', f"-DTABLE={table}",
+                      *(["-DMOVE"] if unit == "tm_movement.hip" else []))
+    r = subprocess.run([exe, variant, *[str(n) for n, _ in edges]], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    got = r.stdout.split("\n")[:-1]
+    for k, (n, want) in enumerate(edges):
+        assert want in got[2 * k] and want in got[2 * k + 1], (n, got[2 * k:2 * k + 2])

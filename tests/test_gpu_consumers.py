@@ -220,3 +220,25 @@ def test_consumers_wide_radii_bit_exact(tm, oracle, model, R):
         got, _ = _run_both(tm, oracle, m, [p], insts, init, 3, variant=v)
         for a, b in zip(base, got):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("ns", [2, 3])
+def test_consumers_vegetation_in_two_passes(tm, ns):
+    """A batch of over 2816 tiles of 64 x 4, where the vegetation's step runs in two passes on
+    64 x 16 tiles, in two groups, against the same instances three at a time, bit for bit."""
+    model = tm.MODEL_DP3 if ns == 3 else tm.MODEL_DP2
+    hi = [20.0, 2.0, 0.5, 0.0, 0.0] if ns == 3 else [20.0, 2.0, 0.0]
+    insts = [tm.Instance(65 if k % 50 == 0 else 23, 0, 5, k) for k in range(471)]
+    tiles = sum(-(-d.L // 64) * -(-d.L // 4) for d in insts)
+    assert tiles > 2816
+    pick = [0, 233, 450]
+    out = []
+    for batch, at in ((insts, pick), ([insts[k] for k in pick], [0, 1, 2])):
+        with tm.Context() as ctx:
+            ctx.configure(model, tm.F64, tm.DPCParams(a=1e-5), batch)
+            ctx.init_uniform([0.0] * len(hi), hi)
+            rows = ctx.run(3)
+            out.append([(ctx.download(k), rows[k]) for k in at])
+    for (f0, r0), (f1, r1) in zip(*out):
+        assert np.array_equal(f0, f1)
+        assert np.array_equal(r0, r1)

@@ -140,3 +140,26 @@ def test_fke_model_many_chunks_matches_oracle(tm, oracle, SP):
     for k, d in enumerate(insts):
         ref, _, _ = _oracle_run(oracle, p[0], SP, f0[k], d, 2)
         assert np.array_equal(got[k], ref), (SP, d.L, np.argwhere(got[k] != ref)[:5])
+
+
+@pytest.mark.parametrize("sp", [2, 3])
+def test_fke_vegetation_in_two_passes(tm, sp):
+    """A batch of over 3072 tiles of 64 x 4, where the vegetation's step runs in two passes
+    on 64 x 16 tiles, in two groups, against the same instances three at a time, bit for
+    bit."""
+    model = tm.MODEL_FKE3 if sp == 3 else tm.MODEL_FKE2
+    hi = [60.0, 3.0, 0.5, 2.0, 2.0, 0.0, 0.0] if sp == 3 else [60.0, 3.0, 2.0, 2.0, 0.0]
+    insts = [tm.Instance(65 if k % 50 == 0 else 23, 0, 5, k) for k in range(471)]
+    tiles = sum(-(-d.L // 64) * -(-d.L // 4) for d in insts)
+    assert tiles > 3072
+    pick = [0, 233, 450]
+    out = []
+    for batch, at in ((insts, pick), ([insts[k] for k in pick], [0, 1, 2])):
+        with tm.Context() as ctx:
+            ctx.configure(model, tm.F64, tm.FKEParams(), batch)
+            ctx.init_uniform([0.0] * len(hi), hi)
+            rows = ctx.run(3)
+            out.append([(ctx.download(k), rows[k]) for k in at])
+    for (f0, r0), (f1, r1) in zip(*out):
+        assert np.array_equal(f0, f1)
+        assert np.array_equal(r0, r1)

@@ -353,3 +353,30 @@ def test_fp32_rietkerk_frames_are_identical(tm, want):
     assert np.array_equal(d0, d1)
     assert np.array_equal(f0, f1)
     assert np.allclose(r0, r1, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("prec,n", [("f64", 1280), ("f64", 1281), ("f32", 384), ("f32", 385), ("f32", 1152), ("f32", 1153)])
+def test_dp_parts_and_tiles_at_the_edges_of_the_rule(tm, prec, n):
+    """Batches on either side of the tiles at which the default DP step changes its kernel,
+    in two groups (sides of 22: one tile each): fields, draws and rho(t) rows are the
+    two-pass tile kernel's."""
+    P = tm.F64 if prec == "f64" else tm.F32
+    names = tm.variant_names(tm.MODEL_DP, P)
+    fixed = "dp_f64_64x32_t256_x8aq" if prec == "f64" else "dp_f32_128x24_t256_w6q"
+    L = 22
+    insts = [tm.Instance(L, 0, 9, k) for k in range(n - 1)]
+    insts.append(tm.Instance(24 if prec == "f32" else 32, 0, 9, n))
+    out = []
+    for v in (-1, names.index(fixed)):
+        with tm.Context() as ctx:
+            ctx.configure(tm.MODEL_DP, P, tm.DPParams(a=0.9), insts)
+            ctx.set_launch(v, 16)
+            ctx.init_uniform([0.0], [1.0])
+            ctx.record_draws(True)
+            rows = ctx.run(4)
+            pick = [0, 1, n // 2 - 1, n // 2, n // 2 + 1, n - 1]
+            out.append((rows, [ctx.download(k) for k in pick], [ctx.draws(k) for k in pick]))
+    (r0, f0, d0), (r1, f1, d1) = out
+    assert np.array_equal(r0, r1)
+    for a, b in zip(f0 + d0, f1 + d1):
+        assert np.array_equal(a, b)

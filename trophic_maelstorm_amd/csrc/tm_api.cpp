@@ -840,7 +840,7 @@ tm_status setup_dpc(tm_ctx* c)
         for (int k = 0; k < nch; ++k) chunks.push_back(make_int2((int)i, k));
     }
     // The vegetation's Dornic step: 64 x 16 tiles in two passes, or 64 x 4 tiles with one
-    // cell a thread where those are at most kVegDirectTiles and the larger would leave
+    // cell a thread where those are at most kVegDirectTilesDpc and the larger would leave
     // CUs idle.
     std::vector<int4> vtiles;
     for (const int ty : {4, 16}) {
@@ -851,7 +851,7 @@ tm_status setup_dpc(tm_ctx* c)
                 for (int x0 = 0; x0 < c->inst[i].L; x0 += 64) vtiles.push_back(make_int4((int)i, x0, y0, 0));
         }
         c->dpc_vdirect = ty == 4;
-        if (vtiles.size() <= (size_t)kVegDirectTiles) break;
+        if (vtiles.size() <= (size_t)kVegDirectTilesDpc) break;
     }
     c->end.vtile = (int)vtiles.size();
     c->end.chunk = (int)chunks.size();

@@ -18,16 +18,18 @@ static void launch_dpk(const StepArgs& a, int grid, hipStream_t s)
     hipLaunchKernelGGL((dp_stepk_kernel<T, TX, TY, NT, K, MINW>), dim3(grid), dim3(NT), 0, s, a);
 }
 
-// The default's single step: a workgroup per part of a tile (dp_part_kernel), one cell
-// a thread up to 256 tiles, three up to 1024, the two-pass tile kernel above.  us a
-// step, one / three cells / tiles: 6.0 / 9.4 / 21.3 at 48 tiles (8 x 128^2), 14.1 / 14.4 /
-// 23.1 at 288, 16.8 / 16.3 / 23.4 at 384, 28.4 / 26.1 / 27.5 at 768, 40.7 / 35.7 / 36.2
-// at 1152.
+// The default's single step: a workgroup per part of a tile (dp_part_kernel), one cell a
+// thread for batches of up to 384 tiles, three up to 1152, the two-pass tile kernel above.
+// us a step, one / three cells / tiles: 6.0 / 9.4 / 21.3 at 48 tiles (8 x 128^2); as two groups
+// of n x 128^2 10.9 / 12.5 / 22.2 at 288, 13.5 / 13.3 / 22.4 at 384, 15.2 / 14.6 / 22.3 at 432,
+// 25.4 / 21.5 / 26.6 at 768, 34.9 / 28.8 / 30.2 at 1056, 37.8 / 31.1 / 31.0 at 1152, 50.4 / 40.5 /
+// 32.4 at 1536.  One lattice: 14.4 / 14.7 / 23.2 at 266 (896^2), 23.5 / 22.8 / 28.0 at 540,
+// 39.0 / 34.8 / 38.1 at 1050, 49.3 / 43.1 / 43.3 at 1376.
 static void launch_dp_default(const StepArgs& a, int grid, hipStream_t s)
 {
-    if (a.ntiles <= 256)
+    if (a.ptiles <= 384)
         hipLaunchKernelGGL((dp_part_kernel<float, 128, 24, 1>), dim3(4 * a.ntiles), dim3(768), 0, s, a);
-    else if (a.ntiles <= 1024)
+    else if (a.ptiles <= 1152)
         hipLaunchKernelGGL((dp_part_kernel<float, 128, 24, 3>), dim3(4 * a.ntiles), dim3(256), 0, s, a);
     else
         launch_dp<float, 128, 24, 256, 0, 6, 1>(a, grid, s);

@@ -20,13 +20,15 @@ static void launch_dpk(const StepArgs& a, int grid, hipStream_t s)
     hipLaunchKernelGGL((dp_stepk_kernel<T, TX, TY, NT, K, MINW>), dim3(grid), dim3(NT), 0, s, a);
 }
 
-// The default's single step: a workgroup per part of a tile (dp_part_kernel) up to
-// 1024 tiles, the two-pass tile kernel above.  us a step, parts against tiles:
-// 8.8 / 31.1 at 64 tiles (8 x 128^2), 17.2 / 31.1 at 256, 28.4 / 37.9 at 512,
-// 50.3 / 56.9 at 1024 (2.1 M cells); the tiles take 97.3 at 2048, under twice 50.3.
+// The default's single step: a workgroup per part of a tile (dp_part_kernel) for batches of
+// up to 1280 tiles, the two-pass tile kernel above.  us a step, parts / tiles: 8.8 / 31.1 at
+// 64 tiles (8 x 128^2); as two groups of n x 128^2 24.9 / 35.7 at 512, 46.9 / 47.6 at 1024,
+// 54.9 / 56.0 at 1200, 60.0 / 59.7 at 1312, 70.3 / 65.8 at 1536, 93.3 / 86.1 at 2048.  One large
+// lattice is one group, and parts hold longer there: 51.8 / 60.3 at 1012 (1408^2), 64.0 / 73.9
+// at 1250, 99.6 / 103.8 at 2048.
 static void launch_dp_default(const StepArgs& a, int grid, hipStream_t s)
 {
-    if (a.ntiles <= 1024)
+    if (a.ptiles <= 1280)
         hipLaunchKernelGGL((dp_part_kernel<double, 64, 32, 1>), dim3(4 * a.ntiles), dim3(512), 0, s, a);
     else
         launch_dp<double, 64, 32, 256, 0, 6, 1>(a, grid, s);

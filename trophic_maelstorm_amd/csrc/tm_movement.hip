@@ -1381,7 +1381,7 @@ template <int SP, int TX, int TY, int NT>
 void launch_fke(const StepArgs& step, int grid, hipStream_t s)
 {
     const ConsumerArgs& a = static_cast<const ConsumerArgs&>(step);
-    if (a.ntiles <= kVegDirectTiles)
+    if (a.ptiles <= kVegDirectTilesFke)
         hipLaunchKernelGGL((fke_head_kernel<SP, true>), dim3((unsigned)(grid + a.nchunks)), dim3(256), 0, s, a, grid);
     else
         hipLaunchKernelGGL((fke_head_kernel<SP, false>), dim3((unsigned)(a.nmtiles + a.nchunks)), dim3(256), 0, s, a,

@@ -79,10 +79,15 @@ __device__ __forceinline__ void queue_push(bool flag, uint16_t e, uint16_t* q, u
 // Rietkerk model in 36 us, with the chunk sums beside it in 30 here.
 constexpr int kVegTX = 64, kVegTY = 16;
 
-// Up to this many 64 x 4 tiles the models run one cell a thread instead: us a step of the
-// three-species Rietkerk model, direct / two passes: 45 / 54 on 4 x 64^2, 54 / 61 on 2 x 256^2,
-// 106 / 107 on 8 x 256^2 (2048 tiles), 175 / 171 on 16 x 256^2.
-constexpr int kVegDirectTiles = 2048;
+// Batches of up to this many 64 x 4 tiles run one cell a thread instead.  us a step, direct /
+// two passes, n x 256^2 (256 tiles each, two groups) and one lattice:
+//   Rietkerk, 3 species  8: 92 / 96   12: 122 / 124   14: 139 / 135   16: 155 / 150   20: 188 / 183
+//                        768^2: 119 / 124   896^2 (3136): 148 / 151   1024^2 (4096): 172 / 172
+//   Rietkerk, 2 species  8: 66 / 69   12: 87 / 87   14: 98 / 93   16: 106 / 101   20: 126 / 121
+//   DP, 2 species        8: 59 / 62   10: 70 / 70   11: 74 / 75   12: 80 / 76   16: 92 / 88
+//                        896^2: 100 / 102   1024^2: 114 / 112
+//   DP, 3 species        8: 83 / 88   11: 108 / 114   12: 115 / 117   16: 143 / 138
+constexpr int kVegDirectTilesFke = 12 * 256, kVegDirectTilesDpc = 11 * 256;
 
 struct VegLds {
     uint32_t n[2];
