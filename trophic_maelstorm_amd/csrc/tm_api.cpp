@@ -312,6 +312,7 @@ const Variant& cur_variant(tm_ctx* c)
 // has nothing to fill the other's gaps with (1024^2 + 64^2 of FP32 Rietkerk 35.8 / 36.7;
 // 1024^2 + 4 x 128^2 of FP64 61.9 / 58.5).
 constexpr int64_t kGroupCells = 12 * 128 * 128;
+constexpr int64_t kOrderCells = 32 * 128 * 128;   // from here on the groups' kernels in different orders (step_args)
 
 int group_cut(tm_ctx* c)
 {
@@ -432,9 +433,12 @@ ConsumerArgs step_args(tm_ctx* c, int parity, int k, int g = kWholeBatch)
     a.nmtiles = hi.mtile - lo.mtile;
     a.move_lds = c->move_lds;
     // Two chains settle into step with each other: in the other order, the second group's
-    // kernels are not the first's beside them (16 x 256^2, three-species Rietkerk consumers:
-    // 154 us, 165 in one order; 7 x 256^2 84 and 88; 16 x 128^2 64 and 62).
-    a.rk_first = g == 1 && c->total_cells >= 2 * kGroupCells;
+    // kernels are not the first's beside them.  us a step of the Rietkerk consumers, other /
+    // one order, three species: 16 x 128^2 64.6 / 60.4, 24 x 128^2 79.1 / 76.7, 28 x 128^2 84.8 /
+    // 83.7, 32 x 128^2 88.2 / 89.1, 128 x 64^2 92.4 / 99.9, 40 x 128^2 106 / 110, 12 x 256^2
+    // 121 / 129, 16 x 256^2 155 / 165; two species: 16 x 128^2 49.7 / 47.6, 28 x 128^2 62.0 / 63.2,
+    // 32 x 128^2 65.0 / 65.5, 12 x 256^2 86.8 / 85.8, 16 x 256^2 106 / 109.
+    a.rk_first = g == 1 && c->total_cells >= kOrderCells;
     a.inst0 = lo.inst;
     a.inst1 = hi.inst;
     a.chunk0 = lo.chunk;
