@@ -163,3 +163,42 @@ def test_fke_vegetation_in_two_passes(tm, sp):
     for (f0, r0), (f1, r1) in zip(*out):
         assert np.array_equal(f0, f1)
         assert np.array_equal(r0, r1)
+
+
+def _move_tile_bytes(tm, p, SP):
+    """LDS of the widest consumer's 64 x 16 movement tile (move_tile_lds in csrc): above
+    128 KiB the step moves them in four passes."""
+    most = 0
+    for s in range(1, SP):
+        (rD, rV, pref), _, _ = tm.fke_move_constants(p.D_mov[s], p.v[s], p.sigma[s], p.dt_analytic, p.dx, p.dt_adv[s],
+                                                     p.mv_invariance, p.CI)
+        S = int((abs(p.v[s] * pref) if SP == 3 else 0.0) + 0.5) + 1
+        R = max(rD, rV)
+        most = max(most, (16 + 2 * S) * (64 + 2 * (R + S)) * 20 + 8 + 16 * (64 + 2 * R) * 32)
+    return most
+
+
+@pytest.mark.parametrize("SP,reach,n", [(2, "tile", 3), (2, "passes", 3), (3, "tile", 3), (3, "passes", 3), (2, "passes", 22),
+                                        (3, "passes", 22)])
+def test_fke_model_wide_movement_matches_oracle(tm, oracle, SP, reach, n):
+    """Consumers that reach far: tiles of 64 to 128 KiB of LDS, and reaches past them, which
+    the whole batch moves in four passes, points of short reach among them; in one group,
+    and in two (22 lattices of 97^2 and more)."""
+    wide = 5.6 if reach == "passes" else 1.4
+    D = (0.0, wide, 0.2) if SP == 2 else (0.0, 0.01028, wide)
+    p = [tm.FKEParams(), tm.FKEParams(D_mov=D, v=(0.0, 0.45427, 2.0))]
+    lds = max(_move_tile_bytes(tm, q, SP) for q in p)
+    assert (lds > 128 << 10) if reach == "passes" else (64 << 10 < lds <= 128 << 10)
+    insts = [tm.Instance([97, 98, 101][k % 3], k % 2, 5, k) for k in range(n)]
+    pick = [0, 1, 2] if n == 3 else [0, 10, 11, 21]
+    f0 = [model_fields(SP, d.L, 200 + k) for k, d in enumerate(insts)]
+    print(f"fke wide SP={SP} {reach} n={n} lds={lds}", flush=True)
+    with tm.Context() as ctx:
+        ctx.configure(tm.MODEL_FKE2 if SP == 2 else tm.MODEL_FKE3, tm.F64, p, insts)
+        for k, f in enumerate(f0):
+            ctx.upload(k, f)
+        ctx.run(2)
+        got = {k: ctx.download(k) for k in pick}
+    for k in pick:
+        ref, _, _ = _oracle_run(oracle, p[insts[k].params_index], SP, f0[k], insts[k], 2)
+        assert np.array_equal(got[k], ref), (SP, k, np.argwhere(got[k] != ref)[:5])
