@@ -277,7 +277,11 @@ inline float cpu_nudge(float x)
 typedef void* hipStream_t;
 typedef void* hipEvent_t;
 enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999, hipErrorNotReady = 600 };
-enum { hipMemcpyHostToDevice, hipMemcpyDeviceToHost };
+typedef void* hipGraph_t;
+typedef void* hipGraphExec_t;
+enum { hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipMemcpyDeviceToDevice };
+enum hipStreamCaptureMode { hipStreamCaptureModeThreadLocal };
+struct hipDeviceProp_t { char gcnArchName[16]; int multiProcessorCount; };
 enum { hipHostMallocDefault = 0, hipStreamNonBlocking = 1, hipEventDisableTiming = 2 };
 enum hipDeviceAttribute_t { hipDeviceAttributeWallClockRate };
 enum hipFuncAttribute { hipFuncAttributeMaxDynamicSharedMemorySize };
@@ -292,24 +296,50 @@ inline int device = 0;
 inline void called(const char* f, const void* p = nullptr) { if (on_call) on_call(f, p); }
 }  // namespace cpu_hip
 
+inline const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "error"; }
+inline hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+inline hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int)
+{
+    strcpy(p->gcnArchName, "gfx950");
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
 inline hipError_t hipGetDevice(int* d) { *d = cpu_hip::device; return hipSuccess; }
 inline hipError_t hipSetDevice(int d) { cpu_hip::device = d; return hipSuccess; }
 inline hipError_t hipMalloc(void** p, size_t n) { *p = calloc(n, 1); cpu_hip::called("hipMalloc", *p); return hipSuccess; }
 inline hipError_t hipFree(void* p) { cpu_hip::called("hipFree", p); free(p); return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(n, 1); return hipSuccess; }
 inline hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }
+template <typename T> hipError_t hipMalloc(T** p, size_t n) { return hipMalloc((void**)p, n); }
 inline hipError_t hipMemcpy(void* d, const void* s, size_t n, int) { std::memcpy(d, s, n); return hipSuccess; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) { std::memcpy(d, s, n); return hipSuccess; }
+inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
+inline hipError_t hipMemcpy2DAsync(void* d, size_t dp, const void* s, size_t sp, size_t w, size_t h, int, hipStream_t)
+{
+    for (size_t i = 0; i < h; ++i) std::memcpy((char*)d + i * dp, (const char*)s + i * sp, w);
+    return hipSuccess;
+}
+// no capture here: what asks for it is told so
+inline hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorUnknown; }
+inline hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorUnknown; }
+inline hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, void*, void*, size_t) { return hipErrorUnknown; }
+inline hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorUnknown; }
+inline hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+inline hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 #define HIP_SYMBOL(x) (&(x))
 inline hipError_t hipGetSymbolAddress(void** p, const void* s) { *p = (void*)s; return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
-inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = malloc(1); return hipSuccess; }
-inline hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
+inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = malloc(1); cpu_hip::called("hipStreamCreate", *s); return hipSuccess; }
+inline hipError_t hipStreamDestroy(hipStream_t s) { cpu_hip::called("hipStreamDestroy", s); free(s); return hipSuccess; }
 inline hipError_t hipStreamQuery(hipStream_t s) { return cpu_hip::on_query ? cpu_hip::on_query(s) : hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t s) { return cpu_hip::on_query ? cpu_hip::on_query(s) : hipSuccess; }
-inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t e, unsigned) { cpu_hip::called("hipStreamWaitEvent", e); return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = malloc(1); return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+inline hipError_t hipEventCreate(hipEvent_t* e) { *e = malloc(1); return hipSuccess; }
+inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 1.0f; return hipSuccess; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 inline hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void* f)
 {

@@ -4,6 +4,7 @@ and the last tile is written, nothing else is, and nothing outside the fields is
 And, the same way, the LDS that the consumers' launches take, the accept estimates of the
 FP64 samplers, the staged downloads' failures, the operators' kept scratch, the lanes of
 runs and the default steps' choice of kernel.  No GPU needed."""
+import concurrent.futures as cf
 import os
 import subprocess
 
@@ -21,6 +22,24 @@ def compile_cpu(src, exe, *extra):
                         os.path.join(CPP, src), "-pthread", "-o", str(exe), *extra], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr
     return str(exe)
+
+
+UNITS = ["tm_kernels_f64.hip", "tm_kernels_f32.hip", "tm_ensemble.hip", "tm_frames.hip", "tm_consumers.hip", "tm_movement.hip",
+         "tm_api.cpp", "tm_io.cpp", "tm_hostcopy.hip", "tm_groups.hip"]
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    """Objects of the whole library for the CPU."""
+    d = tmp_path_factory.mktemp("units")
+
+    def unit(u):
+        obj = d / (u.split(".")[0] + ".o")
+        lds = {"tm_consumers.hip": 1, "tm_movement.hip": 2}.get(u, 0)
+        return compile_cpu("cpu_unit.cpp", obj, "-c", "-x", "c++", f'-DUNIT="{u}"', f"-DLDS={lds}")
+
+    with cf.ThreadPoolExecutor(8) as ex:
+        return list(ex.map(unit, UNITS))
 
 
 @pytest.fixture(scope="module")
@@ -95,3 +114,9 @@ def test_size_rules_hold_for_the_batch(tmp_path, unit, table, variant, edges):
     got = r.stdout.split("\n")[:-1]
     for k, (n, want) in enumerate(edges):
         assert want in got[2 * k] and want in got[2 * k + 1], (n, got[2 * k:2 * k + 2])
+
+
+def test_short_runs_stay_on_their_stream(tmp_path, library):
+    exe = compile_cpu("run_streams.cpp", tmp_path / "run_streams", *library)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout == "ok\n", r.stderr

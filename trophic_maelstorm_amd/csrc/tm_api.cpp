@@ -514,15 +514,36 @@ void launch_fold(tm_ctx* c, int nsteps, int64_t row0)
     launch_combine(a, (int)c->inst.size(), nsteps, c->q);
 }
 
-// A run, from before its first launch to after its last wait: counted, and, with `lanes`,
-// a grouped batch's launches in a lane of its own, after what is on the context's stream.
+// Cell steps of a run from which its lanes pay.  Ordering them, forking and joining takes a
+// call 45 us, and two groups take a tenth off the steps, so: about 400 us of steps.  us a call,
+// one stream / lanes: FP64 Rietkerk 4 x 256^2 1 step 52 / 96, 8 steps 257 / 302, 32 steps 950 /
+// 960, 16 x 512^2 2 steps 396 / 396, 4 steps 704 / 692; FP64 DP 16 x 256^2 8 steps 253 / 255,
+// 12 steps 332 / 302; FP32 DP 16 x 1024^2 2 steps 292 / 302, 4 steps 518 / 496; two-species DP
+// consumers 16 x 256^2 1 step 138 / 163, 4 steps 463 / 435; three-species Rietkerk consumers
+// 4 x 256^2 4 steps 305 / 330, 12 steps 850 / 810, 16 x 256^2 1 step 209 / 254, 3 steps 542 / 543.
+double lane_cell_steps(int model, int prec)
+{
+    switch (model) {
+    case TM_MODEL_DP: return prec == TM_F64 ? 9e6 : 6e7;
+    case TM_MODEL_RIETKERK: return prec == TM_F64 ? 1.1e7 : 2.7e7;
+    case TM_MODEL_DP2: return 4e6;
+    case TM_MODEL_DP3: return 2.9e6;
+    case TM_MODEL_FKE2: return 3.6e6;
+    default: return 2.7e6;   // TM_MODEL_FKE3
+    }
+}
+
+// A run of so many steps, from before its first launch to after its last wait: counted,
+// and, if it is long enough, a grouped batch's launches in a lane of its own, after what is
+// on the context's stream.
 class Run {
 public:
-    Run(tm_ctx* c, bool lanes) : c_(c)
+    Run(tm_ctx* c, int64_t steps) : c_(c)
     {
         if (!c->lanes) return;
         c->lanes->begin();
-        if (!lanes || c->cut.inst == 0 || (c->lane[0] = c->lanes->take()) < 0) return;
+        if (c->cut.inst == 0 || (double)steps * (double)c->total_cells < lane_cell_steps(c->model, c->prec)) return;
+        if ((c->lane[0] = c->lanes->take()) < 0) return;
         c->q = c->lanes->stream(c->lane[0]);
         if (!c->lanes->order(c->lane[0], c->stream, c->q)) c->q = c->stream;
     }
@@ -1343,7 +1364,7 @@ tm_status tm_run(tm_ctx* c, int64_t n_steps, double* rows)
     if (s != TM_OK) return s;
     if (n_steps < 0) return fail(c, TM_ERR_ARG, "negative n_steps");
     if (n_steps == 0) return TM_OK;
-    const Run run(c, true);
+    const Run run(c, n_steps);
     HIPCHK(c, hipEventRecord(c->run_ev[0], c->q));
     if ((s = advance(c, n_steps)) != TM_OK) return s;
     HIPCHK(c, hipEventRecord(c->run_ev[1], c->q));
@@ -1521,7 +1542,7 @@ tm_status tm_time_steps(tm_ctx* c, int64_t n_steps, double* ms_total, int64_t* l
     // Step kernels only (no rows fold): graphs of up to 100 steps, one per
     // starting parity, captured once per context and launch shape and kept with
     // the run graphs, replayed between two events on the context stream.
-    const Run run(c, false);
+    const Run run(c, 0);
     const int B = (int)std::min<int64_t>(std::min<int64_t>(n_steps, 100), c->nslots);
     const int flip = launches_of(c, B) & 1;
     if (c->time_graph_steps != B) {
@@ -1592,7 +1613,7 @@ tm_status tm_autotune(tm_ctx* c, const char* cache_path, int* out_variant, int* 
     }
     // Dry timing: launches read the current buffer and write the other one
     // without advancing the step counter, so the batch state is unchanged.
-    const Run run(c, false);
+    const Run run(c, 0);
     const int nv = tm_variant_count(c->model, c->prec);
     const int graph_steps = c->graph_steps;
     hipEvent_t e0, e1;
@@ -1725,7 +1746,7 @@ tm_status tm_run_series(tm_ctx* c, const int64_t* steps, int n_meas, double* ser
         HIPCHK(c, hipMalloc((void**)&c->d_series_steps, sizeof(int64_t) * (size_t)n_meas));
         c->series_steps_cap = n_meas;
     }
-    const Run run(c, true);
+    const Run run(c, steps[n_meas - 1]);
     HIPCHK(c, hipMemcpyAsync(c->d_series_steps, steps, sizeof(int64_t) * (size_t)n_meas, hipMemcpyHostToDevice,
                              c->q));
     HIPCHK(c, hipEventRecord(c->run_ev[0], c->q));
