@@ -50,10 +50,12 @@ inline thread_local dim3 threadIdx, blockIdx, blockDim, gridDim;
 
 namespace cpu_hip {
 
-// A workgroup: every fiber runs until it ends or waits.  A wave's collective is then done
-// among its lanes that wait for it (the others have passed the branch it is in); a barrier
-// once every lane of the workgroup that has not ended waits for it.
-enum Wait { kRun, kBarrier, kCollective, kDone };
+// A workgroup: every fiber runs until it ends or waits.  The wave votes inside samplers
+// (__builtin_amdgcn_ballot_w64) are in branches that some lanes do not take: each is done
+// first, among the lanes that wait for it.  The other wave operations are where a wave is
+// whole again: done once all its lanes that have not ended wait for one.  A barrier is
+// done once every lane of the workgroup that has not ended waits for it.
+enum Wait { kRun, kBarrier, kVote, kWave, kDone };
 struct Lane {
     ucontext_t ctx;
     Wait wait;
@@ -84,15 +86,15 @@ inline void lane_main()
     group->lanes[group->cur].wait = kDone;
 }
 // This lane's value to the wave; what all of them brought.  Valid until the next one.
-inline const WaveVals& collective(uint64_t v)
+inline const WaveVals& collective(uint64_t v, Wait kind = kWave)
 {
     group->lanes[group->cur].in = v;
-    yield(kCollective);
+    yield(kind);
     return group->waves[group->cur / 64];
 }
-inline uint64_t votes(bool v)
+inline uint64_t votes(bool v, Wait kind)
 {
-    const WaveVals& w = collective(v ? 1 : 0);
+    const WaveVals& w = collective(v ? 1 : 0, kind);
     uint64_t b = 0;
     for (int i = 0; i < 64; ++i) b |= (w.mask >> i & 1 & w.v[i]) << i;
     return b;
@@ -166,18 +168,25 @@ inline void run_workgroup(dim3 grid, dim3 block, dim3 at, std::function<void()> 
         bool any = false, barrier = true;
         for (unsigned w = 0; w < n; w += 64) {
             WaveVals& wave = g.waves[w / 64];
-            uint64_t mask = 0;
-            for (unsigned i = w; i < w + 64 && i < n; ++i) {
+            bool waits[kDone + 1] = {};
+            const unsigned end = w + 64 < n ? w + 64 : n;
+            for (unsigned i = w; i < end; ++i) waits[g.lanes[i].wait] = true;
+            any = any || waits[kBarrier] || waits[kVote] || waits[kWave];
+            barrier = barrier && !waits[kVote] && !waits[kWave];
+            if (!waits[kVote] && waits[kWave] && waits[kBarrier]) {
+                fprintf(stderr, "wave %u: some lanes wait for the wave, some for the workgroup\n", w / 64);
+                abort();
+            }
+            const Wait kind = waits[kVote] ? kVote : kWave;
+            if (!waits[kind]) continue;
+            wave.mask = 0;
+            for (unsigned i = w; i < end; ++i) {
                 Lane& l = g.lanes[i];
-                if (l.wait == kDone) continue;
-                any = true;
-                if (l.wait != kBarrier) barrier = false;
-                if (l.wait != kCollective) continue;
-                mask |= 1ull << (i - w);
+                if (l.wait != kind) continue;
+                wave.mask |= 1ull << (i - w);
                 wave.v[i - w] = l.in;
                 l.wait = kRun;
             }
-            if (mask) wave.mask = mask;
         }
         if (!any) break;
         if (barrier)
@@ -216,7 +225,7 @@ void launch(const char* name, void (*kernel)(P...), dim3 grid, dim3 block, size_
 }  // namespace cpu_hip
 
 inline void __syncthreads() { cpu_hip::yield(cpu_hip::kBarrier); }
-inline uint64_t __ballot(int v) { return cpu_hip::votes(v != 0); }
+inline uint64_t __ballot(int v) { return cpu_hip::votes(v != 0, cpu_hip::kWave); }
 inline int cpu_readfirstlane(int v)
 {
     const cpu_hip::WaveVals& w = cpu_hip::collective((uint32_t)v);
@@ -260,7 +269,7 @@ inline float cpu_nudge(float x)
 #define __builtin_amdgcn_rsqf(x) cpu_nudge((float)(1.0 / std::sqrt((double)(float)(x))))
 #define __builtin_amdgcn_exp2f(x) cpu_nudge((float)std::exp2((double)(float)(x)))
 #define __builtin_amdgcn_readfirstlane(x) cpu_readfirstlane(x)
-#define __builtin_amdgcn_ballot_w64(x) cpu_hip::votes(x)
+#define __builtin_amdgcn_ballot_w64(x) cpu_hip::votes(x, cpu_hip::kVote)
 #define __builtin_amdgcn_s_waitcnt(x) ((void)0)
 #define __builtin_amdgcn_s_sleep(x) ((void)0)
 #define __builtin_amdgcn_update_dpp(old, src, ...) cpu_hip::update_dpp(old, src, __VA_ARGS__)

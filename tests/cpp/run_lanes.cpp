@@ -1,5 +1,6 @@
 // The lanes of runs where the device is busy when they are first measured: a later
-// measurement finds them, a device that has none is not measured for ever.
+// measurement finds them, a device that has none is not measured for ever.  And how long
+// they are kept.
 #include <map>
 
 #include "tm_groups.hip"
@@ -7,7 +8,7 @@
 using namespace tmk;
 
 static bool together;   // streams that run side by side
-static int launches;
+static int launches, streams;
 
 int main()
 {
@@ -23,6 +24,10 @@ int main()
     cpu_hip::on_query = [&](hipStream_t) {
         for (const auto& c : clock) now = max(now, c.second);
         return hipSuccess;
+    };
+    cpu_hip::on_call = [](const char* f, const void*) {
+        if (!strcmp(f, "hipStreamCreate")) ++streams;
+        if (!strcmp(f, "hipStreamDestroy")) --streams;
     };
     int bad = 0;
     auto check = [&](bool ok, const char* what) {
@@ -42,6 +47,20 @@ int main()
         check(g->prepare() && launches == n, "measured again once made");
     }
     {
+        // kept for the next context that wants them, whether its runs take them or not ...
+        for (int life = 0; life < 3; ++life) {
+            std::shared_ptr<RunLanes> g = RunLanes::get(0), h = RunLanes::get(0);
+            const int n = launches;
+            check(g->prepare() && launches == n, "made again for the next context");
+        }
+        // ... and given back at the end of one that does not
+        { std::shared_ptr<RunLanes> g = RunLanes::get(0); }
+        std::shared_ptr<RunLanes> g = RunLanes::get(0);
+        const int n = launches;
+        check(g->prepare() && launches > n, "lanes that nobody wanted were kept");
+    }
+    {
+        { std::shared_ptr<RunLanes> g = RunLanes::get(0); }
         together = false;
         std::shared_ptr<RunLanes> g = RunLanes::get(0);
         int measured = 0;
@@ -52,6 +71,8 @@ int main()
         }
         check(measured >= 2 && measured <= 4, "measurements of a device without lanes");
     }
+    { std::shared_ptr<RunLanes> g = RunLanes::get(0); }   // (an unwanted set of lanes)
+    check(streams == 0, "streams left over");
     if (bad) return 1;
     puts("ok");
     return 0;

@@ -9,7 +9,10 @@
 // streams onto a few queues (four by default, whichever are least used when a stream is
 // made) and queues onto pipes, and two chains that share one take turns: 143 us for the
 // consumer batch above.  So the streams of runs, lanes, are made and measured once per
-// device, and a run takes the free ones whatever the context's own stream shares.  A
+// device, and a run takes the free ones whatever the context's own stream shares.  Making
+// them takes 2 to 8 ms (a hardware queue's first stream 2.8), so they are kept from one
+// context to the next: released with the last of them, they took 10 of the 12 ms of a
+// context that made one short run.  A
 // batch is grouped only while its run is the device's only one in the process: runs of
 // several contexts already overlap (two of half the consumer batch each 92 us a step; four
 // of a quarter 126 on the contexts' streams, 92 to 126 on lanes).  Other processes on the
@@ -25,12 +28,12 @@ namespace tmk {
 
 class RunLanes {
 public:
-    // The device's lanes, shared by its contexts and released with the last of them.
+    // A context's share of the device's lanes.  The last one's end gives the streams back
+    // if no context has prepared them since there last was none.
     static std::shared_ptr<RunLanes> get(int device) noexcept;
-    ~RunLanes();
-    // Makes and measures the lanes at the first call (1 to 2 ms); false where fewer than
-    // two ran side by side.  Work of others on the GPU can make two queues look like one,
-    // so up to kAttempts calls measure until two are found.
+    // Makes and measures the lanes at the first call; false where fewer than two ran side
+    // by side.  Work of others on the GPU can make two queues look like one, so up to
+    // kAttempts calls measure until two are found.
     bool prepare();
     // A free lane of its own, or -1; to be given back when what it was given is done.
     int take();
@@ -49,9 +52,16 @@ public:
 
 private:
     static constexpr int kLanes = 4, kTries = 8, kAttempts = 4;
+    explicit RunLanes(int device) : device_(device) {}
+    void leave();
+    void make();
+    void release();
     bool side_by_side(int n);   // streams 0 .. n
+    const int device_;
     std::mutex mu_;
     std::atomic<int> runs_{0};
+    int contexts_ = 0;
+    bool wanted_ = false;       // since there last was no context
     int attempts_ = 0;
     int n_ = 0;
     hipStream_t s_[kLanes] = {};

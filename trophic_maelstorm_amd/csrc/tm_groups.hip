@@ -1,5 +1,6 @@
 // tm_groups.hip -- see tm_groups.h.
 #include "tm_groups.h"
+#include "tm_ondevice.h"
 
 #include <algorithm>
 #include <cstdint>
@@ -35,28 +36,47 @@ struct DevMem {
 std::shared_ptr<RunLanes> RunLanes::get(int device) noexcept
 {
     static std::mutex mu;
-    static std::weak_ptr<RunLanes> of[64];
+    static RunLanes* of[64];   // never destroyed: a process ends with them
     if (device < 0 || device >= 64) return nullptr;
     try {
-        std::lock_guard<std::mutex> lock(mu);
-        if (std::shared_ptr<RunLanes> g = of[device].lock()) return g;
-        std::shared_ptr<RunLanes> g = std::make_shared<RunLanes>();
-        of[device] = g;
-        return g;
+        RunLanes* l;
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!of[device]) of[device] = new RunLanes(device);
+            l = of[device];
+        }
+        {
+            std::lock_guard<std::mutex> lock(l->mu_);
+            ++l->contexts_;
+        }
+        return std::shared_ptr<RunLanes>(l, [](RunLanes* r) { r->leave(); });
     } catch (...) {   // no memory: runs stay on their contexts' streams
         return nullptr;
     }
 }
 
-RunLanes::~RunLanes()
+void RunLanes::leave()
 {
-    for (hipStream_t s : s_)
+    std::lock_guard<std::mutex> lock(mu_);
+    if (--contexts_ > 0) return;
+    if (!wanted_) release();
+    wanted_ = false;
+}
+
+void RunLanes::release()
+{
+    for (hipStream_t& s : s_)
         if (s) {
             (void)hipStreamSynchronize(s);
             (void)hipStreamDestroy(s);
+            s = nullptr;
         }
-    for (hipEvent_t e : ev_)
-        if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t& e : ev_)
+        if (e) {
+            (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    n_ = attempts_ = 0;
 }
 
 // Whether chains of dependent short launches on streams 0 .. n, queued in turn, take less
@@ -99,8 +119,18 @@ bool RunLanes::side_by_side(int n)
 bool RunLanes::prepare()
 {
     std::lock_guard<std::mutex> lock(mu_);
-    if (n_ >= 2 || attempts_ == kAttempts) return n_ >= 2;
-    ++attempts_;
+    wanted_ = true;
+    if (n_ < 2 && attempts_ < kAttempts) {
+        ++attempts_;
+        make();
+    }
+    return n_ >= 2;
+}
+
+void RunLanes::make()
+{
+    const OnDevice on(device_);
+    if (!on.ok()) return;
     // New streams take the least used queues, so those passed over are kept meanwhile.
     hipStream_t passed_over[kTries];
     int np = 0;
@@ -122,7 +152,6 @@ bool RunLanes::prepare()
     }
     for (int k = 0; k < np; ++k) (void)hipStreamDestroy(passed_over[k]);
     (void)hipGetLastError();
-    return n_ >= 2;
 }
 
 int RunLanes::take()

@@ -1,5 +1,6 @@
 // tm_hostcopy.hip -- see tm_hostcopy.h.
 #include "tm_hostcopy.h"
+#include "tm_ondevice.h"
 
 #include <hip/hip_runtime.h>
 
@@ -35,25 +36,6 @@ __global__ __launch_bounds__(256) void to_pinned_kernel(const char* __restrict__
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x, mark, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-
-// Makes a device current, and the one before it again.
-class OnDevice {
-public:
-    explicit OnDevice(int device)
-    {
-        if (hipGetDevice(&before_) != hipSuccess) before_ = device;
-        ok_ = before_ == device || hipSetDevice(device) == hipSuccess;
-        if (before_ == device || !ok_) before_ = -1;
-    }
-    ~OnDevice() { if (before_ >= 0) (void)hipSetDevice(before_); }
-    OnDevice(const OnDevice&) = delete;
-    OnDevice& operator=(const OnDevice&) = delete;
-    bool ok() const { return ok_; }
-
-private:
-    int before_ = -1;
-    bool ok_ = false;
-};
 
 }  // namespace
 
