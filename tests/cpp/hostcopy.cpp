@@ -34,8 +34,18 @@ int main()
 {
     alarm(100);   // a copy that waits for good ends here
     cpu_hip::device = 3;
-    std::shared_ptr<HostCopier> c = HostCopier::get(1);
-    check(c != nullptr, "no copier");
+    // made once the downloads come to 8 MiB, and again after the last user's end
+    std::shared_ptr<HostCopier> c;
+    for (int life = 0; life < 3; ++life) {
+        c.reset();
+        check(HostCopier::get(1, 5 << 20) == nullptr, "a copier for a first download");
+        check(HostCopier::get(4 + life, 5 << 20) == nullptr, "another device's downloads counted");
+        check(HostCopier::get(1, 2 << 20) == nullptr, "a copier for 7 MiB");
+        c = HostCopier::get(1, 1 << 20);
+        check(c != nullptr, "no copier for 8 MiB");
+        check(HostCopier::get(1, 1 << 18) == c, "not the device's copier");
+        cpu_hip::device = 3;
+    }
     check(cpu_hip::device == 3, "making the copier changed the current device");
     int on = -1;
     auto run = [&](const cpu_hip::Launch& l) {

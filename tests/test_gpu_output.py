@@ -88,3 +88,23 @@ def test_large_downloads_through_staging(tm, prec, L):
             t.join()
         for r in got.values():
             assert len(r) == 12 and all(np.array_equal(x, want[i % 2]) for i, x in enumerate(r))
+
+
+@pytest.mark.parametrize("prec,L", [("f64", 181), ("f64", 182), ("f64", 601), ("f32", 257), ("f32", 1023)])
+def test_downloads_while_the_staging_is_there(tm, tmp_path, prec, L):
+    """The staging is made at 8 MiB of downloads and shared: with a context that holds it,
+    every download from 256 KiB on passes through it, whatever its size and its start."""
+    P = tm.F64 if prec == "f64" else tm.F32
+    with tm.Context() as holder, tm.Context() as ctx:
+        holder.configure(tm.MODEL_DP, tm.F64, tm.DPParams(), [tm.Instance(1500, 0, 1, 0)])
+        holder.init_uniform([0.0], [1.0])
+        held = holder.download(0)
+        ctx.configure(tm.MODEL_DP, P, tm.DPParams(), [tm.Instance(7, 0, 3, 0), tm.Instance(L, 0, 3, 1), tm.Instance(L, 0, 3, 2)])
+        ctx.init_uniform([0.0], [1.0])
+        ctx.run(2)
+        for k in (1, 2):
+            ctx.save_snapshot(k, tmp_path / "s")
+            want = np.frombuffer((tmp_path / "s").read_bytes(), np.float64 if prec == "f64" else np.float32, offset=64)
+            for _ in range(3):
+                assert np.array_equal(ctx.download(k).ravel(), want.astype(np.float64))
+        assert np.array_equal(holder.download(0), held)

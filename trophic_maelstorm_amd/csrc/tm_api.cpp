@@ -148,8 +148,7 @@ struct tm_ctx {
     int move_lds = 0;              // Rietkerk consumers: LDS of the movement tile
     double* d_mov = nullptr;       // tm_mov_stats output [n_inst][4 SpB]
 
-    std::shared_ptr<HostCopier> copier;   // large downloads; taken at the first one
-    bool copier_tried = false;
+    std::shared_ptr<HostCopier> copier;   // large downloads; taken where there is one
 };
 
 namespace {
@@ -1137,10 +1136,7 @@ tm_status tm_download_fields(tm_ctx* c, int i, double* host)
     const char* src = (const char*)c->d_fields[c->parity] + c->esize * c->nf * c->cell_off[i];
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if ((size_t)n * c->esize >= kStagedCopyMin) {
-        if (!c->copier_tried) {
-            c->copier_tried = true;
-            c->copier = HostCopier::get(c->device);
-        }
+        if (!c->copier) c->copier = HostCopier::get(c->device, sizeof(double) * (size_t)n);
         if (c->copier) {
             const HostCopier::Result r = c->copier->copy(host, src, (size_t)n, c->prec == TM_F32);
             if (r == HostCopier::kOk) return TM_OK;

@@ -8,8 +8,11 @@
 // one among them, copy (or widen) the landed pieces out.  Halves of 2 MiB stay in the
 // host's caches: 8 MiB of FP64 in 213 us (480 before; 267 with halves of 8 MiB), 4 MiB of
 // FP32 widened in 129 (514), 256 KiB in 18 (25).
-// One HostCopier per device is shared by the contexts that made a large download (making
-// it takes 0.6 ms) and released with the last of them.
+// One HostCopier per device is shared by the contexts that made a large download and
+// released with the last of them.  Making and releasing it takes 0.8 ms, what it saves on
+// 7 MiB into fresh memory (whose page faults its threads share) or 24 MiB into memory in use,
+// so it is made with the download that brings those without one to 8 MiB: a context that
+// downloads 2 MiB once took 0.6 ms longer for it.
 #pragma once
 #include <cstddef>
 #include <memory>
@@ -20,9 +23,11 @@ class HostCopier {
 public:
     static constexpr int kThreads = 8;        // the calling thread and seven of its own
     static constexpr size_t kHalf = (size_t)2 << 20, kPiece = (size_t)32 << 10;
-    // The device's copier, made if there is none; null where threads, streams or pinned
-    // memory are refused.
-    static std::shared_ptr<HostCopier> get(int device) noexcept;
+    static constexpr size_t kMakeAfter = (size_t)8 << 20;
+    // The device's copier for a download of so many bytes of doubles.  Null where there is
+    // none and the downloads since the last come to less than kMakeAfter with this one, and
+    // where threads, streams or pinned memory are refused (tried again after kRefused more).
+    static std::shared_ptr<HostCopier> get(int device, size_t bytes) noexcept;
     ~HostCopier();
     enum Result { kOk, kBusy, kFailed };
     // n elements at src (device, complete: the caller has waited for its writers) to dst
@@ -32,6 +37,7 @@ public:
     Result copy(double* dst, const void* src, size_t n, bool widen);
 
 private:
+    static constexpr size_t kRefused = (size_t)1 << 30;
     HostCopier() = default;
     struct Impl;
     Impl* impl_ = nullptr;

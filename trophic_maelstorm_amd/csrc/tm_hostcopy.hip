@@ -154,14 +154,19 @@ struct HostCopier::Impl {
     }
 };
 
-std::shared_ptr<HostCopier> HostCopier::get(int device) noexcept
+std::shared_ptr<HostCopier> HostCopier::get(int device, size_t bytes) noexcept
 {
     static std::mutex mu;
     static std::weak_ptr<HostCopier> of[64];
+    static size_t plain[64], after[64];   // bytes downloaded without one since; how many it takes
     if (device < 0 || device >= 64) return nullptr;
     try {
         std::lock_guard<std::mutex> lock(mu);
         if (std::shared_ptr<HostCopier> c = of[device].lock()) return c;
+        plain[device] += bytes;
+        if (plain[device] < std::max(after[device], kMakeAfter)) return nullptr;
+        plain[device] = 0;
+        after[device] = kRefused;
         std::shared_ptr<HostCopier> c(new HostCopier());
         Impl* m = c->impl_ = new Impl();
         m->device = device;
@@ -178,6 +183,7 @@ std::shared_ptr<HostCopier> HostCopier::get(int device) noexcept
         std::memset(m->flags, 0, sizeof(uint64_t) * 2 * Impl::kPer);
         for (std::thread& t : m->threads) t = std::thread([m] { m->loop(); });
         of[device] = c;
+        after[device] = kMakeAfter;
         return c;
     } catch (...) {   // no thread, no memory: the caller copies without staging
         return nullptr;
