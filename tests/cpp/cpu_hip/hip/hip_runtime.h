@@ -285,7 +285,7 @@ inline float cpu_nudge(float x)
 // ---- host API ------------------------------------------------------------------------
 typedef void* hipStream_t;
 typedef void* hipEvent_t;
-enum hipError_t { hipSuccess = 0, hipErrorUnknown = 999, hipErrorNotReady = 600 };
+enum hipError_t { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorUnknown = 999, hipErrorNotReady = 600 };
 typedef void* hipGraph_t;
 typedef void* hipGraphExec_t;
 enum { hipMemcpyHostToDevice, hipMemcpyDeviceToHost, hipMemcpyDeviceToDevice };
@@ -299,6 +299,7 @@ struct hipFuncAttributes { size_t sharedSizeBytes; };
 namespace cpu_hip {
 inline std::function<void(const char*, const void*)> on_call;   // (function, pointer it is about)
 inline std::function<hipError_t(hipStream_t)> on_query;          // hipStreamQuery, hipStreamSynchronize
+inline std::function<bool(size_t)> refuse;                       // device allocations of a size
 inline std::function<size_t(const void*)> static_lds;            // of a kernel
 inline std::function<hipError_t(const void*, int)> on_opt_in;    // to dynamic LDS above the default limit
 inline int device = 0;
@@ -315,7 +316,13 @@ inline hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int)
 }
 inline hipError_t hipGetDevice(int* d) { *d = cpu_hip::device; return hipSuccess; }
 inline hipError_t hipSetDevice(int d) { cpu_hip::device = d; return hipSuccess; }
-inline hipError_t hipMalloc(void** p, size_t n) { *p = calloc(n, 1); cpu_hip::called("hipMalloc", *p); return hipSuccess; }
+inline hipError_t hipMalloc(void** p, size_t n)
+{
+    if (cpu_hip::refuse && cpu_hip::refuse(n)) return hipErrorOutOfMemory;
+    *p = calloc(n, 1); 
+    cpu_hip::called("hipMalloc", *p);
+    return hipSuccess;
+}
 inline hipError_t hipFree(void* p) { cpu_hip::called("hipFree", p); free(p); return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = calloc(n, 1); return hipSuccess; }
 inline hipError_t hipHostFree(void* p) { free(p); return hipSuccess; }

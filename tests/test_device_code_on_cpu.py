@@ -120,3 +120,9 @@ def test_short_runs_stay_on_their_stream(tmp_path, library):
     exe = compile_cpu("run_streams.cpp", tmp_path / "run_streams", *library)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stderr
+
+
+def test_consumer_batch_without_its_scratch(tmp_path, library):
+    exe = compile_cpu("consumer_memory.cpp", tmp_path / "consumer_memory", *library)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stderr)

@@ -886,9 +886,14 @@ tm_status setup_dpc(tm_ctx* c)
     const size_t o_chunks = o_chunk + up(sizeof(double) * 4 * chunks.size());
     const size_t o_disk = o_chunks + up(sizeof(int2) * chunks.size());
     const size_t o_vtiles = o_disk + up(sizeof(int2) * disk.size());
-    const size_t total = o_vtiles + up(sizeof(int4) * vtiles.size());   // of the tables; P* and lambda follow
+    const size_t total = o_vtiles + up(sizeof(int4) * vtiles.size());   // of the tables; lambda follows
     free_dev(c->d_dpc);
-    if (hipMalloc(&c->d_dpc, total + sizeof(double) * (size_t)ns * (size_t)c->total_cells) != hipSuccess) return fail(c, TM_ERR_NOMEM, "consumer tables allocation failed");
+    bool lambda = hipMalloc(&c->d_dpc, total + sizeof(double) * (size_t)(ns - 1) * (size_t)c->total_cells) == hipSuccess;
+    if (!lambda) {   // fields that leave room for the tables only
+        (void)hipGetLastError();
+        c->d_dpc = nullptr;
+        if (hipMalloc(&c->d_dpc, total) != hipSuccess) return fail(c, TM_ERR_NOMEM, "consumer tables allocation failed");
+    }
     char* base = (char*)c->d_dpc;
     DPCWork w{};
     w.params = (const tm_dpc_params*)c->d_params;
@@ -898,8 +903,7 @@ tm_status setup_dpc(tm_ctx* c)
     w.chunks = (const int2*)(base + o_chunks);
     w.disk = (const int2*)(base + o_disk);
     w.vtiles = (const int4*)(base + o_vtiles);
-    w.pstar = (double*)(base + total);
-    w.lambda = w.pstar + c->total_cells;
+    w.lambda = lambda ? (double*)(base + total) : nullptr;
     std::vector<char> host(total, 0);
     std::memcpy(host.data(), &w, sizeof(w));
     std::memcpy(host.data() + o_info, info.data(), sizeof(DPCInstInfo) * info.size());

@@ -90,11 +90,12 @@ __global__ __launch_bounds__(256, 5) void dpc_head_kernel(ConsumerArgs a)
     const DPCConst c = ((const DPCConst*)a.consts)[(int64_t)a.k * a.n_inst + tl.x];
     const VegConst vc = {c.k, di.seed, di.inst_id, c.compat, c.step};
     const double* P = (const double*)a.in + (int64_t)NF * di.cell_off;
+    double* pstar = (double*)a.out + (int64_t)NF * di.cell_off;   // field 0, where the step takes it from
     if (a.vdirect) {   // 64 x 4 tiles, one cell a thread
         const int y = tl.z + (int)(threadIdx.x >> 6), x = tl.y + (int)(threadIdx.x & 63);
-        if (y < di.L && x < di.L) veg_cell(vc, di.L, y, x, P, w->pstar + di.cell_off);
+        if (y < di.L && x < di.L) veg_cell(vc, di.L, y, x, P, pstar);
     } else {
-        veg_tile(vc, di.L, tl.y, tl.z, P, w->pstar + di.cell_off, sm.veg);
+        veg_tile(vc, di.L, tl.y, tl.z, P, pstar, sm.veg);
     }
 }
 
@@ -210,7 +211,7 @@ __device__ __forceinline__ int dpc_consumer(const tm_dpc_params& p, int s, const
 }
 
 // One tile, in phases with a barrier between them: the consumers' perception gamma and
-// first trials per cell (the vegetation's P* is in DPCWork::pstar), the transitions
+// first trials per cell (the vegetation's P* is in its output field), the transitions
 // those leave open from two queues per consumer, densely packed, then the RK4, checks,
 // flush and partials per cell.  Between phases a cell's new densities and gamma wait in
 // the output fields.  In one pass every wave ran every sampler path of its 64 cells and
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
     const int64_t N = (int64_t)L * L;
     const double* fin = (const double*)a.in + (int64_t)NF * tl.cell_off;
     double* fout = (double*)a.out + (int64_t)NF * tl.cell_off;
-    const double* pstar = w->pstar + tl.cell_off;
+    double* const lambdas = w->lambda;
 
     // 32 lanes along a row, NT / 32 rows at a time: no index division
     for (int ry = threadIdx.x >> 5; ry < RH; ry += NT / 32) {
@@ -314,7 +315,10 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
                     if (g > 1) g = 1;
                     double lambda;
                     res = dpc_consumer<true>(p, s, di, cell, c.step, c.compat != 0, g, is, r, RW, y, lambda, words);
-                    if (res == kDornicGamma) w->lambda[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell] = lambda;
+                    if (res == kDornicGamma) {
+                        if (lambdas) lambdas[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell] = lambda;
+                        else res = kDornicRestart;
+                    }
                 }
                 fout[(NS + s - 1) * N + cell] = g;
                 fout[s * N + cell] = y;
@@ -342,7 +346,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
                 Stream sc(di.seed, di.inst_id, cell, c.step);
                 sc.blk = (uint32_t)s << 24;
                 sc.skip(q >> 9);
-                lambda = w->lambda[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell];
+                lambda = lambdas[(int64_t)(NS - 1) * tl.cell_off + (s - 1) * N + cell];
                 y = dornic_gamma_d(sc, fout[s * N + cell], lambda, c.compat != 0);
             }
             fout[s * N + cell] = y;
@@ -359,7 +363,7 @@ __global__ __launch_bounds__(NT, MINW) void dpc_step_kernel(ConsumerArgs a)
         if (gy >= L || gx >= L) continue;
         const uint32_t cell = (uint32_t)gy * (uint32_t)L + (uint32_t)gx;
         double y[NS];
-        y[0] = pstar[cell];
+        y[0] = fout[cell];
 #pragma unroll
         for (int s = 1; s < NS; ++s) y[s] = fout[s * N + cell];
         dpc_rk4<NS>(p, y);

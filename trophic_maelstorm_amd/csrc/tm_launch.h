@@ -60,8 +60,8 @@ struct DPCWork {
     const int2* chunks;   // [nchunks]: (instance, chunk index within it)
     const int2* disk;     // perception offsets (row, column) of every table
     const int4* vtiles;   // the vegetation's Dornic tiles: (instance, x0, y0, 0)
-    double* pstar;        // ... and its result P*, at cell_off
-    double* lambda;       // lambda of the consumers' cells whose Gamma deviate is deferred, (ns - 1) fields
+    double* lambda;       // lambda of the consumers' cells whose Gamma deviate is deferred, (ns - 1)
+                          // fields; null: those cells start again
 };
 // Opts the consumer step kernels in to the LDS they need at this halo on the current
 // device; false where that is refused.
