@@ -120,10 +120,10 @@ struct HostCopier::Impl {
         uint64_t seen = 0;
         for (;;) {
             // copies come in runs (one call per instance): look for the next one for a
-            // while before sleeping
+            // moment before sleeping (10 times as long took as long a copy, and the CPUs)
             const auto t0 = std::chrono::steady_clock::now();
             while (job.load(std::memory_order_acquire) == seen && !stop.load() &&
-                   std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(200))
+                   std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(20))
                 std::this_thread::yield();
             if (job.load(std::memory_order_acquire) == seen && !stop.load()) {
                 std::unique_lock<std::mutex> lock(mu);
