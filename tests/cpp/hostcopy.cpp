@@ -47,6 +47,13 @@ int main()
         cpu_hip::device = 3;
     }
     check(cpu_hip::device == 3, "making the copier changed the current device");
+    c.reset();
+    for (int k = 0; k < 8; ++k) {
+        check(c == nullptr, "a copier for a few small downloads");
+        c = HostCopier::get(1, 1 << 18);
+    }
+    check(c != nullptr, "no copier for many small downloads");
+    cpu_hip::device = 3;
     int on = -1;
     auto run = [&](const cpu_hip::Launch& l) {
         on = cpu_hip::device;

@@ -11,8 +11,9 @@
 // One HostCopier per device is shared by the contexts that made a large download and
 // released with the last of them.  Making and releasing it takes 0.8 ms, what it saves on
 // 7 MiB into fresh memory (whose page faults its threads share) or 24 MiB into memory in use,
-// so it is made with the download that brings those without one to 8 MiB: a context that
-// downloads 2 MiB once took 0.6 ms longer for it.
+// so it is made with the download that brings those without one to 8 MiB, each counted as
+// 1 MiB at least (a plain copy of 256 KiB takes up to 115 us, a staged one 18): a context
+// that downloads 2 MiB once took 0.6 ms longer for it.
 #pragma once
 #include <cstddef>
 #include <memory>
@@ -23,7 +24,7 @@ class HostCopier {
 public:
     static constexpr int kThreads = 8;        // the calling thread and seven of its own
     static constexpr size_t kHalf = (size_t)2 << 20, kPiece = (size_t)32 << 10;
-    static constexpr size_t kMakeAfter = (size_t)8 << 20;
+    static constexpr size_t kMakeAfter = (size_t)8 << 20, kCountedMin = (size_t)1 << 20;
     // The device's copier for a download of so many bytes of doubles.  Null where there is
     // none and the downloads since the last come to less than kMakeAfter with this one, and
     // where threads, streams or pinned memory are refused (tried again after kRefused more).

@@ -163,7 +163,7 @@ std::shared_ptr<HostCopier> HostCopier::get(int device, size_t bytes) noexcept
     try {
         std::lock_guard<std::mutex> lock(mu);
         if (std::shared_ptr<HostCopier> c = of[device].lock()) return c;
-        plain[device] += bytes;
+        plain[device] += std::max(bytes, kCountedMin);
         if (plain[device] < std::max(after[device], kMakeAfter)) return nullptr;
         plain[device] = 0;
         after[device] = kRefused;
