@@ -408,8 +408,8 @@ __device__ __forceinline__ int ptrs_estimate(const PtrsD& p, double z, double kd
 
 // Marsaglia-Tsang's test  log u < x^2 / 2 + d (1 - v + log v), v = (1 + y)^3, y = c x:
 // below |y| = 0.1 the right side from its series in y, which does not cancel, and
-// directly above, where d <= 455 keeps its rounding below 1e-4.  Used for d < 1e9: the
-// FP64 test's own rounding grows as sqrt(d) and passes the margin near d = 1e23.
+// directly above, where d <= 455 keeps its rounding below 1e-4.  The FP64 test's own
+// rounding grows as sqrt(d) and reaches 1e-3 near d = 1e23, so the margin grows with d.
 __device__ __forceinline__ int gamma_estimate(double u, double x2, double y, double v, double d)
 {
     const float yf = (float)y, df = (float)d, vf = (float)v;
@@ -418,7 +418,7 @@ __device__ __forceinline__ int gamma_estimate(double u, double x2, double y, dou
     const float dir = 0.5f * (float)x2 + df * (1.0f - vf + est_log(vf));
     const float rhs = __builtin_fabsf(yf) < 0.1f ? ser : dir;
     const float lhs = est_log((float)u);
-    const float margin = df < 1e9f ? 1e-3f : __builtin_inff();   // a select: no branch in the latency of a draw
+    const float margin = __builtin_fmaf(df, 1e-12f, 1e-3f);   // no branch in the latency of a draw
     return lhs < rhs - margin ? 1 : (lhs > rhs + margin ? -1 : 0);
 }
 
