@@ -315,7 +315,7 @@ tm_status tm_last_run_time(const tm_ctx* ctx, double* ms, int64_t* n_steps);
 tm_status tm_mode_steps(const tm_ctx* ctx, int64_t* single_steps, int64_t* blocked_steps);
 
 /* The context's HIP stream (hipStream_t) for callers that order their own work.  A
- * run of a large batch takes other streams, after what is on this one, and has
+ * long run of a large batch takes other streams, after what is on this one, and has
  * finished when the call returns. */
 void* tm_stream(tm_ctx* ctx);
 
